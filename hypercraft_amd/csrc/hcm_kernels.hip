@@ -11,9 +11,9 @@
 //      with no visible face after step 3's visibility masks.
 //   2. liquid-flow cells take their per-cell face textures (the reference's m_dynamic_block_textures).
 //   3. faces, per (axis, slice, direction) task, each a 16x16 mask:
-//      - visibility, bit-sliced: one lane per column of an axis keeps its cells' face classes as bit
-//        planes, so BlockTexture::Show is a few bit operations (texture codes are compared only for
-//        transparent against transparent); ballots transpose the columns into the tasks' mask rows;
+//      - visibility, bit-parallel: one lane per x-row of blocks has their face classes as bit planes (made
+//        while the row is staged), so BlockTexture::Show is a few logic operations per row and axis (texture
+//        codes are compared only for transparent against transparent);
 //      - face words: visible faces are numbered densely in the reference's scan order and one lane per
 //        face evaluates light4_init; the face word is Light4 plus texture code and pass;
 //      - link masks: each face is compared with its right and lower neighbours, giving the
@@ -35,7 +35,14 @@ namespace hcm {
 constexpr int kHalo = 18;
 constexpr int kHaloVox = kHalo * kHalo * kHalo;
 constexpr int kHaloRows = kHalo * kHalo;
-constexpr int kTasks = 102; // 3 axes x 17 slices x 2 directions
+// A task is the 16 x 16 faces of one axis, layer of owning blocks and direction, in the reference's order
+// (axis, then slice, then direction): t = 32 axis + 2 layer + (1 for the + faces), the - faces of layer l
+// lying in slice l and its + faces in slice l + 1. (The reference's 3 x 17 x 2 also scans the + faces of
+// slice 0 and the - faces of slice 16, which the chunk owns none of.)
+constexpr int kTasks = 96;
+__host__ __device__ constexpr int task_axis(int t) { return t >> 5; }
+__host__ __device__ constexpr int task_layer(int t) { return (t >> 1) & 15; }
+__host__ __device__ constexpr int task_plus(int t) { return t & 1; }
 // Entries of the face-word stage. 1,472 keeps the 256-thread workgroup's LDS within three per CU
 // (static_assert below); the tasks of a chunk with more visible faces are taken in several groups.
 constexpr int kListCap = 1472;
@@ -127,7 +134,13 @@ template <int NT> struct Smem {
 	alignas(16) uint16_t eh[kTasks][16];
 	alignas(16) uint16_t ev[kTasks][16];
 	alignas(16) uint16_t tp[kTasks][16];
-	uint2 key[kListCap];       // face words of the current group of tasks, in dense order
+	union {
+		uint2 key[kListCap]; // face words of the current group of tasks, in dense order
+		struct {             // until the visibility masks are made: the halo rows' face classes as bit planes
+			uint4 planes[kHaloRows];  // of the y faces, then the z faces (row_planes)
+			uint32_t vis_x[256], tt_x[256]; // per chunk row: its visible x faces and those to compare (show_rows)
+		};
+	};
 	uint16_t fpre[kTasks + 2]; // prefix of visible faces per task (the dense face order; at most 24,576)
 	uint32_t qpre_o[kTasks];   // per task: index of its first opaque quad in the opaque pass
 	uint32_t qpre_t[kTasks];   // per task: index of its first transparent quad in the transparent pass
@@ -545,12 +558,12 @@ __device__ __forceinline__ void aabb_merge(Smem<NT> &s, int pass, int k, const u
 	atomicMax(&a[5], hi[2]);
 }
 
-// Regular quad: task t = 34 * axis + 2 * slice + direction, origin (u, v0) on the mask, width w along V,
+// Regular quad: task t, origin (u, v0) on the mask, width w along V,
 // height h along U (:357-460), with the face word of its origin face (Light4 and texture code).
 template <int NT>
 __device__ __forceinline__ void emit_quad(const MeshParams &p, const Smem<NT> &s, int t, int u, int v0, int w, int h,
                                           uint2 word, uint32_t slot, uint32_t vbase, uint32_t lo[3], uint32_t hi[3]) {
-	const int A = t / 34, sl = (t % 34) >> 1, inv = t & 1, face = 2 * A + inv;
+	const int A = task_axis(t), inv = task_plus(t) ^ 1, sl = task_layer(t) + (inv ^ 1), face = 2 * A + inv;
 	const int ua = u_axis(A), va = v_axis(A);
 	const uint2 l = make_uint2(word.x, word.y & 0xffffffu);
 	const uint16_t tex = uint16_t(s.codes[(word.y >> 24) & 0x7fu] & 0xffffu);
@@ -646,77 +659,158 @@ __device__ __forceinline__ void emit_custom(const MeshParams &p, Smem<NT> &s, ui
 }
 
 // ------------------------------------------------------------------------------------------------
-// visibility: one lane per (u, v) column along the slicing axis
+// visibility: one lane per x-row of blocks, its faces as bit planes
 // ------------------------------------------------------------------------------------------------
 // BlockTexture::Show (texture/include/texture/BlockTexture.hpp:68-76) on the 2-bit face classes
 // (empty 0, opaque 1, transparent 2, liquid 3):
 //   opaque self:      visible unless the other face is opaque,
 //   transparent self: visible if the other is empty or liquid, or transparent with another texture,
 //   liquid self:      visible if the other is empty.
-// The face between halo positions a and a + 1 is in slice a; with i = class(+ face of a) |
-// class(- face of a + 1) << 2, bit i of kShowPlus says whether the + face of a shows and bit i of
-// kShowMinus whether the - face of a + 1 does. Transparent against transparent (i = 10) depends on
-// the two texture codes and is resolved from the voxels' texture rows.
-__host__ __device__ constexpr uint32_t show_class(uint32_t self, uint32_t other) {
-	return self == 1 ? (other != 1 ? 1u : 0u) : self == 2 ? ((other == 0 || other == 3) ? 1u : 0u) : self == 3 ? (other == 0 ? 1u : 0u) : 0u;
+// A row's 16 blocks are 16 bits, so the rule is a few logic operations for a whole row, and both directions
+// of an axis share them: the + direction in the low half-word, the - direction in the high one.
+__host__ __device__ constexpr uint32_t show_planes(uint32_t s0, uint32_t s1, uint32_t o0, uint32_t o1) {
+	return (s0 & ~s1 & ~(o0 & ~o1)) | (s1 & ~s0 & ~(o0 ^ o1)) | (s0 & s1 & ~(o0 | o1));
 }
-__host__ __device__ constexpr uint32_t show_table(bool plus) {
-	uint32_t t = 0;
-	for (uint32_t i = 0; i < 16; ++i)
-		t |= (plus ? show_class(i & 3u, i >> 2) : show_class(i >> 2, i & 3u)) << i;
-	return t;
+// Transparent against transparent, which also needs the textures.
+__host__ __device__ constexpr uint32_t tt_planes(uint32_t s0, uint32_t s1, uint32_t o0, uint32_t o1) {
+	return s1 & ~s0 & o1 & ~o0;
 }
-constexpr uint32_t kShowPlus = show_table(true), kShowMinus = show_table(false), kShowTT = 2u | 2u << 2;
-static_assert(kShowPlus == 0x620eu && kShowMinus == 0x19d0u, "Show on face classes");
+namespace check {
+constexpr bool show_matches() {
+	for (uint32_t self = 0; self < 4; ++self)
+		for (uint32_t other = 0; other < 4; ++other) {
+			const bool want = self == 1 ? other != 1 : self == 2 ? (other == 0 || other == 3) : self == 3 ? other == 0 : false;
+			if ((show_planes(self & 1, self >> 1, other & 1, other >> 1) & 1u) != uint32_t(want) ||
+			    (tt_planes(self & 1, self >> 1, other & 1, other >> 1) & 1u) != uint32_t(self == 2 && other == 2))
+				return false;
+		}
+	return true;
+}
+static_assert(show_matches(), "Show on face classes");
+} // namespace check
 
-// Only blocks inside the chunk own faces (:330, :335): + faces of halo positions 1..16 (slices 1..16)
-// and - faces of positions 1..16 (slices 0..15). Ballots over the wave give the 16x16 masks of the
-// (axis, slice, direction) tasks, four mask rows per wave.
-template <int A, int NT> __device__ __forceinline__ void visibility_column(Smem<NT> &s, int col) {
-	const int lane = threadIdx.x & 63;
-	const int u = col >> 4, v = col & 15;
-	constexpr int sa = axis_stride(A);
-	constexpr int shp = kVoxClassShift + 4 * A; // class of face 2A (+); face 2A + 1 (-) follows
-	const uint32_t *cw = s.vox + (u + 1) * axis_stride(u_axis(A)) + (v + 1) * axis_stride(v_axis(A));
-	uint32_t c[kHalo];
+// Bytes of (hi, lo) by selector: selector byte 0-3 takes that byte of lo, 4-7 of hi.
+__device__ __forceinline__ uint32_t byte_perm(uint32_t hi, uint32_t lo, uint32_t sel) {
+	return __builtin_amdgcn_perm(hi, lo, sel);
+}
+
+// One step of four 8 x 8 bit transpositions (one per byte) over eight words: bits and words whose index
+// differs in D change places. (A template argument: the steps in a loop were not unrolled.)
+template <int D> __device__ __forceinline__ void exchange_bits(uint32_t r[8]) {
+	constexpr uint32_t m = D == 4 ? 0x0f0f0f0fu : (D == 2 ? 0x33333333u : 0x55555555u); // bits without D
 #pragma unroll
-	for (int a = 0; a < kHalo; ++a)
-		c[a] = (cw[a * sa] >> shp) & 15u;
-	const int q = (col >> 6) & 3; // this wave's group of four mask rows
-	uint32_t tt_bits = 0;         // 1 << i over all slices: bit kShowTT marks transparent against transparent
+	for (int i = 0; i < 8; ++i)
+		if (!(i & D)) {
+			const uint32_t a = r[i], b = r[i + D];
+			r[i] = (a & m) | ((b << D) & ~m);
+			r[i + D] = ((a >> D) & m) | (b & ~m);
+		}
+}
+
+// The class bits of 16 blocks' templates as planes, two per word: p0[a] holds class bit 0 and p1[a] class
+// bit 1 of the blocks' + faces along axis a in the low half-word (bit i: block i) and of their - faces in
+// the high one. The templates' upper half-words, two to a register, are an 8 x 8 bit matrix per byte;
+// three exchange steps transpose all four at once: 62 VALU instructions a row of 16 blocks, where one
+// shift-and-or per class bit and block would be 192. The phase is bound by instruction issue: with one lane
+// per column of an axis and two ballots per slice the 4,096-chunk cave batch issued 45.5 M instructions in
+// 100.8 us, with the planes 39.4 M in 89.0 us.
+__device__ __forceinline__ void row_planes(const uint32_t tm[16], uint32_t p0[3], uint32_t p1[3]) {
+	static_assert(kVoxClassShift == 20, "class bits 4 .. 15 of the template's upper half-word");
+	uint32_t r[8];
 #pragma unroll
-	for (int a = 0; a <= 16; ++a) {
-		const uint32_t i = (c[a] & 3u) | (c[a + 1] & 12u);
-		const uint64_t bp = a >= 1 ? ballot64((kShowPlus >> i) & 1u) : 0ull;
-		const uint64_t bm = a <= 15 ? ballot64((kShowMinus >> i) & 1u) : 0ull;
-		tt_bits |= 1u << i;
-		if (lane == 0) {
-			reinterpret_cast<uint64_t *>(s.ne[34 * A + 2 * a])[q] = bp;
-			reinterpret_cast<uint64_t *>(s.ne[34 * A + 2 * a + 1])[q] = bm;
-		}
+	for (int i = 0; i < 8; ++i)
+		r[i] = byte_perm(tm[i + 8], tm[i], 0x07060302u);
+	exchange_bits<4>(r);
+	exchange_bits<2>(r);
+	exchange_bits<1>(r);
+	// r[k]: bit k of every block's four bytes; block i < 8 in bit i of bytes 0 (class bits 0-3 in bits 4-7)
+	// and 1 (class bits 4-11), block i + 8 in bit i of bytes 2 and 3
+	p0[0] = byte_perm(r[6], r[4], 0x06040200u), p1[0] = byte_perm(r[7], r[5], 0x06040200u);
+	p0[1] = byte_perm(r[2], r[0], 0x07050301u), p1[1] = byte_perm(r[3], r[1], 0x07050301u);
+	p0[2] = byte_perm(r[6], r[4], 0x07050301u), p1[2] = byte_perm(r[7], r[5], 0x07050301u);
+}
+
+// A halo row's planes (templates tm[0 .. 17] of x = -1 .. 16) to where the rows beside it read them; for a
+// row of the chunk also its visible x faces, which need no other row.
+template <int NT> __device__ __forceinline__ void put_planes(Smem<NT> &s, int hy, int hz, const uint32_t tm[18]) {
+	uint32_t p0[3], p1[3];
+	row_planes(tm + 1, p0, p1);
+	s.planes[hy * kHalo + hz] = make_uint4(p0[1], p1[1], p0[2], p1[2]);
+	if ((unsigned)(hy - 1) < 16u && (unsigned)(hz - 1) < 16u) {
+		// + faces meet the - face of the block at x + 1, - faces the + face of the one at x - 1
+		constexpr int cp = kVoxClassShift, cm = kVoxClassShift + 2; // the rim blocks' + and - class bits
+		const uint32_t o0 = (p0[0] >> 17) | (p0[0] << 17) | ((tm[17] >> (cm - 15)) & 0x8000u) | ((tm[0] >> (cp - 16)) & 0x10000u);
+		const uint32_t o1 = (p1[0] >> 17) | (p1[0] << 17) | ((tm[17] >> (cm - 14)) & 0x8000u) | ((tm[0] >> (cp - 15)) & 0x10000u);
+		const int row = (hy - 1) * 16 + hz - 1;
+		s.vis_x[row] = show_planes(p0[0], p1[0], o0, o1);
+		s.tt_x[row] = tt_planes(p0[0], p1[0], o0, o1);
 	}
-	if (ballot64((tt_bits >> kShowTT) & 1u)) { // such faces show when the two texture codes differ (both directions alike)
-#pragma unroll 1
-		for (int a = 0; a <= 16; ++a) {
-			const uint32_t wa = cw[a * sa], wb = cw[(a + 1) * sa];
-			const bool d = (((wa >> shp) & 3u) | ((wb >> shp) & 12u)) == kShowTT &&
-			               row_code(s, vox_pid(wa), 2 * A) != row_code(s, vox_pid(wb), 2 * A + 1);
-			const uint64_t bd = ballot64(d);
-			if (bd && lane == 0) {
-				if (a >= 1)
-					reinterpret_cast<uint64_t *>(s.ne[34 * A + 2 * a])[q] |= bd;
-				if (a <= 15)
-					reinterpret_cast<uint64_t *>(s.ne[34 * A + 2 * a + 1])[q] |= bd;
-			}
-		}
+}
+
+// Transparent faces of a row against transparent ones (bits tt, both directions along axis A), which show
+// when the two texture codes differ. cell: halo index of the row's first block.
+template <int NT> __device__ uint32_t show_textures(const Smem<NT> &s, uint32_t tt, int A, int cell) {
+	uint32_t vis = 0;
+	while (tt) {
+		const uint32_t bit = __ffs(tt) - 1;
+		tt &= tt - 1u;
+		const int self = cell + int(bit & 15u), other = self + (bit < 16 ? axis_stride(A) : -axis_stride(A));
+		const int f = 2 * A + int(bit >> 4);
+		if (row_code(s, vox_pid(s.vox[self]), f) != row_code(s, vox_pid(s.vox[other]), f ^ 1))
+			vis |= 1u << bit;
 	}
+	return vis;
+}
+
+// One step of a 16 x 16 bit transposition over 16 lanes, for both half-words: bits and lanes whose index
+// differs in d change places. m: the half-words' bits without d, complemented in the lanes with d.
+__device__ __forceinline__ uint32_t transpose_step(uint32_t v, uint32_t other, uint32_t m, bool has, int d) {
+	const uint32_t moved = has ? other >> d : other << d;
+	return (v & m) | (moved & ~m);
+}
+
+// The tasks' masks from the planes, one lane per row (y, z) of the chunk; every mask row is written. The y
+// and z tasks' rows run along x as the planes do; the x tasks' rows run along z, so the 16 rows of a y are
+// transposed over 16 lanes first.
+template <int NT> __device__ __forceinline__ void visibility_row(Smem<NT> &s, int row) {
+	const int y = row >> 4, z = row & 15, h = (y + 1) * kHalo + z + 1, cell = h * kHalo + 1;
+	const uint4 p = s.planes[h];
+	const uint4 yp = s.planes[h + kHalo], ym = s.planes[h - kHalo], zp = s.planes[h + 1], zm = s.planes[h - 1];
+	// the other face of the + direction is the next row's - face (high half-word), of the - direction the
+	// previous row's + face (low half-word)
+	constexpr uint32_t kOther = 0x01000706u;
+	const uint32_t y0 = byte_perm(yp.x, ym.x, kOther), y1 = byte_perm(yp.y, ym.y, kOther);
+	const uint32_t z0 = byte_perm(zp.z, zm.z, kOther), z1 = byte_perm(zp.w, zm.w, kOther);
+	uint32_t vx = s.vis_x[row], vy = show_planes(p.x, p.y, y0, y1), vz = show_planes(p.z, p.w, z0, z1);
+	const uint32_t tx = s.tt_x[row], ty = tt_planes(p.x, p.y, y0, y1), tz = tt_planes(p.z, p.w, z0, z1);
+	if (tx | ty | tz) {
+		vx |= show_textures(s, tx, 0, cell);
+		vy |= show_textures(s, ty, 1, cell);
+		vz |= show_textures(s, tz, 2, cell);
+	}
+	s.ne[32 + 2 * y + 1][z] = uint16_t(vy);
+	s.ne[32 + 2 * y][z] = uint16_t(vy >> 16);
+	s.ne[64 + 2 * z + 1][y] = uint16_t(vz);
+	s.ne[64 + 2 * z][y] = uint16_t(vz >> 16);
+	// lanes 8, 4, 2 and 1 apart within a row of 16: row_ror:8, half-row mirror of the quads mirrored, and
+	// quad_perm 2,3,0,1 and 1,0,3,2
+	uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)vx, 0x128, 0xf, 0xf, true);
+	vx = transpose_step(vx, o, z & 8 ? 0xff00ff00u : 0x00ff00ffu, z & 8, 8);
+	o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)vx, 0x1b, 0xf, 0xf, true);
+	o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)o, 0x141, 0xf, 0xf, true);
+	vx = transpose_step(vx, o, z & 4 ? 0xf0f0f0f0u : 0x0f0f0f0fu, z & 4, 4);
+	o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)vx, 0x4e, 0xf, 0xf, true);
+	vx = transpose_step(vx, o, z & 2 ? 0xccccccccu : 0x33333333u, z & 2, 2);
+	o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)vx, 0xb1, 0xf, 0xf, true);
+	vx = transpose_step(vx, o, z & 1 ? 0xaaaaaaaau : 0x55555555u, z & 1, 1);
+	s.ne[2 * z + 1][y] = uint16_t(vx);
+	s.ne[2 * z][y] = uint16_t(vx >> 16);
 }
 
 // Halo index of the block owning face (task t, row u, column v), and its face.
 __device__ __forceinline__ int face_owner(int t, int u, int v, int &face) {
-	const int A = t / 34, sl = (t % 34) >> 1, inv = t & 1;
-	face = 2 * A + inv;
-	const int layer = inv ? sl : sl - 1;
+	const int A = task_axis(t), layer = task_layer(t);
+	face = 2 * A + (task_plus(t) ^ 1);
 	return (layer + 1) * axis_stride(A) + (u + 1) * axis_stride(u_axis(A)) + (v + 1) * axis_stride(v_axis(A));
 }
 
@@ -1180,6 +1274,7 @@ template <int NT> __device__ __forceinline__ void mesh_chunk(const MeshParams &p
 				tm[x] = tm[x] & kTmplMeta ? v : tm[x];
 			}
 		}
+		put_planes(s, hy, hz, tm);
 		uint32_t and_all = ~0u, or_inner = 0;
 		uint32_t *dst = s.vox + row * kHalo;
 #pragma unroll
@@ -1256,16 +1351,22 @@ template <int NT> __device__ __forceinline__ void mesh_chunk(const MeshParams &p
 			s.vox[i] = (s.vox[i] & kKeep) | (tmpl & ~kKeep);
 		}
 		__syncthreads();
+		// their rows' planes again (the light fields of a voxel word lie below its class bits, which are all
+		// that row_planes takes but for torchlight, in the bits it drops)
+		for (int row = tid; row < kHaloRows; row += NT) {
+			uint32_t w[18];
+#pragma unroll
+			for (int x = 0; x < 18; ++x)
+				w[x] = s.vox[row * kHalo + x];
+			put_planes(s, row / kHalo, row % kHalo, w);
+		}
+		__syncthreads();
 	}
 
 	// 3. faces: visibility masks by bit slices; then, for each group of tasks whose visible faces fit the
 	// stage, the face words (one lane per face, in dense order) and the link masks (one lane per row)
-	for (int col = tid; col < 256; col += NT)
-		visibility_column<0>(s, col);
-	for (int col = tid; col < 256; col += NT)
-		visibility_column<1>(s, col);
-	for (int col = tid; col < 256; col += NT)
-		visibility_column<2>(s, col);
+	for (int row = tid; row < 256; row += NT)
+		visibility_row(s, row);
 	__syncthreads();
 	if (wave == 0) { // exclusive prefix of visible faces over the tasks: lane l counts tasks l and l + 64,
 	                 // packed in one word (a chunk has at most 24,576 visible faces), and one DPP scan
