@@ -46,6 +46,12 @@ __host__ __device__ constexpr int task_plus(int t) { return t & 1; }
 // Entries of the face-word stage. 1,472 keeps the 256-thread workgroup's LDS within three per CU
 // (static_assert below); the tasks of a chunk with more visible faces are taken in several groups.
 constexpr int kListCap = 1472;
+constexpr int kFaceBlocks = kListCap / 64;
+constexpr int kMaskRows = kTasks * 16;
+constexpr int kUnits = kMaskRows / 4; // a unit is four mask rows, 64 faces
+// A group but the last holds more than kListCap - 256 faces (a task has at most 256), of 24,576 at most.
+constexpr int kMaxGroups = kTasks * 256 / (kListCap - 255) + 2;
+static_assert(kListCap % 64 == 0 && kFaceBlocks <= 64, "whole blocks of faces, one lane each");
 constexpr uint32_t kSplitQuads = 16383u; // a BlockMesh holds at most 65,532 vertices (:273-279, :397-403)
 constexpr int kMaxMeshPerPass = 8;
 
@@ -129,11 +135,11 @@ __device__ __forceinline__ int hidx(int x, int y, int z) { return (x + 1) * kSX 
 
 template <int NT> struct Smem {
 	uint32_t vox[kHaloVox];
-	// per task and mask row: visible, equal-to-right, equal-to-below, transparent pass
-	alignas(16) uint16_t ne[kTasks][16];
-	alignas(16) uint16_t eh[kTasks][16];
-	alignas(16) uint16_t ev[kTasks][16];
-	alignas(16) uint16_t tp[kTasks][16];
+	// a mask row of 16 faces per task and row, row 16 t + u: visible faces; equal-to-right faces, then the
+	// faces where a quad starts; equal-to-below faces, then the uncovered visible ones
+	alignas(16) uint16_t ne[kMaskRows];
+	alignas(16) uint16_t eh[kMaskRows];
+	alignas(16) uint16_t ev[kMaskRows];
 	union {
 		uint2 key[kListCap]; // face words of the current group of tasks, in dense order
 		struct {             // until the visibility masks are made: the halo rows' face classes as bit planes
@@ -141,9 +147,10 @@ template <int NT> struct Smem {
 			uint32_t vis_x[256], tt_x[256]; // per chunk row: its visible x faces and those to compare (show_rows)
 		};
 	};
-	uint16_t fpre[kTasks + 2]; // prefix of visible faces per task (the dense face order; at most 24,576)
-	uint32_t qpre_o[kTasks];   // per task: index of its first opaque quad in the opaque pass
-	uint32_t qpre_t[kTasks];   // per task: index of its first transparent quad in the transparent pass
+	alignas(16) uint16_t own[kListCap]; // per face of the group: 1 + its unit where one begins, else 0; then its descriptor
+	uint16_t upre[kUnits + 2]; // visible faces before each unit (the dense face order; at most 24,576), and in all
+	uint32_t bcnt[64];         // per 64 faces of the group: quads that start there, opaque | transparent << 16
+	uint2 grp[kMaxGroups];     // per group of tasks: its first task, and the quads of the groups before it
 	uint2 rows[kMaxPid];
 	uint32_t pid_vox[kMaxPid];
 	uint32_t codes[kMaxCodes];
@@ -153,7 +160,7 @@ template <int NT> struct Smem {
 	uint32_t events[16][2];
 	uint32_t scan_w[NT / 64][4]; // per wavefront: its totals of block_excl_sums
 	uint32_t slots[27];
-	uint32_t job, flags, n_events, n_link;
+	uint32_t job, flags, n_events;
 	uint32_t wave_ref[NT / 64];
 	uint32_t pool_base, mesh_base, group_end;
 };
@@ -788,10 +795,10 @@ template <int NT> __device__ __forceinline__ void visibility_row(Smem<NT> &s, in
 		vy |= show_textures(s, ty, 1, cell);
 		vz |= show_textures(s, tz, 2, cell);
 	}
-	s.ne[32 + 2 * y + 1][z] = uint16_t(vy);
-	s.ne[32 + 2 * y][z] = uint16_t(vy >> 16);
-	s.ne[64 + 2 * z + 1][y] = uint16_t(vz);
-	s.ne[64 + 2 * z][y] = uint16_t(vz >> 16);
+	s.ne[16 * (32 + 2 * y + 1) + z] = uint16_t(vy);
+	s.ne[16 * (32 + 2 * y) + z] = uint16_t(vy >> 16);
+	s.ne[16 * (64 + 2 * z + 1) + y] = uint16_t(vz);
+	s.ne[16 * (64 + 2 * z) + y] = uint16_t(vz >> 16);
 	// lanes 8, 4, 2 and 1 apart within a row of 16: row_ror:8, half-row mirror of the quads mirrored, and
 	// quad_perm 2,3,0,1 and 1,0,3,2
 	uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)vx, 0x128, 0xf, 0xf, true);
@@ -803,96 +810,154 @@ template <int NT> __device__ __forceinline__ void visibility_row(Smem<NT> &s, in
 	vx = transpose_step(vx, o, z & 2 ? 0xccccccccu : 0x33333333u, z & 2, 2);
 	o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)vx, 0xb1, 0xf, 0xf, true);
 	vx = transpose_step(vx, o, z & 1 ? 0xaaaaaaaau : 0x55555555u, z & 1, 1);
-	s.ne[2 * z + 1][y] = uint16_t(vx);
-	s.ne[2 * z][y] = uint16_t(vx >> 16);
+	s.ne[16 * (2 * z + 1) + y] = uint16_t(vx);
+	s.ne[16 * (2 * z) + y] = uint16_t(vx >> 16);
 }
 
-// Halo index of the block owning face (task t, row u, column v), and its face.
-__device__ __forceinline__ int face_owner(int t, int u, int v, int &face) {
+// ------------------------------------------------------------------------------------------------
+// visible faces, numbered densely
+// ------------------------------------------------------------------------------------------------
+// A face's descriptor is its bit among all mask rows: task << 8 | row << 4 | column, with kDescTrans when it
+// goes to the transparent pass.
+constexpr uint32_t kDescTrans = 0x8000u;
+static_assert(kTasks * 256 <= (int)kDescTrans, "descriptors of 15 bits");
+
+// Halo index of the block owning a face, and which of its faces it is.
+__device__ __forceinline__ int face_owner(uint32_t desc, int &face) {
+	const int t = (desc >> 8) & 127, u = (desc >> 4) & 15, v = desc & 15;
 	const int A = task_axis(t), layer = task_layer(t);
 	face = 2 * A + (task_plus(t) ^ 1);
 	return (layer + 1) * axis_stride(A) + (u + 1) * axis_stride(u_axis(A)) + (v + 1) * axis_stride(v_axis(A));
 }
 
-// Task, mask row and column of the visible face with dense index gi (task-major, row-major, as the
-// reference scans them), searched among the tasks [t0, t1), without branches: the task by seven halving
-// steps over the prefix (the last t with fpre[t] <= gi; fpre[t1] > gi and a group spans under 128 tasks),
-// then the task's four 64-bit mask words and the word's four 16-bit rows by comparing the remaining index
-// with their running counts, then the column as the rem-th set bit of the row.
-template <int NT> __device__ __forceinline__ void face_pos(const Smem<NT> &s, int t0, int t1, uint32_t gi, int &t, int &u, int &v) {
-	int lo = t0;
-#pragma unroll
-	for (int step = 64; step >= 1; step >>= 1) {
-		const int m = min(lo + step, t1);
-		lo = s.fpre[m] <= gi ? m : lo;
-	}
-	t = lo;
-	uint32_t rem = gi - s.fpre[t];
-	const uint64_t *rows = reinterpret_cast<const uint64_t *>(s.ne[t]);
-	const uint64_t w0 = rows[0], w1 = rows[1], w2 = rows[2], w3 = rows[3];
-	const uint32_t p1 = __popcll(w0), p2 = p1 + __popcll(w1), p3 = p2 + __popcll(w2);
-	const bool q1 = rem >= p1, q2 = rem >= p2, q3 = rem >= p3;
-	const uint64_t w = q3 ? w3 : (q2 ? w2 : (q1 ? w1 : w0));
-	rem -= q3 ? p3 : (q2 ? p2 : (q1 ? p1 : 0u));
-	const uint32_t lo32 = uint32_t(w), hi32 = uint32_t(w >> 32);
-	const uint32_t r1 = __popc(lo32 & 0xffffu), r2 = __popc(lo32), r3 = r2 + __popc(hi32 & 0xffffu);
-	const bool s1 = rem >= r1, s2 = rem >= r2, s3 = rem >= r3;
-	uint32_t bits = s3 ? hi32 >> 16 : (s2 ? hi32 & 0xffffu : (s1 ? lo32 >> 16 : lo32 & 0xffffu));
-	rem -= s3 ? r3 : (s2 ? r2 : (s1 ? r1 : 0u));
-	u = 4 * (int(q1) + int(q2) + int(q3)) + int(s1) + int(s2) + int(s3);
-	// the column: the rem-th set bit of the row
-	v = 0;
-	const uint32_t c8 = __popc(bits & 0xffu);
-	if (rem >= c8)
-		rem -= c8, bits >>= 8, v += 8;
-	const uint32_t c4 = __popc(bits & 0xfu);
-	if (rem >= c4)
-		rem -= c4, bits >>= 4, v += 4;
-	const uint32_t c2 = __popc(bits & 0x3u);
-	if (rem >= c2)
-		rem -= c2, bits >>= 2, v += 2;
-	if (rem >= (bits & 1u))
-		v += 1;
+// Running maximum over the wavefront, as wave_incl_sum.
+__device__ __forceinline__ uint32_t wave_incl_max(uint32_t v) {
+	v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, true));
+	v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, true));
+	v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, true));
+	v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, true));
+	v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, true));
+	v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, true));
+	return v;
 }
 
-// Word of the visible face with dense index gi (task-major, row-major, as the reference scans them):
-// Light4 (light4_init, :48-163) in x and the low 24 bits of y, the texture code in y bits 24-30 and the
-// transparent-pass flag in bit 31. Faces merge only if their words are equal (Light4::operator==, :44,
-// and the texture compare, :367-368).
+// Units per thread of the numbering: 192 threads hold two each (128 threads: three).
+template <int NT> constexpr int kUnitsPerThread = NT >= 192 ? 2 : 3;
+
+// Numbers the visible faces, task by task and row by row, as the reference scans them: every unit's faces
+// before it into s.upre. first: the faces before this thread's units; cnt: those in each. One barrier; s.upre
+// is complete after the caller's next one. Returns the number of faces.
+template <int NT> __device__ __forceinline__ uint32_t number_faces(Smem<NT> &s, uint32_t &first, uint32_t cnt[3]) {
+	constexpr int U = kUnitsPerThread<NT>;
+	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+	uint32_t c = 0;
+	cnt[0] = cnt[1] = cnt[2] = 0;
+	if (tid < kUnits / U) {
+		const uint64_t *rows = reinterpret_cast<const uint64_t *>(s.ne) + tid * U;
+#pragma unroll
+		for (int k = 0; k < U; ++k)
+			c += cnt[k] = __popcll(rows[k]);
+	}
+	const uint32_t inc = wave_incl_sum(c);
+	if (lane == 63)
+		s.scan_w[wave][0] = inc;
+	__syncthreads();
+	uint32_t before = inc - c, all = 0;
+#pragma unroll
+	for (int w = 0; w < (kUnits / U + 63) / 64; ++w) {
+		const uint32_t x = s.scan_w[w][0];
+		before += w < wave ? x : 0u;
+		all += x;
+	}
+	first = before;
+	if (tid < kUnits / U) {
+		uint32_t at = before;
+#pragma unroll
+		for (int k = 0; k < U; ++k) {
+			s.upre[tid * U + k] = uint16_t(at);
+			at += cnt[k];
+		}
+	}
+	if (tid == 0)
+		s.upre[kUnits] = uint16_t(all);
+	return all;
+}
+
+// Marks the units of the tasks [t0, t1) at their first faces in s.own (all zero before), and again at the
+// first face of a block of 64 where a unit continues into it, so that the unit of every face is the running
+// maximum of the marks over the lanes of its block.
 template <int NT>
-__device__ __forceinline__ uint2 face_word(const Smem<NT> &s, int t0, int t1, uint32_t gi, uint32_t &desc) {
-	int t, u, v;
-	face_pos(s, t0, t1, gi, t, u, v);
-	desc = uint32_t(t) | uint32_t(u) << 7 | uint32_t(v) << 11;
+__device__ __forceinline__ void mark_units(Smem<NT> &s, int t0, int t1, uint32_t g0, uint32_t first, const uint32_t cnt[3]) {
+	constexpr int U = kUnitsPerThread<NT>;
+	uint32_t p = first - g0;
+#pragma unroll
+	for (int k = 0; k < U; ++k) {
+		const int q = (int)threadIdx.x * U + k;
+		if (cnt[k] && q >= 4 * t0 && q < 4 * t1) {
+			const uint32_t next = (p + 63u) & ~63u; // the first block that begins at or after p
+			s.own[p] = uint16_t(q + 1);
+			if (next < p + cnt[k])
+				s.own[next] = uint16_t(q + 1);
+		}
+		p += cnt[k];
+	}
+}
+
+// Position of the n-th set bit (from 0) of the 64-bit word (hi, lo).
+__device__ __forceinline__ uint32_t nth_bit(uint32_t lo, uint32_t hi, uint32_t n) {
+	uint32_t c = __popc(lo);
+	bool up = n >= c;
+	uint32_t w = up ? hi : lo, pos = up ? 32u : 0u;
+	n -= up ? c : 0u;
+#pragma unroll
+	for (int h = 16; h >= 1; h >>= 1) {
+		c = __popc(w & ((1u << h) - 1u));
+		up = n >= c;
+		n -= up ? c : 0u;
+		w = up ? w >> h : w;
+		pos += up ? uint32_t(h) : 0u;
+	}
+	return pos;
+}
+
+// The descriptor of face i of the group (dense index g0 + i); every lane of the wavefront comes here.
+template <int NT> __device__ __forceinline__ uint32_t face_desc(const Smem<NT> &s, uint32_t i, uint32_t g0) {
+	const uint32_t q = max(wave_incl_max(s.own[i]), 1u) - 1u;
+	const uint2 rows = reinterpret_cast<const uint2 *>(s.ne)[q];
+	return (q << 6) + nth_bit(rows.x, rows.y, g0 + i - s.upre[q]);
+}
+
+// Word of a visible face: Light4 (light4_init, :48-163) in x and the low 24 bits of y, the texture code in y
+// bits 24-30 and the transparent-pass flag in bit 31. Faces merge only if their words are equal
+// (Light4::operator==, :44, and the texture compare, :367-368).
+template <int NT> __device__ __forceinline__ uint2 face_word(const Smem<NT> &s, uint32_t desc) {
 	int face;
-	const int self = face_owner(t, u, v, face);
+	const int self = face_owner(desc, face);
 	const uint2 l = light4(s.vox, face, self);
 	const uint32_t tc = row_code(s, vox_pid(s.vox[self]), face);
 	const uint32_t tpass = (s.codes[tc] >> 16) & kCodeTransPass ? 1u : 0u;
 	return make_uint2(l.x, l.y | (tc << 24) | (tpass << 31));
 }
 
-// Equal-to-right, equal-to-below and transparent-pass bits of the visible face with dense index i (local
-// to the group; desc = t | u << 7 | v << 11): its right and lower neighbours, when visible, are at
-// i + 1 and after the rest of row u and the start of row u + 1 in the dense order.
+// Equal-to-right and equal-to-below bits of the visible face with dense index i (local to the group): its
+// right and lower neighbours, when visible, are at i + 1 and after the rest of row u and the start of row
+// u + 1 in the dense order.
 template <int NT> __device__ __forceinline__ void face_links(Smem<NT> &s, uint32_t i, uint32_t desc) {
-	const int t = desc & 127, u = (desc >> 7) & 15, v = (desc >> 11) & 15;
+	const uint32_t r = (desc >> 4) & 0x7ffu, u = r & 15, v = desc & 15;
 	// the neighbours' words are read whether or not the neighbours are visible (positions clamped into the
 	// stage) and compared as whole words, so that only the rare atomics sit behind branches
-	const uint32_t ne_u = s.ne[t][u], ne_d = uint32_t(s.ne[t][min(u + 1, 15)]) & (0u - uint32_t(u < 15));
+	const uint32_t ne_u = s.ne[r], ne_d = uint32_t(s.ne[min(r + 1, uint32_t(kMaskRows - 1))]) & (0u - uint32_t(u < 15));
 	const uint2 w = s.key[i];
 	const uint32_t bit = 1u << (v + 16 * (u & 1));
 	const uint32_t ir = min(i + 1, uint32_t(kListCap - 1));
 	const uint32_t id = min(i + 1 + __popc(ne_u >> (v + 1)) + __popc(ne_d & ((1u << v) - 1u)), uint32_t(kListCap - 1));
-	const uint2 r = s.key[ir], d = s.key[id];
-	const bool eq_r = v < 15 && ((ne_u >> (v + 1)) & 1u) && ((r.x ^ w.x) | (r.y ^ w.y)) == 0;
+	const uint2 right = s.key[ir], d = s.key[id];
+	const bool eq_r = v < 15 && ((ne_u >> (v + 1)) & 1u) && ((right.x ^ w.x) | (right.y ^ w.y)) == 0;
 	const bool eq_d = ((ne_d >> v) & 1u) && ((d.x ^ w.x) | (d.y ^ w.y)) == 0;
 	if (eq_r)
-		atomicOr(reinterpret_cast<uint32_t *>(&s.eh[t][u & ~1]), bit);
+		atomicOr(reinterpret_cast<uint32_t *>(&s.eh[r & ~1u]), bit);
 	if (eq_d)
-		atomicOr(reinterpret_cast<uint32_t *>(&s.ev[t][u & ~1]), bit);
-	if (w.y >> 31)
-		atomicOr(reinterpret_cast<uint32_t *>(&s.tp[t][u & ~1]), bit);
+		atomicOr(reinterpret_cast<uint32_t *>(&s.ev[r & ~1u]), bit);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -929,34 +994,32 @@ __device__ __forceinline__ uint32_t spread_up(uint32_t f, uint32_t link) {
 	return f;
 }
 
-template <int NT>
-__device__ __forceinline__ void greedy_count(Smem<NT> &s, int t, bool active, uint32_t &n_o, uint32_t &n_t) {
+// One task: its quad starts into eh and its uncovered visible cells into ev, in place of the link masks.
+template <int NT> __device__ __forceinline__ void greedy_merge(Smem<NT> &s, int t) {
 	// coverage of the rows below the current one by quads of earlier rows, and the equal-to-below masks,
 	// held in registers as windows that shift up by one row per step (window row k = row u + k)
 	uint32_t cov[8], ev[8];
-	const uint32_t *evs = reinterpret_cast<const uint32_t *>(s.ev[active ? t : 0]);
+	const uint16_t *nes = s.ne + 16 * t;
+	uint16_t *ehs = s.eh + 16 * t, *evs = s.ev + 16 * t;
 #pragma unroll
 	for (int k = 0; k < 8; ++k) {
 		cov[k] = 0;
-		ev[k] = active ? evs[k] : 0u;
+		ev[k] = reinterpret_cast<const uint32_t *>(evs)[k];
 	}
-	n_o = 0, n_t = 0;
 	// a row's masks are read one step ahead, so that their LDS latency overlaps the previous row's work
-	uint32_t ne_n = active ? s.ne[t][0] : 0u, eh_n = active ? s.eh[t][0] : 0u, tp_n = active ? s.tp[t][0] : 0u;
+	uint32_t ne_n = nes[0], eh_n = ehs[0];
 #pragma unroll 1
 	for (int u = 0; u < 16; ++u) {
-		const uint32_t ne = ne_n, eh = eh_n, tp = tp_n;
-		if (u < 15 && active) // row u + 1 is not written before this step writes row u
-			ne_n = s.ne[t][u + 1], eh_n = s.eh[t][u + 1], tp_n = s.tp[t][u + 1];
+		const uint32_t ne = ne_n, eh = eh_n;
+		if (u < 15) // row u + 1 is not written before this step writes row u
+			ne_n = nes[u + 1], eh_n = ehs[u + 1];
 		const uint32_t S = ne & ~(cov[0] & 0xffffu); // uncovered visible cells of row u
 		const uint32_t link = S & ((S & eh) << 1);   // v continues the run of v - 1
 		const uint32_t starts = S & ~link;
-		if (active) { // row u's results replace its (already read) inputs; ev's rows are in registers
-			s.ev[t][u] = uint16_t(S);
-			s.eh[t][u] = uint16_t(starts & ~tp); // opaque quads start here
-			s.tp[t][u] = uint16_t(starts & tp);  // transparent quads start here
-		}
-		if (__ballot(S != 0)) {
+		// row u's results replace its (already read) inputs; ev's rows are in registers
+		evs[u] = uint16_t(S);
+		ehs[u] = uint16_t(starts);
+		if (__ballot(S != 0)) { // branches for the whole wavefront: per-lane ones cost more in execution masks
 			uint32_t alive = starts, cols = S;
 #pragma unroll
 			for (int k = 1; k <= 16; ++k) {
@@ -978,9 +1041,6 @@ __device__ __forceinline__ void greedy_count(Smem<NT> &s, int t, bool active, ui
 				if (k < 16)
 					cov[k >> 1] |= cols << (16 * (k & 1));
 			}
-			const uint32_t nt = __popc(starts & tp);
-			n_t += nt;
-			n_o += __popc(starts) - nt;
 		}
 		// shift the windows up by one row
 #pragma unroll
@@ -992,19 +1052,52 @@ __device__ __forceinline__ void greedy_count(Smem<NT> &s, int t, bool active, ui
 	}
 }
 
+// The quad starts of one task into eh, and its uncovered visible cells into ev, in place of the link masks.
+// A task whose equal neighbouring faces are all side by side (no equal-to-below bit) has one quad per
+// run of equal faces along V: a visible face starts one unless it continues its left neighbour, and no
+// cell is covered from above. One whose equal faces are all above each other (no equal-to-right bit)
+// has one quad per run along U: a face starts one unless it continues the face above, and the cells
+// below a start are covered by its quad. With neither, every visible face is a 1 x 1 quad. These follow
+// from the masks directly (rows are 16-bit fields of the 64-bit words, row u + 4 q at bit 16 u, and a
+// row's equal-to-right bit 15 is never set). Tasks with both are merged row by row.
+template <int NT> __device__ __forceinline__ void quad_starts(Smem<NT> &s, int t) {
+	uint64_t *eh64 = reinterpret_cast<uint64_t *>(s.eh + 16 * t), *ev64 = reinterpret_cast<uint64_t *>(s.ev + 16 * t);
+	const uint64_t *ne64 = reinterpret_cast<const uint64_t *>(s.ne + 16 * t);
+	uint64_t eh[4], ev[4], anyh = 0, anyv = 0;
+#pragma unroll
+	for (int q = 0; q < 4; ++q) {
+		eh[q] = eh64[q], ev[q] = ev64[q];
+		anyh |= eh[q], anyv |= ev[q];
+	}
+	if (anyh && anyv) {
+		greedy_merge(s, t);
+		return;
+	}
+#pragma unroll
+	for (int q = 0; q < 4; ++q) {
+		const uint64_t ne = ne64[q];
+		// equal-to-below bits of the row above each row: the word shifted up one row, with the last
+		// row of the previous word
+		const uint64_t above = (ev[q] << 16) | (q > 0 ? ev[q - 1] >> 48 : 0ull);
+		const uint64_t st = ne & ~(eh[q] << 1) & ~above;
+		ev64[q] = anyv ? st : ne;
+		eh64[q] = st;
+	}
+}
+
 // ------------------------------------------------------------------------------------------------
 // emission of one quad
 // ------------------------------------------------------------------------------------------------
 // The end of the longest run of tasks from t0 whose visible faces fit the face-word stage (one task, at
 // most 256 faces, always fits). Thread 0 searches; a barrier publishes the result.
-template <int NT> __device__ __forceinline__ int group_end(Smem<NT> &s, int t0) {
-	if (s.fpre[kTasks] - s.fpre[t0] <= (uint32_t)kListCap) // the rest fits (the usual case): every thread knows
+template <int NT> __device__ __forceinline__ int group_end(Smem<NT> &s, int t0, uint32_t n_faces) {
+	if (n_faces - s.upre[4 * t0] <= (uint32_t)kListCap) // the rest fits (the usual case): every thread knows
 		return kTasks;
 	if (threadIdx.x == 0) {
-		int lo = t0 + 1, hi = kTasks; // largest t1 with fpre[t1] - fpre[t0] <= kListCap
+		int lo = t0 + 1, hi = kTasks; // largest t1 whose tasks' faces from t0's on fit
 		while (lo < hi) {
 			const int mid = (lo + hi + 1) >> 1;
-			if (s.fpre[mid] - s.fpre[t0] <= (uint32_t)kListCap)
+			if (uint32_t(s.upre[4 * mid] - s.upre[4 * t0]) <= (uint32_t)kListCap)
 				lo = mid;
 			else
 				hi = mid - 1;
@@ -1064,125 +1157,49 @@ __device__ __forceinline__ void quad_done(Smem<NT> &s, uint32_t pass, uint32_t m
 	}
 }
 
-// The quad that starts at the visible face at desc (task t | row u << 7 | column v << 11) with face word
-// `word`, if one does. Per
-// task, ne still holds the visible cells and the counting pass left the opaque quad starts in eh, the
-// transparent ones in tp and the uncovered visible cells S in ev; the covered cells are C = ne & ~S. A
-// quad from (u, v0) spans S's run from v0 to the next start along V, and covers rows u .. u + h - 1 of its
-// columns, so below it column v0 is in C exactly for rows u + 1 .. u + h - 1: the cell under its last row
-// is either not covered or starts a quad. Its index in its pass follows the pass's starts in the task's
-// earlier rows and columns (the reference's order: rows, then columns). kSplit: some pass of the chunk
-// has more than kSplitQuads quads; without, every quad is in the first mesh of its pass.
-template <bool kSplit, int NT>
-__device__ __forceinline__ void emit_face(const MeshParams &p, Smem<NT> &s, uint32_t desc, uint2 word, uint32_t n0,
-                                          uint32_t pool_base, uint32_t box[2][6], bool any_tr) {
-	const int t = desc & 127, u = (desc >> 7) & 15, v = (desc >> 11) & 15;
-	const uint32_t so = s.eh[t][u], st = s.tp[t][u], starts = so | st;
-	if (!((starts >> v) & 1u))
-		return;
-	const uint32_t tr = (st >> v) & 1u, below = (1u << v) - 1u;
-	const uint32_t link = uint32_t(s.ev[t][u]) & ~starts;
+// Whether a quad starts at the face at desc.
+template <int NT> __device__ __forceinline__ bool starts_quad(const Smem<NT> &s, uint32_t desc) {
+	return (s.eh[(desc >> 4) & 0x7ffu] >> (desc & 15)) & 1u;
+}
+
+// Lanes below this one in a ballot.
+__device__ __forceinline__ uint32_t lanes_below(uint64_t ballot) {
+	return __builtin_amdgcn_mbcnt_hi(uint32_t(ballot >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(ballot), 0u));
+}
+
+// The quad that starts at the visible face at desc with face word `word`, quad i of its pass. Per
+// task, ne still holds the visible cells, eh the quad starts and ev the uncovered visible cells S; the
+// covered cells are C = ne & ~S. A quad from (u, v0) spans S's run from v0 to the next start along V, and
+// covers rows u .. u + h - 1 of its columns, so below it column v0 is in C exactly for rows u + 1 ..
+// u + h - 1: the cell under its last row is either not covered or starts a quad. split: some pass of the
+// chunk has more than kSplitQuads quads; else every quad is in the first mesh of its pass. epos: the quads
+// emitted before it, for a split.
+template <int NT>
+__device__ __forceinline__ void emit_face(const MeshParams &p, Smem<NT> &s, uint32_t desc, uint2 word, uint32_t i, uint32_t epos,
+                                          uint32_t n0, uint32_t pool_base, uint32_t box[2][6], bool any_tr, bool split) {
+	const uint32_t r = (desc >> 4) & 0x7ffu, tr = desc >> 15;
+	const int u = r & 15, v = desc & 15;
+	const uint32_t link = uint32_t(s.ev[r] & ~s.eh[r]);
 	const int w = __ffs(~(link >> (v + 1)));
 	// most quads are one row high: the covered cells of the row below are tested before the loop (row 15
 	// has none; its index is clamped so that the load needs no branch)
-	const int ub = min(u + 1, 15);
-	const uint32_t cov_below = uint32_t(s.ne[t][ub] & ~s.ev[t][ub]) & (0u - uint32_t(u < 15));
+	const uint32_t rb = min(r + 1, uint32_t(kMaskRows - 1));
+	const uint32_t cov_below = uint32_t(s.ne[rb] & ~s.ev[rb]) & (0u - uint32_t(u < 15));
 	int h = 1;
 	if ((cov_below >> v) & 1u) {
 		h = 2;
 #pragma unroll 1
-		for (int r = u + 2; r < 16 && ((uint32_t(s.ne[t][r] & ~s.ev[t][r]) >> v) & 1u); ++r)
+		for (int k = 2; u + k < 16 && ((uint32_t(s.ne[r + k] & ~s.ev[r + k]) >> v) & 1u); ++k)
 			++h;
 	}
-	// the pass's starts in rows 0 .. u - 1: words of two rows each, word k whole when k < u / 2 (k = 7
-	// never: u <= 15), and the low row of word u / 2 when u is odd
-	const uint32_t *m32 = reinterpret_cast<const uint32_t *>(tr ? s.tp[t] : s.eh[t]);
-	const uint4 wa = reinterpret_cast<const uint4 *>(m32)[0], wb = reinterpret_cast<const uint4 *>(m32)[1];
-	const uint32_t wk[7] = {wa.x, wa.y, wa.z, wa.w, wb.x, wb.y, wb.z};
-	uint32_t ord = __popc((tr ? st : so) & below);
-	const int half = u >> 1;
-#pragma unroll
-	for (int k = 0; k < 7; ++k)
-		ord += __popc(k < half ? wk[k] : 0u);
-	ord += __popc(m32[half] & (0u - uint32_t(u & 1)) & 0xffffu);
-	const uint32_t i = (tr ? s.qpre_t[t] : s.qpre_o[t]) + ord;
-	uint32_t slot, vbase, mk, mj, lo[3], hi[3];
-	if (!kSplit) {
-		emit_quad(p, s, t, u, v, w, h, word, pool_base + (tr ? n0 : 0u) + i, 4u * i, lo, hi);
+	uint32_t slot = pool_base + (tr ? n0 : 0u) + i, vbase = 4u * i, mk = 0, mj = i, lo[3], hi[3];
+	if (split)
+		quad_slot(tr, i, n0, pool_base, slot, vbase, mk, mj);
+	emit_quad(p, s, int(r >> 4), u, v, w, h, word, slot, vbase, lo, hi);
+	if (split)
+		quad_done(s, tr, mk, mj, epos, lo, hi, box);
+	else
 		box_add(box, tr, lo, hi, any_tr);
-		return;
-	}
-	quad_slot(tr, i, n0, pool_base, slot, vbase, mk, mj);
-	emit_quad(p, s, t, u, v, w, h, word, slot, vbase, lo, hi);
-	uint32_t epos = 0;
-	if (mj == 0 && mk > 0) { // emission position, only needed for a split: both passes' starts before it
-		const uint64_t *o64 = reinterpret_cast<const uint64_t *>(s.eh[t]);
-		const uint64_t *t64 = reinterpret_cast<const uint64_t *>(s.tp[t]);
-		epos = s.qpre_o[t] + s.qpre_t[t] + __popc(starts & below); // custom quads, then the earlier tasks'
-		for (int q = 0; q < 4; ++q) {
-			const int nb = 16 * (u - 4 * q);
-			const uint64_t m = nb >= 64 ? ~0ull : (nb > 0 ? (1ull << nb) - 1ull : 0ull);
-			epos += __popcll(o64[q] & m) + __popcll(t64[q] & m);
-		}
-	}
-	quad_done(s, tr, mk, mj, epos, lo, hi, box);
-}
-
-// The regular quads of a chunk, one lane per visible face (a quad per face that starts one): first the
-// last group of tasks, whose face words are still in key (keep: the lane's face positions, two 15-bit
-// positions to a register, faces tid + 2 k NT and tid + (2 k + 1) NT in register k), then the earlier
-// groups with their words computed again.
-template <bool kSplit, int NT>
-__device__ __forceinline__ void emit_regular(const MeshParams &p, Smem<NT> &s, uint32_t *keep, int t0_last, uint32_t n0,
-                                             uint32_t pool_base, uint32_t box[2][6], bool any_tr) {
-	const int tid = threadIdx.x;
-	constexpr int kMine = (kListCap + NT - 1) / NT, kPairs = (kMine + 1) / 2;
-	{
-		const uint32_t g0 = s.fpre[t0_last], n = s.fpre[kTasks] - g0;
-#pragma unroll 1
-		for (int k = 0; k < kPairs; ++k) {
-			const uint32_t i0 = tid + 2 * k * NT, i1 = i0 + NT;
-			if (i0 < n)
-				emit_face<kSplit>(p, s, keep[0] & 0xffffu, s.key[i0], n0, pool_base, box, any_tr);
-			if (i1 < n)
-				emit_face<kSplit>(p, s, keep[0] >> 16, s.key[i1], n0, pool_base, box, any_tr);
-#pragma unroll
-			for (int j = 0; j + 1 < kPairs; ++j)
-				keep[j] = keep[j + 1];
-		}
-	}
-#pragma unroll 1
-	for (int t0 = 0; t0 < t0_last;) {
-		__syncthreads(); // key is read by the previous group's lanes
-		const int t1 = group_end(s, t0);
-		const uint32_t g0 = s.fpre[t0], n = s.fpre[t1] - g0;
-#pragma unroll 1
-		for (int k = 0; k < kPairs; ++k) {
-			const uint32_t i0 = tid + 2 * k * NT, i1 = i0 + NT;
-			uint32_t d0 = 0, d1 = 0;
-			if (i0 < n)
-				s.key[i0] = face_word(s, t0, t1, g0 + i0, d0);
-			if (i1 < n)
-				s.key[i1] = face_word(s, t0, t1, g0 + i1, d1);
-#pragma unroll
-			for (int j = 0; j + 1 < kPairs; ++j)
-				keep[j] = keep[j + 1];
-			keep[kPairs - 1] = d0 | d1 << 16;
-		}
-		__syncthreads();
-#pragma unroll 1
-		for (int k = 0; k < kPairs; ++k) {
-			const uint32_t i0 = tid + 2 * k * NT, i1 = i0 + NT;
-			if (i0 < n)
-				emit_face<kSplit>(p, s, keep[0] & 0xffffu, s.key[i0], n0, pool_base, box, any_tr);
-			if (i1 < n)
-				emit_face<kSplit>(p, s, keep[0] >> 16, s.key[i1], n0, pool_base, box, any_tr);
-#pragma unroll
-			for (int j = 0; j + 1 < kPairs; ++j)
-				keep[j] = keep[j + 1];
-		}
-		t0 = t1;
-	}
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1198,7 +1215,7 @@ template <int NT> __device__ __forceinline__ void chunk_init(Smem<NT> &s) {
 		a[tid] = (tid % 6) < 3 ? 0xffffffffu : 0u; // AABB<uint32_t>{}: min = max(), max = min() (dep/AABB.hpp:11)
 	}
 	if (tid == 0)
-		s.n_events = 0, s.flags = 0, s.n_link = 0;
+		s.n_events = 0, s.flags = 0;
 }
 
 // One job; s.slots and the state of chunk_init are in place (a barrier after them).
@@ -1363,90 +1380,28 @@ template <int NT> __device__ __forceinline__ void mesh_chunk(const MeshParams &p
 		__syncthreads();
 	}
 
-	// 3. faces: visibility masks by bit slices; then, for each group of tasks whose visible faces fit the
-	// stage, the face words (one lane per face, in dense order) and the link masks (one lane per row)
+	// 3. faces: visibility masks, then the dense numbering of the visible faces. The link masks start empty, and
+	// so do the marks of the numbering.
 	for (int row = tid; row < 256; row += NT)
 		visibility_row(s, row);
-	__syncthreads();
-	if (wave == 0) { // exclusive prefix of visible faces over the tasks: lane l counts tasks l and l + 64,
-	                 // packed in one word (a chunk has at most 24,576 visible faces), and one DPP scan
-		uint32_t c = 0;
-		if (lane < kTasks) {
-			const uint64_t *r = reinterpret_cast<const uint64_t *>(s.ne[lane]);
-			c = __popcll(r[0]) + __popcll(r[1]) + __popcll(r[2]) + __popcll(r[3]);
-		}
-		if (lane + 64 < kTasks) {
-			const uint64_t *r = reinterpret_cast<const uint64_t *>(s.ne[lane + 64]);
-			c |= uint32_t(__popcll(r[0]) + __popcll(r[1]) + __popcll(r[2]) + __popcll(r[3])) << 16;
-		}
-		const uint32_t inc = wave_incl_sum(c), ex = inc - c;
-		const uint32_t tot = (uint32_t)__builtin_amdgcn_readlane((int)inc, 63), tot_a = tot & 0xffffu;
-		if (lane < kTasks)
-			s.fpre[lane] = ex & 0xffffu;
-		if (lane + 64 < kTasks)
-			s.fpre[lane + 64] = tot_a + (ex >> 16);
-		if (lane == 63)
-			s.fpre[kTasks] = tot_a + (tot >> 16);
+	for (int i = tid; i < kMaskRows / 8; i += NT) {
+		reinterpret_cast<uint4 *>(s.eh)[i] = make_uint4(0, 0, 0, 0);
+		reinterpret_cast<uint4 *>(s.ev)[i] = make_uint4(0, 0, 0, 0);
+		if (i < kListCap / 8)
+			reinterpret_cast<uint4 *>(s.own)[i] = make_uint4(0, 0, 0, 0);
 	}
 	__syncthreads();
-	if (s.fpre[kTasks] == 0 && !(flags & kFlagCustom)) { // no visible face and no custom mesh: no quads
+	uint32_t first, cnt[3];
+	const uint32_t n_faces = number_faces(s, first, cnt);
+	if (n_faces == 0 && !(flags & kFlagCustom)) { // no visible face and no custom mesh: no quads
 		if (tid == 0)
 			p.results[job] = hcm_job_result{HCM_OK, 0u, 0u, 0u};
 		return;
 	}
-	// face words per group of tasks, then the group's link masks; the last group's words stay in key. A
-	// lane keeps the positions of its faces (at most kListCap / NT of them, 15 bits each, two to a
-	// register) for the links and the emission, in a register queue shifted once per two faces (static
-	// register indices)
-	constexpr int kMine = (kListCap + NT - 1) / NT, kPairs = (kMine + 1) / 2;
-	int t0_last = 0;
-	uint32_t keep[kPairs]; // the positions of this lane's faces of the last group, for the emission
-#pragma unroll 1
-	for (int t0 = 0; t0 < kTasks;) {
-		const int t1 = group_end(s, t0);
-		const uint32_t g0 = s.fpre[t0], n = s.fpre[t1] - g0;
-		for (int k = tid; k < (t1 - t0) * 8; k += NT) { // clear the group's link masks
-			const int t = t0 + (k >> 3), q = k & 7;
-			reinterpret_cast<uint32_t *>(s.eh[t])[q] = 0;
-			reinterpret_cast<uint32_t *>(s.ev[t])[q] = 0;
-			reinterpret_cast<uint32_t *>(s.tp[t])[q] = 0;
-		}
-		uint32_t mine[kPairs] = {};
-#pragma unroll 1
-		for (int k = 0; k < kPairs; ++k) {
-			const uint32_t i0 = tid + 2 * k * NT, i1 = i0 + NT;
-			uint32_t d0 = 0, d1 = 0;
-			if (i0 < n)
-				s.key[i0] = face_word(s, t0, t1, g0 + i0, d0);
-			if (i1 < n)
-				s.key[i1] = face_word(s, t0, t1, g0 + i1, d1);
-#pragma unroll
-			for (int j = 0; j + 1 < kPairs; ++j)
-				mine[j] = mine[j + 1];
-			mine[kPairs - 1] = d0 | d1 << 16;
-		}
-#pragma unroll
-		for (int j = 0; j < kPairs; ++j)
-			keep[j] = mine[j];
-		__syncthreads();
-#pragma unroll 1
-		for (int k = 0; k < kPairs; ++k) {
-			const uint32_t i0 = tid + 2 * k * NT, i1 = i0 + NT;
-			if (i0 < n)
-				face_links(s, i0, mine[0] & 0xffffu);
-			if (i1 < n)
-				face_links(s, i1, mine[0] >> 16);
-#pragma unroll
-			for (int j = 0; j + 1 < kPairs; ++j)
-				mine[j] = mine[j + 1];
-		}
-		__syncthreads();
-		t0_last = t0;
-		t0 = t1;
-	}
 
-	// 4. counting: custom faces per thread range of cells, greedy quads per task (one lane per task)
-	uint32_t c_o = 0, c_t = 0, q_o = 0, q_t = 0;
+	// custom faces per thread range of cells, and their prefix sums
+	uint32_t c_o = 0, c_t = 0, cust0 = 0, cust1 = 0;
+	uint64_t cust_pre = 0;
 	if (flags & kFlagCustom) {
 		for (int k = 0; k < CPT; ++k) {
 			const int cell = tid * CPT + k;
@@ -1457,112 +1412,139 @@ template <int NT> __device__ __forceinline__ void mesh_chunk(const MeshParams &p
 			c_t += nt;
 			c_o += c.count - nt;
 		}
-	}
-	// A task whose equal neighbouring faces are all side by side (no equal-to-below bit) has one quad per
-	// run of equal faces along V: a visible face starts one unless it continues its left neighbour, and no
-	// cell is covered from above. One whose equal faces are all above each other (no equal-to-right bit)
-	// has one quad per run along U: a face starts one unless it continues the face above, and the cells
-	// below a start are covered by its quad. With neither, every visible face is a 1 x 1 quad. These follow
-	// from the masks directly (rows are 16-bit fields of the 64-bit words, row u + 4 q at bit 16 u, and a
-	// row's equal-to-right bit 15 is never set). Tasks with both are listed and merged by one lane each, in
-	// as few wavefronts as they fill. The list passes through qpre_t and the counts through qpre_o
-	// (o | t << 16) before either holds its own values.
-	if (tid < kTasks) { // the link masks are complete: the group loop ends with a barrier
-		const int t = tid;
-		const uint64_t *eh64 = reinterpret_cast<const uint64_t *>(s.eh[t]);
-		const uint64_t *ev64 = reinterpret_cast<const uint64_t *>(s.ev[t]);
-		uint64_t eh[4], ev[4], anyh = 0, anyv = 0;
-#pragma unroll
-		for (int q = 0; q < 4; ++q) {
-			eh[q] = eh64[q], ev[q] = ev64[q];
-			anyh |= eh[q], anyv |= ev[q];
-		}
-		if (anyh && anyv) {
-			s.qpre_t[atomicAdd(&s.n_link, 1u)] = uint32_t(t);
-		} else {
-			uint32_t no = 0, nt = 0;
-#pragma unroll
-			for (int q = 0; q < 4; ++q) {
-				uint64_t *tp64 = reinterpret_cast<uint64_t *>(s.tp[t]) + q;
-				const uint64_t ne = reinterpret_cast<const uint64_t *>(s.ne[t])[q], tp = *tp64 & ne;
-				// equal-to-below bits of the row above each row: the word shifted up one row, with the last
-				// row of the previous word
-				const uint64_t above = (ev[q] << 16) | (q > 0 ? ev[q - 1] >> 48 : 0ull);
-				const uint64_t st = ne & ~(eh[q] << 1) & ~above;     // quad starts
-				reinterpret_cast<uint64_t *>(s.ev[t])[q] = anyv ? st : ne; // uncovered visible cells
-				reinterpret_cast<uint64_t *>(s.eh[t])[q] = st & ~tp;     // opaque quads start here
-				*tp64 = st & tp;                                         // transparent quads start here
-				no += __popcll(st & ~tp);
-				nt += __popcll(st & tp);
-			}
-			s.qpre_o[t] = no | nt << 16;
-		}
-	}
-	__syncthreads();
-	{
-		const uint32_t n_link = s.n_link;
-		if (wave * 64 < (int)n_link) {
-			const bool active = tid < (int)n_link;
-			const int t = active ? (int)s.qpre_t[tid] : 0;
-			uint32_t no, nt;
-			greedy_count(s, t, active, no, nt);
-			if (active)
-				s.qpre_o[t] = no | nt << 16;
-		}
-	}
-	__syncthreads();
-	if (tid < kTasks) {
-		const uint32_t c = s.qpre_o[tid];
-		q_o = c & 0xffffu, q_t = c >> 16;
-	}
-	// 5. block-wide prefix sums and allocation: the chunk's output is [pool_base, +n0) opaque and
-	// [+n0, +n0+n1) transparent; custom quads come first in each pass, then the tasks' quads in task order
-	// (a chunk's regular quads per pass are at most its 24,576 faces, so both passes' counts share a word)
-	uint32_t scan[3] = {q_o | q_t << 16, c_o, c_t}, tot[3];
-	block_excl_sums(s, scan, tot);
-	const uint64_t cust_pre = (uint64_t)scan[1] | ((uint64_t)scan[2] << 32);
-	const uint32_t cust0 = tot[1], cust1 = tot[2];
-	const uint32_t n0 = cust0 + (tot[0] & 0xffffu), n1 = cust1 + (tot[0] >> 16);
-	const uint32_t total = n0 + n1;
-	if (total == 0) {
-		if (tid == 0)
-			p.results[job] = hcm_job_result{HCM_OK, 0u, 0u, 0u};
-		return;
-	}
-	if (tid < kTasks) {
-		s.qpre_o[tid] = cust0 + (scan[0] & 0xffffu);
-		s.qpre_t[tid] = cust1 + (scan[0] >> 16);
-	}
-	// allocation: the quad range and the mesh records, one atomic each, issued by two lanes of one
-	// instruction so that both are in flight together
-	const uint32_t nm0 = (n0 + kSplitQuads - 1) / kSplitQuads, nm1 = (n1 + kSplitQuads - 1) / kSplitQuads;
-	if (tid < 2) {
-		const uint32_t base = atomicAdd(tid == 0 ? &p.ctr->pool_cursor : &p.ctr->mesh_cursor, tid == 0 ? total : nm0 + nm1);
-		if (tid == 0)
-			s.pool_base = base;
-		else
-			s.mesh_base = base;
-	}
-	__syncthreads();
-	const uint32_t pool_base = s.pool_base;
-	if ((uint64_t)pool_base + total > p.pool_cap || (uint64_t)s.mesh_base + nm0 + nm1 > p.rec_cap) {
-		if (tid == 0)
-			p.results[job] = hcm_job_result{(int32_t)HCM_ERR_POOL_FULL, 0u, 0u, total};
-		return;
+		__syncthreads(); // scan_w is read by number_faces
+		uint32_t scan[3] = {c_o, c_t, 0}, tot[3];
+		block_excl_sums(s, scan, tot);
+		cust_pre = (uint64_t)scan[0] | ((uint64_t)scan[1] << 32);
+		cust0 = tot[0], cust1 = tot[1];
 	}
 
-	// 6. emission. AABB<uint32_t>::Merge (dep/AABB.hpp:52-59) of the first mesh of each pass per lane,
-	// reduced at the end; later meshes of a pass (past 16,383 quads) by LDS atomics
-	uint32_t box[2][6];
+	// 4. groups of tasks whose visible faces fit the stage, twice: first every group's faces, links and quads
+	// (one group but in dense chunks), which gives the chunk's quad counts; then, from the last group, whose
+	// words are still in the stage, the emission, for which an earlier group's words are computed again. A
+	// quad's place in its pass is its start's among the faces, counted by ballots over blocks of 64 faces.
+	const uint32_t wave_u = __builtin_amdgcn_readfirstlane(wave);
+	uint32_t base_o = cust0, base_t = cust1;       // quads of each pass before the group
+	uint32_t n0 = 0, n1 = 0, nm0 = 0, nm1 = 0;      // the chunk's quads and meshes per pass
+	uint32_t pool_base = 0, box[2][6];
+	bool any_tr = false, split = false, collect = true;
+	uint32_t n_saved = 0, next_saved = 0, g0 = 0; // groups before the last; the next to emit; the group's first face
+	int t0 = 0;
+#pragma unroll 1
+	for (bool again = false;; again = true) {
+		int t1 = kTasks;
+		if (again || n_faces > (uint32_t)kListCap) {
+			if (again) {
+				__syncthreads(); // the last group's descriptors are read
+				if (tid < kListCap / 8)
+					reinterpret_cast<uint4 *>(s.own)[tid] = make_uint4(0, 0, 0, 0);
+				if (NT < kListCap / 8 && tid + NT < kListCap / 8)
+					reinterpret_cast<uint4 *>(s.own)[tid + NT] = make_uint4(0, 0, 0, 0);
+			}
+			__syncthreads();
+			t1 = group_end(s, t0, n_faces);
+		}
+		mark_units(s, t0, t1, g0, first, cnt);
+		__syncthreads();
+		const uint32_t n = __builtin_amdgcn_readfirstlane(s.upre[4 * t1]) - g0;
+		// face words
+#pragma unroll 1
+		for (uint32_t b = wave_u; b * 64 < n; b += NT / 64) {
+			const uint32_t i = 64 * b + lane, desc = face_desc(s, i, g0);
+			if (i < n) {
+				const uint2 word = face_word(s, desc);
+				s.key[i] = word;
+				s.own[i] = uint16_t(desc | (word.y >> 31 ? kDescTrans : 0u));
+			}
+		}
+		__syncthreads();
+		if (collect) {
+#pragma unroll 1
+			for (uint32_t i = tid; i < n; i += NT)
+				face_links(s, i, s.own[i]);
+			__syncthreads();
+			if (t0 + tid < t1)
+				quad_starts(s, t0 + tid);
+			__syncthreads();
+		}
+		// quads that start in each block of 64 faces, and before each block in the group (lane b: block b)
+#pragma unroll 1
+		for (uint32_t b = wave_u; b < (uint32_t)kFaceBlocks; b += NT / 64) {
+			uint32_t c = 0;
+			if (b * 64 < n) {
+				const uint32_t i = 64 * b + lane, desc = s.own[i];
+				const bool st = (i < n) & starts_quad(s, desc), tr = desc >> 15;
+				c = (uint32_t)__popcll(ballot64(st & !tr)) | (uint32_t)__popcll(ballot64(st & tr)) << 16;
+			}
+			if (lane == 0)
+				s.bcnt[b] = c;
+		}
+		__syncthreads();
+		const uint32_t c = lane < kFaceBlocks ? s.bcnt[lane] : 0u, inc = wave_incl_sum(c), ex = inc - c;
+		if (collect) {
+			const uint32_t tot = (uint32_t)__builtin_amdgcn_readlane((int)inc, 63);
+			n0 = base_o + (tot & 0xffffu), n1 = base_t + (tot >> 16);
+			if (t1 < kTasks) { // the group waits for the others' counts
+				if (tid == 0)
+					s.grp[n_saved] = make_uint2(uint32_t(t0) | base_o << 8, base_t);
+				++n_saved;
+				base_o = n0, base_t = n1;
+				t0 = t1;
+				g0 += n;
+				continue;
+			}
+			// 5. allocation: the chunk's output is [pool_base, +n0) opaque and [+n0, +n0+n1) transparent, custom
+			// quads first in each pass; the quad range and the mesh records by one atomic each, issued by two
+			// lanes of one instruction so that both are in flight together
+			const uint32_t total = n0 + n1;
+			if (total == 0) {
+				if (tid == 0)
+					p.results[job] = hcm_job_result{HCM_OK, 0u, 0u, 0u};
+				return;
+			}
+			nm0 = (n0 + kSplitQuads - 1) / kSplitQuads, nm1 = (n1 + kSplitQuads - 1) / kSplitQuads;
+			if (tid < 2) {
+				const uint32_t base = atomicAdd(tid == 0 ? &p.ctr->pool_cursor : &p.ctr->mesh_cursor, tid == 0 ? total : nm0 + nm1);
+				if (tid == 0)
+					s.pool_base = base;
+				else
+					s.mesh_base = base;
+			}
+			__syncthreads();
+			pool_base = s.pool_base;
+			if ((uint64_t)pool_base + total > p.pool_cap || (uint64_t)s.mesh_base + nm0 + nm1 > p.rec_cap) {
+				if (tid == 0)
+					p.results[job] = hcm_job_result{(int32_t)HCM_ERR_POOL_FULL, 0u, 0u, total};
+				return;
+			}
+			any_tr = n1 != 0;
+			split = n0 > kSplitQuads || n1 > kSplitQuads;
+			// AABB<uint32_t>::Merge (dep/AABB.hpp:52-59) of the first mesh of each pass per lane, reduced at
+			// the end; later meshes of a pass (past 16,383 quads) by LDS atomics
 #pragma unroll
-	for (int a = 0; a < 6; ++a)
-		box[0][a] = box[1][a] = a < 3 ? ~0u : 0u;
-	// regular quads, one lane per visible face (a quad per face that starts one)
-	const bool any_tr = __builtin_amdgcn_readfirstlane(int(n1)) != 0; // the same in every lane
-	if (n0 > kSplitQuads || n1 > kSplitQuads)
-		emit_regular<true>(p, s, keep, t0_last, n0, pool_base, box, any_tr);
-	else
-		emit_regular<false>(p, s, keep, t0_last, n0, pool_base, box, any_tr);
+			for (int a = 0; a < 6; ++a)
+				box[0][a] = box[1][a] = a < 3 ? ~0u : 0u;
+			collect = false;
+		}
+		// 6. emission: one lane per visible face, a quad per face that starts one
+#pragma unroll 1
+		for (uint32_t b = wave_u; b * 64 < n; b += NT / 64) {
+			const uint32_t i = 64 * b + lane, desc = s.own[i];
+			const bool st = (i < n) & starts_quad(s, desc), tr = desc >> 15;
+			const uint64_t opaque = ballot64(st & !tr), trans = ballot64(st & tr);
+			const uint32_t before = (uint32_t)__builtin_amdgcn_readlane((int)ex, (int)b);
+			if (st) {
+				const uint32_t io = base_o + (before & 0xffffu) + lanes_below(opaque);
+				const uint32_t it = base_t + (before >> 16) + lanes_below(trans);
+				emit_face(p, s, desc, s.key[i], tr ? it : io, io + it, n0, pool_base, box, any_tr, split);
+			}
+		}
+		if (next_saved == n_saved)
+			break;
+		const uint2 saved = s.grp[next_saved++];
+		t0 = int(saved.x & 0xffu), base_o = saved.x >> 8, base_t = saved.y;
+		g0 = s.upre[4 * t0];
+	}
 	// custom quads, after the regular ones (their positions in the output are fixed by the prefix sums): in
 	// windows of the face-word stage, the threads list their cells' quads (cells in YZX order, faces in
 	// mesh order, each thread its range of cells), then one lane per listed quad writes it
@@ -1646,7 +1628,7 @@ template <int NT> __device__ __forceinline__ void mesh_chunk(const MeshParams &p
 			put(0, nm0 - 1);
 		if (nm1)
 			put(1, nm1 - 1);
-		p.results[job] = hcm_job_result{HCM_OK, mbase, m, total};
+		p.results[job] = hcm_job_result{HCM_OK, mbase, m, n0 + n1};
 	}
 }
 
@@ -1664,27 +1646,19 @@ template <int NT> __global__ __launch_bounds__(NT, NT >= 512 ? 2 : 3) void mesh_
 		const uint32_t q = p.reg.pid_of[65536 + i];
 		s.tmpl_id[i] = q == 0xffu ? kTmplMeta : p.reg.pid_vox[q];
 	}
-	if (!p.persistent) {
-		const uint32_t job = p.job_base + blockIdx.x;
-		if (job < p.n_jobs && threadIdx.x < 27)
-			s.slots[threadIdx.x] = p.nbr[27 * (size_t)job + threadIdx.x];
-		chunk_init(s);
-		__syncthreads();
-		if (job < p.n_jobs)
-			mesh_chunk(p, s, job);
-		return;
-	}
 	// part q of the job list is [q * n / kQueues, (q + 1) * n / kQueues); a part is empty once its
 	// counter reaches its length, and the workgroup moves on to the next part
 	const uint32_t home = blockIdx.x % kQueues;
 	uint32_t tried = 0; // lane 0 of wavefront 0 only
 	const int lane = threadIdx.x & 63;
+	const uint32_t given = p.persistent ? ~0u : p.job_base + blockIdx.x; // per-chunk launches: the workgroup's one job
 	for (;;) {
 		// wavefront 0 claims the next job and loads its slot list while the others set up its LDS state
 		if (threadIdx.x < 64) {
 			uint32_t job = ~0u;
 			if (lane == 0) {
-				while (job == ~0u && tried < kQueues) {
+				job = given;
+				while (p.persistent && job == ~0u && tried < kQueues) {
 					const uint32_t q = (home + tried) % kQueues;
 					const uint32_t lo = uint32_t(uint64_t(q) * p.n_jobs / kQueues);
 					const uint32_t len = uint32_t(uint64_t(q + 1) * p.n_jobs / kQueues) - lo;
@@ -1706,6 +1680,8 @@ template <int NT> __global__ __launch_bounds__(NT, NT >= 512 ? 2 : 3) void mesh_
 		if (job >= p.n_jobs)
 			break;
 		mesh_chunk(p, s, job);
+		if (!p.persistent)
+			break;
 		__syncthreads();
 	}
 	// every claim and allocation of this workgroup precedes its increment of `done`, so the last

@@ -91,6 +91,8 @@ inline dim3 grid_dim() { return current()->gdim; }
 
 #define __syncthreads() ::hipcpu::wait_barrier()
 #define __threadfence() ((void)0)
+#define __builtin_amdgcn_s_barrier() ::hipcpu::wait_barrier()
+#define __builtin_amdgcn_fence(...) ((void)0)
 namespace hipcpu {
 // wavefront operations: a call site is told apart by the return address into its caller (each
 // inlined copy of a caller has its own); the last argument is unused
@@ -119,6 +121,15 @@ inline uint32_t __builtin_amdgcn_perm(uint32_t hi, uint32_t lo, uint32_t sel) {
 	for (int i = 0; i < 4; ++i)
 		r |= uint32_t((v >> (8 * ((sel >> (8 * i)) & 7u))) & 0xffu) << (8 * i);
 	return r;
+}
+// v_mbcnt: the set bits of a mask below this lane, added up over its two halves
+inline uint32_t __builtin_amdgcn_mbcnt_lo(uint32_t m, uint32_t a) {
+	const uint32_t l = hipcpu::current()->cur->tid & 63u;
+	return a + (uint32_t)__builtin_popcount(l >= 32 ? m : m & ((1u << l) - 1u));
+}
+inline uint32_t __builtin_amdgcn_mbcnt_hi(uint32_t m, uint32_t a) {
+	const uint32_t l = hipcpu::current()->cur->tid & 63u;
+	return a + (l > 32 ? (uint32_t)__builtin_popcount(m & ((1u << (l - 32)) - 1u)) : 0u);
 }
 // integer intrinsics
 inline int __popc(uint32_t v) { return __builtin_popcount(v); }

@@ -59,3 +59,56 @@ def test_meshes_of_blocks_with_six_textures(tmp_path, seed, density, threads):
     batch.close()
     store.close()
     ctx.close()
+
+
+def chunk_with_faces(n):
+    """27 chunks whose middle one has exactly n visible faces: stone blocks apart from each other (six faces each), with
+    stone beyond x, y and z = 15, which hides a face of the blocks along those sides."""
+    fours = [(x, 15, 15) for x in range(1, 14, 2)]
+    put = {0: [], 1: [(15, 15, 15)] + fours[:1], 2: fours[:2], 3: [(15, 15, 15)], 4: fours[:1], 5: [(15, 15, 15)] + fours[:2]}[n % 6]
+    left = n - sum(3 if at[0] == 15 else 4 for at in put)
+    inner = [(x, y, z) for y in range(14) for z in range(14) for x in range(14) if (x + y + z) % 2 == 0]
+    put += inner[:left // 6]
+    left -= 6 * min(left // 6, len(inner))
+    b = np.zeros((16, 16, 16), np.uint16)  # [y, z, x]
+    for x, y, z in put:
+        b[y, z, x] = 1
+    out = []
+    for d in workloads.SLOT_OFFSETS:
+        c = np.zeros((16, 16, 16), np.uint16)
+        if not d.any():
+            c = b
+        elif (d == 1).any():
+            c[0 if d[1] == 1 else slice(None), 0 if d[2] == 1 else slice(None), 0 if d[0] == 1 else slice(None)] = 1
+        out.append(c.reshape(-1))
+    return np.stack(out), left
+
+
+@pytest.mark.parametrize("merge", [False, True])
+@pytest.mark.parametrize("faces", [1, 2, 63, 64, 65, 128, 1471, 1472, 1473, 1536, 2944, 2945, 4416, 4417, 8232])
+def test_face_counts_at_block_and_group_edges(ctx, oracle, faces, merge):
+    """Visible faces are numbered by units of 64 mask bits, handled in blocks of 64 lanes and held in groups of up to
+    1,472: counts at and beside those edges, with light that lets faces merge and light that does not."""
+    if faces < 3:  # nothing apart has so few: a slab's top, and two
+        b27 = [np.zeros(4096, np.uint16) if d[1] == 1 else np.ones(4096, np.uint16) for d in workloads.SLOT_OFFSETS]
+        l27 = [np.zeros(4096, np.uint8)] * 27
+    else:
+        blocks, left = chunk_with_faces(faces)
+        assert left == 0, (faces, left)
+        b27 = list(blocks)
+        rng = np.random.default_rng(faces)
+        l27 = [np.full(4096, 0x3A, np.uint8) if merge else rng.integers(0, 256, 4096).astype(np.uint8) for _ in range(27)]
+    print(f"{faces} faces, merge {merge}", flush=True)
+    want = oracle.mesh(b27, l27)
+    assert meshdigest.digest(ctx.mesh_chunk(b27, l27)) == meshdigest.digest(want)
+    store = hcm.Store(ctx, 27)
+    store.upload(np.stack(b27), np.stack(l27))
+    for threads in (128, 256, 512):
+        ctx.set_tuning(wg_per_cu=0, threads=threads)
+        batch = hcm.Batch(ctx, store, np.arange(27, dtype=np.uint32).reshape(1, 27))
+        batch.run()
+        out = batch.download()
+        batch.close()
+        assert meshdigest.digest(hcm.job_meshes(0, *out)) == meshdigest.digest(want), threads
+    ctx.set_tuning(wg_per_cu=0, threads=256)
+    store.close()
