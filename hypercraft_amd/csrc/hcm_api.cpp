@@ -983,7 +983,7 @@ static hipError_t enqueue_light(hcm_batch *b, hipStream_t st) {
 	hipError_t e = launch_light_prep(lp, st);
 	if (e == hipSuccess) {
 		const int per_cu = std::max(1, std::min(3, (160 * 1024) / std::max(1, light_lds_bytes())));
-		e = launch_light(lp, per_cu * b->ctx->n_cu, st);
+		e = launch_light(lp, (int)std::min((uint32_t)(per_cu * b->ctx->n_cu), b->n_jobs), st);
 	}
 	return e;
 }
@@ -999,6 +999,7 @@ static int batch_run(hcm_batch *b, uint32_t mode, uint32_t times) {
 	hipStream_t st = c->stream;
 	const uint32_t threads = c->tuning.threads;
 	MeshParams p = batch_params(b);
+	const uint32_t grid = std::min((uint32_t)persistent_grid(c, threads), b->n_jobs);
 	if (mode == HCM_RUN_PERSISTENT && !b->launched) {
 		// first persistent run: launched directly, since capturing and instantiating a graph costs more
 		// than the launches it replaces; the graph is captured when the batch runs again
@@ -1009,12 +1010,11 @@ static int batch_run(hcm_batch *b, uint32_t mode, uint32_t times) {
 			HCM_HIP(enqueue_light(b, st));
 		p.persistent = 1;
 		p.self_reset = 1;
-		HCM_HIP(launch_mesh(p, (int)threads, persistent_grid(c, threads), st));
+		HCM_HIP(launch_mesh(p, (int)threads, (int)grid, st));
 		HCM_HIP(hipEventRecord(b->ev1, st));
 		b->ctr_clean = true;
 		b->launched = true;
 	} else if (mode == HCM_RUN_PERSISTENT) {
-		const uint32_t grid = (uint32_t)persistent_grid(c, threads);
 		if (!b->graph_exec || b->graph_threads != threads || b->graph_grid != grid || b->graph_light != b->light_mode) {
 			if (b->graph_exec)
 				(void)hipGraphExecDestroy(b->graph_exec), b->graph_exec = nullptr;

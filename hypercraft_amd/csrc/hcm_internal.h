@@ -52,24 +52,62 @@ struct DevReg {
 	uint32_t flow_tex, src_id, flow_id, pad;
 };
 
-// The persistent kernel's job list is cut into kQueues contiguous parts, one per XCD (gfx950 has 8,
+// The persistent kernels' job list is cut into kQueues contiguous parts, one per XCD (gfx950 has 8,
 // and workgroups are dispatched to them round-robin by workgroup id). A workgroup takes jobs from its
 // own XCD's part first, so neighbouring chunks, which share halo data, are read through one L2; then it
-// takes jobs from the other parts. Each counter sits on its own 256-byte line: all are hit by
-// device-scope atomics, and atomics on one line are serialised where that line lives.
+// takes jobs from the other parts. The first jobs of a part belong to its workgroups, one each, so that only
+// jobs beyond those are claimed by atomics, and a launch with no more jobs than workgroups makes none. Each
+// counter sits on its own 256-byte line: all are hit by device-scope atomics, and atomics on one line are
+// serialised where that line lives.
 constexpr uint32_t kQueues = 8;
 
 struct Counters {
 	struct alignas(256) Line {
 		uint32_t v;
 	};
-	Line queue[kQueues];               // jobs taken from each part of the job list
+	Line queue[kQueues];               // jobs claimed from each part of the job list, past its workgroups' first ones
+	Line dry;                          // bit q: part q had no job left for a claim
 	alignas(256) uint32_t pool_cursor; // quads allocated in the pool
 	alignas(256) uint32_t mesh_cursor; // mesh records allocated
 	// self-resetting persistent runs: workgroups done; the last one copies the run's totals below and
 	// clears every counter for the next run
 	alignas(256) uint32_t done;
 	uint32_t total_quads, total_meshes;
+};
+
+// The jobs of one workgroup of a persistent launch, by one lane.
+struct JobClaims {
+	uint32_t n_jobs, tried = 0;
+	bool first = true;
+	__device__ explicit JobClaims(uint32_t n) : n_jobs(n) {}
+	__device__ uint32_t part(uint32_t q) const { return uint32_t(uint64_t(q) * n_jobs / kQueues); }
+	// The next job, or ~0. A part is left for the next one once its counter has passed its end; whoever finds
+	// that out first sets its bit in `dry`, so that a workgroup that runs out of its own part's jobs reads one
+	// word instead of failing a claim in every other part: eight failed claims of 768 workgroups, one after
+	// another, were 26 us of every launch, that of one job too (a 37-chunk batch: 57 us).
+	__device__ uint32_t next(Counters *ctr) {
+		const uint32_t home = blockIdx.x % kQueues;
+		if (first) {
+			first = false;
+			const uint32_t job = part(home) + blockIdx.x / kQueues;
+			if (job < part(home + 1))
+				return job;
+		}
+		uint32_t dry = 0;
+		for (; tried < kQueues; ++tried) {
+			const uint32_t q = (home + tried) % kQueues, lo = part(q), len = part(q + 1) - lo;
+			const uint32_t given = (gridDim.x - q + kQueues - 1) / kQueues; // its workgroups
+			if (given >= len || ((dry >> q) & 1u))
+				continue;
+			const uint32_t k = given + atomicAdd(&ctr->queue[q].v, 1u);
+			if (k < len)
+				return lo + k;
+			if (k == len)
+				atomicOr(&ctr->dry.v, 1u << q);
+			dry = atomicOr(&ctr->dry.v, 0u);
+		}
+		return ~0u;
+	}
 };
 
 struct MeshParams {

@@ -270,24 +270,12 @@ __global__ __launch_bounds__(256) void light_prep_kernel(LightParams p) {
 
 template <int NT> __global__ __launch_bounds__(NT, 3) void light_kernel(LightParams p) {
 	__shared__ LightSmem s;
-	// part q of the job list is [q * n / kQueues, (q + 1) * n / kQueues): a workgroup takes jobs from
-	// its own XCD's part first, then from the others
-	const uint32_t home = blockIdx.x % kQueues;
-	uint32_t tried = 0; // lane 0 of wavefront 0 only
+	JobClaims claims(p.n_jobs); // lane 0 of wavefront 0 only
 	for (;;) {
 		if (threadIdx.x < 64) { // wavefront 0 claims the next job and loads its slot list and levels
 			uint32_t job = ~0u;
 			if (threadIdx.x == 0) {
-				while (job == ~0u && tried < kQueues) {
-					const uint32_t q = (home + tried) % kQueues;
-					const uint32_t lo = uint32_t(uint64_t(q) * p.n_jobs / kQueues);
-					const uint32_t len = uint32_t(uint64_t(q + 1) * p.n_jobs / kQueues) - lo;
-					const uint32_t k = atomicAdd(&p.ctr->queue[q].v, 1u);
-					if (k < len)
-						job = lo + k;
-					else
-						++tried;
-				}
+				job = claims.next(p.ctr);
 				s.job = job;
 			}
 			job = (uint32_t)__shfl((int)job, 0);
@@ -303,10 +291,10 @@ template <int NT> __global__ __launch_bounds__(NT, 3) void light_kernel(LightPar
 	}
 	// as in the mesh kernel: the last workgroup to finish clears the queues for the next run
 	if (p.self_reset && threadIdx.x == 0) {
-		__threadfence();
 		if (atomicAdd(&p.ctr->done, 1u) == gridDim.x - 1) {
 			for (uint32_t q = 0; q < kQueues; ++q)
 				p.ctr->queue[q].v = 0;
+			p.ctr->dry.v = 0;
 			p.ctr->done = 0;
 		}
 	}
