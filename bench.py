@@ -4,13 +4,13 @@ plus the serving loop's p50/p99 remesh latency.
 Headline workload: the 4096-chunk cave-terrain batch -- a 16x16x16-chunk region (256^3 voxels) plus
 a one-chunk rim, seeded 3D fBm caves under a surface cap, ~15% all-air and ~10% all-stone chunks,
 spatially correlated random sun/torch light. Inputs are resident in HBM before timing. One step =
-one batched meshing pass over all 4096 chunks (HIP-graph replay of counter reset + persistent
+one batched meshing pass over all 4096 chunks (a launch of the persistent
 kernel) with the autotuned workgroup shape. Output is checked bit-exact against the digests the
 reference mesher produced for the same chunks.
 
 More legs go into the same JSON line:
   mixed_batches  200 batches of log-uniform size in [1, 4096] drawn from the cave region and a
-                 plant-covered terrain region: captured-graph runs vs per-chunk launches, bit-exact;
+                 plant-covered terrain region: persistent launches vs per-chunk launches, bit-exact;
   serving        a spiral load trace (radius 24 columns x 16 chunks, ~29k terrain chunks, Poisson
                  arrivals at 20k chunks/s) with concurrent single-voxel edits at 2k/s through the
                  continuous-batching server (16 GB vertex pool): p50/p99 request latency; also with the
@@ -162,7 +162,7 @@ def workloads_slice(blocks, light, nbr, j):
 def relight_leg(ctx, hcm, workloads, meshdigest, steps, cpu_threads, with_cpu, order="linear"):
     """The whole mesh task on the lit cave region (the cave region with glowstone in 0.05% of its air and
     sunlight heights from its columns): light rebuilt from blocks and heights (ChunkMeshTask.cpp:48-111),
-    then meshing, one captured graph per step, with the job order the tuner chose for the cave batch
+    then meshing, three launches per step, with the job order the tuner chose for the cave batch
     (both kernels cut the job list into per-XCD parts). Bit-exact against the reference's mesh digests."""
     import hashlib
 
@@ -293,8 +293,8 @@ def percentile(a, q):
 
 
 def mixed_leg(ctx, hcm, workloads, meshdigest, golden):
-    """Uneven batches: a new batch's first run (cold: launched directly, wall time), its graph replay (warm,
-    captured on the second run, HIP-event time), and per-chunk launches of the same jobs."""
+    """Uneven batches: a new batch's first run (cold, wall time), a further run (warm,
+    HIP-event time), and per-chunk launches of the same jobs."""
     blocks, light, nbr, _ = workloads.mixed_pool()
     want = np.concatenate([golden["cave_region_digest"], golden["terrain_plants_region_digest"]])
     store = hcm.Store(ctx, blocks.shape[0])
@@ -463,7 +463,7 @@ def main():
     batch.sync()
 
     log(f"timing {args.steps} steps")
-    # the timed region: K graph replays back to back, bracketed by device synchronisation on the host
+    # the timed region: K launches back to back, bracketed by device synchronisation on the host
     # and by HIP events on the context's stream (the kernel time per launch is their time over K)
     batch.sync()
     t0 = time.perf_counter()

@@ -1,8 +1,8 @@
 // hcm_api.cpp -- host side of the C ABI declared in include/hcm.h.
 //
-// Owns device memory (registry tables, quad pools, chunk stores, job tables, depth hierarchies), the HIP
-// stream each context works on, and the HIP graph that replays the batched pipeline (the light rebuild
-// when asked for, then the persistent meshing kernel; both clear their own counters). Kernels live in
+// Owns device memory (registry tables, quad pools, chunk stores, job tables, depth hierarchies) and the HIP
+// stream each context works on, and launches the batched pipeline (the light rebuild when asked for, then the
+// persistent meshing kernel; both clear their own counters). Kernels live in
 // hcm_kernels.hip, hcm_light.hip and hcm_draw.hip.
 #include <hip/hip_runtime.h>
 
@@ -287,15 +287,11 @@ struct hcm_batch {
 	hcm_mesh_rec *d_recs = nullptr;
 	hcm_job_result *d_res = nullptr;
 	hipEvent_t ev0 = nullptr, ev1 = nullptr;
-	hipGraph_t graph = nullptr;
-	hipGraphExec_t graph_exec = nullptr;
-	uint32_t graph_threads = 0, graph_grid = 0;
 	uint32_t last_mode = 0;
 	bool ran = false;
 	bool ctr_clean = false; // the counters are zero: a persistent run needs no reset kernel
-	bool launched = false;  // a persistent run has been launched directly: the next one captures the graph
 	// light rebuild (HCM_LIGHT_REBUILD)
-	uint32_t light_mode = HCM_LIGHT_STORE, graph_light = HCM_LIGHT_STORE;
+	uint32_t light_mode = HCM_LIGHT_STORE;
 	uint32_t n_read_slots = 0;
 	uint32_t *d_read_slots = nullptr; // the distinct store slots the jobs read
 	Counters *d_lctr = nullptr;
@@ -919,10 +915,6 @@ extern "C" void hcm_batch_destroy(hcm_batch *b) {
 		return;
 	if (b->ctx && b->ctx->stream)
 		(void)hipStreamSynchronize(b->ctx->stream);
-	if (b->graph_exec)
-		(void)hipGraphExecDestroy(b->graph_exec);
-	if (b->graph)
-		(void)hipGraphDestroy(b->graph);
 	if (b->ev0)
 		(void)hipEventDestroy(b->ev0);
 	if (b->ev1)
@@ -988,7 +980,10 @@ static hipError_t enqueue_light(hcm_batch *b, hipStream_t st) {
 	return e;
 }
 
-// `times` graph replays back to back between the timing events (persistent runs after the first)
+// `times` persistent passes back to back between the timing events. Each is launched directly: a graph of the
+// same one or three kernels, replayed, took 5 us longer per pass back to back (4,096 cave chunks 86.2 against
+// 81.0 us, 37 plant chunks 46.1 against 41.2, with the light rebuild 327.5 against 321.8) and 10 to 20 us longer
+// alone.
 static int batch_run(hcm_batch *b, uint32_t mode, uint32_t times) {
 	if (!b || (mode != HCM_RUN_PERSISTENT && mode != HCM_RUN_PER_CHUNK))
 		return HCM_ERR_INVALID;
@@ -999,47 +994,19 @@ static int batch_run(hcm_batch *b, uint32_t mode, uint32_t times) {
 	hipStream_t st = c->stream;
 	const uint32_t threads = c->tuning.threads;
 	MeshParams p = batch_params(b);
-	const uint32_t grid = std::min((uint32_t)persistent_grid(c, threads), b->n_jobs);
-	if (mode == HCM_RUN_PERSISTENT && !b->launched) {
-		// first persistent run: launched directly, since capturing and instantiating a graph costs more
-		// than the launches it replaces; the graph is captured when the batch runs again
-		if (!b->ctr_clean)
-			HCM_HIP(launch_reset(b->d_ctr, st));
-		HCM_HIP(hipEventRecord(b->ev0, st));
-		if (b->light_mode == HCM_LIGHT_REBUILD)
-			HCM_HIP(enqueue_light(b, st));
-		p.persistent = 1;
-		p.self_reset = 1;
-		HCM_HIP(launch_mesh(p, (int)threads, (int)grid, st));
-		HCM_HIP(hipEventRecord(b->ev1, st));
-		b->ctr_clean = true;
-		b->launched = true;
-	} else if (mode == HCM_RUN_PERSISTENT) {
-		if (!b->graph_exec || b->graph_threads != threads || b->graph_grid != grid || b->graph_light != b->light_mode) {
-			if (b->graph_exec)
-				(void)hipGraphExecDestroy(b->graph_exec), b->graph_exec = nullptr;
-			if (b->graph)
-				(void)hipGraphDestroy(b->graph), b->graph = nullptr;
-			p.persistent = 1;
-			p.self_reset = 1; // the counters start at zero and the run's last workgroup zeroes them again
-			HCM_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-			hipError_t e1 = b->light_mode == HCM_LIGHT_REBUILD ? enqueue_light(b, st) : hipSuccess;
-			hipError_t e2 = e1 == hipSuccess ? launch_mesh(p, (int)threads, (int)grid, st) : hipSuccess;
-			hipError_t e3 = hipStreamEndCapture(st, &b->graph);
-			if (e1 != hipSuccess || e2 != hipSuccess || e3 != hipSuccess) {
-				g_last_hip = (int)(e1 != hipSuccess ? e1 : (e2 != hipSuccess ? e2 : e3));
-				return HCM_ERR_HIP;
-			}
-			HCM_HIP(hipGraphInstantiate(&b->graph_exec, b->graph, nullptr, nullptr, 0));
-			b->graph_threads = threads;
-			b->graph_grid = grid;
-			b->graph_light = b->light_mode;
-		}
+	if (mode == HCM_RUN_PERSISTENT) {
 		if (!b->ctr_clean) // after per-chunk launches
 			HCM_HIP(launch_reset(b->d_ctr, st));
+		b->ctr_clean = false;
+		p.persistent = 1;
+		p.self_reset = 1; // the counters start at zero and the run's last workgroup zeroes them again
+		const int grid = (int)std::min((uint32_t)persistent_grid(c, threads), b->n_jobs);
 		HCM_HIP(hipEventRecord(b->ev0, st));
-		for (uint32_t k = 0; k < times; ++k)
-			HCM_HIP(hipGraphLaunch(b->graph_exec, st));
+		for (uint32_t k = 0; k < times; ++k) {
+			if (b->light_mode == HCM_LIGHT_REBUILD)
+				HCM_HIP(enqueue_light(b, st));
+			HCM_HIP(launch_mesh(p, (int)threads, grid, st));
+		}
 		HCM_HIP(hipEventRecord(b->ev1, st));
 		b->ctr_clean = true;
 	} else {
@@ -1067,11 +1034,6 @@ extern "C" int hcm_batch_run(hcm_batch *b, uint32_t mode) { return batch_run(b, 
 extern "C" int hcm_batch_run_repeat(hcm_batch *b, uint32_t times) {
 	if (!b || times == 0)
 		return HCM_ERR_INVALID;
-	if (!b->launched) { // the first persistent run is a direct launch
-		const int r = batch_run(b, HCM_RUN_PERSISTENT, 1);
-		if (r != HCM_OK || --times == 0)
-			return r;
-	}
 	return batch_run(b, HCM_RUN_PERSISTENT, times);
 }
 

@@ -212,7 +212,7 @@ int hcm_mesh_halos_noalloc(hcm_ctx *ctx, const uint16_t *halo_blocks, const uint
 
 typedef struct hcm_batch hcm_batch;
 
-#define HCM_RUN_PERSISTENT 0u /* one persistent launch with a work queue, replayed as a HIP graph */
+#define HCM_RUN_PERSISTENT 0u /* one persistent launch with a work queue */
 #define HCM_RUN_PER_CHUNK 1u  /* one kernel launch per chunk (the plain per-chunk path) */
 
 /* A batch of n_jobs chunk jobs over a store: nbr holds 27 slot indices per job (host array, copied
@@ -223,7 +223,7 @@ void hcm_batch_destroy(hcm_batch *batch);
 int hcm_batch_run(hcm_batch *batch, uint32_t mode);
 /* Enqueues `times` persistent passes back to back, as many calls of hcm_batch_run(batch,
  * HCM_RUN_PERSISTENT) would (each pass's output replaces the previous one's); hcm_batch_sync then gives
- * the HIP-event time of all of them but a batch's first pass, which is launched on its own. A throughput
+ * the HIP-event time of all of them. A throughput
  * form for repeated meshing of resident chunks; no counterpart in the reference. Asynchronous. */
 int hcm_batch_run_repeat(hcm_batch *batch, uint32_t times);
 /* Waits for the last run; *kernel_ms receives the HIP-event time of its kernels (with HCM_LIGHT_REBUILD
