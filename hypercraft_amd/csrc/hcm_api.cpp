@@ -193,23 +193,24 @@ constexpr uint32_t kPlainRecs = 64;
 // a lone workgroup has the GPU to itself, so more lanes per chunk shorten it (cave chunks: 23.9 us at 512
 // threads, 27.7 us at 256, 37.3 us at 128). The persistent batch keeps its tuned shape.
 constexpr int kChunkLaunchThreads = 512;
-// A one-chunk call copies back this many quads with its result, records and vertices in one go; a chunk
-// with more takes a second round trip.
-constexpr uint32_t kPlainFastQuads = 2048;
+// One-chunk calls read their input from pinned host memory and write their result, records and quads there, so
+// that such a call is one launch and one synchronisation (with the light rebuild three launches): with copies
+// each way beside the launches a cave chunk took 71 us. Chunks of more quads than this are meshed again
+// into the context's device buffers and copied.
+constexpr uint32_t kPlainFastQuads = 8192;
 constexpr size_t kHaloBytes = HCM_HALO_BLOCKS * 2 + HCM_HALO_LIGHT;
 constexpr size_t kPoutRecs = 64, kPoutVerts = 64 + kPlainRecs * sizeof(hcm_mesh_rec);
 constexpr size_t kPoutIdx = kPoutVerts + kPlainFastQuads * 4 * sizeof(uint2);
-constexpr size_t kPoutBytes = kPoutIdx + kPlainFastQuads * 6 * 2;
+constexpr size_t kPoutLight = kPoutIdx + kPlainFastQuads * 6 * 2;
+constexpr size_t kPoutBytes = kPoutLight + kLightJobBytes;
+static_assert(kPoutVerts % 16 == 0 && kPoutIdx % 16 == 0 && kPoutLight % 4 == 0 && HCM_HALO_BLOCKS * 2 % 16 == 0,
+              "aligned for the kernels' widest stores and loads");
 
 // Scratch of hcm_mesh_halos_noalloc: the device memory its kernels use beyond the caller's inputs and
-// outputs -- work counters, the job table (job j reads slots 27 j .. 27 j + 26) and the 27-slot stores
-// its halos are scattered into -- for at most kNoAllocMaxJobs chunks per call, 2.7 MB. Each GPU holds its
-// own copy from the library's load to the end of the process; calls on one GPU share it.
+// outputs, the work counters. Each GPU holds its own copy from the library's load to the end of the process;
+// calls on one GPU share it.
 constexpr uint32_t kNoAllocMaxJobs = 8;
-constexpr size_t kScratchNbr = (sizeof(Counters) + 255) / 256 * 256;
-constexpr size_t kScratchBlocks = kScratchNbr + (kNoAllocMaxJobs * 27 * 4 + 255) / 256 * 256;
-constexpr size_t kScratchLight = kScratchBlocks + (size_t)kNoAllocMaxJobs * 27 * HCM_CHUNK_VOXELS * 2;
-constexpr size_t kScratchBytes = kScratchLight + (size_t)kNoAllocMaxJobs * 27 * HCM_CHUNK_VOXELS;
+constexpr size_t kScratchBytes = sizeof(Counters);
 static __device__ __align__(256) uint8_t scratch[kScratchBytes];
 static_assert(kNoAllocMaxJobs == HCM_NOALLOC_MAX_CHUNKS, "documented limit");
 
@@ -236,29 +237,22 @@ struct hcm_ctx {
 	uint16_t *d_idx = nullptr;
 	// plain path
 	uint16_t *d_pblocks = nullptr;
-	uint8_t *d_plight = nullptr;
 	uint32_t *d_pnbr = nullptr;
-	Counters *d_pctr = nullptr;
 	uint2 *d_pverts = nullptr;
 	uint16_t *d_pidx = nullptr;
 	hcm_mesh_rec *d_precs = nullptr;
-	hcm_job_result *d_pres = nullptr;
 	uint16_t *h_pblocks = nullptr; // pinned staging
-	uint8_t *h_plight = nullptr;
-	// plain path from a packed halo: the halo on the device and in pinned memory, and a pinned copy of
-	// the result, the mesh records and the first kPlainFastQuads quads
-	uint8_t *d_halo_in = nullptr;
+	// pinned memory that the one-chunk calls' kernels read and write: the packed halo, and the result, the mesh
+	// records, up to kPlainFastQuads quads and the rebuilt light
 	uint8_t *h_halo_in = nullptr;
 	uint8_t *h_pout = nullptr;
 	// this device's copy of `scratch` (hcm_mesh_halos_noalloc); host code uses this address, never the
 	// array's name, which on the host is only a stand-in
 	uint8_t *d_scratch = nullptr;
 	// plain path light rebuild
-	int8_t *d_pheights = nullptr;
 	int8_t *h_pheights = nullptr;
 	uint16_t *d_ppacked = nullptr;
 	uint32_t *d_plevels = nullptr;
-	Counters *d_plctr = nullptr;
 	uint8_t *d_phalo = nullptr;
 	// depth hierarchy for occlusion culling (hcm_ctx_set_depth)
 	float *d_depth = nullptr;
@@ -339,26 +333,18 @@ static void free_ctx(hcm_ctx *c) {
 	dfree(c->d_verts);
 	dfree(c->d_idx);
 	dfree(c->d_pblocks);
-	dfree(c->d_plight);
 	dfree(c->d_pnbr);
-	dfree(c->d_pctr);
 	dfree(c->d_pverts);
 	dfree(c->d_pidx);
 	dfree(c->d_precs);
-	dfree(c->d_pres);
 	if (c->h_pblocks)
 		(void)hipHostFree(c->h_pblocks);
-	if (c->h_plight)
-		(void)hipHostFree(c->h_plight);
-	dfree(c->d_halo_in);
 	if (c->h_halo_in)
 		(void)hipHostFree(c->h_halo_in);
 	if (c->h_pout)
 		(void)hipHostFree(c->h_pout);
-	dfree(c->d_pheights);
 	dfree(c->d_ppacked);
 	dfree(c->d_plevels);
-	dfree(c->d_plctr);
 	dfree(c->d_phalo);
 	dfree(c->d_depth);
 	if (c->h_pheights)
@@ -419,35 +405,23 @@ static int create_impl(hcm_ctx *c, const hcm_registry *registry, uint64_t pool_q
 		HCM_HIP(dmalloc(&c->d_idx, (size_t)c->pool_quads * 6));
 	}
 	HCM_HIP(dmalloc(&c->d_pblocks, 27 * HCM_CHUNK_VOXELS));
-	HCM_HIP(dmalloc(&c->d_plight, 27 * HCM_CHUNK_VOXELS));
 	HCM_HIP(dmalloc(&c->d_pnbr, 27));
-	HCM_HIP(dmalloc(&c->d_pctr, 1));
 	HCM_HIP(dmalloc(&c->d_pverts, (size_t)kPlainPoolQuads * 4));
 	HCM_HIP(dmalloc(&c->d_pidx, (size_t)kPlainPoolQuads * 6));
 	HCM_HIP(dmalloc(&c->d_precs, kPlainRecs));
-	HCM_HIP(dmalloc(&c->d_pres, 1));
 	HCM_HIP(hipHostMalloc(reinterpret_cast<void **>(&c->h_pblocks), 27 * HCM_CHUNK_VOXELS * 2));
-	HCM_HIP(hipHostMalloc(reinterpret_cast<void **>(&c->h_plight), 27 * HCM_CHUNK_VOXELS));
-	HCM_HIP(dmalloc(&c->d_halo_in, kHaloBytes));
 	HCM_HIP(hipHostMalloc(reinterpret_cast<void **>(&c->h_halo_in), kHaloBytes));
 	HCM_HIP(hipHostMalloc(reinterpret_cast<void **>(&c->h_pout), kPoutBytes));
-	HCM_HIP(dmalloc(&c->d_pheights, 27 * 256));
 	HCM_HIP(hipHostMalloc(reinterpret_cast<void **>(&c->h_pheights), 27 * 256));
 	HCM_HIP(dmalloc(&c->d_ppacked, 27 * kLightPlanes * 256));
 	HCM_HIP(dmalloc(&c->d_plevels, 27));
-	HCM_HIP(dmalloc(&c->d_plctr, 1));
 	HCM_HIP(dmalloc(&c->d_phalo, kLightJobBytes));
 	uint32_t ident[27];
 	for (uint32_t i = 0; i < 27; ++i)
 		ident[i] = i;
 	HCM_HIP(hipMemcpy(c->d_pnbr, ident, sizeof(ident), hipMemcpyHostToDevice));
-	// the no-allocation entry point's scratch on this (current) device, and its constant job table; every
-	// context on the device writes the same table
+	// the no-allocation entry point's scratch on this (current) device
 	HCM_HIP(hipGetSymbolAddress(reinterpret_cast<void **>(&c->d_scratch), HIP_SYMBOL(scratch)));
-	uint32_t jobs[kNoAllocMaxJobs * 27];
-	for (uint32_t i = 0; i < kNoAllocMaxJobs * 27; ++i)
-		jobs[i] = i;
-	HCM_HIP(hipMemcpy(c->d_scratch + kScratchNbr, jobs, sizeof(jobs), hipMemcpyHostToDevice));
 	return HCM_OK;
 }
 
@@ -562,47 +536,39 @@ static int fetch_job(hipStream_t stream, const hcm_job_result &res, const hcm_me
 	return HCM_OK;
 }
 
-// One chunk from the packed halo in ctx->h_halo_in (context lock held): one upload, the halo scattered into
-// the plain path's 27 slots on the device, one meshing workgroup, then the result, the mesh records and
-// the first kPlainFastQuads quads copied back together; the meshes of such a chunk are assembled from that
-// copy after one synchronisation, a larger chunk's are fetched mesh by mesh.
-static int mesh_halo_locked(hcm_ctx *ctx, hcm_host_result *out) {
+// Meshes the one job of p (its input filled in, context lock held) into the context's pinned output and
+// assembles the meshes from there after one synchronisation; a chunk that does not fit it is meshed again into
+// the device buffers and fetched mesh by mesh.
+static int mesh_alone(hcm_ctx *ctx, MeshParams &p, hcm_host_result *out) {
 	hipStream_t st = ctx->stream;
-	HCM_HIP(hipMemcpyAsync(ctx->d_halo_in, ctx->h_halo_in, kHaloBytes, hipMemcpyHostToDevice, st));
-	HCM_HIP(launch_halo_unpack(reinterpret_cast<const uint16_t *>(ctx->d_halo_in), ctx->d_halo_in + HCM_HALO_BLOCKS * 2,
-	                           1, ctx->d_pblocks, ctx->d_plight, st));
-	HCM_HIP(launch_reset(ctx->d_pctr, st));
-	MeshParams p = base_params(ctx);
-	p.blocks = ctx->d_pblocks;
-	p.light = ctx->d_plight;
-	p.nbr = ctx->d_pnbr;
+	uint8_t *po = ctx->h_pout;
 	p.n_jobs = 1;
 	p.job_base = 0;
 	p.persistent = 0;
-	p.pool_cap = kPlainPoolQuads;
-	p.ctr = ctx->d_pctr;
-	p.pool_verts = ctx->d_pverts;
-	p.pool_idx = ctx->d_pidx;
-	p.recs = ctx->d_precs;
+	p.alone = 1;
+	p.pool_cap = kPlainFastQuads;
+	p.pool_verts = reinterpret_cast<uint2 *>(po + kPoutVerts);
+	p.pool_idx = reinterpret_cast<uint16_t *>(po + kPoutIdx);
+	p.recs = reinterpret_cast<hcm_mesh_rec *>(po + kPoutRecs);
 	p.rec_cap = kPlainRecs;
-	p.results = ctx->d_pres;
+	p.results = reinterpret_cast<hcm_job_result *>(po);
 	HCM_HIP(launch_mesh(p, kChunkLaunchThreads, 1, st));
-	uint8_t *po = ctx->h_pout;
-	HCM_HIP(hipMemcpyAsync(po, ctx->d_pres, sizeof(hcm_job_result), hipMemcpyDeviceToHost, st));
-	HCM_HIP(hipMemcpyAsync(po + kPoutRecs, ctx->d_precs, kPlainRecs * sizeof(hcm_mesh_rec), hipMemcpyDeviceToHost, st));
-	HCM_HIP(hipMemcpyAsync(po + kPoutVerts, ctx->d_pverts, kPlainFastQuads * 4 * sizeof(uint2), hipMemcpyDeviceToHost, st));
-	HCM_HIP(hipMemcpyAsync(po + kPoutIdx, ctx->d_pidx, kPlainFastQuads * 6 * 2, hipMemcpyDeviceToHost, st));
 	HCM_HIP(hipStreamSynchronize(st));
 	hcm_job_result res;
 	std::memcpy(&res, po, sizeof(res));
+	if (res.status == HCM_ERR_POOL_FULL) {
+		p.pool_cap = kPlainPoolQuads;
+		p.pool_verts = ctx->d_pverts;
+		p.pool_idx = ctx->d_pidx;
+		p.recs = ctx->d_precs;
+		HCM_HIP(launch_mesh(p, kChunkLaunchThreads, 1, st));
+		HCM_HIP(hipStreamSynchronize(st));
+		std::memcpy(&res, po, sizeof(res));
+		return fetch_job(st, res, ctx->d_precs, ctx->d_pverts, ctx->d_pidx, out);
+	}
 	if (res.status != HCM_OK)
 		return res.status;
 	const hcm_mesh_rec *recs = reinterpret_cast<const hcm_mesh_rec *>(po + kPoutRecs);
-	bool fits = res.first_mesh + res.mesh_count <= kPlainRecs;
-	for (uint32_t m = 0; fits && m < res.mesh_count; ++m)
-		fits = (uint64_t)recs[res.first_mesh + m].first_quad + recs[res.first_mesh + m].quad_count <= kPlainFastQuads;
-	if (!fits)
-		return fetch_job(st, res, ctx->d_precs, ctx->d_pverts, ctx->d_pidx, out);
 	uint64_t nv = 0, ni = 0;
 	for (uint32_t m = 0; m < res.mesh_count; ++m)
 		nv += 4ull * recs[res.first_mesh + m].quad_count, ni += 6ull * recs[res.first_mesh + m].quad_count;
@@ -629,6 +595,14 @@ static int mesh_halo_locked(hcm_ctx *ctx, hcm_host_result *out) {
 	return HCM_OK;
 }
 
+// One chunk from the packed halo in ctx->h_halo_in (context lock held).
+static int mesh_halo_locked(hcm_ctx *ctx, hcm_host_result *out) {
+	MeshParams p = base_params(ctx);
+	p.halo_in = reinterpret_cast<const uint16_t *>(ctx->h_halo_in);
+	p.halo_in_light = ctx->h_halo_in + HCM_HALO_BLOCKS * 2;
+	return mesh_alone(ctx, p, out);
+}
+
 extern "C" int hcm_mesh_halo(hcm_ctx *ctx, const uint16_t *blocks, const uint8_t *light, hcm_host_result *out) {
 	if (!ctx || !blocks || !light || !out)
 		return HCM_ERR_INVALID;
@@ -650,17 +624,15 @@ extern "C" int hcm_mesh_halos_noalloc(hcm_ctx *ctx, const uint16_t *halo_blocks,
 		return HCM_ERR_INVALID;
 	hipStream_t st = reinterpret_cast<hipStream_t>(stream);
 	Counters *ctr = reinterpret_cast<Counters *>(ctx->d_scratch);
-	uint16_t *blocks = reinterpret_cast<uint16_t *>(ctx->d_scratch + kScratchBlocks);
-	uint8_t *light = ctx->d_scratch + kScratchLight;
-	HCM_HIP(launch_halo_unpack(halo_blocks, halo_light, n, blocks, light, st));
-	HCM_HIP(launch_reset(ctr, st)); // a kernel, not a memset, so that a captured graph replays it correctly
+	if (n > 1)
+		HCM_HIP(launch_reset(ctr, st)); // a kernel, not a memset, so that a captured graph replays it correctly
 	MeshParams p = base_params(ctx);
-	p.blocks = blocks;
-	p.light = light;
-	p.nbr = reinterpret_cast<const uint32_t *>(ctx->d_scratch + kScratchNbr);
+	p.halo_in = halo_blocks;
+	p.halo_in_light = halo_light;
 	p.n_jobs = n;
 	p.job_base = 0;
 	p.persistent = 0;
+	p.alone = n == 1;
 	p.pool_cap = quad_cap;
 	p.ctr = ctr;
 	p.pool_verts = reinterpret_cast<uint2 *>(vertices);
@@ -718,13 +690,13 @@ extern "C" int hcm_mesh_chunk_relight(hcm_ctx *ctx, const uint16_t *const blocks
 		std::memcpy(ctx->h_pheights + (size_t)i * 256, heights[i], 256);
 	}
 	hipStream_t st = ctx->stream;
-	HCM_HIP(hipMemcpyAsync(ctx->d_pblocks, ctx->h_pblocks, 27 * HCM_CHUNK_VOXELS * 2, hipMemcpyHostToDevice, st));
-	HCM_HIP(hipMemcpyAsync(ctx->d_pheights, ctx->h_pheights, 27 * 256, hipMemcpyHostToDevice, st));
-	// light rebuild of the one job (slots 0..26 in neighbour-slot order)
+	// light rebuild of the one job (slots 0..26 in neighbour-slot order); the packing pass reads the pinned
+	// blocks and leaves them on the device for the mesher
 	LightParams lp;
 	std::memset(&lp, 0, sizeof(lp));
-	lp.blocks = ctx->d_pblocks;
-	lp.heights = ctx->d_pheights;
+	lp.blocks = ctx->h_pblocks;
+	lp.blocks_copy = ctx->d_pblocks;
+	lp.heights = ctx->h_pheights;
 	lp.light_info = ctx->d_light_info;
 	lp.slots = ctx->d_pnbr;
 	lp.n_slots = 27;
@@ -732,41 +704,20 @@ extern "C" int hcm_mesh_chunk_relight(hcm_ctx *ctx, const uint16_t *const blocks
 	lp.packed = ctx->d_ppacked;
 	lp.levels = ctx->d_plevels;
 	lp.nbr = ctx->d_pnbr;
-	lp.ctr = ctx->d_plctr;
 	lp.halo_light = ctx->d_phalo;
-	HCM_HIP(launch_reset(ctx->d_plctr, st));
+	lp.halo_light_copy = light_out ? ctx->h_pout + kPoutLight : nullptr;
 	HCM_HIP(launch_light_prep(lp, st));
-	HCM_HIP(launch_light(lp, 1, st));
+	HCM_HIP(launch_light(lp, 1, st)); // one workgroup has its one job without a claim
 	// meshing over the rebuilt light
-	HCM_HIP(launch_reset(ctx->d_pctr, st));
 	MeshParams p = base_params(ctx);
 	p.blocks = ctx->d_pblocks;
-	p.light = ctx->d_plight;
 	p.halo_light = ctx->d_phalo;
 	p.nbr = ctx->d_pnbr;
-	p.n_jobs = 1;
-	p.job_base = 0;
-	p.persistent = 0;
-	p.pool_cap = kPlainPoolQuads;
-	p.ctr = ctx->d_pctr;
-	p.pool_verts = ctx->d_pverts;
-	p.pool_idx = ctx->d_pidx;
-	p.recs = ctx->d_precs;
-	p.rec_cap = kPlainRecs;
-	p.results = ctx->d_pres;
-	HCM_HIP(launch_mesh(p, kChunkLaunchThreads, 1, st));
-	hcm_job_result res;
-	HCM_HIP(hipMemcpyAsync(&res, ctx->d_pres, sizeof(res), hipMemcpyDeviceToHost, st));
-	std::vector<uint8_t> rows;
-	if (light_out) {
-		rows.resize(kLightJobBytes);
-		HCM_HIP(hipMemcpyAsync(rows.data(), ctx->d_phalo, kLightJobBytes, hipMemcpyDeviceToHost, st));
-	}
-	HCM_HIP(hipStreamSynchronize(st));
-	if (light_out)
-		for (uint32_t r = 0; r < 18 * 18; ++r) // row hz + 18 hy holds x = -1 .. 16
-			std::memcpy(light_out + 18 * r, rows.data() + r * kLightRowBytes, 18);
-	return fetch_job(st, res, ctx->d_precs, ctx->d_pverts, ctx->d_pidx, out);
+	const int r = mesh_alone(ctx, p, out);
+	if (light_out && r != HCM_ERR_HIP)
+		for (uint32_t k = 0; k < 18 * 18; ++k) // row hz + 18 hy holds x = -1 .. 16
+			std::memcpy(light_out + 18 * k, ctx->h_pout + kPoutLight + k * kLightRowBytes, 18);
+	return r;
 }
 
 // ------------------------------------------------------------------------------------------------

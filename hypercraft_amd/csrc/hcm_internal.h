@@ -86,10 +86,16 @@ struct JobClaims {
 	// word instead of failing a claim in every other part: eight failed claims of 768 workgroups, one after
 	// another, were 26 us of every launch, that of one job too (a 37-chunk batch: 57 us).
 	__device__ uint32_t next(Counters *ctr) {
-		const uint32_t home = blockIdx.x % kQueues;
+		const uint32_t home = blockIdx.x % kQueues, turn = blockIdx.x / kQueues;
+		if (gridDim.x >= n_jobs) { // one job each: parts as long as the XCDs have workgroups, and no claims
+			const uint32_t len = n_jobs / kQueues, more = n_jobs % kQueues; // the first `more` parts hold one more
+			const bool mine = first && turn < len + (home < more ? 1u : 0u);
+			first = false;
+			return mine ? home * len + min(home, more) + turn : ~0u;
+		}
 		if (first) {
 			first = false;
-			const uint32_t job = part(home) + blockIdx.x / kQueues;
+			const uint32_t job = part(home) + turn;
 			if (job < part(home + 1))
 				return job;
 		}
@@ -128,6 +134,11 @@ struct MeshParams {
 	hcm_job_result *results;
 	// [n_jobs][kLightJobBytes]: each job's rebuilt light over its halo, or null: light from the store
 	const uint8_t *halo_light;
+	// Packed halos (include/hcm.h), job j's at j HCM_HALO_BLOCKS and j HCM_HALO_LIGHT, instead of a store (null:
+	// the store). Launches of 512 threads. Any alignment, device or pinned host memory.
+	const uint16_t *halo_in;
+	const uint8_t *halo_in_light;
+	uint32_t alone; // the launch's one job: its output starts at quad and record 0, the counters are not touched
 };
 
 // ---- light rebuild before meshing (client/src/ChunkMeshTask.cpp:48-111) ----
@@ -152,6 +163,8 @@ struct LightParams {
 	const uint32_t *nbr;       // 27 slots per job
 	Counters *ctr;             // work queues of the persistent light kernel
 	uint8_t *halo_light;       // [n_jobs][kLightJobBytes]
+	uint8_t *halo_light_copy;  // a second copy of the same, or null
+	uint16_t *blocks_copy;     // the packed slots' blocks as the packing pass read them, or null: slot * 4096 + local
 	uint32_t self_reset;       // the last workgroup to finish clears the work queues (no reset kernel)
 };
 
@@ -164,8 +177,6 @@ struct VoxelEdit {
 // Launchers (hcm_kernels.hip)
 hipError_t launch_reset(Counters *ctr, hipStream_t stream);
 hipError_t launch_mesh(const MeshParams &p, int threads, int grid, hipStream_t stream);
-hipError_t launch_halo_unpack(const uint16_t *hblocks, const uint8_t *hlight, uint32_t n, uint16_t *blocks,
-                              uint8_t *light, hipStream_t stream);
 // staged chunk k (sblocks + 4096 k, and slight + 4096 k or sheights + 256 k; the unused one null) to store
 // slot moves[i].y for k = moves[i].x, i < n; all arrays 16-byte aligned
 hipError_t launch_upload_scatter(const uint16_t *sblocks, const uint8_t *slight, const int8_t *sheights,

@@ -135,17 +135,25 @@ __device__ __forceinline__ int hidx(int x, int y, int z) { return (x + 1) * kSX 
 
 template <int NT> struct Smem {
 	uint32_t vox[kHaloVox];
-	// a mask row of 16 faces per task and row, row 16 t + u: visible faces; equal-to-right faces, then the
-	// faces where a quad starts; equal-to-below faces, then the uncovered visible ones
-	alignas(16) uint16_t ne[kMaskRows];
-	alignas(16) uint16_t eh[kMaskRows];
-	alignas(16) uint16_t ev[kMaskRows];
 	union {
-		uint2 key[kListCap]; // face words of the current group of tasks, in dense order
-		struct {             // until the visibility masks are made: the halo rows' face classes as bit planes
-			uint4 planes[kHaloRows];  // of the y faces, then the z faces (row_planes)
-			uint32_t vis_x[256], tt_x[256]; // per chunk row: its visible x faces and those to compare (show_rows)
+		struct {
+			// a mask row of 16 faces per task and row, row 16 t + u: visible faces; equal-to-right faces, then
+			// the faces where a quad starts; equal-to-below faces, then the uncovered visible ones
+			alignas(16) uint16_t ne[kMaskRows];
+			alignas(16) uint16_t eh[kMaskRows];
+			alignas(16) uint16_t ev[kMaskRows];
+			union {
+				uint2 key[kListCap]; // face words of the current group of tasks, in dense order
+				struct {             // until the visibility masks are made: the halo rows' face classes as bit planes
+					uint4 planes[kHaloRows];  // of the y faces, then the z faces (row_planes)
+					uint32_t vis_x[256], tt_x[256]; // per chunk row: its visible x faces and those to compare
+				};
+			};
 		};
+		struct { // while a packed halo is staged: its bytes
+			alignas(16) uint16_t blocks[HCM_HALO_BLOCKS];
+			alignas(8) uint8_t light[HCM_HALO_LIGHT];
+		} halo;
 	};
 	alignas(16) uint16_t own[kListCap]; // per face of the group: 1 + its unit where one begins, else 0; then its descriptor
 	uint16_t upre[kUnits + 2]; // visible faces before each unit (the dense face order; at most 24,576), and in all
@@ -353,9 +361,17 @@ struct Flow {
 
 __device__ __forceinline__ uint32_t flow_h(const Flow &f, int i) { return (f.h >> (8 * i)) & 0xffu; }
 
-__device__ __forceinline__ uint16_t global_block(const MeshParams &p, const uint32_t *slots, int x, int y, int z) {
-	return p.blocks[(size_t)slots[slot27(x, y, z)] * HCM_CHUNK_VOXELS + local16(x, y, z)];
-}
+// Where a job's blocks are in global memory: the store's slots, or its packed halo.
+struct JobBlocks {
+	const uint16_t *store;  // p.blocks
+	const uint32_t *slots;  // s.slots
+	const uint16_t *halo;   // null: the store
+	__device__ __forceinline__ uint16_t at(int x, int y, int z) const {
+		if (halo)
+			return halo[(x + 2) + 20 * ((z + 2) + 20 * (y + 1))];
+		return store[(size_t)slots[slot27(x, y, z)] * HCM_CHUNK_VOXELS + local16(x, y, z)];
+	}
+};
 
 // get_nei_height (:164-169) as a signed integer: the reference returns it as int8_t, so a flow level's
 // uint8_t height max(meta * 2, 1) wraps to [-128, 127].
@@ -378,14 +394,14 @@ __device__ __forceinline__ uint32_t flow_vh(int nb, int a, int b, int c) {
 	return (mx != 16u && zeros >= 3) ? 0u : mx;
 }
 
-__device__ __forceinline__ Flow flow_heights(const MeshParams &p, const uint32_t *slots, int x, int y, int z,
+__device__ __forceinline__ Flow flow_heights(const MeshParams &p, const JobBlocks &blocks, int x, int y, int z,
                                           uint32_t nb_height) {
 	const uint32_t src = p.reg.src_id, fid = p.reg.flow_id;
 	// neighbours (:291-300): 0 (-1,-1) 1 (0,-1) 2 (1,-1) 3 (-1,0) 4 (1,0) 5 (-1,1) 6 (0,1) 7 (1,1) in (x, z)
-	const uint32_t b0 = global_block(p, slots, x - 1, y, z - 1), b1 = global_block(p, slots, x, y, z - 1);
-	const uint32_t b2 = global_block(p, slots, x + 1, y, z - 1), b3 = global_block(p, slots, x - 1, y, z);
-	const uint32_t b4 = global_block(p, slots, x + 1, y, z), b5 = global_block(p, slots, x - 1, y, z + 1);
-	const uint32_t b6 = global_block(p, slots, x, y, z + 1), b7 = global_block(p, slots, x + 1, y, z + 1);
+	const uint32_t b0 = blocks.at(x - 1, y, z - 1), b1 = blocks.at(x, y, z - 1);
+	const uint32_t b2 = blocks.at(x + 1, y, z - 1), b3 = blocks.at(x - 1, y, z);
+	const uint32_t b4 = blocks.at(x + 1, y, z), b5 = blocks.at(x - 1, y, z + 1);
+	const uint32_t b6 = blocks.at(x, y, z + 1), b7 = blocks.at(x + 1, y, z + 1);
 	const int n0 = flow_nei_height(b0, src, fid), n1 = flow_nei_height(b1, src, fid);
 	const int n2 = flow_nei_height(b2, src, fid), n3 = flow_nei_height(b3, src, fid);
 	const int n4 = flow_nei_height(b4, src, fid), n5 = flow_nei_height(b5, src, fid);
@@ -486,10 +502,13 @@ __device__ __forceinline__ bool tex_trans_pass(const MeshParams &p, uint16_t t) 
 	return id < p.reg.n_tex && (p.reg.tex_flags[id] & HCM_TEX_TRANS_PASS);
 }
 
-template <int NT> __device__ __forceinline__ CustomCell custom_cell(const MeshParams &p, const Smem<NT> &s, int cell) {
+template <int NT>
+__device__ __forceinline__ CustomCell custom_cell(const MeshParams &p, const Smem<NT> &s, const JobBlocks &blocks, int cell) {
 	const int x = cell & 15, z = (cell >> 4) & 15, y = cell >> 8;
-	const uint16_t b = p.blocks[(size_t)s.slots[26] * HCM_CHUNK_VOXELS + (uint32_t)cell];
-	const uint32_t pid = block_pid(p, s, b);
+	// the voxel word has the block's row but for flow cells, whose words took a row of face textures
+	uint32_t pid = vox_pid(s.vox[hidx(x, y, z)]);
+	if (pid >= p.reg.flow_pid_base)
+		pid = block_pid(p, s, blocks.at(x, y, z));
 	CustomCell c;
 	c.mesh = s.rows[pid].y >> 24;
 	c.flow = (s.pid_vox[pid] & kVoxFlow) ? 1u : 0u;
@@ -498,7 +517,7 @@ template <int NT> __device__ __forceinline__ CustomCell custom_cell(const MeshPa
 	c.fl.h = 0, c.fl.liq_side = 0;
 	const hcm_custom_mesh &m = p.reg.meshes[c.mesh];
 	if (c.flow) {
-		c.fl = flow_heights(p, s.slots, x, y, z, m.flow_height);
+		c.fl = flow_heights(p, blocks, x, y, z, m.flow_height);
 		c.flow_set = flow_face_set(c.fl);
 		c.count = __popc(c.flow_set);
 		if (tex_trans_pass(p, uint16_t(p.reg.flow_tex)))
@@ -613,11 +632,11 @@ __device__ __forceinline__ uint32_t interp(uint32_t l0, uint32_t l1, uint32_t l2
 }
 
 template <int NT>
-__device__ __forceinline__ void emit_custom(const MeshParams &p, Smem<NT> &s, uint32_t desc, uint32_t slot,
+__device__ __forceinline__ void emit_custom(const MeshParams &p, Smem<NT> &s, const JobBlocks &blocks, uint32_t desc, uint32_t slot,
                                          uint32_t vbase, uint32_t lo[3], uint32_t hi[3]) {
 	const int cell = desc & 4095, j = (desc >> 12) & 15;
 	const int x = cell & 15, z = (cell >> 4) & 15, y = cell >> 8;
-	const CustomCell c = custom_cell(p, s, cell);
+	const CustomCell c = custom_cell(p, s, blocks, cell);
 	const hcm_mesh_face f = custom_face(p, c, j);
 	const int lf = f.light_face, la = lf >> 1, sg = (lf & 1) ? -1 : 1;
 	const int pos = hidx(x, y, z);
@@ -1218,6 +1237,66 @@ template <int NT> __device__ __forceinline__ void chunk_init(Smem<NT> &s) {
 		s.n_events = 0, s.flags = 0;
 }
 
+// A packed halo (include/hcm.h, HCM_HALO_BLOCKS / HCM_HALO_LIGHT) into LDS as it is, in whole 16-byte loads
+// where it is aligned (its job's place keeps the alignment of the first: 14,400 and 5,832 bytes a halo), so that
+// each of its lines is read once also where it lies in host memory.
+template <int NT> __device__ __forceinline__ void load_halo(const MeshParams &p, Smem<NT> &s, uint32_t job) {
+	const uint16_t *b = p.halo_in + (size_t)job * HCM_HALO_BLOCKS;
+	const uint8_t *l = p.halo_in_light + (size_t)job * HCM_HALO_LIGHT;
+	const int tid = threadIdx.x;
+	if (((uintptr_t(b) & 15u) | (uintptr_t(l) & 7u)) == 0) {
+		constexpr int nb = HCM_HALO_BLOCKS * 2 / 16, nl = HCM_HALO_LIGHT / 8, kb = (nb + NT - 1) / NT, kl = (nl + NT - 1) / NT;
+		static_assert(nb * 16 == HCM_HALO_BLOCKS * 2 && nl * 8 == HCM_HALO_LIGHT, "whole words");
+		uint4 vb[kb];
+		uint2 vl[kl];
+#pragma unroll
+		for (int k = 0; k < kb; ++k)
+			vb[k] = reinterpret_cast<const uint4 *>(b)[min(tid + k * NT, nb - 1)];
+#pragma unroll
+		for (int k = 0; k < kl; ++k)
+			vl[k] = reinterpret_cast<const uint2 *>(l)[min(tid + k * NT, nl - 1)];
+#pragma unroll
+		for (int k = 0; k < kb; ++k)
+			if (tid + k * NT < nb)
+				reinterpret_cast<uint4 *>(s.halo.blocks)[tid + k * NT] = vb[k];
+#pragma unroll
+		for (int k = 0; k < kl; ++k)
+			if (tid + k * NT < nl)
+				reinterpret_cast<uint2 *>(s.halo.light)[tid + k * NT] = vl[k];
+	} else {
+		for (int i = tid; i < HCM_HALO_BLOCKS; i += NT)
+			s.halo.blocks[i] = b[i];
+		for (int i = tid; i < HCM_HALO_LIGHT; i += NT)
+			s.halo.light[i] = l[i];
+	}
+}
+
+// One halo row of 18 voxels: blocks at x = -1, 0 .. 15 (two per word) and 16, light bytes from x = -1 on.
+struct HaloRow {
+	uint32_t bw[8], bl, br, lw[5];
+};
+template <int NT> __device__ __forceinline__ HaloRow halo_row(const Smem<NT> &s, int row) {
+	// the packed halo's blocks reach from x = -2 to 17: 20 per row, ten words that start at an even word
+	const int hz = row % kHalo, hy = row / kHalo;
+	const uint2 *hb = reinterpret_cast<const uint2 *>(s.halo.blocks + 20 * (hz + 1 + 20 * hy));
+	const uint16_t *hl = reinterpret_cast<const uint16_t *>(s.halo.light + kHalo * row);
+	HaloRow r;
+	uint32_t d[10];
+#pragma unroll
+	for (int k = 0; k < 5; ++k) {
+		const uint2 w = hb[k];
+		d[2 * k] = w.x, d[2 * k + 1] = w.y;
+	}
+	r.bl = d[0] >> 16, r.br = d[9] & 0xffffu;
+#pragma unroll
+	for (int k = 0; k < 8; ++k)
+		r.bw[k] = d[k + 1];
+#pragma unroll
+	for (int k = 0; k < 5; ++k)
+		r.lw[k] = hl[2 * k] | (k < 4 ? uint32_t(hl[2 * k + 1]) << 16 : 0u);
+	return r;
+}
+
 // One job; s.slots and the state of chunk_init are in place (a barrier after them).
 template <int NT> __device__ __forceinline__ void mesh_chunk(const MeshParams &p, Smem<NT> &s, uint32_t job) {
 	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -1228,32 +1307,52 @@ template <int NT> __device__ __forceinline__ void mesh_chunk(const MeshParams &p
 	// changes the texture row); the row's flags come from an AND and an OR over its templates and from
 	// comparing packed block pairs, the custom-mesh cells only when some template has a mesh.
 	uint32_t my_flags = 0, wave_ref = 0xffffffffu;
+	const JobBlocks blocks{p.blocks, s.slots, p.halo_in ? p.halo_in + (size_t)job * HCM_HALO_BLOCKS : nullptr};
+	HaloRow given; // a packed halo's row: one per thread, all read before the first is staged over them
+	if constexpr (NT >= kHaloRows)
+		if (p.halo_in) {
+			load_halo(p, s, job);
+			__syncthreads();
+			if (tid < kHaloRows)
+				given = halo_row(s, tid);
+			__syncthreads();
+		}
 	for (int row = tid; row < kHaloRows; row += NT) {
 		const int hz = row % kHalo, hy = row / kHalo, y = hy - 1, z = hz - 1;
-		const size_t lrow = 16u * (uint32_t(z & 15) + 16u * uint32_t(y & 15));
-		const int syz = slot27_yz(hy, hz); // slot27(x, y, z) = 9 * (x term) + syz: 18 at x = 0, 9 at -1, 0 at 16
-		const size_t cm = (size_t)s.slots[18 + syz] * HCM_CHUNK_VOXELS + lrow;
-		const size_t cl = (size_t)s.slots[9 + syz] * HCM_CHUNK_VOXELS + lrow + 15;
-		const size_t cr = (size_t)s.slots[syz] * HCM_CHUNK_VOXELS + lrow;
-		const uint4 b0 = *reinterpret_cast<const uint4 *>(p.blocks + cm);
-		const uint4 b1 = *reinterpret_cast<const uint4 *>(p.blocks + cm + 8);
-		const uint32_t bw[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
-		const uint32_t bl = p.blocks[cl], br = p.blocks[cr];
-		uint32_t lw[5];
-		if (p.halo_light) { // the job's rebuilt light, one 20-byte record per halo x-row
-			const uint32_t *hl = reinterpret_cast<const uint32_t *>(p.halo_light + (size_t)job * kLightJobBytes +
-			                                                        row * kLightRowBytes);
+		uint32_t bw[8], bl, br, lw[5];
+		if (NT >= kHaloRows && p.halo_in) {
+			bl = given.bl, br = given.br;
+#pragma unroll
+			for (int k = 0; k < 8; ++k)
+				bw[k] = given.bw[k];
 #pragma unroll
 			for (int k = 0; k < 5; ++k)
-				lw[k] = hl[k];
-		} else { // the same layout from the store: x = -1 in byte 0, x = 0 .. 15 in bytes 1 .. 16, x = 16 in 17
-			const uint4 lm = *reinterpret_cast<const uint4 *>(p.light + cm);
-			const uint32_t ll = p.light[cl], lr = p.light[cr];
-			lw[0] = ll | (lm.x << 8);
-			lw[1] = (lm.x >> 24) | (lm.y << 8);
-			lw[2] = (lm.y >> 24) | (lm.z << 8);
-			lw[3] = (lm.z >> 24) | (lm.w << 8);
-			lw[4] = (lm.w >> 24) | (lr << 8);
+				lw[k] = given.lw[k];
+		} else {
+			const size_t lrow = 16u * (uint32_t(z & 15) + 16u * uint32_t(y & 15));
+			const int syz = slot27_yz(hy, hz); // slot27(x, y, z) = 9 * (x term) + syz: 18 at x = 0, 9 at -1, 0 at 16
+			const size_t cm = (size_t)s.slots[18 + syz] * HCM_CHUNK_VOXELS + lrow;
+			const size_t cl = (size_t)s.slots[9 + syz] * HCM_CHUNK_VOXELS + lrow + 15;
+			const size_t cr = (size_t)s.slots[syz] * HCM_CHUNK_VOXELS + lrow;
+			const uint4 b0 = *reinterpret_cast<const uint4 *>(p.blocks + cm);
+			const uint4 b1 = *reinterpret_cast<const uint4 *>(p.blocks + cm + 8);
+			bw[0] = b0.x, bw[1] = b0.y, bw[2] = b0.z, bw[3] = b0.w, bw[4] = b1.x, bw[5] = b1.y, bw[6] = b1.z, bw[7] = b1.w;
+			bl = p.blocks[cl], br = p.blocks[cr];
+			if (p.halo_light) { // the job's rebuilt light, one 20-byte record per halo x-row
+				const uint32_t *hl = reinterpret_cast<const uint32_t *>(p.halo_light + (size_t)job * kLightJobBytes +
+				                                                        row * kLightRowBytes);
+#pragma unroll
+				for (int k = 0; k < 5; ++k)
+					lw[k] = hl[k];
+			} else { // the same layout from the store: x = -1 in byte 0, x = 0 .. 15 in bytes 1 .. 16, x = 16 in 17
+				const uint4 lm = *reinterpret_cast<const uint4 *>(p.light + cm);
+				const uint32_t ll = p.light[cl], lr = p.light[cr];
+				lw[0] = ll | (lm.x << 8);
+				lw[1] = (lm.x >> 24) | (lm.y << 8);
+				lw[2] = (lm.y >> 24) | (lm.z << 8);
+				lw[3] = (lm.z >> 24) | (lm.w << 8);
+				lw[4] = (lm.w >> 24) | (lr << 8);
+			}
 		}
 		// one reference value per wavefront (its first row's first voxel): a halo of one block value has
 		// every voxel equal to it and all wavefronts' references equal
@@ -1363,7 +1462,7 @@ template <int NT> __device__ __forceinline__ void mesh_chunk(const MeshParams &p
 			const int hx = i % kHalo, rest = i / kHalo, hz = rest % kHalo, hy = rest / kHalo;
 			const uint32_t pid = vox_pid(s.vox[i]);
 			const uint32_t mesh = s.rows[pid].y >> 24;
-			const Flow f = flow_heights(p, s.slots, hx - 1, hy - 1, hz - 1, p.reg.meshes[mesh].flow_height);
+			const Flow f = flow_heights(p, blocks, hx - 1, hy - 1, hz - 1, p.reg.meshes[mesh].flow_height);
 			const uint32_t tmpl = s.pid_vox[p.reg.flow_pid_base + flow_pattern(f)];
 			s.vox[i] = (s.vox[i] & kKeep) | (tmpl & ~kKeep);
 		}
@@ -1407,7 +1506,7 @@ template <int NT> __device__ __forceinline__ void mesh_chunk(const MeshParams &p
 			const int cell = tid * CPT + k;
 			if (!((s.custom_bits[cell >> 5] >> (cell & 31)) & 1u))
 				continue;
-			const CustomCell c = custom_cell(p, s, cell);
+			const CustomCell c = custom_cell(p, s, blocks, cell);
 			const uint32_t nt = __popc(c.trans);
 			c_t += nt;
 			c_o += c.count - nt;
@@ -1503,8 +1602,9 @@ template <int NT> __device__ __forceinline__ void mesh_chunk(const MeshParams &p
 				return;
 			}
 			nm0 = (n0 + kSplitQuads - 1) / kSplitQuads, nm1 = (n1 + kSplitQuads - 1) / kSplitQuads;
+			// (a launch of one job has the pool to itself)
 			if (tid < 2) {
-				const uint32_t base = atomicAdd(tid == 0 ? &p.ctr->pool_cursor : &p.ctr->mesh_cursor, tid == 0 ? total : nm0 + nm1);
+				const uint32_t base = p.alone ? 0u : atomicAdd(tid == 0 ? &p.ctr->pool_cursor : &p.ctr->mesh_cursor, tid == 0 ? total : nm0 + nm1);
 				if (tid == 0)
 					s.pool_base = base;
 				else
@@ -1560,7 +1660,7 @@ template <int NT> __device__ __forceinline__ void mesh_chunk(const MeshParams &p
 					const int cell = tid * CPT + k;
 					if (!((s.custom_bits[cell >> 5] >> (cell & 31)) & 1u))
 						continue;
-					const CustomCell c = custom_cell(p, s, cell);
+					const CustomCell c = custom_cell(p, s, blocks, cell);
 					for (uint32_t j = 0; j < c.count; ++j) {
 						const uint32_t tr = (c.trans >> j) & 1u, g = io + it, i = tr ? it++ : io++;
 						if (g >= w0 && g < w1)
@@ -1575,7 +1675,7 @@ template <int NT> __device__ __forceinline__ void mesh_chunk(const MeshParams &p
 				const uint32_t tr = ent.x >> 31;
 				uint32_t slot, vbase, mk, mj, lo[3], hi[3];
 				quad_slot(tr, ent.y, n0, pool_base, slot, vbase, mk, mj);
-				emit_custom(p, s, ent.x & 0xffffu, slot, vbase, lo, hi);
+				emit_custom(p, s, blocks, ent.x & 0xffffu, slot, vbase, lo, hi);
 				quad_done(s, tr, mk, mj, w0 + e, lo, hi, box);
 			}
 		}
@@ -1658,7 +1758,7 @@ template <int NT> __global__ __launch_bounds__(NT, NT >= 512 ? 2 : 3) void mesh_
 				s.job = job;
 			}
 			job = (uint32_t)__builtin_amdgcn_readfirstlane((int)job);
-			if (job < p.n_jobs && lane < 27)
+			if (job < p.n_jobs && lane < 27 && !p.halo_in)
 				s.slots[lane] = p.nbr[27 * (size_t)job + lane];
 		}
 		chunk_init(s);
@@ -1755,39 +1855,14 @@ hipError_t launch_upload_scatter(const uint16_t *sblocks, const uint8_t *slight,
 	return hipGetLastError();
 }
 
-// Scatters n packed chunk halos (include/hcm.h, HCM_HALO_BLOCKS / HCM_HALO_LIGHT; halo j at j times those
-// sizes) into 27 store slots each, job j's chunks at slots 27 j .. 27 j + 26 in neighbour-slot order, where
-// the mesher reads them; cells of the slots outside the halo are not written (the mesher never reads them).
-constexpr int kUnpackBlocksPerHalo = (HCM_HALO_BLOCKS + 255) / 256;
-__global__ void halo_unpack_kernel(const uint16_t *hblocks, const uint8_t *hlight, uint16_t *blocks, uint8_t *light) {
-	const int job = blockIdx.x / kUnpackBlocksPerHalo;
-	const int i = (blockIdx.x % kUnpackBlocksPerHalo) * 256 + threadIdx.x;
-	const size_t base = (size_t)job * 27;
-	if (i < HCM_HALO_BLOCKS) {
-		const int x = i % 20 - 2, z = (i / 20) % 20 - 2, y = i / 400 - 1;
-		blocks[(base + slot27(x, y, z)) * HCM_CHUNK_VOXELS + local16(x, y, z)] = hblocks[(size_t)job * HCM_HALO_BLOCKS + i];
-	}
-	if (i < HCM_HALO_LIGHT) {
-		const int x = i % 18 - 1, z = (i / 18) % 18 - 1, y = i / 324 - 1;
-		light[(base + slot27(x, y, z)) * HCM_CHUNK_VOXELS + local16(x, y, z)] = hlight[(size_t)job * HCM_HALO_LIGHT + i];
-	}
-}
-
-hipError_t launch_halo_unpack(const uint16_t *hblocks, const uint8_t *hlight, uint32_t n, uint16_t *blocks,
-                              uint8_t *light, hipStream_t stream) {
-	if (n == 0)
-		return hipSuccess;
-	hipLaunchKernelGGL(halo_unpack_kernel, dim3(n * kUnpackBlocksPerHalo), dim3(256), 0, stream, hblocks, hlight, blocks,
-	                   light);
-	return hipGetLastError();
-}
-
 hipError_t launch_reset(Counters *ctr, hipStream_t stream) {
 	hipLaunchKernelGGL(reset_kernel, dim3(1), dim3(64), 0, stream, ctr);
 	return hipGetLastError();
 }
 
 hipError_t launch_mesh(const MeshParams &p, int threads, int grid, hipStream_t stream) {
+	if (p.halo_in && threads < kHaloRows) // packed halos are staged one row per thread
+		return hipErrorInvalidValue;
 	switch (threads) {
 	case 128:
 		hipLaunchKernelGGL(mesh_kernel<128>, dim3(grid), dim3(128), 0, stream, p);

@@ -221,6 +221,12 @@ template <int NT> __device__ __forceinline__ void light_job(const LightParams &p
 #pragma unroll
 		for (int q = 0; q < 5; ++q)
 			o[q] = w[q];
+		if (p.halo_light_copy) {
+			o = reinterpret_cast<uint32_t *>(p.halo_light_copy + (size_t)job * kLightJobBytes) + hr * (kLightRowBytes / 4);
+#pragma unroll
+			for (int q = 0; q < 5; ++q)
+				o[q] = w[q];
+		}
 	}
 }
 
@@ -235,6 +241,10 @@ __global__ __launch_bounds__(256) void light_prep_kernel(LightParams p) {
 	const uint16_t *src = p.blocks + (size_t)slot * HCM_CHUNK_VOXELS + row * 16;
 	const uint4 b0 = *reinterpret_cast<const uint4 *>(src), b1 = *reinterpret_cast<const uint4 *>(src + 8);
 	const uint4 hv = *reinterpret_cast<const uint4 *>(p.heights + (size_t)slot * 256 + 16 * z);
+	if (p.blocks_copy) {
+		uint4 *copy = reinterpret_cast<uint4 *>(p.blocks_copy + (size_t)slot * HCM_CHUNK_VOXELS + row * 16);
+		copy[0] = b0, copy[1] = b1;
+	}
 	const uint32_t bw[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
 	const uint32_t hw[4] = {hv.x, hv.y, hv.z, hv.w};
 	uint32_t info[16];

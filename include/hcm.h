@@ -149,8 +149,8 @@ int hcm_mesh_chunk(hcm_ctx *ctx, const uint16_t *const blocks[27], const uint8_t
 /* Meshes one chunk from its packed halo, like Generate(get_block, get_light)
  * (client/include/client/BlockMeshAlgo.hpp:494-521) at the reference's call site
  * (client/src/ChunkMeshTask.cpp:113-122), whose lambdas are evaluated exactly over these voxels. The
- * halo (20 KB) is the only upload; the results of a chunk of up to 2,048 quads come back with one
- * synchronisation. Same output and errors as hcm_mesh_chunk. */
+ * halo (20 KB) is the only upload; the kernel reads it from pinned host memory and writes a chunk of up to
+ * 8,192 quads back there, one launch and one synchronisation. Same output and errors as hcm_mesh_chunk. */
 int hcm_mesh_halo(hcm_ctx *ctx, const uint16_t *blocks, const uint8_t *light, hcm_host_result *out);
 
 /* The whole mesh task of ChunkTaskRunner<kMesh>::Run (client/src/ChunkMeshTask.cpp:41-122): rebuilds light
@@ -200,10 +200,9 @@ typedef struct hcm_job_result {
  * j HCM_HALO_LIGHT) are meshed on `stream` (a hipStream_t; NULL: the default stream) into the caller's
  * device buffers: quads in vertices[4 q ..]/indices[6 q ..] for q < quad_cap, mesh records in
  * recs[0 .. rec_cap) (first_quad into those buffers), per-halo results in results[0 .. n) -- the
- * hcm_batch_download layout. The kernels' other memory (work counters, job table, the 27-slot stores the
- * halos are scattered into) is a fixed device array of the library, one per GPU, held until the process
- * ends: n is at most HCM_NOALLOC_MAX_CHUNKS (HCM_ERR_INVALID beyond). Calls that overlap on one GPU share
- * that array and race; calls on one stream do not. A halo whose output does not fit gets
+ * hcm_batch_download layout. The kernels' other memory (the work counters) is a fixed device array of the
+ * library, one per GPU, held until the process ends; n is at most HCM_NOALLOC_MAX_CHUNKS (HCM_ERR_INVALID
+ * beyond). Calls that overlap on one GPU share that array and race; calls on one stream do not. A halo whose output does not fit gets
  * HCM_ERR_POOL_FULL in its result. */
 #define HCM_NOALLOC_MAX_CHUNKS 8
 int hcm_mesh_halos_noalloc(hcm_ctx *ctx, const uint16_t *halo_blocks, const uint8_t *halo_light, uint32_t n,
