@@ -267,7 +267,7 @@ struct hcm_store {
 	uint16_t *d_blocks = nullptr;
 	uint8_t *d_light = nullptr;
 	int8_t *d_heights = nullptr;  // [n_slots][256] sunlight heights
-	uint16_t *d_packed = nullptr; // [n_slots][kLightPlanes][256] light-rebuild inputs, packed per batch run
+	uint16_t *d_packed = nullptr; // [n_slots][kLightSlotBytes / 2] light-rebuild inputs, packed per batch run
 	uint32_t *d_levels = nullptr; // [n_slots] torchlight levels present
 };
 
@@ -413,7 +413,7 @@ static int create_impl(hcm_ctx *c, const hcm_registry *registry, uint64_t pool_q
 	HCM_HIP(hipHostMalloc(reinterpret_cast<void **>(&c->h_halo_in), kHaloBytes));
 	HCM_HIP(hipHostMalloc(reinterpret_cast<void **>(&c->h_pout), kPoutBytes));
 	HCM_HIP(hipHostMalloc(reinterpret_cast<void **>(&c->h_pheights), 27 * 256));
-	HCM_HIP(dmalloc(&c->d_ppacked, 27 * kLightPlanes * 256));
+	HCM_HIP(dmalloc(&c->d_ppacked, 27 * kLightSlotBytes / 2));
 	HCM_HIP(dmalloc(&c->d_plevels, 27));
 	HCM_HIP(dmalloc(&c->d_phalo, kLightJobBytes));
 	uint32_t ident[27];
@@ -834,7 +834,7 @@ extern "C" int hcm_batch_set_light(hcm_batch *b, uint32_t light_mode) {
 	if (light_mode == HCM_LIGHT_REBUILD) {
 		hcm_store *st = b->store;
 		if (!st->d_packed) {
-			HCM_HIP(dmalloc(&st->d_packed, (size_t)st->n_slots * kLightPlanes * 256));
+			HCM_HIP(dmalloc(&st->d_packed, (size_t)st->n_slots * kLightSlotBytes / 2));
 			HCM_HIP(dmalloc(&st->d_levels, st->n_slots));
 		}
 		if (!b->d_lctr) { // zero once: each light run's last workgroup clears the queues again
@@ -925,7 +925,7 @@ static hipError_t enqueue_light(hcm_batch *b, hipStream_t st) {
 	lp.self_reset = 1;
 	hipError_t e = launch_light_prep(lp, st);
 	if (e == hipSuccess) {
-		const int per_cu = std::max(1, std::min(3, (160 * 1024) / std::max(1, light_lds_bytes())));
+		const int per_cu = std::max(1, std::min(kLightPerCu, (160 * 1024) / std::max(1, light_lds_bytes())));
 		e = launch_light(lp, (int)std::min((uint32_t)(per_cu * b->ctx->n_cu), b->n_jobs), st);
 	}
 	return e;

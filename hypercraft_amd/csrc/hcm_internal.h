@@ -75,6 +75,19 @@ struct Counters {
 	uint32_t total_quads, total_meshes;
 };
 
+// One step of four 8 x 8 bit transpositions (one per byte) over eight words: bits and words whose index
+// differs in D change places. (A template argument: the steps in a loop were not unrolled.)
+template <int D> __device__ __forceinline__ void exchange_bits(uint32_t r[8]) {
+	constexpr uint32_t m = D == 4 ? 0x0f0f0f0fu : (D == 2 ? 0x33333333u : 0x55555555u); // bits without D
+#pragma unroll
+	for (int i = 0; i < 8; ++i)
+		if (!(i & D)) {
+			const uint32_t a = r[i], b = r[i + D];
+			r[i] = (a & m) | ((b << D) & ~m);
+			r[i + D] = ((a >> D) & m) | (b & ~m);
+		}
+}
+
 // The jobs of one workgroup of a persistent launch, by one lane.
 struct JobClaims {
 	uint32_t n_jobs, tried = 0;
@@ -142,12 +155,13 @@ struct MeshParams {
 };
 
 // ---- light rebuild before meshing (client/src/ChunkMeshTask.cpp:48-111) ----
-// Per store slot, the inputs of the light rebuild packed as 16-bit x-rows (row z + 16 y, bit x):
-// plane 0 the indirect light pass, plane 1 sunlight, planes 2..5 the bits of the torchlight level,
-// plane 6 the cells of torchlight level 15.
-constexpr int kLightPlanes = 7;
+// Per store slot, the inputs of the light rebuild packed as 16-bit x-rows (bit x), two 8-byte records per row
+// z + 16 y: first, for every row, the indirect light pass, the sunlit cells and the cells of torchlight level 15
+// (16 bits unused); then, for every row, the four bits of the torchlight level.
+constexpr size_t kLightSlotBytes = 2 * 256 * 8;
 constexpr uint32_t kLightRowBytes = 20;                        // one halo x-row of rebuilt light (18 used)
 constexpr uint32_t kLightJobBytes = 18 * 18 * kLightRowBytes; // rows hz + 18 hy
+constexpr int kLightPerCu = 4; // workgroups of the persistent light kernel per CU: its 32 wavefronts
 constexpr uint8_t kLightInfoPass = 0x10;     // light_info: level | kLightInfoPass when the block passes light
 constexpr uint8_t kLightInfoVertical = 0x20; // ... | kLightInfoVertical when it passes sunlight straight down
 
@@ -158,7 +172,7 @@ struct LightParams {
 	const uint32_t *slots;     // the store slots the batch reads
 	uint32_t n_slots;
 	uint32_t n_jobs;
-	uint16_t *packed;          // [store slots][kLightPlanes][256]
+	uint16_t *packed;          // [store slots][kLightSlotBytes / 2]
 	uint32_t *levels;          // [store slots]: bit l set when a voxel emits torchlight level l
 	const uint32_t *nbr;       // 27 slots per job
 	Counters *ctr;             // work queues of the persistent light kernel

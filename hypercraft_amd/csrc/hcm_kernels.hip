@@ -720,19 +720,6 @@ __device__ __forceinline__ uint32_t byte_perm(uint32_t hi, uint32_t lo, uint32_t
 	return __builtin_amdgcn_perm(hi, lo, sel);
 }
 
-// One step of four 8 x 8 bit transpositions (one per byte) over eight words: bits and words whose index
-// differs in D change places. (A template argument: the steps in a loop were not unrolled.)
-template <int D> __device__ __forceinline__ void exchange_bits(uint32_t r[8]) {
-	constexpr uint32_t m = D == 4 ? 0x0f0f0f0fu : (D == 2 ? 0x33333333u : 0x55555555u); // bits without D
-#pragma unroll
-	for (int i = 0; i < 8; ++i)
-		if (!(i & D)) {
-			const uint32_t a = r[i], b = r[i + D];
-			r[i] = (a & m) | ((b << D) & ~m);
-			r[i + D] = ((a >> D) & m) | (b & ~m);
-		}
-}
-
 // The class bits of 16 blocks' templates as planes, two per word: p0[a] holds class bit 0 and p1[a] class
 // bit 1 of the blocks' + faces along axis a in the low half-word (bit i: block i) and of their - faces in
 // the high one. The templates' upper half-words, two to a register, are an 8 x 8 bit matrix per byte;

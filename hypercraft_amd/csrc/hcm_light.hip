@@ -12,17 +12,16 @@
 // whatever order the propagation runs in. This file computes it level by level on bit masks. With G_k
 // the cells of level >= k,
 //     G_15 = sources of level 15,   G_k = G_{k+1} | sources of level k | (dilate(G_{k+1}) & passable),
-// one 64-bit word per x-row of the 46-wide window; at step k only rows within distance k - 1 of the
+// one 46-bit x-row of the 46-wide window per lane; at step k only rows within distance k - 1 of the
 // bound can still reach it. A cell's level is the largest k with the cell in G_k.
 //
 // Two kernels:
 //   light_prep_kernel  one workgroup per store slot the batch reads: packs its blocks' light pass, its
-//                      sunlit cells (from the sunlight heights), its torchlight levels and its level-15
-//                      torchlight sources into 16-bit x-rows (3.5 KB per slot);
-//   light_kernel       one workgroup per job (persistent, per-XCD work queues, three per CU): assembles
-//                      the 46^3 window from the 27 slots' packed rows in LDS, runs the sunlight and
-//                      torchlight levels, and writes the 18^3 rebuilt light bytes (sun | torch << 4) the
-//                      mesher reads.
+//                      sunlit cells (from the sunlight heights), its level-15 torchlight sources and its
+//                      torchlight levels into 16-bit x-rows (4 KB per slot);
+//   light_kernel       one workgroup per job (persistent, per-XCD work queues): assembles the 46^3 window
+//                      from the 27 slots' packed rows in registers, runs the sunlight and torchlight levels,
+//                      and writes the 18^3 rebuilt light bytes (sun | torch << 4) the mesher reads.
 #include <hip/hip_runtime.h>
 
 #include "hcm_internal.h"
@@ -32,117 +31,160 @@ namespace hcm {
 namespace {
 
 constexpr int kW = 46;                 // window [-15, 31) per axis
-constexpr int kWRows = kW * kW;        // x-rows, index wz + 46 wy
 constexpr int kH = 18;                 // the mesher's halo [-1, 17) per axis
 constexpr int kHRows = kH * kH;        // halo x-rows, index hz + 18 hy
 constexpr int kHOff = 14;              // window index of halo index 0
-constexpr uint64_t kWMask = (1ull << kW) - 1ull;
 constexpr int kLightThreads = 512;
-constexpr int kIn = kW - 2;          // the level steps update rows y, z in [-14, 30): window rows 1 .. 44
-constexpr int kInRows = kIn * kIn;
+constexpr int kLightWaves = kLightThreads / 64;
+// A wavefront holds kPlanes layers of the window along y, a lane one row z of each (46 of the 64 lanes): a
+// row's neighbours along z are the neighbouring lanes', those along y are in the lane's own registers but for
+// the wavefront's first and last layer, which go through LDS. A level step of a layer is 16 VALU instructions
+// and no LDS; eight wavefronts of six layers at 64 registers fill a CU's wavefronts four workgroups deep. The
+// step is bound by VALU issue (88.6 M instructions for 4,096 jobs of the lit cave region, 144 us at full issue,
+// 174 us measured). The earlier kernel kept the whole window in LDS, one row per thread and step, with six LDS
+// reads and a write per row: 223 us. Six wavefronts of eight layers took 207 us, a wavefront skipping steps that
+// can change none of its rows 181 us (the skipped work is less than the bookkeeping).
+constexpr int kPlanes = 6;
+static_assert(kLightWaves * kPlanes >= kW && kW <= 64, "the wavefronts' layers cover the window");
+constexpr int kEdgeLanes = 48; // rows of an exchanged layer: 46 and two that are always empty
 
-// 53.4 KB: three workgroups per CU
+// The wavefronts whose layers meet the halo record all of theirs: layers kHFirst .. kHFirst + kHLayers - 1.
+constexpr int kHWave = kHOff / kPlanes, kHFirst = kHWave * kPlanes;
+constexpr int kHWaves = (kHOff + kH + kPlanes - 1) / kPlanes - kHWave, kHLayers = kHWaves * kPlanes;
+constexpr int kHRec = kHLayers * kH, kHBefore = (kHOff - kHFirst) * kH; // rows recorded per level, and those before the halo's
+
 struct LightSmem {
-	uint64_t pass[kInRows]; // cells that pass light indirectly (Block::GetIndirectLightPass, Block.hpp:70)
-	uint64_t g[2][kWRows];  // G_{k+1} and G_k
-	uint64_t lv012[kHRows]; // the channel's level of each halo cell: bit planes 0, 1, 2 at bits 0, 18, 36
-	uint32_t lv3[kHRows];   // and bit plane 3
+	uint2 edge[2][kLightWaves][2][kEdgeLanes]; // by the step's parity: each wavefront's first and last layer
+	uint32_t halo[15][kHRec];                  // G_1 .. G_15 over the halo's x-rows (bits past the 18th are others'), see kHRec
 	uint32_t slots[27];
 	uint32_t changed[3]; // per level step (rotating): some row of the step changed
 	uint32_t levels;     // torchlight levels present in the 27 chunks
 	uint32_t job;
 };
 
-// CmpXYZ2NeighbourIndex (common/include/common/Position.hpp:138-145): L(-1) = 1, L(0) = 2, L(1) = 0
-__device__ __forceinline__ int nbr_slot(int x, int y, int z) {
-	const int cx = x < 0 ? -1 : (x >= 16 ? 1 : 0), cy = y < 0 ? -1 : (y >= 16 ? 1 : 0), cz = z < 0 ? -1 : (z >= 16 ? 1 : 0);
-	return ((cx + 2) % 3) * 9 + ((cy + 2) % 3) * 3 + (cz + 2) % 3;
-}
+// Neighbour-slot terms along an axis (CmpXYZ2NeighbourIndex, common/include/common/Position.hpp:138-145):
+// L(-1) = 1, L(0) = 2, L(1) = 0.
+__device__ __forceinline__ int slot_term(int v) { return v < 0 ? 1 : (v >= 16 ? 0 : 2); }
 
-// The packed rows of window row (wy, wz): x in [-15, 0) from the -x chunk, [0, 16) from the centre
-// column, [16, 31) from the +x chunk.
+// The packed records of a window row: x in [-15, 0) from the -x chunk, [0, 16) from the centre column,
+// [16, 31) from the +x chunk.
 struct RowSrc {
-	const uint16_t *l, *c, *r;
+	uint2 l, c, r;
 };
-__device__ __forceinline__ RowSrc row_src(const LightParams &p, const LightSmem &s, int wy, int wz) {
-	const int y = wy - 15, z = wz - 15;
-	const uint32_t lr = uint32_t(z & 15) + 16u * uint32_t(y & 15);
-	const size_t stride = (size_t)kLightPlanes * 256;
-	return {p.packed + s.slots[nbr_slot(-1, y, z)] * stride + lr, p.packed + s.slots[nbr_slot(0, y, z)] * stride + lr,
-	        p.packed + s.slots[nbr_slot(16, y, z)] * stride + lr};
+// record 0: x = light pass | sunlit << 16, y = level-15 torchlight sources; record 1: the four bits of the
+// torchlight level.
+__device__ __forceinline__ RowSrc row_src(const LightParams &p, const LightSmem &s, int wy, int wz, int record) {
+	const int y = wy - 15, z = wz - 15, yz = 3 * slot_term(y) + slot_term(z);
+	const uint2 *rows = reinterpret_cast<const uint2 *>(p.packed) + 256 * record + (z & 15) + 16 * (y & 15);
+	constexpr size_t stride = kLightSlotBytes / sizeof(uint2);
+	return {rows[s.slots[9 + yz] * stride], rows[s.slots[18 + yz] * stride], rows[s.slots[yz] * stride]};
 }
-__device__ __forceinline__ uint64_t plane_row(const RowSrc &r, int q) {
-	const uint64_t a = r.l[q * 256], b = r.c[q * 256], c = r.r[q * 256];
-	return (a >> 1) | (b << 15) | ((c & 0x7fffu) << 31);
-}
-// Cells of the row whose torchlight level is exactly k.
-__device__ __forceinline__ uint64_t level_row(const RowSrc &r, uint32_t k) {
-	uint64_t m = kWMask;
-#pragma unroll
-	for (int b = 0; b < 4; ++b) {
-		const uint64_t t = plane_row(r, 2 + b);
-		m &= (k >> b) & 1u ? t : ~t;
-	}
-	return m;
+// The window row (lo, hi) of three 16-bit rows.
+__device__ __forceinline__ uint2 window_row(uint32_t l, uint32_t c, uint32_t r) {
+	return make_uint2((l >> 1) | (c << 15) | (r << 31), (r >> 1) & 0x3fffu);
 }
 
-// One channel: G_15 is in s.g[0]; records each halo cell's level in s.lv012 / s.lv3. A step that adds
-// no cell to its rows leaves G unchanged for every later step (each later step reads only rows of the
-// earlier step), so the channel ends there unless sources enter at a lower level.
-template <int NT>
-__device__ __forceinline__ void propagate(const LightParams &p, LightSmem &s, bool inject) {
-	const int tid = threadIdx.x;
-	if (tid < 3)
-		s.changed[tid] = 0;
-	for (int hr = tid; hr < kHRows; hr += NT) {
-		const int hy = hr / kH, hz = hr % kH;
-		const uint64_t bits = (s.g[0][(hz + kHOff) + kW * (hy + kHOff)] >> kHOff) & 0x3ffffu;
-		s.lv012[hr] = bits | (bits << 18) | (bits << 36); // level 15
-		s.lv3[hr] = uint32_t(bits);
+// Lane z's value from lane z - 1 and z + 1 (0 beyond the wavefront): wave_shr:1, wave_shl:1.
+__device__ __forceinline__ uint32_t from_prev(uint32_t v) { return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x138, 0xf, 0xf, true); }
+__device__ __forceinline__ uint32_t from_next(uint32_t v) { return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x130, 0xf, 0xf, true); }
+
+// The halo's x and z part of this wavefront's layers of G_k into s.halo.
+__device__ __forceinline__ void record_halo(LightSmem &s, uint32_t k, int wave, int lane, const uint2 g[kPlanes]) {
+	if ((unsigned)(wave - kHWave) >= (unsigned)kHWaves) // the same for the whole wavefront
+		return;
+	const int hz = lane - kHOff;
+	if ((unsigned)hz < (unsigned)kH) {
+		uint32_t *rec = s.halo[k - 1] + (wave - kHWave) * kPlanes * kH + hz;
+#pragma unroll
+		for (int q = 0; q < kPlanes; ++q)
+			rec[q * kH] = (g[q].x >> kHOff) | (g[q].y << (32 - kHOff));
 	}
-	__syncthreads();
-	int cur = 0;
+}
+
+// One channel from its G_15, with s.changed clear: G_k over the halo into s.halo[k - 1] for k down to the
+// returned level; the lower ones equal that one. A step that adds no cell to its rows leaves G unchanged for
+// every later step (each later step reads only rows of the earlier step), so the channel ends there unless
+// sources enter at a lower level; one without a cell of level 15 ends at once.
+__device__ __forceinline__ uint32_t propagate(const LightParams &p, LightSmem &s, int wave, int lane, uint2 g[kPlanes],
+                                              const uint2 pass[kPlanes], bool inject) {
+	record_halo(s, 15, wave, lane, g);
+	uint32_t any = 0;
+#pragma unroll
+	for (int q = 0; q < kPlanes; ++q)
+		any |= g[q].x | g[q].y;
+	if (__ballot(any != 0) && lane == 0)
+		s.changed[15 % 3] = 1;
+	uint32_t end = 15;
 #pragma unroll 1
 	for (uint32_t k = 14; k >= 1; --k) {
-		const int lo = 15 - int(k), n = 16 + 2 * int(k);
-		const uint32_t inv = ((1u << 20) + uint32_t(n) - 1u) / uint32_t(n); // i / n = (i * inv) >> 20, i < n * n
+		uint2(*edge)[2][kEdgeLanes] = s.edge[k & 1];
+		if (lane < kEdgeLanes) {
+			edge[wave][0][lane] = g[0];
+			edge[wave][1][lane] = g[kPlanes - 1];
+		}
+		__syncthreads();
+		if (!s.changed[(k + 1) % 3] && !(inject && (s.levels & ((2u << k) - 1u))))
+			break;
+		end = k;
+		if (threadIdx.x == 0)
+			s.changed[(k + 2) % 3] = 0; // the flag of step k - 1, last read before this step's barrier
+		// rows past distance k - 1 of the bound cannot reach it any more
+		if (kPlanes * wave + kPlanes <= 15 - int(k) || kPlanes * wave >= 31 + int(k))
+			continue;
+		const int el = min(lane, kEdgeLanes - 1);
+		uint2 before = wave > 0 ? edge[wave - 1][1][el] : make_uint2(0, 0);
+		const uint2 after = wave < kLightWaves - 1 ? edge[wave + 1][0][el] : make_uint2(0, 0);
 		const bool inj = inject && ((s.levels >> k) & 1u);
-		const uint64_t *gi = s.g[cur];
-		uint64_t *go = s.g[cur ^ 1];
-		if (tid == 0)
-			s.changed[(k + 2) % 3] = 0; // the flag of step k - 1, last read before the previous barrier
-		bool changed = false;
-		for (int i = tid; i < n * n; i += NT) {
-			const int qy = int((uint32_t(i) * inv) >> 20), wy = lo + qy, wz = lo + (i - qy * n);
-			const int r = wz + kW * wy;
-			const uint64_t g = gi[r];
-			const uint64_t d = (g << 1) | (g >> 1) | gi[r - 1] | gi[r + 1] | gi[r - kW] | gi[r + kW];
-			uint64_t nw = g | (d & s.pass[(wz - 1) + kIn * (wy - 1)]);
-			if (inj)
-				nw |= level_row(row_src(p, s, wy, wz), k);
-			go[r] = nw;
-			changed |= nw != g;
-			const int hy = wy - kHOff, hz = wz - kHOff;
-			if ((unsigned)hy < (unsigned)kH && (unsigned)hz < (unsigned)kH) {
-				const uint64_t add = ((nw & ~g) >> kHOff) & 0x3ffffu;
-				if (add) {
-					const int hr = hz + kH * hy;
-					const uint64_t m =
-					    ((k & 1u) ? add : 0ull) | ((k & 2u) ? add << 18 : 0ull) | ((k & 4u) ? add << 36 : 0ull);
-					if (m)
-						s.lv012[hr] |= m;
-					if (k & 8u)
-						s.lv3[hr] |= uint32_t(add);
+		uint32_t changed = 0;
+#pragma unroll
+		for (int q = 0; q < kPlanes; ++q) {
+			const uint2 o = g[q], up = q < kPlanes - 1 ? g[q + 1] : after;
+			const uint32_t dx = (o.x << 1) | ((o.x >> 1) | (o.y << 31)) | before.x | up.x | from_prev(o.x) | from_next(o.x);
+			const uint32_t dy = ((o.y << 1) | (o.x >> 31)) | (o.y >> 1) | before.y | up.y | from_prev(o.y) | from_next(o.y);
+			uint2 n = make_uint2(o.x | (dx & pass[q].x), o.y | (dy & pass[q].y));
+			changed |= (n.x ^ o.x) | (n.y ^ o.y);
+			before = o;
+			g[q] = n;
+		}
+		if (inj) { // sources of level k
+			// (the layer index by way of readfirstlane, so that the addresses are not computed ahead of the steps and
+			// held in registers through all of them)
+			const int w0 = kPlanes * __builtin_amdgcn_readfirstlane(wave);
+#pragma unroll
+			for (int q = 0; q < kPlanes; ++q) {
+				const RowSrc t = row_src(p, s, min(w0 + q, kW - 1), min(lane, kW - 1), 1);
+				uint32_t ml = w0 + q < kW && lane < kW ? 0xffffu : 0u, mc = ml, mr = ml;
+#pragma unroll
+				for (int b = 0; b < 4; ++b) {
+					const uint32_t flip = (k >> b) & 1u ? 0u : 0xffffu;
+					ml &= ((b < 2 ? t.l.x : t.l.y) >> (16 * (b & 1))) ^ flip;
+					mc &= ((b < 2 ? t.c.x : t.c.y) >> (16 * (b & 1))) ^ flip;
+					mr &= ((b < 2 ? t.r.x : t.r.y) >> (16 * (b & 1))) ^ flip;
 				}
+				const uint2 src = window_row(ml, mc, mr);
+				changed |= (src.x & ~g[q].x) | (src.y & ~g[q].y);
+				g[q].x |= src.x, g[q].y |= src.y;
 			}
 		}
-		if (__ballot(changed) && (tid & 63) == 0)
+		record_halo(s, k, wave, lane, g);
+		if (__ballot(changed != 0) && lane == 0)
 			s.changed[k % 3] = 1;
-		__syncthreads();
-		cur ^= 1;
-		if (!s.changed[k % 3] && !(inject && (s.levels & ((1u << k) - 1u))))
-			break;
 	}
+	__syncthreads();
+	return end;
+}
+
+// The levels of halo row hr as four bit planes, from G_1 .. G_15 (each within the next lower one).
+__device__ __forceinline__ void level_planes(const LightSmem &s, int hr, uint32_t end, uint32_t pl[4]) {
+	uint32_t G[16];
+#pragma unroll
+	for (uint32_t k = 1; k < 16; ++k)
+		G[k] = s.halo[max(k, end) - 1][kHBefore + hr];
+	pl[3] = G[8];
+	pl[2] = (G[4] & ~G[8]) | G[12];
+	pl[1] = (G[2] & ~G[4]) | (G[6] & ~G[8]) | (G[10] & ~G[12]) | G[14];
+	pl[0] = (G[1] & ~G[2]) | (G[3] & ~G[4]) | (G[5] & ~G[6]) | (G[7] & ~G[8]) | (G[9] & ~G[10]) | (G[11] & ~G[12]) |
+	        (G[13] & ~G[14]) | G[15];
 }
 
 // Wavefront 0: the slot list of `job` and the torchlight levels present in its 27 chunks, into LDS.
@@ -161,72 +203,61 @@ __device__ __forceinline__ void light_slots(const LightParams &p, LightSmem &s, 
 		s.levels = lv & ~1u;
 }
 
-// One job; s.slots and s.levels are in place (a barrier after them). Every window row is read from the
-// packed planes once: its light pass and sunlit cells into LDS, its level-15 torchlight sources into
-// the reading thread's registers until the torchlight channel starts.
-template <int NT> __device__ __forceinline__ void light_job(const LightParams &p, LightSmem &s, uint32_t job) {
-	static_assert(NT >= kHRows, "one halo x-row per thread");
-	constexpr int kRowsPerThread = (kWRows + NT - 1) / NT;
-	const int tid = threadIdx.x;
-	const bool torch = s.levels != 0, torch15 = (s.levels >> 15) & 1u;
-	uint64_t src15[kRowsPerThread];
+// One job; s.slots and s.levels are in place and s.changed is clear (a barrier after them).
+__device__ __forceinline__ void light_job(const LightParams &p, LightSmem &s, uint32_t job) {
+	static_assert(kLightThreads >= kHRows, "one halo x-row per thread");
+	const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+	const bool torch = s.levels != 0;
+	uint2 g[kPlanes], pass[kPlanes];
+	uint32_t pl[8] = {}; // bit planes of the light bytes sun | torch << 4 (block/include/block/Light.hpp)
+#pragma unroll 1
+	for (int channel = 0;; ++channel) { // sunlight: 15 at and above the sunlight height (Chunk.hpp:73-79); then torchlight
+		// (the layer index by way of readfirstlane, so that the addresses are not kept in registers through a channel)
+		const int w0 = kPlanes * __builtin_amdgcn_readfirstlane(wave);
 #pragma unroll
-	for (int k = 0; k < kRowsPerThread; ++k) {
-		const int r = tid + k * NT;
-		src15[k] = 0;
-		if (r < kWRows) {
-			const int wy = r / kW, wz = r % kW;
-			const RowSrc src = row_src(p, s, wy, wz);
-			if (unsigned(wy - 1) < unsigned(kIn) && unsigned(wz - 1) < unsigned(kIn))
-				s.pass[(wz - 1) + kIn * (wy - 1)] = plane_row(src, 0);
-			s.g[0][r] = plane_row(src, 1); // sunlight: 15 at and above the sunlight height (Chunk.hpp:73-79)
-			if (torch15)
-				src15[k] = plane_row(src, 6);
+		for (int q = 0; q < kPlanes; ++q) { // lanes and layers past the window read some row of it and drop it
+			const RowSrc t = row_src(p, s, min(w0 + q, kW - 1), min(lane, kW - 1), 0);
+			const uint32_t in = w0 + q < kW && lane < kW ? ~0u : 0u, l = t.l.x & in, c = t.c.x & in, r = t.r.x & in;
+			if (channel == 0) {
+				pass[q] = window_row(l & 0xffffu, c & 0xffffu, r & 0xffffu);
+				g[q] = window_row(l >> 16, c >> 16, r >> 16);
+			} else
+				g[q] = window_row(t.l.y & in, t.c.y & in, t.r.y & in);
 		}
-	}
-	__syncthreads();
-	// light bytes sun | torch << 4 (block/include/block/Light.hpp), one 20-byte record per halo x-row,
-	// written once: a thread's halo row's sunlight nibbles wait in its registers for the torchlight ones
-	const int hr = tid;
-	uint32_t w[5] = {0, 0, 0, 0, 0};
-	auto nibbles = [&](int shift) {
-		if (hr < kHRows) {
-			const uint64_t l012 = s.lv012[hr];
-			const uint32_t pl[4] = {uint32_t(l012) & 0x3ffffu, uint32_t(l012 >> 18) & 0x3ffffu,
-			                        uint32_t(l012 >> 36) & 0x3ffffu, s.lv3[hr]};
+		const uint32_t end = propagate(p, s, wave, lane, g, pass, channel != 0);
+		if (tid < kHRows)
+			level_planes(s, tid, end, pl + 4);
+		if (channel != 0)
+			break;
 #pragma unroll
-			for (int x = 0; x < kH; ++x) {
-				uint32_t v = 0;
-#pragma unroll
-				for (int b = 0; b < 4; ++b)
-					v |= ((pl[b] >> x) & 1u) << b;
-				w[x >> 2] |= v << (8 * (x & 3) + shift);
-			}
-		}
-	};
-	propagate<NT>(p, s, false);
-	nibbles(0);
-	if (torch) {
+		for (int b = 0; b < 4; ++b)
+			pl[b] = pl[4 + b], pl[4 + b] = 0;
+		if (!torch)
+			break;
+		if (tid < 3)
+			s.changed[tid] = 0;
 		__syncthreads(); // every halo row's sunlight level is read
-#pragma unroll
-		for (int k = 0; k < kRowsPerThread; ++k)
-			if (tid + k * NT < kWRows)
-				s.g[0][tid + k * NT] = src15[k];
-		__syncthreads();
-		propagate<NT>(p, s, true);
-		nibbles(4);
 	}
-	if (hr < kHRows) {
-		uint32_t *o = reinterpret_cast<uint32_t *>(p.halo_light + (size_t)job * kLightJobBytes) + hr * (kLightRowBytes / 4);
+	if (tid < kHRows) { // one 20-byte record per halo x-row: the planes' bits 8 j + b transposed are byte j of word b
+		exchange_bits<4>(pl);
+		exchange_bits<2>(pl);
+		exchange_bits<1>(pl);
+		uint32_t w[5];
+#pragma unroll
+		for (int j = 0; j < 4; ++j) { // bytes x = 4 j .. 4 j + 3
+			const int b = 4 * (j & 1), sh = 8 * (j >> 1);
+			w[j] = ((pl[b] >> sh) & 0xffu) | ((pl[b + 1] >> sh) & 0xffu) << 8 | ((pl[b + 2] >> sh) & 0xffu) << 16 |
+			       ((pl[b + 3] >> sh) & 0xffu) << 24;
+		}
+		w[4] = ((pl[0] >> 16) & 0xffu) | ((pl[1] >> 16) & 0xffu) << 8;
+		const size_t at = (size_t)job * (kLightJobBytes / 4) + tid * (kLightRowBytes / 4);
 #pragma unroll
 		for (int q = 0; q < 5; ++q)
-			o[q] = w[q];
-		if (p.halo_light_copy) {
-			o = reinterpret_cast<uint32_t *>(p.halo_light_copy + (size_t)job * kLightJobBytes) + hr * (kLightRowBytes / 4);
+			reinterpret_cast<uint32_t *>(p.halo_light)[at + q] = w[q];
+		if (p.halo_light_copy)
 #pragma unroll
 			for (int q = 0; q < 5; ++q)
-				o[q] = w[q];
-		}
+				reinterpret_cast<uint32_t *>(p.halo_light_copy)[at + q] = w[q];
 	}
 }
 
@@ -262,14 +293,9 @@ __global__ __launch_bounds__(256) void light_prep_kernel(LightParams p) {
 		t15 |= (l == 15u ? 1u : 0u) << x;
 		lv |= 1u << l;
 	}
-	uint16_t *dst = p.packed + (size_t)slot * kLightPlanes * 256 + row;
-	dst[0] = uint16_t(pass);
-	dst[256] = uint16_t(sun);
-	dst[512] = uint16_t(t0);
-	dst[768] = uint16_t(t1);
-	dst[1024] = uint16_t(t2);
-	dst[1280] = uint16_t(t3);
-	dst[1536] = uint16_t(t15);
+	uint2 *dst = reinterpret_cast<uint2 *>(p.packed + (size_t)slot * (kLightSlotBytes / 2)) + row;
+	dst[0] = make_uint2(pass | sun << 16, t15);
+	dst[256] = make_uint2(t0 | t1 << 16, t2 | t3 << 16);
 	__syncthreads();
 	if (lv & ~1u)
 		atomicOr(&s_levels, lv & ~1u);
@@ -278,7 +304,7 @@ __global__ __launch_bounds__(256) void light_prep_kernel(LightParams p) {
 		p.levels[slot] = s_levels;
 }
 
-template <int NT> __global__ __launch_bounds__(NT, 3) void light_kernel(LightParams p) {
+__global__ __launch_bounds__(kLightThreads, 8) void light_kernel(LightParams p) {
 	__shared__ LightSmem s;
 	JobClaims claims(p.n_jobs); // lane 0 of wavefront 0 only
 	for (;;) {
@@ -287,6 +313,7 @@ template <int NT> __global__ __launch_bounds__(NT, 3) void light_kernel(LightPar
 			if (threadIdx.x == 0) {
 				job = claims.next(p.ctr);
 				s.job = job;
+				s.changed[0] = s.changed[1] = s.changed[2] = 0;
 			}
 			job = (uint32_t)__shfl((int)job, 0);
 			if (job < p.n_jobs)
@@ -296,7 +323,7 @@ template <int NT> __global__ __launch_bounds__(NT, 3) void light_kernel(LightPar
 		const uint32_t job = s.job;
 		if (job >= p.n_jobs)
 			break;
-		light_job<NT>(p, s, job);
+		light_job(p, s, job);
 		__syncthreads();
 	}
 	// as in the mesh kernel: the last workgroup to finish clears the queues for the next run
@@ -318,7 +345,7 @@ hipError_t launch_light_prep(const LightParams &p, hipStream_t stream) {
 }
 
 hipError_t launch_light(const LightParams &p, int grid, hipStream_t stream) {
-	hipLaunchKernelGGL(light_kernel<kLightThreads>, dim3(grid), dim3(kLightThreads), 0, stream, p);
+	hipLaunchKernelGGL(light_kernel, dim3(grid), dim3(kLightThreads), 0, stream, p);
 	return hipGetLastError();
 }
 

@@ -162,7 +162,7 @@ struct hcm_server {
 	uint16_t *d_blocks = nullptr;
 	uint8_t *d_light = nullptr;
 	int8_t *d_heights = nullptr;  // HCM_LIGHT_REBUILD: [slot][256] sunlight heights
-	uint16_t *d_packed = nullptr; // HCM_LIGHT_REBUILD: [slot][kLightPlanes][256]
+	uint16_t *d_packed = nullptr; // HCM_LIGHT_REBUILD: [slot][kLightSlotBytes / 2]
 	uint32_t *d_levels = nullptr;
 	uint2 *d_verts = nullptr;
 	uint16_t *d_idx = nullptr;
@@ -514,7 +514,7 @@ struct hcm_server {
 				lp.halo_light = b.d_halo;
 				lp.self_reset = 1; // the slot's light queues start at zero; the run's last workgroup clears them
 				HCM_CHECK(launch_light_prep(lp, s_comp));
-				HCM_CHECK(launch_light(lp, std::max(1, std::min(info.n_cu * 3, (int)b.jobs.size())), s_comp));
+				HCM_CHECK(launch_light(lp, std::max(1, std::min(info.n_cu * kLightPerCu, (int)b.jobs.size())), s_comp));
 			}
 			MeshParams p;
 			std::memset(&p, 0, sizeof(p));
@@ -796,7 +796,7 @@ static int server_init(hcm_server *s) {
 	HCM_CHECK(dalloc(&s->d_light, (size_t)c.max_chunks * HCM_CHUNK_VOXELS));
 	if (s->relight()) {
 		HCM_CHECK(dalloc(&s->d_heights, (size_t)c.max_chunks * 256));
-		HCM_CHECK(dalloc(&s->d_packed, (size_t)c.max_chunks * kLightPlanes * 256));
+		HCM_CHECK(dalloc(&s->d_packed, (size_t)c.max_chunks * kLightSlotBytes / 2));
 		HCM_CHECK(dalloc(&s->d_levels, (size_t)c.max_chunks));
 	}
 	HCM_CHECK(dalloc(&s->d_verts, (size_t)c.pool_quads * 4));

@@ -46,6 +46,8 @@ static int dpp_src(uint32_t ctrl, int lane) {
 		const int n = int(ctrl & 15u);
 		return in >= n ? lane - n : -1;
 	}
+	case 0x138: return lane - 1;                                 // wave_shr:1
+	case 0x130: return lane < 63 ? lane + 1 : -1;                // wave_shl:1
 	case 0x128: return (row << 4) | ((in + 8) & 15);             // row_ror:8
 	case 0x142: return row >= 1 ? ((row - 1) << 4) | 15 : -1;    // row_bcast:15
 	case 0x143: return row >= 2 ? 31 : -1;                       // row_bcast:31
