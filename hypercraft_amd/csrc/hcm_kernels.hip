@@ -28,7 +28,7 @@
 // All arithmetic is integer. References are to client/include/client/BlockMeshAlgo.hpp unless noted.
 #include <hip/hip_runtime.h>
 
-#include "hcm_internal.h"
+#include "hcm_device.h"
 
 namespace hcm {
 

@@ -24,7 +24,7 @@
 //                      and writes the 18^3 rebuilt light bytes (sun | torch << 4) the mesher reads.
 #include <hip/hip_runtime.h>
 
-#include "hcm_internal.h"
+#include "hcm_device.h"
 
 namespace hcm {
 
