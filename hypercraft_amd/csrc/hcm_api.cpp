@@ -202,7 +202,10 @@ constexpr size_t kHaloBytes = HCM_HALO_BLOCKS * 2 + HCM_HALO_LIGHT;
 constexpr size_t kPoutRecs = 64, kPoutVerts = 64 + kPlainRecs * sizeof(hcm_mesh_rec);
 constexpr size_t kPoutIdx = kPoutVerts + kPlainFastQuads * 4 * sizeof(uint2);
 constexpr size_t kPoutLight = kPoutIdx + kPlainFastQuads * 6 * 2;
-constexpr size_t kPoutBytes = kPoutLight + kLightJobBytes;
+// The same pinned memory takes what batches hand out, where it fits: a run's totals, results, records and
+// quads, mesh infos, draws.
+constexpr size_t kPoutBytes = size_t(2) << 20;
+static_assert(kPoutLight + kLightJobBytes <= kPoutBytes, "a one-chunk call's output fits");
 static_assert(kPoutVerts % 16 == 0 && kPoutIdx % 16 == 0 && kPoutLight % 4 == 0 && HCM_HALO_BLOCKS * 2 % 16 == 0,
               "aligned for the kernels' widest stores and loads");
 
@@ -295,7 +298,7 @@ struct hcm_batch {
 	int32_t *d_chunk_pos = nullptr;
 	hcm_mesh_info *d_infos = nullptr;
 	hcm_draw_cmd *d_draws = nullptr; // [2][rec_cap]: opaque, transparent
-	uint32_t *d_draw_counts = nullptr;
+	CullCounts *d_draw_counts = nullptr;
 	uint32_t n_infos = 0;
 	bool infos_ready = false;
 };
@@ -997,40 +1000,73 @@ extern "C" int hcm_batch_sync(hcm_batch *b, float *kernel_ms) {
 	return HCM_OK;
 }
 
-extern "C" int hcm_batch_results(hcm_batch *b, hcm_job_result *results) {
-	if (!b || !results || !b->ran)
-		return HCM_ERR_INVALID;
-	hipStream_t st = b->ctx->stream;
-	HCM_HIP(hipMemcpyAsync(results, b->d_res, (size_t)b->n_jobs * sizeof(hcm_job_result), hipMemcpyDeviceToHost, st));
+// The run's totals, results (n_jobs), records and, where all of them fit, quads, copied to the context's pinned
+// memory (context lock held). `what` receives where; a part that was not wanted or does not fit is null.
+struct Exported {
+	uint32_t quads = 0, meshes = 0;
+	const hcm_job_result *results = nullptr;
+	const hcm_mesh_rec *recs = nullptr;
+	const uint2 *verts = nullptr;
+	const uint16_t *idx = nullptr;
+};
+static int export_run(hcm_batch *b, bool results, bool recs, bool quads, Exported *what) {
+	hcm_ctx *c = b->ctx;
+	hipStream_t st = c->stream;
+	ExportParams p;
+	p.ctr = b->d_ctr;
+	p.persistent = b->last_mode == HCM_RUN_PERSISTENT;
+	size_t at = 64;
+	const auto place = [&](size_t bytes) { // 16-byte aligned; null when it does not fit
+		if (at + bytes > kPoutBytes)
+			return (uint8_t *)nullptr;
+		uint8_t *q = c->h_pout + at;
+		at += (bytes + 15) / 16 * 16;
+		return q;
+	};
+	p.out_totals = reinterpret_cast<uint32_t *>(c->h_pout);
+	p.n_jobs = b->n_jobs;
+	if (results && (p.out_results = reinterpret_cast<hcm_job_result *>(place((size_t)b->n_jobs * sizeof(hcm_job_result)))))
+		p.results = b->d_res;
+	p.rec_cap = b->rec_cap;
+	if (recs && (p.out_recs = reinterpret_cast<hcm_mesh_rec *>(place((size_t)b->rec_cap * sizeof(hcm_mesh_rec)))))
+		p.recs = b->d_recs;
+	if (quads) {
+		p.quad_cap = (uint32_t)((kPoutBytes - at - 32) / 44);
+		p.out_verts = reinterpret_cast<uint2 *>(place((size_t)p.quad_cap * 4 * sizeof(uint2)));
+		p.out_idx = reinterpret_cast<uint16_t *>(place((size_t)p.quad_cap * 12));
+		if (p.out_verts && p.out_idx)
+			p.verts = c->d_verts, p.idx = c->d_idx;
+	}
+	HCM_HIP(launch_export(p, st));
 	HCM_HIP(hipStreamSynchronize(st));
+	what->quads = p.out_totals[0], what->meshes = p.out_totals[1];
+	if (p.results)
+		what->results = p.out_results;
+	if (p.recs)
+		what->recs = p.out_recs;
+	if (p.verts && what->quads <= p.quad_cap && what->quads <= c->pool_quads)
+		what->verts = p.out_verts, what->idx = p.out_idx;
 	return HCM_OK;
 }
 
-// The quads and mesh records of the batch's last run: a persistent run's last workgroup copies them to
-// total_quads / total_meshes before it clears the cursors; per-chunk launches leave them in the cursors.
-static hipError_t run_totals(hcm_batch *b, uint32_t *quads, uint32_t *meshes) {
-	Counters ctr;
-	hipStream_t st = b->ctx->stream;
-	hipError_t e = hipMemcpyAsync(&ctr, b->d_ctr, sizeof(ctr), hipMemcpyDeviceToHost, st);
-	if (e == hipSuccess)
-		e = hipStreamSynchronize(st);
-	if (e != hipSuccess)
-		return e;
-	const bool persistent = b->last_mode == HCM_RUN_PERSISTENT;
-	*quads = persistent ? ctr.total_quads : ctr.pool_cursor;
-	*meshes = persistent ? ctr.total_meshes : ctr.mesh_cursor;
-	return hipSuccess;
+extern "C" int hcm_batch_results(hcm_batch *b, hcm_job_result *results) {
+	if (!b || !results || !b->ran)
+		return HCM_ERR_INVALID;
+	return hcm_batch_download(b, results, nullptr, 0, nullptr, nullptr, 0);
 }
 
 extern "C" int hcm_batch_totals(hcm_batch *b, uint64_t *quads, uint64_t *meshes) {
 	if (!b || !b->ran)
 		return HCM_ERR_INVALID;
-	uint32_t nq, nm;
-	HCM_HIP(run_totals(b, &nq, &nm));
+	std::lock_guard<std::mutex> lk(b->ctx->mu);
+	Exported e;
+	const int r = export_run(b, false, false, false, &e);
+	if (r != HCM_OK)
+		return r;
 	if (quads)
-		*quads = nq;
+		*quads = e.quads;
 	if (meshes)
-		*meshes = nm;
+		*meshes = e.meshes;
 	return HCM_OK;
 }
 
@@ -1055,22 +1091,36 @@ extern "C" int hcm_batch_mesh_infos(hcm_batch *b, const int32_t *chunk_pos, hcm_
 		HCM_HIP(dmalloc(&b->d_chunk_pos, 3ull * b->n_jobs));
 		HCM_HIP(dmalloc(&b->d_infos, b->rec_cap));
 		HCM_HIP(dmalloc(&b->d_draws, 2ull * b->rec_cap));
-		HCM_HIP(dmalloc(&b->d_draw_counts, 2));
+		HCM_HIP(dmalloc(&b->d_draw_counts, 1));
+		HCM_HIP(hipMemsetAsync(b->d_draw_counts, 0, sizeof(CullCounts), st)); // zero once: each cull clears them again
 	}
-	uint32_t total_quads, total_meshes;
-	HCM_HIP(run_totals(b, &total_quads, &total_meshes));
-	HCM_HIP(hipMemcpyAsync(b->d_chunk_pos, chunk_pos, 12ull * b->n_jobs, hipMemcpyHostToDevice, st));
-	const uint32_t nr = std::min<uint32_t>(total_meshes, b->rec_cap);
-	HCM_HIP(launch_mesh_infos(b->d_recs, nr, b->d_chunk_pos, b->d_infos, st));
+	// one launch from and to pinned memory where the positions and the infos fit, else by way of the device
+	const size_t pos_bytes = 12ull * b->n_jobs, at_infos = 64 + (pos_bytes + 15) / 16 * 16;
+	const bool pinned = at_infos + (size_t)b->rec_cap * sizeof(hcm_mesh_info) <= kPoutBytes;
+	uint32_t *count = reinterpret_cast<uint32_t *>(c->h_pout);
+	int32_t *pos = reinterpret_cast<int32_t *>(pinned ? c->h_pout + 64 : reinterpret_cast<uint8_t *>(b->d_chunk_pos));
+	hcm_mesh_info *copy = pinned && out ? reinterpret_cast<hcm_mesh_info *>(c->h_pout + at_infos) : nullptr;
+	if (pinned)
+		std::memcpy(pos, chunk_pos, pos_bytes);
+	else
+		HCM_HIP(hipMemcpyAsync(pos, chunk_pos, pos_bytes, hipMemcpyHostToDevice, st));
+	HCM_HIP(launch_mesh_infos(b->d_recs, b->d_ctr, b->last_mode == HCM_RUN_PERSISTENT, b->rec_cap, pos, b->d_infos, copy,
+	                          count, st));
+	HCM_HIP(hipStreamSynchronize(st));
+	const uint32_t nr = *count;
 	*n = nr;
 	b->n_infos = nr;
 	b->infos_ready = true;
 	if (out) {
 		if (nr > cap)
 			return HCM_ERR_CAPACITY;
-		HCM_HIP(hipMemcpyAsync(out, b->d_infos, (size_t)nr * sizeof(hcm_mesh_info), hipMemcpyDeviceToHost, st));
+		if (copy) {
+			std::memcpy(out, copy, (size_t)nr * sizeof(hcm_mesh_info));
+		} else {
+			HCM_HIP(hipMemcpyAsync(out, b->d_infos, (size_t)nr * sizeof(hcm_mesh_info), hipMemcpyDeviceToHost, st));
+			HCM_HIP(hipStreamSynchronize(st));
+		}
 	}
-	HCM_HIP(hipStreamSynchronize(st));
 	return HCM_OK;
 }
 
@@ -1090,21 +1140,32 @@ static int cull_batch(hcm_batch *b, const float view_position[3], const float vi
 	std::memcpy(cp.view_proj, view_projection, sizeof(cp.view_proj));
 	if (occlusion)
 		cp.hiz = c->hiz;
-	HCM_HIP(hipMemsetAsync(b->d_draw_counts, 0, 2 * sizeof(uint32_t), st));
-	HCM_HIP(launch_cull(b->d_infos, b->n_infos, cp, b->d_draws, b->d_draws + b->rec_cap, b->d_draw_counts, st));
-	uint32_t counts[2];
-	HCM_HIP(hipMemcpyAsync(counts, b->d_draw_counts, sizeof(counts), hipMemcpyDeviceToHost, st));
+	// the draws go straight to pinned memory where both lists fit, else by way of the device
+	const size_t list = (size_t)b->rec_cap * sizeof(hcm_draw_cmd);
+	const bool pinned = 64 + 2 * list <= kPoutBytes;
+	uint32_t *counts = reinterpret_cast<uint32_t *>(c->h_pout);
+	hcm_draw_cmd *lists[2] = {b->d_draws, b->d_draws + b->rec_cap};
+	if (pinned)
+		for (int k = 0; k < 2; ++k)
+			lists[k] = reinterpret_cast<hcm_draw_cmd *>(c->h_pout + 64 + k * list);
+	HCM_HIP(launch_cull(b->d_infos, b->n_infos, cp, lists[0], lists[1], b->d_draw_counts, counts, st));
 	HCM_HIP(hipStreamSynchronize(st));
 	*n_opaque = counts[0];
 	*n_transparent = counts[1];
 	if ((opaque && counts[0] > opaque_cap) || (transparent && counts[1] > transparent_cap))
 		return HCM_ERR_CAPACITY;
-	if (opaque && counts[0])
-		HCM_HIP(hipMemcpyAsync(opaque, b->d_draws, counts[0] * sizeof(hcm_draw_cmd), hipMemcpyDeviceToHost, st));
-	if (transparent && counts[1])
-		HCM_HIP(hipMemcpyAsync(transparent, b->d_draws + b->rec_cap, counts[1] * sizeof(hcm_draw_cmd),
-		                       hipMemcpyDeviceToHost, st));
-	HCM_HIP(hipStreamSynchronize(st));
+	hcm_draw_cmd *const to[2] = {opaque, transparent};
+	const uint32_t kept[2] = {counts[0], counts[1]};
+	for (int k = 0; k < 2; ++k) {
+		if (!to[k] || !kept[k])
+			continue;
+		if (pinned)
+			std::memcpy(to[k], lists[k], kept[k] * sizeof(hcm_draw_cmd));
+		else
+			HCM_HIP(hipMemcpyAsync(to[k], lists[k], kept[k] * sizeof(hcm_draw_cmd), hipMemcpyDeviceToHost, st));
+	}
+	if (!pinned)
+		HCM_HIP(hipStreamSynchronize(st));
 	return HCM_OK;
 }
 
@@ -1153,9 +1214,7 @@ extern "C" int hcm_ctx_set_depth(hcm_ctx *ctx, const float *depth, uint32_t widt
 		ctx->depth_cap = total;
 	}
 	HCM_HIP(hipMemcpyAsync(ctx->d_depth, depth, (size_t)width * height * sizeof(float), hipMemcpyHostToDevice, st));
-	for (uint32_t i = 1; i < h.n_levels; ++i)
-		HCM_HIP(launch_depth_level(ctx->d_depth + h.offset[i - 1], h.width[i - 1], h.height[i - 1],
-		                           ctx->d_depth + h.offset[i], h.width[i], h.height[i], st));
+	HCM_HIP(launch_depth_levels(h, ctx->d_depth, st));
 	HCM_HIP(hipStreamSynchronize(st));
 	h.data = ctx->d_depth;
 	ctx->hiz = h;
@@ -1186,27 +1245,38 @@ extern "C" int hcm_batch_download(hcm_batch *b, hcm_job_result *results, hcm_mes
                                   uint32_t (*vertices)[2], uint16_t *indices, uint64_t quad_cap) {
 	if (!b || !b->ran)
 		return HCM_ERR_INVALID;
-	hipStream_t st = b->ctx->stream;
-	uint32_t total_quads, total_meshes;
-	HCM_HIP(run_totals(b, &total_quads, &total_meshes));
-	const uint64_t nq = std::min<uint64_t>(total_quads, b->ctx->pool_quads);
-	const uint32_t nr = std::min<uint32_t>(total_meshes, b->rec_cap);
+	hcm_ctx *c = b->ctx;
+	std::lock_guard<std::mutex> lk(c->mu);
+	hipStream_t st = c->stream;
+	Exported e;
+	const int r = export_run(b, results, recs, vertices || indices, &e);
+	if (r != HCM_OK)
+		return r;
+	const uint64_t nq = std::min<uint64_t>(e.quads, c->pool_quads);
+	const uint32_t nr = std::min<uint32_t>(e.meshes, b->rec_cap);
+	// what did not fit the pinned memory is copied from the device
+	const auto give = [&](void *to, const void *pinned, const void *device, size_t bytes) -> hipError_t {
+		if (!bytes)
+			return hipSuccess;
+		if (!pinned)
+			return hipMemcpyAsync(to, device, bytes, hipMemcpyDeviceToHost, st);
+		std::memcpy(to, pinned, bytes);
+		return hipSuccess;
+	};
 	if (results)
-		HCM_HIP(hipMemcpyAsync(results, b->d_res, (size_t)b->n_jobs * sizeof(hcm_job_result), hipMemcpyDeviceToHost,
-		                       st));
+		HCM_HIP(give(results, e.results, b->d_res, (size_t)b->n_jobs * sizeof(hcm_job_result)));
 	if (recs) {
 		if (nr > rec_cap)
 			return HCM_ERR_CAPACITY;
-		if (nr)
-			HCM_HIP(hipMemcpyAsync(recs, b->d_recs, (size_t)nr * sizeof(hcm_mesh_rec), hipMemcpyDeviceToHost, st));
+		HCM_HIP(give(recs, e.recs, b->d_recs, (size_t)nr * sizeof(hcm_mesh_rec)));
 	}
 	if (vertices || indices) {
 		if (nq > quad_cap)
 			return HCM_ERR_CAPACITY;
-		if (nq && vertices)
-			HCM_HIP(hipMemcpyAsync(vertices, b->ctx->d_verts, (size_t)nq * 4 * sizeof(uint2), hipMemcpyDeviceToHost, st));
-		if (nq && indices)
-			HCM_HIP(hipMemcpyAsync(indices, b->ctx->d_idx, (size_t)nq * 12, hipMemcpyDeviceToHost, st));
+		if (vertices)
+			HCM_HIP(give(vertices, e.verts, c->d_verts, (size_t)nq * 4 * sizeof(uint2)));
+		if (indices)
+			HCM_HIP(give(indices, e.idx, c->d_idx, (size_t)nq * 12));
 	}
 	HCM_HIP(hipStreamSynchronize(st));
 	return HCM_OK;

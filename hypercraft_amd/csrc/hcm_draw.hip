@@ -14,7 +14,10 @@
 //   depth_level_kernel one thread per texel of a depth-hierarchy level: the largest of the 2x2 texels under
 //                     it in the level above, plus the third column / row where that level's width / height
 //                     is odd (client/shader/src/depth_hierarchy.comp, DepthHierarchyPass.hpp:166-196).
+//   depth_tail_kernel the small levels, one after another in one workgroup.
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 #include "hcm_internal.h"
 
@@ -33,8 +36,12 @@ __device__ __forceinline__ float f_div(float a, float b) { return a / b; }
 
 } // namespace
 
-__global__ void mesh_info_kernel(const hcm_mesh_rec *recs, uint32_t n, const int32_t *chunk_pos, hcm_mesh_info *out) {
+__global__ void mesh_info_kernel(const hcm_mesh_rec *recs, const Counters *ctr, uint32_t persistent, uint32_t rec_cap,
+                                 const int32_t *chunk_pos, hcm_mesh_info *out, hcm_mesh_info *out2, uint32_t *count) {
 	const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+	const uint32_t n = min(persistent ? ctr->total_meshes : ctr->mesh_cursor, rec_cap);
+	if (i == 0)
+		*count = n;
 	if (i >= n)
 		return;
 	const hcm_mesh_rec r = recs[i];
@@ -50,6 +57,8 @@ __global__ void mesh_info_kernel(const hcm_mesh_rec *recs, uint32_t n, const int
 	}
 	m.transparent = r.transparent;
 	out[i] = m;
+	if (out2)
+		out2[i] = m;
 }
 
 namespace {
@@ -104,10 +113,10 @@ __device__ __forceinline__ bool occluded(const DepthPyramid &h, const float cmin
 
 } // namespace
 
-__global__ void depth_level_kernel(const float *prev, uint32_t pw, uint32_t ph, float *cur, uint32_t cw, uint32_t ch) {
-	const uint32_t x = blockIdx.x * blockDim.x + threadIdx.x, y = blockIdx.y * blockDim.y + threadIdx.y;
-	if (x >= cw || y >= ch)
-		return;
+namespace {
+
+// One texel of a depth-hierarchy level from the level above.
+__device__ __forceinline__ float depth_texel(const float *prev, uint32_t pw, uint32_t ph, uint32_t x, uint32_t y) {
 	// texels outside the level above read 0 (robust image access), which never raises a depth in [0, 1]
 	auto at = [&](uint32_t px, uint32_t py) { return px < pw && py < ph ? prev[py * pw + px] : 0.0f; };
 	const uint32_t bx = 2 * x, by = 2 * y;
@@ -119,11 +128,35 @@ __global__ void depth_level_kernel(const float *prev, uint32_t pw, uint32_t ph, 
 	}
 	if (ph & 1u)
 		d = gmax(d, gmax(at(bx, by + 2), at(bx + 1, by + 2)));
-	cur[y * cw + x] = d;
+	return d;
+}
+
+// Levels of at most this many texels are made by one workgroup, level after level: a launch of its own per
+// level takes longer than such a level (1080p: seven launches of 2 to 5 us against one of the seven levels).
+constexpr uint32_t kTailTexels = 16384;
+
+} // namespace
+
+__global__ void depth_level_kernel(const float *prev, uint32_t pw, uint32_t ph, float *cur, uint32_t cw, uint32_t ch) {
+	const uint32_t x = blockIdx.x * blockDim.x + threadIdx.x, y = blockIdx.y * blockDim.y + threadIdx.y;
+	if (x < cw && y < ch)
+		cur[y * cw + x] = depth_texel(prev, pw, ph, x, y);
+}
+
+// Levels first .. n_levels - 1, each of at most kTailTexels texels.
+__global__ __launch_bounds__(1024) void depth_tail_kernel(DepthPyramid h, float *levels, uint32_t first) {
+	for (uint32_t i = first; i < h.n_levels; ++i) {
+		const float *prev = levels + h.offset[i - 1];
+		float *cur = levels + h.offset[i];
+		const uint32_t w = h.width[i], n = w * h.height[i];
+		for (uint32_t t = threadIdx.x; t < n; t += blockDim.x)
+			cur[t] = depth_texel(prev, h.width[i - 1], h.height[i - 1], t % w, t / w);
+		__syncthreads(); // the level is in memory for the whole workgroup
+	}
 }
 
 __global__ void cull_kernel(const hcm_mesh_info *infos, uint32_t n, CullParams cp, hcm_draw_cmd *opaque,
-                            hcm_draw_cmd *transparent, uint32_t *counts) {
+                            hcm_draw_cmd *transparent, CullCounts *counts, uint32_t *out_counts) {
 	const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
 	bool keep = false;
 	hcm_mesh_info m;
@@ -161,36 +194,48 @@ __global__ void cull_kernel(const hcm_mesh_info *infos, uint32_t n, CullParams c
 			continue;
 		uint32_t base = 0;
 		if (lane == __ffsll((unsigned long long)ballot) - 1)
-			base = atomicAdd(&counts[pass], (uint32_t)__popcll(ballot));
+			base = atomicAdd(&counts->kept[pass], (uint32_t)__popcll(ballot));
 		base = (uint32_t)__shfl((int)base, __ffsll((unsigned long long)ballot) - 1);
 		if (mine) {
 			const uint32_t slot = base + (uint32_t)__popcll(ballot & ((1ull << lane) - 1ull));
 			(pass ? transparent : opaque)[slot] = hcm_draw_cmd{m.index_count, 1u, m.first_index, m.vertex_offset, i};
 		}
 	}
+	// the last workgroup hands out the counts and clears them for the next launch (its own and the others' atomics
+	// have returned: their results gave the slots)
+	__syncthreads();
+	if (threadIdx.x == 0 && atomicAdd(&counts->done, 1u) == gridDim.x - 1) {
+		out_counts[0] = atomicAdd(&counts->kept[0], 0u);
+		out_counts[1] = atomicAdd(&counts->kept[1], 0u);
+		counts->kept[0] = counts->kept[1] = counts->done = 0;
+	}
 }
 
-hipError_t launch_mesh_infos(const hcm_mesh_rec *recs, uint32_t n, const int32_t *chunk_pos, hcm_mesh_info *out,
+hipError_t launch_mesh_infos(const hcm_mesh_rec *recs, const Counters *ctr, uint32_t persistent, uint32_t rec_cap,
+                             const int32_t *chunk_pos, hcm_mesh_info *out, hcm_mesh_info *out2, uint32_t *n,
                              hipStream_t stream) {
-	if (n == 0)
-		return hipSuccess;
-	hipLaunchKernelGGL(mesh_info_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, recs, n, chunk_pos, out);
+	hipLaunchKernelGGL(mesh_info_kernel, dim3((rec_cap + 255) / 256), dim3(256), 0, stream, recs, ctr, persistent, rec_cap,
+	                   chunk_pos, out, out2, n);
 	return hipGetLastError();
 }
 
-hipError_t launch_depth_level(const float *prev, uint32_t pw, uint32_t ph, float *cur, uint32_t cw, uint32_t ch,
-                              hipStream_t stream) {
-	const dim3 block(16, 16), grid((cw + 15) / 16, (ch + 15) / 16);
-	hipLaunchKernelGGL(depth_level_kernel, grid, block, 0, stream, prev, pw, ph, cur, cw, ch);
+hipError_t launch_depth_levels(const DepthPyramid &h, float *levels, hipStream_t stream) {
+	uint32_t i = 1;
+	for (; i < h.n_levels && (uint64_t)h.width[i] * h.height[i] > kTailTexels; ++i) {
+		const dim3 block(16, 16), grid((h.width[i] + 15) / 16, (h.height[i] + 15) / 16);
+		hipLaunchKernelGGL(depth_level_kernel, grid, block, 0, stream, levels + h.offset[i - 1], h.width[i - 1],
+		                   h.height[i - 1], levels + h.offset[i], h.width[i], h.height[i]);
+	}
+	if (i < h.n_levels)
+		hipLaunchKernelGGL(depth_tail_kernel, dim3(1), dim3(1024), 0, stream, h, levels, i);
 	return hipGetLastError();
 }
 
 hipError_t launch_cull(const hcm_mesh_info *infos, uint32_t n, const CullParams &cp, hcm_draw_cmd *opaque,
-                       hcm_draw_cmd *transparent, uint32_t *counts, hipStream_t stream) {
-	if (n == 0)
-		return hipSuccess;
-	hipLaunchKernelGGL(cull_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, infos, n, cp, opaque, transparent,
-	                   counts);
+                       hcm_draw_cmd *transparent, CullCounts *counts, uint32_t *out_counts, hipStream_t stream) {
+	// (without meshes one workgroup hands out the zero counts)
+	hipLaunchKernelGGL(cull_kernel, dim3((std::max(n, 1u) + 255) / 256), dim3(256), 0, stream, infos, n, cp, opaque,
+	                   transparent, counts, out_counts);
 	return hipGetLastError();
 }
 

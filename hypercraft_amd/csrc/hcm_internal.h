@@ -145,6 +145,26 @@ hipError_t launch_upload_scatter(const uint16_t *sblocks, const uint8_t *slight,
 hipError_t launch_edits(uint16_t *blocks, uint8_t *light, int8_t *heights, const VoxelEdit *edits, uint32_t n,
                         hipStream_t stream);
 int mesh_lds_bytes(int threads);
+
+// What a run left on the device, copied to pinned host memory by one kernel: a launch and a synchronisation
+// instead of copies that wait for one another (the totals say how much there is to copy).
+struct ExportParams {
+	const Counters *ctr = nullptr;
+	uint32_t persistent = 1; // totals: a persistent run's, else the cursors
+	const hcm_job_result *results = nullptr;
+	uint32_t n_jobs = 0;
+	const hcm_mesh_rec *recs = nullptr;
+	uint32_t rec_cap = 0; // records there can be, and that fit out_recs
+	const uint2 *verts = nullptr;
+	const uint16_t *idx = nullptr;
+	uint32_t quad_cap = 0; // quads that fit out_verts and out_idx: all of the run's or none
+	uint32_t *out_totals = nullptr; // quads, mesh records
+	hcm_job_result *out_results = nullptr;
+	hcm_mesh_rec *out_recs = nullptr;
+	uint2 *out_verts = nullptr;
+	uint16_t *out_idx = nullptr;
+};
+hipError_t launch_export(const ExportParams &p, hipStream_t stream);
 // Launchers (hcm_draw.hip)
 // Depth hierarchy of the renderer's depth image (client/include/client/rg/DepthHierarchyPass.hpp:166-196):
 // level 0 is the image, level i >= 1 is max(level i - 1 size >> 1, 1) per axis; the culling shader's
@@ -160,12 +180,18 @@ struct CullParams {
 	float view_proj[16]; // column-major
 	DepthPyramid hiz;    // data == nullptr: frustum test only
 };
-hipError_t launch_depth_level(const float *prev, uint32_t pw, uint32_t ph, float *cur, uint32_t cw, uint32_t ch,
-                              hipStream_t stream);
-hipError_t launch_mesh_infos(const hcm_mesh_rec *recs, uint32_t n, const int32_t *chunk_pos, hcm_mesh_info *out,
+// levels 1 .. h.n_levels - 1 from level 0, in `levels` (h.data's memory)
+hipError_t launch_depth_levels(const DepthPyramid &h, float *levels, hipStream_t stream);
+// The infos of the run's records (at most rec_cap); n receives their number, out2 (may be null) a second copy.
+hipError_t launch_mesh_infos(const hcm_mesh_rec *recs, const Counters *ctr, uint32_t persistent, uint32_t rec_cap,
+                             const int32_t *chunk_pos, hcm_mesh_info *out, hcm_mesh_info *out2, uint32_t *n,
                              hipStream_t stream);
+struct CullCounts { // zero between launches
+	uint32_t kept[2], done;
+};
+// out_counts: opaque and transparent draws
 hipError_t launch_cull(const hcm_mesh_info *infos, uint32_t n, const CullParams &cp, hcm_draw_cmd *opaque,
-                       hcm_draw_cmd *transparent, uint32_t *counts, hipStream_t stream);
+                       hcm_draw_cmd *transparent, CullCounts *counts, uint32_t *out_counts, hipStream_t stream);
 // Launchers (hcm_light.hip)
 hipError_t launch_light_prep(const LightParams &p, hipStream_t stream);
 hipError_t launch_light(const LightParams &p, int grid, hipStream_t stream);

@@ -1842,6 +1842,36 @@ hipError_t launch_upload_scatter(const uint16_t *sblocks, const uint8_t *slight,
 	return hipGetLastError();
 }
 
+// n words of type T from src to dst by the whole grid.
+template <typename T> __device__ __forceinline__ void copy_words(void *dst, const void *src, size_t n) {
+	for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
+		reinterpret_cast<T *>(dst)[i] = reinterpret_cast<const T *>(src)[i];
+}
+
+// Bound by the link to the host (56 GB/s): 64 KB of results and 120 KB of records of 4,096 jobs take about 7 us
+// with the launch, where three copies and two synchronisations took about 75.
+__global__ __launch_bounds__(256) void export_kernel(ExportParams p) {
+	const uint32_t quads = p.persistent ? p.ctr->total_quads : p.ctr->pool_cursor;
+	const uint32_t meshes = p.persistent ? p.ctr->total_meshes : p.ctr->mesh_cursor;
+	if (blockIdx.x == 0 && threadIdx.x == 0)
+		p.out_totals[0] = quads, p.out_totals[1] = meshes;
+	if (p.results)
+		copy_words<uint4>(p.out_results, p.results, p.n_jobs);
+	if (p.recs)
+		copy_words<uint2>(p.out_recs, p.recs, (size_t)min(meshes, p.rec_cap) * (sizeof(hcm_mesh_rec) / sizeof(uint2)));
+	if (p.verts && quads <= p.quad_cap) {
+		copy_words<uint4>(p.out_verts, p.verts, 2 * (size_t)quads);
+		copy_words<uint32_t>(p.out_idx, p.idx, 3 * (size_t)quads);
+	}
+}
+static_assert(sizeof(hcm_job_result) == sizeof(uint4) && sizeof(hcm_mesh_rec) % sizeof(uint2) == 0, "whole words");
+
+hipError_t launch_export(const ExportParams &p, hipStream_t stream) {
+	const int grid = p.verts ? 256 : 64;
+	hipLaunchKernelGGL(export_kernel, dim3(grid), dim3(256), 0, stream, p);
+	return hipGetLastError();
+}
+
 hipError_t launch_reset(Counters *ctr, hipStream_t stream) {
 	hipLaunchKernelGGL(reset_kernel, dim3(1), dim3(64), 0, stream, ctr);
 	return hipGetLastError();
