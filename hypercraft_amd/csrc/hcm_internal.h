@@ -149,8 +149,9 @@ int mesh_lds_bytes(int threads);
 // What a run left on the device, copied to pinned host memory by one kernel: a launch and a synchronisation
 // instead of copies that wait for one another (the totals say how much there is to copy).
 struct ExportParams {
-	const Counters *ctr = nullptr;
-	uint32_t persistent = 1; // totals: a persistent run's, else the cursors
+	const Counters *ctr = nullptr; // null: given_quads quads, no records
+	uint32_t persistent = 1;       // totals: a persistent run's, else the cursors
+	uint32_t given_quads = 0;
 	const hcm_job_result *results = nullptr;
 	uint32_t n_jobs = 0;
 	const hcm_mesh_rec *recs = nullptr;

@@ -1851,9 +1851,12 @@ template <typename T> __device__ __forceinline__ void copy_words(void *dst, cons
 // Bound by the link to the host (56 GB/s): 64 KB of results and 120 KB of records of 4,096 jobs take about 7 us
 // with the launch, where three copies and two synchronisations took about 75.
 __global__ __launch_bounds__(256) void export_kernel(ExportParams p) {
-	const uint32_t quads = p.persistent ? p.ctr->total_quads : p.ctr->pool_cursor;
-	const uint32_t meshes = p.persistent ? p.ctr->total_meshes : p.ctr->mesh_cursor;
-	if (blockIdx.x == 0 && threadIdx.x == 0)
+	uint32_t quads = p.given_quads, meshes = 0;
+	if (p.ctr) {
+		quads = p.persistent ? p.ctr->total_quads : p.ctr->pool_cursor;
+		meshes = p.persistent ? p.ctr->total_meshes : p.ctr->mesh_cursor;
+	}
+	if (p.out_totals && blockIdx.x == 0 && threadIdx.x == 0)
 		p.out_totals[0] = quads, p.out_totals[1] = meshes;
 	if (p.results)
 		copy_words<uint4>(p.out_results, p.results, p.n_jobs);

@@ -4,11 +4,12 @@
 // applies them to the world model in arrival order (request k gets epoch k), keeps the set of chunks whose
 // mesh is stale, and, whenever fewer than max_inflight batches are on the device, forms a batch from what
 // is pending:
-//   copy stream:    first-time chunk loads -> their fresh slots (no running batch reads a fresh slot);
+//   copy stream:    first-time chunk loads -> their fresh slots (no running batch reads a fresh slot), by a
+//                   kernel that reads them where the host staged them, in pinned memory;
 //   compute stream: wait for those copies; reloads of resident chunks (in stream order, after every
 //                   earlier batch that may read them); the batch's voxel edits; then up to max_batch stale
 //                   chunks meshed by the persistent kernel into an arena taken from the vertex pool, and
-//                   the per-chunk results copied back.
+//                   the per-chunk results written back to pinned memory.
 // Uploads of batch i+1 overlap the meshing of batch i. A batch meshes chunks only when every pending data
 // change has been flushed into it, so its meshes reflect all requests up to the epoch at its launch; a
 // batch that cannot flush everything (upload or edit limits) carries data only, and its "applied epoch"
@@ -111,9 +112,16 @@ struct PendingEdit {
 	uint64_t first_epoch; // earliest request still pending for this voxel
 };
 
+// Batches of up to this many jobs mesh from their job table in pinned memory; the kernels of larger ones would
+// wait for it at every job, and it is copied.
+constexpr uint32_t kPinnedJobs = 256;
+// A chunk's meshes of up to this many quads are handed out by way of pinned memory, by one kernel.
+constexpr uint32_t kPinnedQuads = 8192;
+
+// The kernels read what the host staged, and write what it reads back, in pinned memory: an edit's batch is three
+// launches (edits, meshing, results) where it was two, two copies up and three copies down.
 struct BatchSlot { // device and pinned buffers of one in-flight batch
 	uint32_t *d_nbr = nullptr;
-	VoxelEdit *d_edits = nullptr;
 	Counters *d_ctr = nullptr;
 	hcm_job_result *d_res = nullptr;
 	hcm_mesh_rec *d_recs = nullptr;
@@ -123,22 +131,18 @@ struct BatchSlot { // device and pinned buffers of one in-flight batch
 	uint8_t *h_light = nullptr;
 	int8_t *h_heights = nullptr;
 	hcm_job_result *h_res = nullptr;
-	// the batch's chunk uploads: staged on the host, copied once, then scattered to their slots on the device
-	uint16_t *d_up_blocks = nullptr;
-	uint8_t *d_up_light = nullptr;
-	int8_t *d_up_heights = nullptr;
-	uint2 *d_moves = nullptr, *h_moves = nullptr;
+	// the batch's chunk uploads: staged on the host (h_blocks, ...) and scattered to their slots from there
+	uint2 *h_moves = nullptr;
 	// light rebuild (HCM_LIGHT_REBUILD): the slots the jobs read, queues, rebuilt halo light
-	uint32_t *d_rslots = nullptr, *h_rslots = nullptr;
+	uint32_t *h_rslots = nullptr;
 	Counters *d_lctr = nullptr;
 	uint8_t *d_halo = nullptr;
 	hcm_mesh_rec *h_recs = nullptr;
-	Counters *h_ctr = nullptr;
+	uint32_t *h_totals = nullptr; // quads, mesh records
 	hipEvent_t ev_up = nullptr, ev_k0 = nullptr, ev_k1 = nullptr, ev_done = nullptr;
 	bool busy = false;
 	bool arena_was_largest = false; // the arena took the largest free range there was
 	uint64_t id = 0, epoch = 0;     // epoch: every request up to it is applied on the device
-	uint32_t recs_copied = 0;       // mesh records copied back with the results (the usual count)
 	std::vector<uint64_t> jobs;     // the first n_urgent were taken from the high-priority queue
 	uint32_t n_urgent = 0;
 	Range arena;
@@ -166,6 +170,7 @@ struct hcm_server {
 	uint32_t *d_levels = nullptr;
 	uint2 *d_verts = nullptr;
 	uint16_t *d_idx = nullptr;
+	uint8_t *h_mesh = nullptr; // pinned: a chunk's quads on their way to hcm_server_chunk_mesh's caller (world_mu)
 	std::vector<BatchSlot> slots;
 	std::atomic<int> error{HCM_OK};
 
@@ -449,9 +454,8 @@ struct hcm_server {
 			std::vector<uint8_t>().swap(r->light);
 			std::vector<int8_t>().swap(r->heights);
 		}
-		// a slot's data, blocks and light bytes or sunlight heights, goes up with the batch's others in one
-		// copy per array; first-time loads are scattered to their slots on the copy stream, reloads on the
-		// compute stream after it, in order with the earlier batches that may read their slots
+		// one kernel takes the staged chunks to their slots, first-time loads on the copy stream, reloads on the
+		// compute stream, in order with the earlier batches that may read their slots
 		uint32_t n_fresh = 0;
 		for (uint32_t i = 0; i < n_up; ++i)
 			if (!uploads[i].reload)
@@ -459,20 +463,14 @@ struct hcm_server {
 		for (uint32_t i = 0, k = n_fresh; i < n_up; ++i)
 			if (uploads[i].reload)
 				b.h_moves[k++] = make_uint2(i, uploads[i].slot);
-		if (n_up) {
-			HCM_CHECK(hipMemcpyAsync(b.d_up_blocks, b.h_blocks, n_up * V * 2, hipMemcpyHostToDevice, s_copy));
-			if (relight())
-				HCM_CHECK(hipMemcpyAsync(b.d_up_heights, b.h_heights, n_up * 256, hipMemcpyHostToDevice, s_copy));
-			else
-				HCM_CHECK(hipMemcpyAsync(b.d_up_light, b.h_light, n_up * V, hipMemcpyHostToDevice, s_copy));
-			HCM_CHECK(hipMemcpyAsync(b.d_moves, b.h_moves, n_up * sizeof(uint2), hipMemcpyHostToDevice, s_copy));
+		if (n_fresh) {
+			HCM_CHECK(launch_upload_scatter(b.h_blocks, b.h_light, b.h_heights, b.h_moves, n_fresh, d_blocks, d_light,
+			                                d_heights, s_copy));
+			HCM_CHECK(hipEventRecord(b.ev_up, s_copy));
+			HCM_CHECK(hipStreamWaitEvent(s_comp, b.ev_up, 0));
 		}
-		HCM_CHECK(launch_upload_scatter(b.d_up_blocks, b.d_up_light, b.d_up_heights, b.d_moves, n_fresh, d_blocks,
-		                                d_light, d_heights, s_copy));
-		HCM_CHECK(hipEventRecord(b.ev_up, s_copy));
-		HCM_CHECK(hipStreamWaitEvent(s_comp, b.ev_up, 0));
-		HCM_CHECK(launch_upload_scatter(b.d_up_blocks, b.d_up_light, b.d_up_heights, b.d_moves + n_fresh,
-		                                n_up - n_fresh, d_blocks, d_light, d_heights, s_comp));
+		HCM_CHECK(launch_upload_scatter(b.h_blocks, b.h_light, b.h_heights, b.h_moves + n_fresh, n_up - n_fresh, d_blocks,
+		                                d_light, d_heights, s_comp));
 		uploads.erase(uploads.begin(), uploads.begin() + n_up);
 
 		uint32_t k = 0;
@@ -483,33 +481,34 @@ struct hcm_server {
 		for (auto &e : edits)
 			applied = std::min(applied, e.second.first_epoch - 1);
 		b.epoch = applied;
-		if (n_ed) {
-			HCM_CHECK(hipMemcpyAsync(b.d_edits, b.h_edits, n_ed * sizeof(VoxelEdit), hipMemcpyHostToDevice, s_comp));
-			HCM_CHECK(launch_edits(d_blocks, d_light, d_heights, b.d_edits, n_ed, s_comp));
-		}
+		if (n_ed)
+			HCM_CHECK(launch_edits(d_blocks, d_light, d_heights, b.h_edits, n_ed, s_comp));
 
 		if (!b.jobs.empty()) {
 			for (size_t j = 0; j < b.jobs.size(); ++j)
 				std::memcpy(b.h_nbr + 27 * j, world.at(b.jobs[j]).nbr, 27 * sizeof(uint32_t));
-			HCM_CHECK(hipMemcpyAsync(b.d_nbr, b.h_nbr, b.jobs.size() * 27 * 4, hipMemcpyHostToDevice, s_comp));
+			const uint32_t *nbr = b.h_nbr;
+			if (b.jobs.size() > kPinnedJobs) {
+				HCM_CHECK(hipMemcpyAsync(b.d_nbr, b.h_nbr, b.jobs.size() * 27 * 4, hipMemcpyHostToDevice, s_comp));
+				nbr = b.d_nbr;
+			}
 			HCM_CHECK(hipEventRecord(b.ev_k0, s_comp));
 			if (relight()) { // rebuild the jobs' light from the slots they read (ChunkMeshTask.cpp:48-111)
 				std::vector<uint32_t> rs(b.h_nbr, b.h_nbr + 27 * b.jobs.size());
 				std::sort(rs.begin(), rs.end());
 				rs.erase(std::unique(rs.begin(), rs.end()), rs.end());
 				std::memcpy(b.h_rslots, rs.data(), rs.size() * 4);
-				HCM_CHECK(hipMemcpyAsync(b.d_rslots, b.h_rslots, rs.size() * 4, hipMemcpyHostToDevice, s_comp));
 				LightParams lp;
 				std::memset(&lp, 0, sizeof(lp));
 				lp.blocks = d_blocks;
 				lp.heights = d_heights;
 				lp.light_info = info.light_info;
-				lp.slots = b.d_rslots;
+				lp.slots = b.h_rslots;
 				lp.n_slots = (uint32_t)rs.size();
 				lp.n_jobs = (uint32_t)b.jobs.size();
 				lp.packed = d_packed;
 				lp.levels = d_levels;
-				lp.nbr = b.d_nbr;
+				lp.nbr = nbr;
 				lp.ctr = b.d_lctr;
 				lp.halo_light = b.d_halo;
 				lp.self_reset = 1; // the slot's light queues start at zero; the run's last workgroup clears them
@@ -521,7 +520,7 @@ struct hcm_server {
 			p.reg = info.reg;
 			p.blocks = d_blocks;
 			p.light = d_light;
-			p.nbr = b.d_nbr;
+			p.nbr = nbr;
 			p.n_jobs = (uint32_t)b.jobs.size();
 			p.persistent = 1;
 			p.pool_cap = (uint32_t)b.arena.count;
@@ -536,12 +535,14 @@ struct hcm_server {
 			const int grid = (int)std::max<uint32_t>(1, std::min<uint32_t>(info.grid, (uint32_t)b.jobs.size()));
 			HCM_CHECK(launch_mesh(p, (int)info.threads, grid, s_comp));
 			HCM_CHECK(hipEventRecord(b.ev_k1, s_comp));
-			HCM_CHECK(hipMemcpyAsync(b.h_res, b.d_res, b.jobs.size() * sizeof(hcm_job_result), hipMemcpyDeviceToHost,
-			                         s_comp));
-			HCM_CHECK(hipMemcpyAsync(b.h_ctr, b.d_ctr, sizeof(Counters), hipMemcpyDeviceToHost, s_comp));
-			b.recs_copied = std::min<uint32_t>(rec_cap(), 3 * (uint32_t)b.jobs.size() + 64);
-			HCM_CHECK(hipMemcpyAsync(b.h_recs, b.d_recs, b.recs_copied * sizeof(hcm_mesh_rec), hipMemcpyDeviceToHost,
-			                         s_comp));
+			ExportParams e;
+			e.ctr = b.d_ctr;
+			e.results = b.d_res, e.out_results = b.h_res;
+			e.n_jobs = (uint32_t)b.jobs.size();
+			e.recs = b.d_recs, e.out_recs = b.h_recs;
+			e.rec_cap = rec_cap();
+			e.out_totals = b.h_totals;
+			HCM_CHECK(launch_export(e, s_comp));
 		}
 		HCM_CHECK(hipEventRecord(b.ev_done, s_comp));
 		return 0;
@@ -553,13 +554,9 @@ struct hcm_server {
 		if (!b.jobs.empty()) {
 			float ms = 0;
 			HCM_CHECK(hipEventElapsedTime(&ms, b.ev_k0, b.ev_k1));
-			const uint32_t n_recs = std::min(b.h_ctr->total_meshes, rec_cap());
-			if (n_recs > b.recs_copied) // more overflow meshes than usual: fetch the rest
-				HCM_CHECK(hipMemcpy(b.h_recs + b.recs_copied, b.d_recs + b.recs_copied,
-				                    (n_recs - b.recs_copied) * sizeof(hcm_mesh_rec), hipMemcpyDeviceToHost));
 			std::vector<uint2> hv;
 			std::vector<uint16_t> hi;
-			const uint64_t used = std::min<uint64_t>(b.h_ctr->total_quads, b.arena.count);
+			const uint64_t used = std::min<uint64_t>(b.h_totals[0], b.arena.count);
 			if (cfg.keep_history && used) {
 				hv.resize(used * 4);
 				hi.resize(used * 6);
@@ -753,13 +750,12 @@ struct hcm_server {
 
 static void free_server(hcm_server *s) {
 	for (auto &b : s->slots) {
-		for (void *p : {(void *)b.d_nbr, (void *)b.d_edits, (void *)b.d_ctr, (void *)b.d_res, (void *)b.d_recs,
-		                (void *)b.d_rslots, (void *)b.d_lctr, (void *)b.d_halo, (void *)b.d_up_blocks,
-		                (void *)b.d_up_light, (void *)b.d_up_heights, (void *)b.d_moves})
+		for (void *p : {(void *)b.d_nbr, (void *)b.d_ctr, (void *)b.d_res, (void *)b.d_recs, (void *)b.d_lctr,
+		                (void *)b.d_halo})
 			if (p)
 				(void)hipFree(p);
 		for (void *p : {(void *)b.h_nbr, (void *)b.h_edits, (void *)b.h_blocks, (void *)b.h_light, (void *)b.h_res,
-		                (void *)b.h_recs, (void *)b.h_ctr, (void *)b.h_heights, (void *)b.h_rslots, (void *)b.h_moves})
+		                (void *)b.h_recs, (void *)b.h_totals, (void *)b.h_heights, (void *)b.h_rslots, (void *)b.h_moves})
 			if (p)
 				(void)hipHostFree(p);
 		for (hipEvent_t e : {b.ev_up, b.ev_k0, b.ev_k1, b.ev_done})
@@ -770,6 +766,8 @@ static void free_server(hcm_server *s) {
 	                (void *)s->d_packed, (void *)s->d_levels})
 		if (p)
 			(void)hipFree(p);
+	if (s->h_mesh)
+		(void)hipHostFree(s->h_mesh);
 	if (s->s_copy)
 		(void)hipStreamDestroy(s->s_copy);
 	if (s->s_comp)
@@ -801,11 +799,11 @@ static int server_init(hcm_server *s) {
 	}
 	HCM_CHECK(dalloc(&s->d_verts, (size_t)c.pool_quads * 4));
 	HCM_CHECK(dalloc(&s->d_idx, (size_t)c.pool_quads * 6));
+	HCM_CHECK(halloc(&s->h_mesh, (size_t)kPinnedQuads * 44));
 	s->pool = new RangeAllocator(c.pool_quads);
 	s->slots.resize(c.max_inflight);
 	for (auto &b : s->slots) {
 		HCM_CHECK(dalloc(&b.d_nbr, (size_t)c.max_batch * 27));
-		HCM_CHECK(dalloc(&b.d_edits, kMaxEdits));
 		HCM_CHECK(dalloc(&b.d_ctr, 1));
 		HCM_CHECK(hipMemset(b.d_ctr, 0, sizeof(Counters)));
 		HCM_CHECK(dalloc(&b.d_res, c.max_batch));
@@ -813,17 +811,11 @@ static int server_init(hcm_server *s) {
 		HCM_CHECK(halloc(&b.h_nbr, (size_t)c.max_batch * 27));
 		HCM_CHECK(halloc(&b.h_edits, kMaxEdits));
 		HCM_CHECK(halloc(&b.h_blocks, (size_t)kMaxUploads * HCM_CHUNK_VOXELS));
-		HCM_CHECK(dalloc(&b.d_up_blocks, (size_t)kMaxUploads * HCM_CHUNK_VOXELS));
 		HCM_CHECK(halloc(&b.h_moves, kMaxUploads));
-		HCM_CHECK(dalloc(&b.d_moves, kMaxUploads));
-		if (!s->relight()) {
+		if (!s->relight())
 			HCM_CHECK(halloc(&b.h_light, (size_t)kMaxUploads * HCM_CHUNK_VOXELS));
-			HCM_CHECK(dalloc(&b.d_up_light, (size_t)kMaxUploads * HCM_CHUNK_VOXELS));
-		}
 		if (s->relight()) {
 			HCM_CHECK(halloc(&b.h_heights, (size_t)kMaxUploads * 256));
-			HCM_CHECK(dalloc(&b.d_up_heights, (size_t)kMaxUploads * 256));
-			HCM_CHECK(dalloc(&b.d_rslots, (size_t)c.max_batch * 27));
 			HCM_CHECK(halloc(&b.h_rslots, (size_t)c.max_batch * 27));
 			HCM_CHECK(dalloc(&b.d_lctr, 1));
 			HCM_CHECK(hipMemset(b.d_lctr, 0, sizeof(Counters)));
@@ -831,7 +823,7 @@ static int server_init(hcm_server *s) {
 		}
 		HCM_CHECK(halloc(&b.h_res, c.max_batch));
 		HCM_CHECK(halloc(&b.h_recs, s->rec_cap()));
-		HCM_CHECK(halloc(&b.h_ctr, 1));
+		HCM_CHECK(halloc(&b.h_totals, 2));
 		HCM_CHECK(hipEventCreateWithFlags(&b.ev_up, hipEventDisableTiming));
 		HCM_CHECK(hipEventCreate(&b.ev_k0));
 		HCM_CHECK(hipEventCreate(&b.ev_k1));
@@ -1014,7 +1006,23 @@ extern "C" int hcm_server_chunk_mesh(hcm_server *s, int32_t cx, int32_t cy, int3
 	auto it = s->world.find(chunk_key(cx, cy, cz));
 	if (it == s->world.end() || !it->second.has_mesh)
 		return HCM_ERR_INVALID;
-	return copy_meshes(it->second.recs, s->d_verts, s->d_idx, true, out);
+	const Chunk &c = it->second;
+	if (c.mesh.count == 0 || c.mesh.count > kPinnedQuads)
+		return copy_meshes(c.recs, s->d_verts, s->d_idx, true, out);
+	// the chunk's quads lie together: one kernel brings them to pinned memory (on the copy stream: they were made
+	// by a finished batch, and later ones may be running)
+	ExportParams e;
+	e.given_quads = e.quad_cap = (uint32_t)c.mesh.count;
+	e.verts = s->d_verts + 4 * c.mesh.first;
+	e.idx = s->d_idx + 6 * c.mesh.first;
+	e.out_verts = reinterpret_cast<uint2 *>(s->h_mesh);
+	e.out_idx = reinterpret_cast<uint16_t *>(s->h_mesh + (size_t)kPinnedQuads * 32);
+	HCM_CHECK(launch_export(e, s->s_copy));
+	HCM_CHECK(hipStreamSynchronize(s->s_copy));
+	std::vector<hcm_mesh_rec> recs = c.recs;
+	for (auto &rec : recs)
+		rec.first_quad -= (uint32_t)c.mesh.first;
+	return copy_meshes(recs, e.out_verts, e.out_idx, false, out);
 }
 
 extern "C" int hcm_server_get_stats(hcm_server *s, hcm_server_stats *out) {

@@ -101,6 +101,20 @@ hipError_t launch_light(const LightParams &p, int, hipStream_t) {
 	std::memset(p.halo_light, 0, (size_t)p.n_jobs * kLightJobBytes);
 	return hipSuccess;
 }
+hipError_t launch_export(const ExportParams &p, hipStream_t) {
+	const uint32_t quads = p.ctr ? p.ctr->total_quads : p.given_quads, meshes = p.ctr ? p.ctr->total_meshes : 0;
+	if (p.out_totals)
+		p.out_totals[0] = quads, p.out_totals[1] = meshes;
+	if (p.results)
+		std::memcpy(p.out_results, p.results, p.n_jobs * sizeof(hcm_job_result));
+	if (p.recs)
+		std::memcpy(p.out_recs, p.recs, (meshes < p.rec_cap ? meshes : p.rec_cap) * sizeof(hcm_mesh_rec));
+	if (p.verts && quads <= p.quad_cap) {
+		std::memcpy(p.out_verts, p.verts, (size_t)quads * 4 * sizeof(uint2));
+		std::memcpy(p.out_idx, p.idx, (size_t)quads * 12);
+	}
+	return hipSuccess;
+}
 hipError_t launch_reset(Counters *ctr, hipStream_t) {
 	*ctr = Counters{};
 	return hipSuccess;
