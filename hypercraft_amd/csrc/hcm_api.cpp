@@ -41,9 +41,9 @@ struct DeviceTables {
 	std::vector<uint32_t> pid_vox;
 	std::vector<uint32_t> codes;
 	std::vector<hcm_custom_mesh> meshes;
-	std::vector<uint8_t> tex_flags;
+	std::vector<uint32_t> mesh_sums;
 	std::vector<uint8_t> light_info; // [65536]: light level | kLightInfoPass
-	uint32_t flow_pid_base = 0, flow_tex = 0, src_id = 0, flow_id = 0;
+	uint32_t flow_pid_base = 0, flow_tex = 0, flow_trans = 0, src_id = 0, flow_id = 0;
 };
 
 int build_tables(const hcm_registry *r, DeviceTables *t) {
@@ -178,8 +178,14 @@ int build_tables(const hcm_registry *r, DeviceTables *t) {
 		t->light_info[d] = uint8_t(lv | (tr != 0 ? kLightInfoPass : 0u) | (tr == 2 ? kLightInfoVertical : 0u));
 	}
 	t->meshes.assign(r->meshes, r->meshes + r->n_meshes);
-	t->tex_flags.assign(r->tex_flags, r->tex_flags + r->n_tex);
+	for (const hcm_custom_mesh &m : t->meshes) {
+		uint32_t n = std::min<uint32_t>(m.face_count, HCM_MAX_FACES), trans = 0;
+		for (uint32_t j = 0; j < n; ++j)
+			trans |= (tex_flags(m.faces[j].texture) & HCM_TEX_TRANS_PASS ? 1u : 0u) << j;
+		t->mesh_sums.push_back(n | trans << 16);
+	}
 	t->flow_tex = r->liquid_flow_tex;
+	t->flow_trans = tex_flags(r->liquid_flow_tex) & HCM_TEX_TRANS_PASS ? 1u : 0u;
 	t->src_id = r->liquid_source_id;
 	t->flow_id = r->liquid_flow_id;
 	return HCM_OK;
@@ -231,7 +237,7 @@ struct hcm_ctx {
 	uint32_t *d_pid_vox = nullptr;
 	uint32_t *d_codes = nullptr;
 	hcm_custom_mesh *d_meshes = nullptr;
-	uint8_t *d_tex_flags = nullptr;
+	uint32_t *d_mesh_sums = nullptr;
 	uint8_t *d_light_info = nullptr;
 	std::vector<uint8_t> light_info; // host copy
 	// batched pool
@@ -331,7 +337,7 @@ static void free_ctx(hcm_ctx *c) {
 	dfree(c->d_pid_vox);
 	dfree(c->d_codes);
 	dfree(c->d_meshes);
-	dfree(c->d_tex_flags);
+	dfree(c->d_mesh_sums);
 	dfree(c->d_light_info);
 	dfree(c->d_verts);
 	dfree(c->d_idx);
@@ -375,7 +381,7 @@ static int create_impl(hcm_ctx *c, const hcm_registry *registry, uint64_t pool_q
 	HCM_HIP(dmalloc(&c->d_pid_vox, t.pid_vox.size()));
 	HCM_HIP(dmalloc(&c->d_codes, t.codes.size()));
 	HCM_HIP(dmalloc(&c->d_meshes, t.meshes.size()));
-	HCM_HIP(dmalloc(&c->d_tex_flags, t.tex_flags.size()));
+	HCM_HIP(dmalloc(&c->d_mesh_sums, t.mesh_sums.size()));
 	HCM_HIP(dmalloc(&c->d_light_info, t.light_info.size()));
 	HCM_HIP(hipMemcpy(c->d_light_info, t.light_info.data(), t.light_info.size(), hipMemcpyHostToDevice));
 	c->light_info = t.light_info;
@@ -386,19 +392,19 @@ static int create_impl(hcm_ctx *c, const hcm_registry *registry, uint64_t pool_q
 	if (!t.meshes.empty())
 		HCM_HIP(hipMemcpy(c->d_meshes, t.meshes.data(), t.meshes.size() * sizeof(hcm_custom_mesh),
 		                  hipMemcpyHostToDevice));
-	if (!t.tex_flags.empty())
-		HCM_HIP(hipMemcpy(c->d_tex_flags, t.tex_flags.data(), t.tex_flags.size(), hipMemcpyHostToDevice));
+	if (!t.mesh_sums.empty())
+		HCM_HIP(hipMemcpy(c->d_mesh_sums, t.mesh_sums.data(), t.mesh_sums.size() * 4, hipMemcpyHostToDevice));
 	c->reg.pid_of = c->d_pid_of;
 	c->reg.rows = c->d_rows;
 	c->reg.pid_vox = c->d_pid_vox;
 	c->reg.codes = c->d_codes;
 	c->reg.meshes = c->d_meshes;
-	c->reg.tex_flags = c->d_tex_flags;
+	c->reg.mesh_sums = c->d_mesh_sums;
 	c->reg.n_pid = (uint32_t)t.rows.size();
 	c->reg.n_codes = (uint32_t)t.codes.size();
-	c->reg.n_tex = (uint32_t)t.tex_flags.size();
 	c->reg.flow_pid_base = t.flow_pid_base;
 	c->reg.flow_tex = t.flow_tex;
+	c->reg.flow_trans = t.flow_trans;
 	c->reg.src_id = t.src_id;
 	c->reg.flow_id = t.flow_id;
 

@@ -47,9 +47,9 @@ struct DevReg {
 	const uint32_t *pid_vox;       // [n_pid]: voxel-word template (everything but the light fields)
 	const uint32_t *codes;         // [n_codes]
 	const hcm_custom_mesh *meshes; // [n_meshes]
-	const uint8_t *tex_flags;      // [n_tex] by texture id
-	uint32_t n_pid, n_codes, n_tex, flow_pid_base;
-	uint32_t flow_tex, src_id, flow_id, pad;
+	const uint32_t *mesh_sums;     // [n_meshes]: faces | (bit j: face j goes to the transparent pass) << 16
+	uint32_t n_pid, n_codes, flow_pid_base;
+	uint32_t flow_tex, flow_trans, src_id, flow_id;
 };
 
 // The persistent kernels' job list is cut into kQueues contiguous parts, one per XCD (gfx950 has 8,

@@ -497,11 +497,6 @@ struct CustomCell {
 	uint32_t flow_set; // liquid flow: emitted face kinds
 };
 
-__device__ __forceinline__ bool tex_trans_pass(const MeshParams &p, uint16_t t) {
-	const uint32_t id = t & 0x1fffu;
-	return id < p.reg.n_tex && (p.reg.tex_flags[id] & HCM_TEX_TRANS_PASS);
-}
-
 template <int NT>
 __device__ __forceinline__ CustomCell custom_cell(const MeshParams &p, const Smem<NT> &s, const JobBlocks &blocks, int cell) {
 	const int x = cell & 15, z = (cell >> 4) & 15, y = cell >> 8;
@@ -515,20 +510,26 @@ __device__ __forceinline__ CustomCell custom_cell(const MeshParams &p, const Sme
 	c.trans = 0;
 	c.flow_set = 0;
 	c.fl.h = 0, c.fl.liq_side = 0;
-	const hcm_custom_mesh &m = p.reg.meshes[c.mesh];
+	const uint32_t sum = p.reg.mesh_sums[c.mesh]; // (one load: the faces' textures and flags would be two per face)
 	if (c.flow) {
-		c.fl = flow_heights(p, blocks, x, y, z, m.flow_height);
+		c.fl = flow_heights(p, blocks, x, y, z, p.reg.meshes[c.mesh].flow_height);
 		c.flow_set = flow_face_set(c.fl);
 		c.count = __popc(c.flow_set);
-		if (tex_trans_pass(p, uint16_t(p.reg.flow_tex)))
+		if (p.reg.flow_trans)
 			c.trans = (1u << c.count) - 1u;
 	} else {
-		c.count = m.face_count > HCM_MAX_FACES ? HCM_MAX_FACES : m.face_count;
-		for (uint32_t j = 0; j < c.count; ++j)
-			if (tex_trans_pass(p, m.faces[j].texture))
-				c.trans |= 1u << j;
+		c.count = sum & 0x1fu;
+		c.trans = sum >> 16;
 	}
 	return c;
+}
+
+// The custom-mesh cells among this thread's 4096 / NT.
+template <int NT> __device__ __forceinline__ uint32_t custom_cells(const Smem<NT> &s) {
+	constexpr int n = HCM_CHUNK_VOXELS / NT;
+	static_assert(n <= 32 && 32 % n == 0, "a thread's cells in one word");
+	const uint32_t at = threadIdx.x * n;
+	return (s.custom_bits[at >> 5] >> (at & 31)) & uint32_t((1ull << n) - 1ull);
 }
 
 __device__ __forceinline__ hcm_mesh_face custom_face(const MeshParams &p, const CustomCell &c, int j) {
@@ -621,19 +622,46 @@ __device__ __forceinline__ void emit_quad(const MeshParams &p, const Smem<NT> &s
 	}
 }
 
-__device__ __forceinline__ uint32_t lerp16(uint32_t a, uint32_t b, uint32_t t) { return a * (16u - t) + b * t; }
-__device__ __forceinline__ uint32_t interp(uint32_t l0, uint32_t l1, uint32_t l2, uint32_t l3, uint32_t h0, uint32_t h1,
-                                           uint32_t h2, uint32_t h3, uint32_t du, uint32_t dv, uint32_t dw) {
-	// light4_interpolate (:165-196): trilinear in 1/16 steps, rounded up
-	const uint32_t lo = lerp16(lerp16(l0, l1, du), lerp16(l3, l2, du), dv);
-	const uint32_t hi = lerp16(lerp16(h0, h1, du), lerp16(h3, h2, du), dv);
-	const uint32_t sum = lerp16(lo, hi, dw);
+// light4_interpolate (:165-196): trilinear in 1/16 steps, rounded up, for two values of at most 63 in the
+// half-words of each corner word. The corners' plane (du, dv) stays within 16 bits (63 * 256); the last step, between
+// the planes (dw), is in 32.
+typedef uint16_t halves __attribute__((vector_size(4)));
+__device__ __forceinline__ halves lerp16(halves a, halves b, uint32_t t) {
+	const halves s = {uint16_t(16u - t), uint16_t(16u - t)}, u = {uint16_t(t), uint16_t(t)};
+	return a * s + b * u;
+}
+__device__ __forceinline__ halves as_halves(uint32_t v) {
+	const halves h = {uint16_t(v), uint16_t(v >> 16)};
+	return h;
+}
+struct Interp {
+	uint32_t first, second;
+};
+__device__ __forceinline__ uint32_t interp32(const uint32_t l[4], const uint32_t h[4], int shift, uint32_t du, uint32_t dv,
+                                             uint32_t dw) {
+	const auto v = [shift](uint32_t w) { return (w >> shift) & 0xffffu; };
+	const auto lerp = [](uint32_t a, uint32_t b, uint32_t t) { return a * (16u - t) + b * t; };
+	const uint32_t lo = lerp(lerp(v(l[0]), v(l[1]), du), lerp(v(l[3]), v(l[2]), du), dv);
+	const uint32_t hi = lerp(lerp(v(h[0]), v(h[1]), du), lerp(v(h[3]), v(h[2]), du), dv);
+	const uint32_t sum = lerp(lo, hi, dw);
 	return sum / 4096u + (sum % 4096u ? 1u : 0u);
 }
+__device__ __forceinline__ Interp interp(const uint32_t l[4], const uint32_t h[4], uint32_t du, uint32_t dv, uint32_t dw) {
+	if (du > 16u || dv > 16u) // a vertex outside its block: in 32 bits throughout, which wrap as the reference's do
+		return {interp32(l, h, 0, du, dv, dw), interp32(l, h, 16, du, dv, dw)};
+	const halves lo = lerp16(lerp16(as_halves(l[0]), as_halves(l[1]), du), lerp16(as_halves(l[3]), as_halves(l[2]), du), dv);
+	const halves hi = lerp16(lerp16(as_halves(h[0]), as_halves(h[1]), du), lerp16(as_halves(h[3]), as_halves(h[2]), du), dv);
+	const uint32_t a = uint32_t(lo[0]) * (16u - dw) + uint32_t(hi[0]) * dw, b = uint32_t(lo[1]) * (16u - dw) + uint32_t(hi[1]) * dw;
+	return {(a + 4095u) >> 12, (b + 4095u) >> 12};
+}
 
+// Vertex k of custom quad desc (cell | face << 12); its box is the vertex. A chunk has few custom quads, so their time
+// is the length of one's chain of loads and operations: four lanes share a quad's vertices, the face counts and passes
+// come from one word per mesh, and light is interpolated two values at a time. 768 chunks of terrain with plants
+// took 47.7 us with a lane per quad and two loads per face, 31.9 so; one such chunk from host memory 41.4 and 33.3.
 template <int NT>
-__device__ __forceinline__ void emit_custom(const MeshParams &p, Smem<NT> &s, const JobBlocks &blocks, uint32_t desc, uint32_t slot,
-                                         uint32_t vbase, uint32_t lo[3], uint32_t hi[3]) {
+__device__ __forceinline__ void emit_custom(const MeshParams &p, Smem<NT> &s, const JobBlocks &blocks, uint32_t desc, uint32_t k,
+                                         uint32_t slot, uint32_t vbase, uint32_t lo[3], uint32_t hi[3]) {
 	const int cell = desc & 4095, j = (desc >> 12) & 15;
 	const int x = cell & 15, z = (cell >> 4) & 15, y = cell >> 8;
 	const CustomCell c = custom_cell(p, s, blocks, cell);
@@ -648,40 +676,31 @@ __device__ __forceinline__ void emit_custom(const MeshParams &p, Smem<NT> &s, co
 		const int tmp = ua;
 		ua = va, va = tmp;
 	}
-	const uint32_t bx = uint32_t(x) << 4, by = uint32_t(y) << 4, bz = uint32_t(z) << 4;
-	lo[0] = lo[1] = lo[2] = ~0u;
-	hi[0] = hi[1] = hi[2] = 0u;
-	// vertices one at a time (custom faces are rare; this keeps the register footprint small), each
-	// picked from packed words so that nothing is indexed at run time
-	uint32_t vw[4];
+	const hcm_mesh_vertex v = k == 0 ? f.v[0] : (k == 1 ? f.v[1] : (k == 2 ? f.v[2] : f.v[3]));
+	const uint32_t vx = v.x, vy = v.y, vz = v.z;
+	auto pick = [&](int a) { return a == 0 ? vx : (a == 1 ? vy : vz); };
+	lo[0] = hi[0] = (uint32_t(x) << 4) + vx, lo[1] = hi[1] = (uint32_t(y) << 4) + vy, lo[2] = hi[2] = (uint32_t(z) << 4) + vz;
+	const uint32_t du = pick(ua), dv = pick(va);
+	uint32_t dw = min(pick(la), 16u);
+	if (lf & 1)
+		dw = 16u - dw;
+	uint32_t l[4], h[4];
 #pragma unroll
-	for (int k = 0; k < 4; ++k)
-		vw[k] = uint32_t(f.v[k].x) | uint32_t(f.v[k].y) << 8 | uint32_t(f.v[k].z) << 16 | uint32_t(f.v[k].ao) << 24;
-#pragma unroll 1
-	for (int k = 0; k < 4; ++k) {
-		const uint32_t w = k == 0 ? vw[0] : (k == 1 ? vw[1] : (k == 2 ? vw[2] : vw[3]));
-		const uint32_t vx = w & 0xffu, vy = (w >> 8) & 0xffu, vz = (w >> 16) & 0xffu;
-		auto pick = [&](int a) { return a == 0 ? vx : (a == 1 ? vy : vz); };
-		const uint32_t px = bx + vx, py = by + vy, pz = bz + vz;
-		lo[0] = min(lo[0], px), lo[1] = min(lo[1], py), lo[2] = min(lo[2], pz);
-		hi[0] = max(hi[0], px), hi[1] = max(hi[1], py), hi[2] = max(hi[2], pz);
-		const uint32_t du = pick(ua), dv = pick(va);
-		uint32_t dw = pick(la) < 16u ? pick(la) : 16u;
-		if (lf & 1)
-			dw = 16u - dw;
-		uint32_t ao = w >> 24;
-		if (ao == 4)
-			ao = interp(l4_ao(lo4, 0), l4_ao(lo4, 1), l4_ao(lo4, 2), l4_ao(lo4, 3), l4_ao(hi4, 0), l4_ao(hi4, 1),
-			            l4_ao(hi4, 2), l4_ao(hi4, 3), du, dv, dw) & 0xffu;
-		const uint32_t sun = interp(l4_sun(lo4, 0), l4_sun(lo4, 1), l4_sun(lo4, 2), l4_sun(lo4, 3), l4_sun(hi4, 0),
-		                            l4_sun(hi4, 1), l4_sun(hi4, 2), l4_sun(hi4, 3), du, dv, dw) & 0xffu;
-		const uint32_t torch = interp(l4_torch(lo4, 0), l4_torch(lo4, 1), l4_torch(lo4, 2), l4_torch(lo4, 3),
-		                              l4_torch(hi4, 0), l4_torch(hi4, 1), l4_torch(hi4, 2), l4_torch(hi4, 3), du, dv,
-		                              dw) & 0xffu;
-		p.pool_verts[4 * (size_t)slot + k] = make_uint2(px | (py << 10) | (pz << 20) | (uint32_t(f.axis) << 30),
-		                                                vword1(f.texture, f.render_face, ao, sun, torch));
+	for (int i = 0; i < 4; ++i)
+		l[i] = l4_sun(lo4, i) | l4_torch(lo4, i) << 16, h[i] = l4_sun(hi4, i) | l4_torch(hi4, i) << 16;
+	const Interp light = interp(l, h, du, dv, dw);
+	uint32_t ao = v.ao;
+	if (ao == 4) {
+#pragma unroll
+		for (int i = 0; i < 4; ++i)
+			l[i] = l4_ao(lo4, i), h[i] = l4_ao(hi4, i);
+		ao = interp(l, h, du, dv, dw).first & 0xffu;
 	}
-	put_indices(p, slot, vbase, true);
+	p.pool_verts[4 * (size_t)slot + k] =
+	    make_uint2(lo[0] | (lo[1] << 10) | (lo[2] << 20) | (uint32_t(f.axis) << 30),
+	               vword1(f.texture, f.render_face, ao, light.first & 0xffu, light.second & 0xffu));
+	if (k == 0)
+		put_indices(p, slot, vbase, true);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1489,11 +1508,8 @@ template <int NT> __device__ __forceinline__ void mesh_chunk(const MeshParams &p
 	uint32_t c_o = 0, c_t = 0, cust0 = 0, cust1 = 0;
 	uint64_t cust_pre = 0;
 	if (flags & kFlagCustom) {
-		for (int k = 0; k < CPT; ++k) {
-			const int cell = tid * CPT + k;
-			if (!((s.custom_bits[cell >> 5] >> (cell & 31)) & 1u))
-				continue;
-			const CustomCell c = custom_cell(p, s, blocks, cell);
+		for (uint32_t bits = custom_cells(s); bits; bits &= bits - 1) {
+			const CustomCell c = custom_cell(p, s, blocks, tid * CPT + __ffs(bits) - 1);
 			const uint32_t nt = __popc(c.trans);
 			c_t += nt;
 			c_o += c.count - nt;
@@ -1643,10 +1659,8 @@ template <int NT> __device__ __forceinline__ void mesh_chunk(const MeshParams &p
 			const uint32_t w1 = w0 + kListCap;
 			uint32_t io = (uint32_t)cust_pre, it = (uint32_t)(cust_pre >> 32);
 			if (io + it < w1 && io + it + c_o + c_t > w0) {
-				for (int k = 0; k < CPT && io + it < w1; ++k) {
-					const int cell = tid * CPT + k;
-					if (!((s.custom_bits[cell >> 5] >> (cell & 31)) & 1u))
-						continue;
+				for (uint32_t bits = custom_cells(s); bits && io + it < w1; bits &= bits - 1) {
+					const int cell = tid * CPT + __ffs(bits) - 1;
 					const CustomCell c = custom_cell(p, s, blocks, cell);
 					for (uint32_t j = 0; j < c.count; ++j) {
 						const uint32_t tr = (c.trans >> j) & 1u, g = io + it, i = tr ? it++ : io++;
@@ -1657,13 +1671,14 @@ template <int NT> __device__ __forceinline__ void mesh_chunk(const MeshParams &p
 			}
 			__syncthreads();
 			const uint32_t n = min(n_cust - w0, (uint32_t)kListCap);
-			for (uint32_t e = tid; e < n; e += NT) {
+			for (uint32_t v = tid; v < 4 * n; v += NT) { // a lane per vertex
+				const uint32_t e = v >> 2;
 				const uint2 ent = s.key[e];
 				const uint32_t tr = ent.x >> 31;
 				uint32_t slot, vbase, mk, mj, lo[3], hi[3];
 				quad_slot(tr, ent.y, n0, pool_base, slot, vbase, mk, mj);
-				emit_custom(p, s, blocks, ent.x & 0xffffu, slot, vbase, lo, hi);
-				quad_done(s, tr, mk, mj, w0 + e, lo, hi, box);
+				emit_custom(p, s, blocks, ent.x & 0xffffu, v & 3, slot, vbase, lo, hi);
+				quad_done(s, tr, mk, (v & 3) ? ~0u : mj, w0 + e, lo, hi, box); // (a split is one lane's to note)
 			}
 		}
 	}

@@ -112,3 +112,51 @@ def test_face_counts_at_block_and_group_edges(ctx, oracle, faces, merge):
         assert meshdigest.digest(hcm.job_meshes(0, *out)) == meshdigest.digest(want), threads
     ctx.set_tuning(wg_per_cu=0, threads=256)
     store.close()
+
+
+@pytest.mark.parametrize("seed,reach,threads", [(1, 16, 256), (2, 17, 256), (3, 40, 512), (4, 255, 128), (5, 16, 512)])
+def test_custom_meshes_with_any_vertices(tmp_path, seed, reach, threads):
+    """Custom meshes whose faces have random corners, axes, light faces and textures (opaque and transparent pass), within
+    their block (the light's interpolation in 16 bits) and past it (in 32, wrapping)."""
+    import cpu_oracle
+
+    reg = cases.RegistryFile(REGISTRY)
+    rng = np.random.default_rng(seed)
+    tex = np.unique(reg.rows["tex"])
+    tex = tex[tex != 0]
+    for m in reg.meshes:
+        head = m[:16].view(np.uint32)
+        if head[1] != 0:
+            continue  # liquid flow
+        head[0] = rng.integers(1, 17)
+        faces = m[16:].reshape(16, 24)
+        faces[:, 0] = rng.integers(0, 3, 16)
+        faces[:, 1:3] = rng.integers(0, 6, (16, 2))
+        faces[:, 4:6] = rng.choice(tex, 16).astype(np.uint16).reshape(16, 1).view(np.uint8)
+        corners = faces[:, 8:].reshape(16, 4, 4)
+        corners[..., :3] = rng.integers(0, reach + 1, (16, 4, 3))
+        corners[..., 3] = rng.integers(0, 5, (16, 4))
+    path = str(tmp_path / f"registry_custom_{seed}.bin")
+    reg.write(path)
+    orc = cpu_oracle.Oracle(path)
+    values = cases.CUSTOM
+    n = 4
+    blocks = np.where(rng.random((27 * n, 4096)) < (0.02, 0.4)[seed % 2], values[rng.integers(0, values.size, (27 * n, 4096))], 0).astype(np.uint16)
+    light = rng.integers(0, 256, blocks.shape).astype(np.uint8)
+    nbr = np.arange(27 * n, dtype=np.uint32).reshape(n, 27)
+    ctx = hcm.Context(pool_quads=1 << 20, registry=reg.c_registry(hcm))
+    ctx.set_tuning(wg_per_cu=0, threads=threads)
+    store = hcm.Store(ctx, blocks.shape[0])
+    store.upload(blocks, light)
+    batch = hcm.Batch(ctx, store, nbr)
+    print(f"custom meshes: seed {seed}, reach {reach}, threads {threads}", flush=True)
+    batch.run()
+    out = batch.download()
+    for j in range(n):
+        b27, l27 = workloads.slice_jobs(blocks, light, nbr, j)
+        want = meshdigest.digest(orc.mesh(b27, l27))
+        assert meshdigest.digest(hcm.job_meshes(j, *out)) == want, f"job {j}"
+        assert meshdigest.digest(ctx.mesh_chunk(b27, l27)) == want, f"job {j}, plain"
+    batch.close()
+    store.close()
+    ctx.close()
