@@ -268,6 +268,7 @@ struct hcm_ctx {
 	size_t depth_cap = 0; // floats
 	DepthPyramid hiz;
 	hcm_tuning tuning{0, 256, {0, 0}};
+	bool threads_given = false; // hcm_set_tuning named the workgroup size: no launch takes another
 };
 
 struct hcm_store {
@@ -466,6 +467,7 @@ extern "C" int hcm_set_tuning(hcm_ctx *ctx, const hcm_tuning *t) {
 	std::lock_guard<std::mutex> lk(ctx->mu);
 	ctx->tuning = *t;
 	ctx->tuning.threads = th;
+	ctx->threads_given = t->threads != 0;
 	return HCM_OK;
 }
 
@@ -495,6 +497,14 @@ static int persistent_grid(hcm_ctx *c, uint32_t threads) {
 	return (int)(per_cu * (uint32_t)c->n_cu);
 }
 
+// Workgroup size of a persistent launch of n_jobs. With a CU per job, 512 threads are the fastest (per pass, 256 against
+// 512 threads: 37 cave chunks 19.7 and 17.4 us, 256 of them 32.1 and 27.3, 256 plant chunks 26.7 and 24.7); one
+// such workgroup fills a CU's registers, so that past that many jobs it is the slower (400 jobs: 35.8 and 38.5, 28.9
+// and 41.0).
+static uint32_t batch_threads(const hcm_ctx *c, uint32_t n_jobs) {
+	return !c->threads_given && n_jobs <= (uint32_t)c->n_cu ? 512u : c->tuning.threads;
+}
+
 int hcm::ctx_info(hcm_ctx *ctx, uint32_t threads, CtxInfo *out) {
 	if (!ctx || !out)
 		return HCM_ERR_INVALID;
@@ -503,6 +513,7 @@ int hcm::ctx_info(hcm_ctx *ctx, uint32_t threads, CtxInfo *out) {
 	out->n_cu = ctx->n_cu;
 	out->threads = threads ? threads : ctx->tuning.threads;
 	out->grid = (uint32_t)persistent_grid(ctx, out->threads);
+	out->threads_few = threads ? threads : batch_threads(ctx, 1);
 	out->light_info = ctx->d_light_info;
 	out->light_info_host = ctx->light_info.data();
 	return HCM_OK;
@@ -952,7 +963,7 @@ static int batch_run(hcm_batch *b, uint32_t mode, uint32_t times) {
 	if (!c->pool_quads)
 		return HCM_ERR_POOL_FULL;
 	hipStream_t st = c->stream;
-	const uint32_t threads = c->tuning.threads;
+	const uint32_t threads = batch_threads(c, b->n_jobs);
 	MeshParams p = batch_params(b);
 	if (mode == HCM_RUN_PERSISTENT) {
 		if (!b->ctr_clean) // after per-chunk launches

@@ -204,6 +204,7 @@ struct CtxInfo {
 	int n_cu;
 	uint32_t threads;
 	uint32_t grid;              // persistent grid for `threads`
+	uint32_t threads_few;       // workgroup size of launches of at most n_cu jobs
 	const uint8_t *light_info;  // [65536] for the light rebuild
 	const uint8_t *light_info_host; // the same table in host memory
 };

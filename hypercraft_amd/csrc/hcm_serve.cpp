@@ -532,8 +532,9 @@ struct hcm_server {
 			p.results = b.d_res;
 			p.halo_light = relight() ? b.d_halo : nullptr;
 			p.self_reset = 1; // the slot's counters start at zero; the run's last workgroup clears them
-			const int grid = (int)std::max<uint32_t>(1, std::min<uint32_t>(info.grid, (uint32_t)b.jobs.size()));
-			HCM_CHECK(launch_mesh(p, (int)info.threads, grid, s_comp));
+			const uint32_t n = (uint32_t)b.jobs.size();
+			const bool few = n <= (uint32_t)info.n_cu;
+			HCM_CHECK(launch_mesh(p, (int)(few ? info.threads_few : info.threads), (int)(few ? n : std::min(info.grid, n)), s_comp));
 			HCM_CHECK(hipEventRecord(b.ev_k1, s_comp));
 			ExportParams e;
 			e.ctr = b.d_ctr;

@@ -298,7 +298,7 @@ int hcm_batch_cull_occlusion(hcm_batch *batch, const float view_position[3], con
 /* Launch shape of the meshing kernel. 0 = default. */
 typedef struct hcm_tuning {
 	uint32_t wg_per_cu; /* persistent workgroups per compute unit */
-	uint32_t threads;   /* workgroup size: 128, 256 or 512 */
+	uint32_t threads;   /* workgroup size: 128, 256 or 512; 0: 256, and 512 for batches of few jobs */
 	uint32_t reserved[2];
 } hcm_tuning;
 int hcm_set_tuning(hcm_ctx *ctx, const hcm_tuning *t);

@@ -160,3 +160,30 @@ def test_custom_meshes_with_any_vertices(tmp_path, seed, reach, threads):
     batch.close()
     store.close()
     ctx.close()
+
+
+@pytest.mark.parametrize("n", [255, 256, 257])
+def test_batches_around_a_job_per_cu(n, oracle):
+    """Up to a job per CU a batch runs in workgroups of 512 threads, unless a size was asked for; beyond, in 256."""
+    rng = np.random.default_rng(n)
+    values = np.concatenate([cases.CUSTOM, np.arange(1, 9, dtype=np.uint16)])
+    blocks = np.where(rng.random((54, 4096)) < 0.1, values[rng.integers(0, values.size, (54, 4096))], 0).astype(np.uint16)
+    light = rng.integers(0, 256, blocks.shape).astype(np.uint8)
+    nbr = np.tile(np.arange(54, dtype=np.uint32).reshape(2, 27), (n, 1))[:n]
+    want = [meshdigest.digest(oracle.mesh(*workloads.slice_jobs(blocks, light, nbr, j))) for j in range(2)]
+    ctx = hcm.Context(pool_quads=1 << 21)
+    store = hcm.Store(ctx, 54)
+    store.upload(blocks, light)
+    for asked in (None, 256, 512):
+        if asked:
+            ctx.set_tuning(wg_per_cu=0, threads=asked)
+        batch = hcm.Batch(ctx, store, nbr)
+        print(f"{n} jobs, threads {asked}", flush=True)
+        for _ in range(2):
+            batch.run()
+        out = batch.download()
+        for j in range(n):
+            assert meshdigest.digest(hcm.job_meshes(j, *out)) == want[j & 1], (asked, j)
+        batch.close()
+    store.close()
+    ctx.close()
