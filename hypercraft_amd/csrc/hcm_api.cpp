@@ -139,17 +139,10 @@ int build_tables(const hcm_registry *r, DeviceTables *t) {
 	if (code_tex.size() > (size_t)kMaxCodes)
 		return HCM_ERR_INVALID;
 	t->codes.clear();
-	for (uint16_t tex : code_tex) {
-		uint32_t f = tex_flags(tex), cf = 0;
-		if (f & HCM_TEX_TRANSPARENT)
-			cf |= kCodeTransparent;
-		if (f & HCM_TEX_TRANS_PASS)
-			cf |= kCodeTransPass;
-		if (f & HCM_TEX_LIQUID)
-			cf |= kCodeLiquid;
-		if ((tex & 0x1fffu) == 0)
-			cf |= kCodeEmpty;
-		t->codes.push_back(uint32_t(tex) | cf << 16);
+	for (size_t i = 0; i < code_tex.size(); ++i) { // (a texture of id 0 is on no visible face)
+		const uint32_t tex = code_tex[i], vertex = ((tex & 0x1fffu) - 1u) | (tex >> 13) << 10;
+		const uint32_t pass = tex_flags(uint16_t(tex)) & HCM_TEX_TRANS_PASS ? kCodeTransPass : 0u;
+		t->codes.push_back((vertex & kCodeVertex) | uint32_t(i >> 4) << 28 | pass);
 	}
 	t->pid_of.resize(65536 + 256);
 	for (uint32_t d = 0; d < 65536; ++d) {

@@ -30,11 +30,11 @@ __host__ __device__ constexpr uint32_t vox_light(uint32_t byte) { return (byte *
 // Face classes for BlockTexture::Show (texture/include/texture/BlockTexture.hpp:68-76)
 constexpr uint32_t kClassEmpty = 0, kClassOpaque = 1, kClassTransparent = 2, kClassLiquid = 3;
 
-// Texture-code flags (code word = texture value | flags << 16)
-constexpr uint32_t kCodeTransparent = 1u;
-constexpr uint32_t kCodeTransPass = 2u;
-constexpr uint32_t kCodeLiquid = 4u;
-constexpr uint32_t kCodeEmpty = 8u;
+// Code words: texture bits as the second word of a vertex has them, and in the upper bits, as a face word has them,
+// the upper three of the code's own seven bits and whether its faces go to the transparent pass.
+constexpr uint32_t kCodeVertex = 0x1fffu;
+constexpr uint32_t kCodeLow = 0x0fffffffu;
+constexpr uint32_t kCodeTransPass = 1u << 31;
 
 // Texture-row flag (in rows[pid].y): a halo made of this row's block alone has visible faces.
 constexpr uint32_t kRowSelfShow = 1u << 16;

@@ -241,18 +241,18 @@ __device__ __forceinline__ uint32_t lpass(uint32_t c) { return c & kVoxLight & (
 // One vertex of light4_init (:114-162), without branches, from its side cells a and b, corner cell c and
 // the front cell: the side cells count when they pass indirect light, the corner when it does and a side
 // cell does; sunlight and torchlight are averaged as (sum << 2) / count, the front cell always counted.
-// Returns sun | torch << 8 | ao << 16.
+// Returns ao | sun << 2 | torch << 8.
 __device__ __forceinline__ uint32_t light_vertex(uint32_t a, uint32_t c, uint32_t b, uint32_t pf, uint32_t d3) {
 	const uint32_t g = 0u - (((a | b) >> 12) & 1u);
 	const uint32_t sum = pf + lpass(a) + lpass(b) + (lpass(c) & g); // count - 1 in bits 12-13
 	const uint32_t r = uint32_t(kRecip >> ((sum >> 8) & 0x30u)) & 0x3ffu;
 	const uint32_t prod = (sum & 0x003f003fu) * r;
 	const uint32_t idx = ((a >> 11) & 1u) | ((c >> 10) & 2u) | ((b >> 9) & 4u) | d3;
-	return ((prod >> 7) & 63u) | (((prod >> 23) & 63u) << 8) | (((kAoTable >> (2 * idx)) & 3u) << 16);
+	return ((prod >> 5) & 0xfcu) | (((prod >> 23) & 63u) << 8) | ((kAoTable >> (2 * idx)) & 3u);
 }
 
-// light4_init (:48-163) for face `face` of the block at halo index self. Returns the packed Light4:
-//   x = sun0 | sun1 << 6 | sun2 << 12 | sun3 << 18 | ao4 << 24,   y = torch0 | ... | torch3 << 18.
+// light4_init (:48-163) for face `face` of the block at halo index self. Returns the packed Light4, a vertex in 14 bits
+// as a vertex word holds it from bit 16 on: vertex 0 | vertex 1 << 14 in x, vertex 2 | vertex 3 << 14 in y.
 // The front cell F and its eight neighbours in the face's plane; vertex k's side cells along the plane
 // axes Q and P and the corner between them have (P, Q) signs (-,-), then (+,-) or (-,+) by the winding,
 // then (+,+), then the other of (+,-) and (-,+).
@@ -272,37 +272,40 @@ __device__ __forceinline__ uint2 light4(const uint32_t *vox, int face, int self)
 	const uint32_t vpm = light_vertex(qm, pmq, pp, pf, d3), vmp = light_vertex(qp, mp, pm, pf, d3);
 	const uint32_t v0 = light_vertex(qm, mm, pm, pf, d3), v1 = wa ? vpm : vmp;
 	const uint32_t v2 = light_vertex(qp, ppq, pp, pf, d3), v3 = wa ? vmp : vpm;
-	const uint32_t lo = (v0 & 63u) | (v1 & 63u) << 6 | (v2 & 63u) << 12 | (v3 & 63u) << 18;
-	const uint32_t hi = ((v0 >> 8) & 63u) | ((v1 >> 8) & 63u) << 6 | ((v2 >> 8) & 63u) << 12 | ((v3 >> 8) & 63u) << 18;
-	const uint32_t ao4 = (v0 >> 16) | (v1 >> 16) << 2 | (v2 >> 16) << 4 | (v3 >> 16) << 6;
-	return make_uint2(lo | (ao4 << 24), hi);
+	return make_uint2(v0 | v1 << 14, v2 | v3 << 14);
 }
 
-__device__ __forceinline__ uint32_t l4_sun(uint2 l, int k) { return (l.x >> (6 * k)) & 63u; }
-__device__ __forceinline__ uint32_t l4_torch(uint2 l, int k) { return (l.y >> (6 * k)) & 63u; }
-__device__ __forceinline__ uint32_t l4_ao(uint2 l, int k) { return (l.x >> (24 + 2 * k)) & 3u; }
+__device__ __forceinline__ uint32_t l4_at(uint2 l, int k, int bit) { return (k < 2 ? l.x : l.y) >> (14 * (k & 1) + bit); }
+__device__ __forceinline__ uint32_t l4_ao(uint2 l, int k) { return l4_at(l, k, 0) & 3u; }
+__device__ __forceinline__ uint32_t l4_sun(uint2 l, int k) { return l4_at(l, k, 2) & 63u; }
+__device__ __forceinline__ uint32_t l4_torch(uint2 l, int k) { return l4_at(l, k, 8) & 63u; }
 
 // Light4::GetFlip (:38-43): sunlight and AO only.
 __device__ __forceinline__ bool l4_flip(uint2 l) {
-	const int d02 = int(l4_ao(l, 0) + 1) * int(l4_sun(l, 0) + 1) - int(l4_ao(l, 2) + 1) * int(l4_sun(l, 2) + 1);
-	const int d13 = int(l4_ao(l, 1) + 1) * int(l4_sun(l, 1) + 1) - int(l4_ao(l, 3) + 1) * int(l4_sun(l, 3) + 1);
-	return abs(d02) < abs(d13);
+	const uint2 more = make_uint2(l.x + (4u | 4u << 14), l.y + (4u | 4u << 14)); // sunlight + 1 (at most 61)
+	const auto product = [&](int k) { return l4_ao(l, k) * l4_sun(more, k) + l4_sun(more, k); };
+	return abs(int(product(0) - product(2))) < abs(int(product(1) - product(3)));
 }
 
 __device__ __forceinline__ uint64_t ballot64(bool b) { return __ballot(b); }
 
-// Minimum / maximum over the wavefront with DPP lane moves (no LDS): swaps within quads, the half-row
+// Minima of the 16-bit halves of two words.
+__device__ __forceinline__ uint32_t min_halves(uint32_t a, uint32_t b) {
+	typedef uint16_t halves __attribute__((vector_size(4)));
+	const halves x = __builtin_bit_cast(halves, a), y = __builtin_bit_cast(halves, b);
+	return __builtin_bit_cast(uint32_t, x < y ? x : y);
+}
+
+// The minima over the wavefront with DPP lane moves (no LDS): swaps within quads, the half-row
 // and row mirrors leave every lane of a 16-lane row with the row's result, then the row broadcasts of
 // lanes 15 and 31 fold the rows into lane 63. Lanes a move does not write keep the identity.
-template <bool kMax> __device__ __forceinline__ uint32_t wave_fold(uint32_t v) {
-	constexpr uint32_t id = kMax ? 0u : 0xffffffffu;
-	auto op = [](uint32_t a, uint32_t b) { return kMax ? max(a, b) : min(a, b); };
-	v = op(v, (uint32_t)__builtin_amdgcn_update_dpp((int)id, (int)v, 0xb1, 0xf, 0xf, false));  // quad_perm 1,0,3,2
-	v = op(v, (uint32_t)__builtin_amdgcn_update_dpp((int)id, (int)v, 0x4e, 0xf, 0xf, false));  // quad_perm 2,3,0,1
-	v = op(v, (uint32_t)__builtin_amdgcn_update_dpp((int)id, (int)v, 0x141, 0xf, 0xf, false)); // row_half_mirror
-	v = op(v, (uint32_t)__builtin_amdgcn_update_dpp((int)id, (int)v, 0x140, 0xf, 0xf, false)); // row_mirror
-	v = op(v, (uint32_t)__builtin_amdgcn_update_dpp((int)id, (int)v, 0x142, 0xa, 0xf, false)); // row_bcast:15
-	v = op(v, (uint32_t)__builtin_amdgcn_update_dpp((int)id, (int)v, 0x143, 0xc, 0xf, false)); // row_bcast:31
+__device__ __forceinline__ uint32_t wave_min_halves(uint32_t v) {
+	v = min_halves(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0xb1, 0xf, 0xf, false));  // quad_perm 1,0,3,2
+	v = min_halves(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x4e, 0xf, 0xf, false));  // quad_perm 2,3,0,1
+	v = min_halves(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x141, 0xf, 0xf, false)); // row_half_mirror
+	v = min_halves(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x140, 0xf, 0xf, false)); // row_mirror
+	v = min_halves(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x142, 0xa, 0xf, false)); // row_bcast:15
+	v = min_halves(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x143, 0xc, 0xf, false)); // row_bcast:31
 	return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
 
@@ -544,28 +547,13 @@ __device__ __forceinline__ hcm_mesh_face custom_face(const MeshParams &p, const 
 // ------------------------------------------------------------------------------------------------
 // writing one quad
 // ------------------------------------------------------------------------------------------------
-__device__ __forceinline__ void put_indices(const MeshParams &p, uint32_t slot, uint32_t base, bool flip) {
+__device__ __forceinline__ void put_indices(uint32_t *ip, uint32_t base, bool flip) {
 	// index patterns: flip (0,1,2, 0,2,3) (:440-446) -- also the custom-mesh pattern (:295-301) --
 	// and no flip (1,2,3, 0,1,3) (:453-459)
-	const uint32_t b0 = base, b1 = base + 1, b2 = base + 2, b3 = base + 3;
-	uint32_t *ip = reinterpret_cast<uint32_t *>(p.pool_idx + 6 * (size_t)slot);
-	if (flip) {
-		ip[0] = b0 | (b1 << 16);
-		ip[1] = b2 | (b0 << 16);
-		ip[2] = b2 | (b3 << 16);
-	} else {
-		ip[0] = b1 | (b2 << 16);
-		ip[1] = b3 | (b0 << 16);
-		ip[2] = b1 | (b3 << 16);
-	}
-}
-
-__device__ __forceinline__ void put_quad(const MeshParams &p, uint32_t slot, const uint32_t w0[4], const uint32_t w1[4],
-                                         uint32_t base, bool flip) {
-	uint4 *vp = reinterpret_cast<uint4 *>(p.pool_verts + 4 * (size_t)slot);
-	vp[0] = make_uint4(w0[0], w1[0], w0[1], w1[1]);
-	vp[1] = make_uint4(w0[2], w1[2], w0[3], w1[3]);
-	put_indices(p, slot, base, flip);
+	const uint32_t two = base | base << 16; // at most 65,532 each: no carry
+	ip[0] = two + (flip ? 0u | 1u << 16 : 1u | 2u << 16);
+	ip[1] = two + (flip ? 2u | 0u << 16 : 3u | 0u << 16);
+	ip[2] = two + (flip ? 2u | 3u << 16 : 1u | 3u << 16);
 }
 
 // BlockVertex word 1 (client/include/client/BlockVertex.hpp:13-14)
@@ -574,52 +562,59 @@ __device__ __forceinline__ uint32_t vword1(uint16_t tex, uint32_t face, uint32_t
 	       (torch << 24);
 }
 
-template <int NT>
-__device__ __forceinline__ void aabb_merge(Smem<NT> &s, int pass, int k, const uint32_t lo[3], const uint32_t hi[3]) {
-	uint32_t *a = s.aabb[pass][k];
-	atomicMin(&a[0], lo[0]);
-	atomicMin(&a[1], lo[1]);
-	atomicMin(&a[2], lo[2]);
-	atomicMax(&a[3], hi[0]);
-	atomicMax(&a[4], hi[1]);
-	atomicMax(&a[5], hi[2]);
+// The box of a pass, over words of vertices (x, y, z in 10 bits each): the lowest x, y and z and the lowest complements
+// of the highest, in the upper bits of six 16-bit halves, whose lower bits are of no account; all of them are minima,
+// of all ones where there is none.
+struct Box {
+	uint32_t lo_xy, hi_xy, z;
+};
+__device__ __forceinline__ uint32_t low_high(uint32_t low, uint32_t high) { return (low & 0xffffu) | (high & 0xffff0000u); }
+// The box of the vertex words lo and hi.
+__device__ __forceinline__ Box word_box(uint32_t lo, uint32_t hi) {
+	return {low_high(lo << 6, lo << 12), low_high(~hi << 6, ~hi << 12), low_high(lo >> 14, ~hi << 2)};
+}
+__device__ __forceinline__ void box_min(Box &b, const Box &a, uint32_t m) {
+	b.lo_xy = min_halves(b.lo_xy, a.lo_xy | m), b.hi_xy = min_halves(b.hi_xy, a.hi_xy | m), b.z = min_halves(b.z, a.z | m);
+}
+__device__ __forceinline__ Box wave_box(const Box &b) {
+	return {wave_min_halves(b.lo_xy), wave_min_halves(b.hi_xy), wave_min_halves(b.z)};
 }
 
-// Regular quad: task t, origin (u, v0) on the mask, width w along V,
-// height h along U (:357-460), with the face word of its origin face (Light4 and texture code).
+template <int NT> __device__ __forceinline__ void aabb_merge(Smem<NT> &s, int pass, int k, const Box &b) {
+	uint32_t *a = s.aabb[pass][k];
+	atomicMin(&a[0], (b.lo_xy >> 6) & 0x3ffu);
+	atomicMin(&a[1], b.lo_xy >> 22);
+	atomicMin(&a[2], (b.z >> 6) & 0x3ffu);
+	atomicMax(&a[3], ~(b.hi_xy >> 6) & 0x3ffu);
+	atomicMax(&a[4], ~b.hi_xy >> 22);
+	atomicMax(&a[5], ~b.z >> 22);
+}
+
+// Regular quad at the face at desc (task, row u, column v0), width w along V, height h along U (:357-460), with the
+// face word of its origin face (Light4 and texture code), to quad i of the chunk, whose pool range starts at verts
+// and idx. Returns its box.
 template <int NT>
-__device__ __forceinline__ void emit_quad(const MeshParams &p, const Smem<NT> &s, int t, int u, int v0, int w, int h,
-                                          uint2 word, uint32_t slot, uint32_t vbase, uint32_t lo[3], uint32_t hi[3]) {
-	const int A = task_axis(t), inv = task_plus(t) ^ 1, sl = task_layer(t) + (inv ^ 1), face = 2 * A + inv;
-	const int ua = u_axis(A), va = v_axis(A);
-	const uint2 l = make_uint2(word.x, word.y & 0xffffffu);
-	const uint16_t tex = uint16_t(s.codes[(word.y >> 24) & 0x7fu] & 0xffffu);
+__device__ __forceinline__ Box emit_quad(const Smem<NT> &s, uint32_t desc, uint32_t w, uint32_t h, uint2 word, uint4 *verts,
+                                         uint32_t *idx, uint32_t i, uint32_t vbase) {
+	const int t = (desc >> 8) & 127, A = task_axis(t), plus = task_plus(t);
+	const uint32_t u = (desc >> 4) & 15, v0 = desc & 15;
+	// a vertex word has x, y and z (1/16 units, at most 256) in 10-bit fields: the origin's word and the packed
+	// vectors along U and V, with no carry between fields
+	const uint32_t at_u = A == 1 ? 24 : 14, at_v = A == 0 ? 24 : 4, at_a = 42 - at_u - at_v;
+	const uint32_t base = uint32_t(task_layer(t) + plus) << at_a | u << at_u | v0 << at_v | uint32_t(A) << 30;
+	const uint32_t pu = h << at_u, pv = w << at_v;
 	// quad vectors (:383-390): (U+1)%3 == V holds for the x and y axes
-	const bool height_on_u = (inv != 0) != (A != 2);
-	int du[3], dv[3], o[3];
-#pragma unroll
-	for (int a = 0; a < 3; ++a) {
-		const int on_u = a == ua, on_v = a == va;
-		o[a] = a == A ? sl : (on_u ? u : v0);
-		du[a] = height_on_u ? on_u * h : on_v * w;
-		dv[a] = height_on_u ? on_v * w : on_u * h;
-	}
-	// word 0 packs x, y, z (1/16 units, at most 256) in 10-bit fields: the corners are the origin's word
-	// plus the packed quad vectors, with no carry between fields
-	const auto pack = [](uint32_t x, uint32_t y, uint32_t z) { return (x << 4) | (y << 14) | (z << 24); };
-	const uint32_t base = pack(o[0], o[1], o[2]) | (uint32_t(A) << 30);
-	const uint32_t pu = pack(du[0], du[1], du[2]), pv = pack(dv[0], dv[1], dv[2]);
-	const uint32_t w0[4] = {base, base + pu, base + pu + pv, base + pv};
-	uint32_t w1[4];
-#pragma unroll
-	for (int k = 0; k < 4; ++k)
-		w1[k] = vword1(tex, uint32_t(face), l4_ao(l, k), l4_sun(l, k), l4_torch(l, k));
-	put_quad(p, slot, w0, w1, vbase, l4_flip(l));
-#pragma unroll
-	for (int a = 0; a < 3; ++a) {
-		lo[a] = uint32_t(o[a]) << 4;
-		hi[a] = uint32_t(o[a] + du[a] + dv[a]) << 4;
-	}
+	const bool height_first = (plus == 0) != (A != 2);
+	const uint32_t second = base + (height_first ? pu : pv), opposite = base + pu + pv, fourth = base + (height_first ? pv : pu);
+	// BlockVertex word 1 (client/include/client/BlockVertex.hpp:13-14): texture, face, and the vertex's light
+	const uint32_t code = (word.x >> 28) | ((word.y >> 24) & 0x70u);
+	const uint32_t common = (s.codes[code] & kCodeVertex) | uint32_t(2 * A + (plus ^ 1)) << 13;
+	constexpr uint32_t kLight = 0x3fff0000u;
+	uint4 *vp = verts + 2 * (size_t)i;
+	vp[0] = make_uint4(base, common | (word.x << 16 & kLight), second, common | (word.x << 2 & kLight));
+	vp[1] = make_uint4(opposite, common | (word.y << 16 & kLight), fourth, common | (word.y << 2 & kLight));
+	put_indices(idx + 3 * (size_t)i, vbase, l4_flip(word));
+	return word_box(base, opposite);
 }
 
 // light4_interpolate (:165-196): trilinear in 1/16 steps, rounded up, for two values of at most 63 in the
@@ -655,13 +650,13 @@ __device__ __forceinline__ Interp interp(const uint32_t l[4], const uint32_t h[4
 	return {(a + 4095u) >> 12, (b + 4095u) >> 12};
 }
 
-// Vertex k of custom quad desc (cell | face << 12); its box is the vertex. A chunk has few custom quads, so their time
+// Vertex k of custom quad desc (cell | face << 12), to quad `slot` of the pool. Returns its word, which is its box. A chunk has few custom quads, so their time
 // is the length of one's chain of loads and operations: four lanes share a quad's vertices, the face counts and passes
 // come from one word per mesh, and light is interpolated two values at a time. 768 chunks of terrain with plants
 // took 47.7 us with a lane per quad and two loads per face, 31.9 so; one such chunk from host memory 41.4 and 33.3.
 template <int NT>
-__device__ __forceinline__ void emit_custom(const MeshParams &p, Smem<NT> &s, const JobBlocks &blocks, uint32_t desc, uint32_t k,
-                                         uint32_t slot, uint32_t vbase, uint32_t lo[3], uint32_t hi[3]) {
+__device__ __forceinline__ uint32_t emit_custom(const MeshParams &p, Smem<NT> &s, const JobBlocks &blocks, uint32_t desc,
+                                                uint32_t k, uint32_t slot, uint32_t vbase) {
 	const int cell = desc & 4095, j = (desc >> 12) & 15;
 	const int x = cell & 15, z = (cell >> 4) & 15, y = cell >> 8;
 	const CustomCell c = custom_cell(p, s, blocks, cell);
@@ -679,7 +674,7 @@ __device__ __forceinline__ void emit_custom(const MeshParams &p, Smem<NT> &s, co
 	const hcm_mesh_vertex v = k == 0 ? f.v[0] : (k == 1 ? f.v[1] : (k == 2 ? f.v[2] : f.v[3]));
 	const uint32_t vx = v.x, vy = v.y, vz = v.z;
 	auto pick = [&](int a) { return a == 0 ? vx : (a == 1 ? vy : vz); };
-	lo[0] = hi[0] = (uint32_t(x) << 4) + vx, lo[1] = hi[1] = (uint32_t(y) << 4) + vy, lo[2] = hi[2] = (uint32_t(z) << 4) + vz;
+	const uint32_t at = ((uint32_t(x) << 4) + vx) | ((uint32_t(y) << 4) + vy) << 10 | ((uint32_t(z) << 4) + vz) << 20;
 	const uint32_t du = pick(ua), dv = pick(va);
 	uint32_t dw = min(pick(la), 16u);
 	if (lf & 1)
@@ -697,10 +692,10 @@ __device__ __forceinline__ void emit_custom(const MeshParams &p, Smem<NT> &s, co
 		ao = interp(l, h, du, dv, dw).first & 0xffu;
 	}
 	p.pool_verts[4 * (size_t)slot + k] =
-	    make_uint2(lo[0] | (lo[1] << 10) | (lo[2] << 20) | (uint32_t(f.axis) << 30),
-	               vword1(f.texture, f.render_face, ao, light.first & 0xffu, light.second & 0xffu));
+	    make_uint2(at | (uint32_t(f.axis) << 30), vword1(f.texture, f.render_face, ao, light.first & 0xffu, light.second & 0xffu));
 	if (k == 0)
-		put_indices(p, slot, vbase, true);
+		put_indices(reinterpret_cast<uint32_t *>(p.pool_idx) + 3 * (size_t)slot, vbase, true);
+	return at;
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -952,16 +947,16 @@ template <int NT> __device__ __forceinline__ uint32_t face_desc(const Smem<NT> &
 	return (q << 6) + nth_bit(rows.x, rows.y, g0 + i - s.upre[q]);
 }
 
-// Word of a visible face: Light4 (light4_init, :48-163) in x and the low 24 bits of y, the texture code in y
-// bits 24-30 and the transparent-pass flag in bit 31. Faces merge only if their words are equal
-// (Light4::operator==, :44, and the texture compare, :367-368).
+// Word of a visible face: Light4 (light4_init, :48-163) in the low 28 bits of x and y, the texture code in the upper
+// four of x and bits 28-30 of y and the transparent-pass flag in bit 31. Faces merge only if their words are equal
+// (Light4::operator==, :44, and the texture compare, :367-368). The code's upper three bits and the flag come from
+// the table of codes as they lie in the word.
 template <int NT> __device__ __forceinline__ uint2 face_word(const Smem<NT> &s, uint32_t desc) {
 	int face;
 	const int self = face_owner(desc, face);
 	const uint2 l = light4(s.vox, face, self);
 	const uint32_t tc = row_code(s, vox_pid(s.vox[self]), face);
-	const uint32_t tpass = (s.codes[tc] >> 16) & kCodeTransPass ? 1u : 0u;
-	return make_uint2(l.x, l.y | (tc << 24) | (tpass << 31));
+	return make_uint2(l.x | tc << 28, l.y | (s.codes[tc] & ~kCodeLow));
 }
 
 // Equal-to-right and equal-to-below bits of the visible face with dense index i (local to the group): its
@@ -1133,46 +1128,33 @@ template <int NT> __device__ __forceinline__ int group_end(Smem<NT> &s, int t0, 
 	return s.group_end;
 }
 
-// Where quad i of a pass goes: its pool slot, the base vertex of its mesh, the mesh of the pass (mk) and
-// its index in that mesh (mj). The reference reads the 16-bit vertex count before splitting, so the first
+// Where quad i of a pass goes: the base vertex of its mesh, the mesh of the pass (mk) and its index in that mesh (mj). The reference reads the 16-bit vertex count before splitting, so the first
 // quad of a continuation mesh keeps base 65,532 (:273-279, :397-403).
-__device__ __forceinline__ void quad_slot(uint32_t pass, uint32_t i, uint32_t n0, uint32_t pool_base, uint32_t &slot,
-                                          uint32_t &vbase, uint32_t &mk, uint32_t &mj) {
-	slot = pool_base + (pass ? n0 : 0u) + i;
+__device__ __forceinline__ void quad_place(uint32_t i, uint32_t &vbase, uint32_t &mk, uint32_t &mj) {
 	mk = i / kSplitQuads;
 	mj = i - mk * kSplitQuads;
 	vbase = (mj == 0 && mk > 0) ? 65532u : 4u * mj;
 }
 
-// A written quad's box into its mesh's AABB (per lane for the first mesh of a pass, LDS atomics for the
-// others) and, when it starts a continuation mesh, a split event at its emission position epos.
-// A quad's box into the lane's box of the first mesh of its pass (static register indices only): the
-// other pass's box takes the empty box (lower corner all ones, upper zero), which changes nothing, and the
-// transparent pass's box is left alone in chunks without transparent quads (any_tr, the same in every lane).
-__device__ __forceinline__ void box_add(uint32_t box[2][6], uint32_t pass, const uint32_t lo[3], const uint32_t hi[3],
-                                        bool any_tr = true) {
+// A quad's box into the lane's box of the first mesh of its pass: the other pass's box takes the empty box, which
+// changes nothing, and the transparent pass's box is left alone in chunks without transparent quads (any_tr, the same
+// in every lane).
+__device__ __forceinline__ void box_add(Box box[2], uint32_t pass, const Box &b, bool any_tr = true) {
 	const uint32_t m = 0u - pass; // all ones for the transparent pass
-#pragma unroll
-	for (int a = 0; a < 3; ++a) {
-		box[0][a] = min(box[0][a], lo[a] | m);
-		box[0][3 + a] = max(box[0][3 + a], hi[a] & ~m);
-	}
-	if (any_tr) {
-#pragma unroll
-		for (int a = 0; a < 3; ++a) {
-			box[1][a] = min(box[1][a], lo[a] | ~m);
-			box[1][3 + a] = max(box[1][3 + a], hi[a] & m);
-		}
-	}
+	box_min(box[0], b, m);
+	if (any_tr)
+		box_min(box[1], b, ~m);
 }
 
+// A written quad's box into its mesh's AABB (per lane for the first mesh of a pass, LDS atomics for the
+// others) and, when it starts a continuation mesh, a split event at its emission position epos.
 template <int NT>
-__device__ __forceinline__ void quad_done(Smem<NT> &s, uint32_t pass, uint32_t mk, uint32_t mj, uint32_t epos,
-                                          const uint32_t lo[3], const uint32_t hi[3], uint32_t box[2][6]) {
+__device__ __forceinline__ void quad_done(Smem<NT> &s, uint32_t pass, uint32_t mk, uint32_t mj, uint32_t epos, const Box &b,
+                                          Box box[2]) {
 	if (mk == 0)
-		box_add(box, pass, lo, hi);
+		box_add(box, pass, b);
 	else
-		aabb_merge(s, pass, mk, lo, hi);
+		aabb_merge(s, pass, mk, b);
 	if (mj == 0 && mk > 0) { // a split happened right before this quad (:397-403)
 		const uint32_t ev = atomicAdd(&s.n_events, 1u);
 		if (ev < 16) {
@@ -1200,8 +1182,8 @@ __device__ __forceinline__ uint32_t lanes_below(uint64_t ballot) {
 // chunk has more than kSplitQuads quads; else every quad is in the first mesh of its pass. epos: the quads
 // emitted before it, for a split.
 template <int NT>
-__device__ __forceinline__ void emit_face(const MeshParams &p, Smem<NT> &s, uint32_t desc, uint2 word, uint32_t i, uint32_t epos,
-                                          uint32_t n0, uint32_t pool_base, uint32_t box[2][6], bool any_tr, bool split) {
+__device__ __forceinline__ void emit_face(Smem<NT> &s, uint32_t desc, uint2 word, uint32_t i, uint32_t epos, uint32_t n0,
+                                          uint4 *verts, uint32_t *idx, Box box[2], bool any_tr, bool split) {
 	const uint32_t r = (desc >> 4) & 0x7ffu, tr = desc >> 15;
 	const int u = r & 15, v = desc & 15;
 	const uint32_t link = uint32_t(s.ev[r] & ~s.eh[r]);
@@ -1217,14 +1199,14 @@ __device__ __forceinline__ void emit_face(const MeshParams &p, Smem<NT> &s, uint
 		for (int k = 2; u + k < 16 && ((uint32_t(s.ne[r + k] & ~s.ev[r + k]) >> v) & 1u); ++k)
 			++h;
 	}
-	uint32_t slot = pool_base + (tr ? n0 : 0u) + i, vbase = 4u * i, mk = 0, mj = i, lo[3], hi[3];
+	uint32_t vbase = 4u * i, mk = 0, mj = i;
 	if (split)
-		quad_slot(tr, i, n0, pool_base, slot, vbase, mk, mj);
-	emit_quad(p, s, int(r >> 4), u, v, w, h, word, slot, vbase, lo, hi);
+		quad_place(i, vbase, mk, mj);
+	const Box b = emit_quad(s, desc, w, h, word, verts, idx, (tr ? n0 : 0u) + i, vbase);
 	if (split)
-		quad_done(s, tr, mk, mj, epos, lo, hi, box);
+		quad_done(s, tr, mk, mj, epos, b, box);
 	else
-		box_add(box, tr, lo, hi, any_tr);
+		box_add(box, tr, b, any_tr);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1528,7 +1510,12 @@ template <int NT> __device__ __forceinline__ void mesh_chunk(const MeshParams &p
 	const uint32_t wave_u = __builtin_amdgcn_readfirstlane(wave);
 	uint32_t base_o = cust0, base_t = cust1;       // quads of each pass before the group
 	uint32_t n0 = 0, n1 = 0, nm0 = 0, nm1 = 0;      // the chunk's quads and meshes per pass
-	uint32_t pool_base = 0, box[2][6];
+	uint32_t pool_base = 0;
+	uint4 *verts = nullptr;  // the chunk's range of the pool
+	uint32_t *idx = nullptr;
+	// AABB<uint32_t>::Merge (dep/AABB.hpp:52-59) of the first mesh of each pass per lane, reduced at the end; later
+	// meshes of a pass (past 16,383 quads) by LDS atomics
+	Box box[2] = {{~0u, ~0u, ~0u}, {~0u, ~0u, ~0u}};
 	bool any_tr = false, split = false, collect = true;
 	uint32_t n_saved = 0, next_saved = 0, g0 = 0; // groups before the last; the next to emit; the group's first face
 	int t0 = 0;
@@ -1614,7 +1601,9 @@ template <int NT> __device__ __forceinline__ void mesh_chunk(const MeshParams &p
 					s.mesh_base = base;
 			}
 			__syncthreads();
-			pool_base = s.pool_base;
+			pool_base = __builtin_amdgcn_readfirstlane(s.pool_base);
+			verts = reinterpret_cast<uint4 *>(p.pool_verts) + 2 * (size_t)pool_base;
+			idx = reinterpret_cast<uint32_t *>(p.pool_idx) + 3 * (size_t)pool_base;
 			if ((uint64_t)pool_base + total > p.pool_cap || (uint64_t)s.mesh_base + nm0 + nm1 > p.rec_cap) {
 				if (tid == 0)
 					p.results[job] = hcm_job_result{(int32_t)HCM_ERR_POOL_FULL, 0u, 0u, total};
@@ -1622,11 +1611,6 @@ template <int NT> __device__ __forceinline__ void mesh_chunk(const MeshParams &p
 			}
 			any_tr = n1 != 0;
 			split = n0 > kSplitQuads || n1 > kSplitQuads;
-			// AABB<uint32_t>::Merge (dep/AABB.hpp:52-59) of the first mesh of each pass per lane, reduced at
-			// the end; later meshes of a pass (past 16,383 quads) by LDS atomics
-#pragma unroll
-			for (int a = 0; a < 6; ++a)
-				box[0][a] = box[1][a] = a < 3 ? ~0u : 0u;
 			collect = false;
 		}
 		// 6. emission: one lane per visible face, a quad per face that starts one
@@ -1639,7 +1623,7 @@ template <int NT> __device__ __forceinline__ void mesh_chunk(const MeshParams &p
 			if (st) {
 				const uint32_t io = base_o + (before & 0xffffu) + lanes_below(opaque);
 				const uint32_t it = base_t + (before >> 16) + lanes_below(trans);
-				emit_face(p, s, desc, s.key[i], tr ? it : io, io + it, n0, pool_base, box, any_tr, split);
+				emit_face(s, desc, s.key[i], tr ? it : io, io + it, n0, verts, idx, box, any_tr, split);
 			}
 		}
 		if (next_saved == n_saved)
@@ -1675,30 +1659,25 @@ template <int NT> __device__ __forceinline__ void mesh_chunk(const MeshParams &p
 				const uint32_t e = v >> 2;
 				const uint2 ent = s.key[e];
 				const uint32_t tr = ent.x >> 31;
-				uint32_t slot, vbase, mk, mj, lo[3], hi[3];
-				quad_slot(tr, ent.y, n0, pool_base, slot, vbase, mk, mj);
-				emit_custom(p, s, blocks, ent.x & 0xffffu, v & 3, slot, vbase, lo, hi);
-				quad_done(s, tr, mk, (v & 3) ? ~0u : mj, w0 + e, lo, hi, box); // (a split is one lane's to note)
+				uint32_t vbase, mk, mj;
+				quad_place(ent.y, vbase, mk, mj);
+				const uint32_t slot = pool_base + (tr ? n0 : 0u) + ent.y;
+				const uint32_t at = emit_custom(p, s, blocks, ent.x & 0xffffu, v & 3, slot, vbase);
+				quad_done(s, tr, mk, (v & 3) ? ~0u : mj, w0 + e, word_box(at, at), box); // (a split is one lane's to note)
 			}
 		}
 	}
 
 	// the passes' boxes over the wavefront (a pass without quads is skipped: its boxes are empty)
 	if (n0) {
-#pragma unroll
-		for (int a = 0; a < 6; ++a)
-			box[0][a] = a < 3 ? wave_fold<false>(box[0][a]) : wave_fold<true>(box[0][a]);
+		const Box b = wave_box(box[0]);
+		if (lane == 0)
+			aabb_merge(s, 0, 0, b);
 	}
 	if (n1) {
-#pragma unroll
-		for (int a = 0; a < 6; ++a)
-			box[1][a] = a < 3 ? wave_fold<false>(box[1][a]) : wave_fold<true>(box[1][a]);
-	}
-	if (lane == 0 && (n0 | n1)) {
-		if (n0)
-			aabb_merge(s, 0, 0, box[0], box[0] + 3);
-		if (n1)
-			aabb_merge(s, 1, 0, box[1], box[1] + 3);
+		const Box b = wave_box(box[1]);
+		if (lane == 0)
+			aabb_merge(s, 1, 0, b);
 	}
 	__syncthreads();
 
@@ -1742,7 +1721,7 @@ template <int NT> __global__ __launch_bounds__(NT, NT >= 512 ? 2 : 3) void mesh_
 		s.pid_vox[i] = ok ? p.reg.pid_vox[i] : (uint32_t(i) << kVoxPidShift);
 	}
 	for (int i = threadIdx.x; i < kMaxCodes; i += NT)
-		s.codes[i] = i < (int)p.reg.n_codes ? p.reg.codes[i] : (kCodeEmpty | kCodeTransparent) << 16;
+		s.codes[i] = i < (int)p.reg.n_codes ? p.reg.codes[i] : 0u;
 	for (int i = threadIdx.x; i < 256; i += NT)
 	{
 		const uint32_t q = p.reg.pid_of[65536 + i];
