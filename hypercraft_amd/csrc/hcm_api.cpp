@@ -38,12 +38,12 @@ template <typename T> hipError_t dmalloc(T **p, size_t count) {
 struct DeviceTables {
 	std::vector<uint8_t> pid_of;
 	std::vector<uint2> rows;
-	std::vector<uint32_t> pid_vox;
+	std::vector<uint2> pid_vox;
 	std::vector<uint32_t> codes;
 	std::vector<hcm_custom_mesh> meshes;
 	std::vector<uint32_t> mesh_sums;
 	std::vector<uint8_t> light_info; // [65536]: light level | kLightInfoPass
-	uint32_t flow_pid_base = 0, flow_tex = 0, flow_trans = 0, src_id = 0, flow_id = 0;
+	uint32_t flow_pid_base = 0, flow_tex = 0, flow_trans = 0, src_id = 0, flow_id = 0, raw_front = 0;
 };
 
 int build_tables(const hcm_registry *r, DeviceTables *t) {
@@ -85,7 +85,7 @@ int build_tables(const hcm_registry *r, DeviceTables *t) {
 			return false;
 		return !s_t || o_t || o_l;
 	};
-	auto add_row = [&](const uint16_t tex[6], uint32_t dp, uint32_t ip, uint32_t mesh, uint32_t flags) {
+	auto add_row = [&](const uint16_t tex[6], uint32_t dp, uint32_t ip, uint32_t mesh, uint32_t flags, bool of_block) {
 		uint32_t tc[6], cls = 0;
 		for (int f = 0; f < 6; ++f) {
 			tc[f] = code_of(tex[f]);
@@ -101,8 +101,12 @@ int build_tables(const hcm_registry *r, DeviceTables *t) {
 		const uint32_t pid = (uint32_t)t->rows.size();
 		t->rows.push_back(make_uint2(tc[0] | tc[1] << 8 | tc[2] << 16 | tc[3] << 24,
 		                             tc[4] | tc[5] << 8 | self_show | mesh << 24));
-		t->pid_vox.push_back((dp ? kVoxDirect : 0u) | (ip ? kVoxIndirect : 0u) | cls << kVoxClassShift | flags |
-		                     pid << kVoxPidShift);
+		t->pid_vox.push_back(make_uint2(cls << kVoxClassShift | flags | (ip ? kVoxSunTorch : 0u),
+		                                (dp ? kVoxDirect : 0u) | (ip ? kVoxIndirect : 0u) |
+		                                    (flags & kTmplFlow ? kVoxFlow : 0u) | pid << kVoxPidShift));
+		// (a face shows only towards a face that is not opaque, and a mesh's light is its own cell's too)
+		if (!ip && of_block && ((flags & kTmplMesh) || cls != 0x555u))
+			t->raw_front = 1;
 	};
 	t->rows.clear();
 	t->pid_vox.clear();
@@ -113,13 +117,13 @@ int build_tables(const hcm_registry *r, DeviceTables *t) {
 			if (row.mesh >= r->n_meshes)
 				return HCM_ERR_INVALID;
 			mesh = row.mesh;
-			flags |= kVoxMesh;
+			flags |= kTmplMesh;
 			if (r->meshes[row.mesh].kind == HCM_MESH_LIQUID_FLOW)
-				flags |= kVoxFlow;
+				flags |= kTmplFlow;
 			else if (r->meshes[row.mesh].face_count > HCM_MAX_FACES)
 				return HCM_ERR_INVALID;
 		}
-		add_row(row.tex, row.transparency == 2 || row.collision != 1, row.transparency != 0, mesh, flags);
+		add_row(row.tex, row.transparency == 2 || row.collision != 1, row.transparency != 0, mesh, flags, true);
 	}
 	// dynamic liquid-flow textures: 16 = all faces liquid; else bits right, left, front, back full
 	// (the voxel keeps its own light-pass bits; only the face textures come from these rows)
@@ -134,8 +138,11 @@ int build_tables(const hcm_registry *r, DeviceTables *t) {
 			tex[0] = (p & 1) ? ft : 0, tex[1] = (p & 2) ? ft : 0, tex[2] = 0, tex[3] = ft;
 			tex[4] = (p & 4) ? ft : 0, tex[5] = (p & 8) ? ft : 0;
 		}
-		add_row(tex, 0, 0, 0xffu, 0);
+		add_row(tex, 0, 0, 0xffu, 0, false); // (no block's own row)
 	}
+	if (t->raw_front)
+		for (uint2 &q : t->pid_vox)
+			q.x |= kVoxSunTorch;
 	if (code_tex.size() > (size_t)kMaxCodes)
 		return HCM_ERR_INVALID;
 	t->codes.clear();
@@ -227,7 +234,7 @@ struct hcm_ctx {
 	// device registry buffers
 	uint8_t *d_pid_of = nullptr;
 	uint2 *d_rows = nullptr;
-	uint32_t *d_pid_vox = nullptr;
+	uint2 *d_pid_vox = nullptr;
 	uint32_t *d_codes = nullptr;
 	hcm_custom_mesh *d_meshes = nullptr;
 	uint32_t *d_mesh_sums = nullptr;
@@ -381,7 +388,7 @@ static int create_impl(hcm_ctx *c, const hcm_registry *registry, uint64_t pool_q
 	c->light_info = t.light_info;
 	HCM_HIP(hipMemcpy(c->d_pid_of, t.pid_of.data(), t.pid_of.size(), hipMemcpyHostToDevice));
 	HCM_HIP(hipMemcpy(c->d_rows, t.rows.data(), t.rows.size() * sizeof(uint2), hipMemcpyHostToDevice));
-	HCM_HIP(hipMemcpy(c->d_pid_vox, t.pid_vox.data(), t.pid_vox.size() * 4, hipMemcpyHostToDevice));
+	HCM_HIP(hipMemcpy(c->d_pid_vox, t.pid_vox.data(), t.pid_vox.size() * sizeof(uint2), hipMemcpyHostToDevice));
 	HCM_HIP(hipMemcpy(c->d_codes, t.codes.data(), t.codes.size() * 4, hipMemcpyHostToDevice));
 	if (!t.meshes.empty())
 		HCM_HIP(hipMemcpy(c->d_meshes, t.meshes.data(), t.meshes.size() * sizeof(hcm_custom_mesh),
@@ -391,6 +398,7 @@ static int create_impl(hcm_ctx *c, const hcm_registry *registry, uint64_t pool_q
 	c->reg.pid_of = c->d_pid_of;
 	c->reg.rows = c->d_rows;
 	c->reg.pid_vox = c->d_pid_vox;
+	c->reg.raw_front = t.raw_front;
 	c->reg.codes = c->d_codes;
 	c->reg.meshes = c->d_meshes;
 	c->reg.mesh_sums = c->d_mesh_sums;

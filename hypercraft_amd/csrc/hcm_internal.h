@@ -12,21 +12,23 @@ constexpr int kMaxPid = 128;   // registry rows + dynamic liquid-texture rows ke
 constexpr int kMaxCodes = 128; // distinct face textures kept in LDS
 constexpr int kFlowPatterns = 17;
 
-// Voxel word staged in LDS per halo voxel: sunlight in bits 0-3 and torchlight in bits 16-19 (the light
-// byte's low and high nibbles), and the per-row template below. With the indirect-pass bit at 12, a cell's
-// contribution to a light4_init corner sum is the word masked to kVoxLight when it passes light: adding
-// such words sums sunlight in bits 0-5, the count of cells in bits 12-13 and torchlight in bits 16-21.
-constexpr int kVoxPidShift = 4;            // texture row, 7 bits
-constexpr uint32_t kVoxPidMask = 0x7fu;
-constexpr uint32_t kVoxDirect = 1u << 11;   // VerticalLightPass || collision != solid (BlockMeshAlgo.hpp:119)
-constexpr uint32_t kVoxIndirect = 1u << 12; // transparency != opaque (block/include/block/Block.hpp:70)
-constexpr uint32_t kVoxMesh = 1u << 13;     // has a custom mesh
-constexpr uint32_t kVoxFlow = 1u << 14;     // liquid flow (dynamic mesh and face textures)
-constexpr int kVoxClassShift = 20;          // 2-bit face class per BlockFace f at bit 20 + 2 f
-constexpr uint32_t kVoxSunTorch = 0x000f000fu;
+// Voxel word staged in LDS per halo voxel, laid out so that light4_init adds words as they are (the fields above the
+// sums do not reach down into them): bit 0 zero and bits 1-4 the direct light pass, each four times; sunlight in bits
+// 8-11, 1 for a block that passes indirect light in bit 14 and torchlight in bits 16-19, so that a sum of four
+// has sunlight in bits 8-13, a count in bits 14-15 and torchlight in bits 16-21; the texture row in bits 23-29; flow.
+constexpr int kVoxSunBit = 8, kVoxIndirectBit = 14, kVoxTorchBit = 16;
+constexpr uint32_t kVoxDirect = 0x1eu;                   // VerticalLightPass || collision != solid (BlockMeshAlgo.hpp:119)
+constexpr uint32_t kVoxIndirect = 1u << kVoxIndirectBit; // transparency != opaque (block/include/block/Block.hpp:70)
+constexpr uint32_t kVoxSunTorch = 0xfu << kVoxSunBit | 0xfu << kVoxTorchBit;
 constexpr uint32_t kVoxLight = kVoxSunTorch | kVoxIndirect;
-// The light byte (sun | torch << 4) moved to the word's light fields.
-__host__ __device__ constexpr uint32_t vox_light(uint32_t byte) { return (byte * 0x1001u) & kVoxSunTorch; }
+constexpr int kVoxPidShift = 23; // texture row, 7 bits
+constexpr uint32_t kVoxPidMask = 0x7fu;
+constexpr uint32_t kVoxFlow = 1u << 30; // liquid flow (dynamic mesh and face textures)
+// A block's template: in y its voxel word but for light; in x its face classes, flags, and kVoxSunTorch if its light counts.
+constexpr uint32_t kTmplMesh = 1u; // has a custom mesh
+constexpr uint32_t kTmplFlow = 2u;
+constexpr uint32_t kTmplMeta = 4u; // (by block id) the texture row depends on the meta byte: the full table decides
+constexpr int kVoxClassShift = 20; // 2-bit face class per BlockFace f at bit 20 + 2 f
 // Face classes for BlockTexture::Show (texture/include/texture/BlockTexture.hpp:68-76)
 constexpr uint32_t kClassEmpty = 0, kClassOpaque = 1, kClassTransparent = 2, kClassLiquid = 3;
 
@@ -44,12 +46,13 @@ struct DevReg {
 	                               // the row when the meta byte does not change it, else 0xff
 	const uint2 *rows;             // [n_pid]: x = tc0..tc3 (8 bits each),
 	                               // y = tc4 | tc5 << 8 | kRowSelfShow | mesh << 24
-	const uint32_t *pid_vox;       // [n_pid]: voxel-word template (everything but the light fields)
+	const uint2 *pid_vox;          // [n_pid]: templates
 	const uint32_t *codes;         // [n_codes]
 	const hcm_custom_mesh *meshes; // [n_meshes]
 	const uint32_t *mesh_sums;     // [n_meshes]: faces | (bit j: face j goes to the transparent pass) << 16
 	uint32_t n_pid, n_codes, flow_pid_base;
 	uint32_t flow_tex, flow_trans, src_id, flow_id;
+	uint32_t raw_front; // a block that passes no indirect light may stand in front of a visible face (or have a mesh)
 };
 
 // The persistent kernels' job list is cut into kQueues contiguous parts, one per XCD (gfx950 has 8,

@@ -43,9 +43,9 @@ constexpr int kTasks = 96;
 __host__ __device__ constexpr int task_axis(int t) { return t >> 5; }
 __host__ __device__ constexpr int task_layer(int t) { return (t >> 1) & 15; }
 __host__ __device__ constexpr int task_plus(int t) { return t & 1; }
-// Entries of the face-word stage. 1,472 keeps the 256-thread workgroup's LDS within three per CU
+// Entries of the face-word stage. 1,344 keeps the 256-thread workgroup's LDS within three per CU
 // (static_assert below); the tasks of a chunk with more visible faces are taken in several groups.
-constexpr int kListCap = 1472;
+constexpr int kListCap = 1344;
 constexpr int kFaceBlocks = kListCap / 64;
 constexpr int kMaskRows = kTasks * 16;
 constexpr int kUnits = kMaskRows / 4; // a unit is four mask rows, 64 faces
@@ -150,9 +150,9 @@ template <int NT> struct Smem {
 				};
 			};
 		};
-		struct { // while a packed halo is staged: its bytes
-			alignas(16) uint16_t blocks[HCM_HALO_BLOCKS];
-			alignas(8) uint8_t light[HCM_HALO_LIGHT];
+		struct { // while a packed halo is staged (a row per thread): its bytes
+			alignas(16) uint16_t blocks[NT >= kHaloRows ? HCM_HALO_BLOCKS : 8];
+			alignas(8) uint8_t light[NT >= kHaloRows ? HCM_HALO_LIGHT : 8];
 		} halo;
 	};
 	alignas(16) uint16_t own[kListCap]; // per face of the group: 1 + its unit where one begins, else 0; then its descriptor
@@ -160,10 +160,11 @@ template <int NT> struct Smem {
 	uint32_t bcnt[64];         // per 64 faces of the group: quads that start there, opaque | transparent << 16
 	uint2 grp[kMaxGroups];     // per group of tasks: its first task, and the quads of the groups before it
 	uint2 rows[kMaxPid];
-	uint32_t pid_vox[kMaxPid];
+	uint2 pid_vox[kMaxPid];    // templates by texture row
 	uint32_t codes[kMaxCodes];
 	uint32_t custom_bits[128]; // in-chunk cells with a custom mesh
-	uint32_t tmpl_id[256];     // voxel-word template by block id when the meta byte does not change it, else kTmplMeta
+	uint2 tmpl_id[256];        // template by block id when the meta byte does not change it, else kTmplMeta
+	uint8_t sun_of[256], torch_of[256]; // averages of light4_init (fill_averages)
 	uint32_t aabb[2][kMaxMeshPerPass][6];
 	uint32_t events[16][2];
 	uint32_t scan_w[NT / 64][4]; // per wavefront: its totals of block_excl_sums
@@ -179,7 +180,7 @@ constexpr uint32_t kFlagNonUniform = 1u, kFlagCustom = 2u, kFlagFlow = 4u;
 // without either has no visible face: BlockTexture::Show never shows an empty face, nor an opaque face
 // against an opaque one (texture/include/texture/BlockTexture.hpp:68-76).
 constexpr uint32_t kFlagMixed = 8u, kFlagInnerFaces = 16u;
-constexpr uint32_t kVoxShape = 0xfff00000u | kVoxMesh | kVoxFlow; // the face classes and the mesh and flow bits
+constexpr uint32_t kVoxShape = 0xfff00000u | kTmplMesh | kTmplFlow; // the face classes and the mesh and flow bits
 constexpr uint32_t kVoxOpaqueCube = 0x555u << kVoxClassShift; // opaque on all six faces
 
 // ------------------------------------------------------------------------------------------------
@@ -194,17 +195,9 @@ template <int NT> __device__ __forceinline__ uint32_t row_code(const Smem<NT> &s
 }
 
 // Texture row of a block value: from LDS for most ids, from the full table for meta-dependent ones.
-// A template word flag (bit 15 of the voxel word is otherwise unused): the block id's texture row depends
-// on the meta byte, so the full table decides.
-constexpr uint32_t kTmplMeta = 1u << 15;
-
 template <int NT> __device__ __forceinline__ uint32_t block_pid(const MeshParams &p, const Smem<NT> &s, uint32_t b) {
-	const uint32_t q = s.tmpl_id[b & 0xffu];
-	return q & kTmplMeta ? p.reg.pid_of[b] : vox_pid(q);
-}
-
-__device__ __forceinline__ uint32_t face_class(uint32_t vox, int face) {
-	return (vox >> (kVoxClassShift + 2 * face)) & 3u;
+	const uint2 q = s.tmpl_id[b & 0xffu];
+	return q.x & kTmplMeta ? p.reg.pid_of[b] : vox_pid(q.y);
 }
 
 // AO of a light4_init vertex (:126-130) by side, corner and side cell direct-pass bits and the front cell's:
@@ -221,58 +214,75 @@ constexpr uint32_t ao_table() {
 }
 constexpr uint32_t kAoTable = ao_table();
 static_assert(kAoTable == 0xe9849040u, "AO table");
+constexpr uint32_t rotate_left(uint32_t v, int n) { return n ? v << n | v >> (32 - n) : v; }
 
-// (sum << 2) / cnt for cnt in 1..4 and sum <= 15 cnt, exactly: (sum * R) >> 7 with R = 512, 256, 171, 128,
-// packed 16 bits apart by cnt - 1. Checked below for every possible sum.
-constexpr uint64_t kRecip = 0x008000ab01000200ull;
-constexpr bool recip_exact() {
-	for (uint32_t cnt = 1; cnt <= 4; ++cnt)
-		for (uint32_t sum = 0; sum <= 15 * cnt; ++sum)
-			if (((sum * uint32_t((kRecip >> (16 * (cnt - 1))) & 0x3ffu)) >> 7) != (sum << 2) / cnt)
-				return false;
-	return true;
-}
-static_assert(recip_exact(), "reciprocal table");
-
-// A cell's light in a light4_init sum: its word masked to the light fields and the count bit when it
-// passes indirect light (:132-161), else 0.
-__device__ __forceinline__ uint32_t lpass(uint32_t c) { return c & kVoxLight & (0u - ((c >> 12) & 1u)); }
-
-// One vertex of light4_init (:114-162), without branches, from its side cells a and b, corner cell c and
-// the front cell: the side cells count when they pass indirect light, the corner when it does and a side
-// cell does; sunlight and torchlight are averaged as (sum << 2) / count, the front cell always counted.
-// Returns ao | sun << 2 | torch << 8.
-__device__ __forceinline__ uint32_t light_vertex(uint32_t a, uint32_t c, uint32_t b, uint32_t pf, uint32_t d3) {
-	const uint32_t g = 0u - (((a | b) >> 12) & 1u);
-	const uint32_t sum = pf + lpass(a) + lpass(b) + (lpass(c) & g); // count - 1 in bits 12-13
-	const uint32_t r = uint32_t(kRecip >> ((sum >> 8) & 0x30u)) & 0x3ffu;
-	const uint32_t prod = (sum & 0x003f003fu) * r;
-	const uint32_t idx = ((a >> 11) & 1u) | ((c >> 10) & 2u) | ((b >> 9) & 4u) | d3;
-	return ((prod >> 5) & 0xfcu) | (((prod >> 23) & 63u) << 8) | ((kAoTable >> (2 * idx)) & 3u);
+// (sum << 2) / count for every sum of lights of 0 to 15, as bytes by the fields of a sum of voxel words: sunlight by
+// sum | (count - 1) << 6 and moved up by the two bits a face word has it at, torchlight by (count - 1) | sum << 2.
+template <int NT> __device__ __forceinline__ void fill_averages(Smem<NT> &s) {
+	for (uint32_t i = threadIdx.x; i < 256; i += NT) {
+		s.sun_of[i] = uint8_t((i & 63u) * 4u / ((i >> 6) + 1u) << 2);
+		s.torch_of[i] = uint8_t((i >> 2) * 4u / ((i & 3u) + 1u));
+	}
 }
 
-// light4_init (:48-163) for face `face` of the block at halo index self. Returns the packed Light4, a vertex in 14 bits
-// as a vertex word holds it from bit 16 on: vertex 0 | vertex 1 << 14 in x, vertex 2 | vertex 3 << 14 in y.
-// The front cell F and its eight neighbours in the face's plane; vertex k's side cells along the plane
-// axes Q and P and the corner between them have (P, Q) signs (-,-), then (+,-) or (-,+) by the winding,
-// then (+,+), then the other of (+,-) and (-,+).
-__device__ __forceinline__ uint2 light4(const uint32_t *vox, int face, int self) {
+// A cell's word in a light4_init sum when it passes indirect light (:132-161). Voxel words have no light where their
+// block does not pass it, so that words are added as they are, unless the registry has such a block in front of
+// visible faces (kRaw), whose light counts there.
+template <bool kRaw> __device__ __forceinline__ uint32_t lpass(uint32_t c) {
+	return kRaw ? c & (uint32_t(int32_t(c << (31 - kVoxIndirectBit)) >> 31) | ~kVoxLight) : c;
+}
+
+// Sum of one vertex of light4_init (:114-162), without branches, from its side cells a and b, corner cell c and f, the
+// sum of the front cell and a: the corner counts when a side cell passes indirect light.
+__device__ __forceinline__ uint32_t light_sum(uint32_t a, uint32_t c, uint32_t b, uint32_t f) {
+	return f + b + (c & uint32_t(int32_t((a | b) << (31 - kVoxIndirectBit)) >> 31));
+}
+
+// light4_init (:48-163) for the face whose front cell is at byte f of vox. P and Q: the byte strides of its plane's axes
+// in the order of its winding, so that its vertices 0 to 3 have the corner cells (-,-), (+,-), (+,+) and (-,+) and the
+// side cells along each axis. Returns the packed Light4, a vertex in 14 bits as a vertex word holds it from
+// bit 16 on: vertex 0 | vertex 1 << 14 in x, vertex 2 | vertex 3 << 14 in y.
+//
+// Dense chunks issue most of their instructions here. Sums of whole words (no masks), averages by LDS look-ups at the
+// sums' fields and AO by a table rotated by the cells' direct-pass bits, which each word has at the four places its cell
+// may take: the loop around it is 174 VALU instructions per 64 faces, where masked sums with reciprocals made it 247.
+// 2,304 chunks of random blocks took 724 us so, now 659; 768 plant chunks 30.7 and 30.1.
+template <bool kRaw, int NT> __device__ __forceinline__ uint2 light4(const Smem<NT> &s, int f, int P, int Q) {
+	const char *vox = reinterpret_cast<const char *>(s.vox);
+	const auto cell = [vox](int at) { return *reinterpret_cast<const uint32_t *>(vox + at); };
+	const int fm = f - P, fp = f + P;
+	const uint32_t F = cell(f);
+	const uint32_t qm = lpass<kRaw>(cell(f - Q)), qp = lpass<kRaw>(cell(f + Q));
+	const uint32_t pm = lpass<kRaw>(cell(fm)), pp = lpass<kRaw>(cell(fp));
+	const uint32_t c0 = lpass<kRaw>(cell(fm - Q)), c1 = lpass<kRaw>(cell(fp - Q));
+	const uint32_t c2 = lpass<kRaw>(cell(fp + Q)), c3 = lpass<kRaw>(cell(fm + Q));
+	const uint32_t front = F & ~kVoxIndirect; // counted always, as the 1 of count - 1
+	const uint32_t fqm = front + qm, fqp = front + qp;
+	const uint32_t s0 = light_sum(qm, c0, pm, fqm), s1 = light_sum(qm, c1, pp, fqm);
+	const uint32_t s2 = light_sum(qp, c2, pp, fqp), s3 = light_sum(qp, c3, pm, fqp);
+	const auto vertex = [&s](uint32_t sum) {
+		return uint32_t(s.sun_of[(sum >> kVoxSunBit) & 0xffu]) | uint32_t(s.torch_of[(sum >> (kVoxTorchBit - 2)) & 0xffu]) << 8;
+	};
+	uint32_t x = vertex(s0) | vertex(s1) << 14, y = vertex(s2) | vertex(s3) << 14;
+	// AO: bits 1 to 4 of a word, of which bit 0 is zero, rotate the table by the two bits of each cell's flag
+	const auto direct = [](uint32_t bit, uint32_t a, uint32_t b) { return (a & bit) | (b & ~bit); };
+	const uint32_t dqm = direct(2u, qm, F), dqp = direct(2u, qp, F);
+	const auto ao = [&](uint32_t dq, uint32_t c, uint32_t b, uint32_t table) {
+		return __builtin_amdgcn_alignbit(table, table, direct(8u, b, direct(4u, c, dq)));
+	};
+	constexpr uint32_t table1 = rotate_left(kAoTable, 14);
+	x = direct(3u << 14, ao(dqm, c1, pp, table1), direct(3u, ao(dqm, c0, pm, kAoTable), x));
+	y = direct(3u << 14, ao(dqp, c3, pm, table1), direct(3u, ao(dqp, c2, pp, kAoTable), y));
+	return make_uint2(x, y);
+}
+
+// The same for face `face` of the block at halo index self. Winding a (faces 0, 3 and 4) has the plane axes in order.
+template <bool kRaw, int NT> __device__ __forceinline__ uint2 light4_of(const Smem<NT> &s, int face, int self) {
 	const int a = face >> 1;
 	const int sn = a == 0 ? kSX : (a == 1 ? kSY : kSZ);
-	const int sp = a == 0 ? kSY : kSX; // plane axis P
-	const int sq = a == 2 ? kSY : kSZ; // plane axis Q
-	const int f = self + ((face & 1) ? -sn : sn);
-	const uint32_t F = vox[f];
-	const uint32_t qm = vox[f - sq], qp = vox[f + sq], pm = vox[f - sp], pp = vox[f + sp];
-	const uint32_t mm = vox[f - sp - sq], mp = vox[f - sp + sq], pmq = vox[f + sp - sq], ppq = vox[f + sp + sq];
+	const int sp = a == 0 ? kSY : kSX, sq = a == 2 ? kSY : kSZ;
 	const bool wa = face == 0 || face == 3 || face == 4;
-	const uint32_t pf = F & kVoxSunTorch, d3 = ((F >> 11) & 1u) << 3;
-	// the corners (+,-) and (-,+): vertex 1 is the first with winding a, else the second; vertex 3 the
-	// other (each side cell then enters two vertices through the same expressions)
-	const uint32_t vpm = light_vertex(qm, pmq, pp, pf, d3), vmp = light_vertex(qp, mp, pm, pf, d3);
-	const uint32_t v0 = light_vertex(qm, mm, pm, pf, d3), v1 = wa ? vpm : vmp;
-	const uint32_t v2 = light_vertex(qp, ppq, pp, pf, d3), v3 = wa ? vmp : vpm;
-	return make_uint2(v0 | v1 << 14, v2 | v3 << 14);
+	return light4<kRaw>(s, 4 * (self + ((face & 1) ? -sn : sn)), 4 * (wa ? sp : sq), 4 * (wa ? sq : sp));
 }
 
 __device__ __forceinline__ uint32_t l4_at(uint2 l, int k, int bit) { return (k < 2 ? l.x : l.y) >> (14 * (k & 1) + bit); }
@@ -509,7 +519,7 @@ __device__ __forceinline__ CustomCell custom_cell(const MeshParams &p, const Sme
 		pid = block_pid(p, s, blocks.at(x, y, z));
 	CustomCell c;
 	c.mesh = s.rows[pid].y >> 24;
-	c.flow = (s.pid_vox[pid] & kVoxFlow) ? 1u : 0u;
+	c.flow = (s.pid_vox[pid].x & kTmplFlow) ? 1u : 0u;
 	c.trans = 0;
 	c.flow_set = 0;
 	c.fl.h = 0, c.fl.liq_side = 0;
@@ -654,7 +664,7 @@ __device__ __forceinline__ Interp interp(const uint32_t l[4], const uint32_t h[4
 // is the length of one's chain of loads and operations: four lanes share a quad's vertices, the face counts and passes
 // come from one word per mesh, and light is interpolated two values at a time. 768 chunks of terrain with plants
 // took 47.7 us with a lane per quad and two loads per face, 31.9 so; one such chunk from host memory 41.4 and 33.3.
-template <int NT>
+template <bool kRaw, int NT>
 __device__ __forceinline__ uint32_t emit_custom(const MeshParams &p, Smem<NT> &s, const JobBlocks &blocks, uint32_t desc,
                                                 uint32_t k, uint32_t slot, uint32_t vbase) {
 	const int cell = desc & 4095, j = (desc >> 12) & 15;
@@ -664,8 +674,8 @@ __device__ __forceinline__ uint32_t emit_custom(const MeshParams &p, Smem<NT> &s
 	const int lf = f.light_face, la = lf >> 1, sg = (lf & 1) ? -1 : 1;
 	const int pos = hidx(x, y, z);
 	// low: the face of the cell behind; high: this cell's own face if the next cell passes light (:259-267)
-	const uint2 lo4 = light4(s.vox, lf, pos - sg * axis_stride(la));
-	const uint2 hi4 = (s.vox[pos + sg * axis_stride(la)] & kVoxIndirect) ? light4(s.vox, lf, pos) : lo4;
+	const uint2 lo4 = light4_of<kRaw>(s, lf, pos - sg * axis_stride(la));
+	const uint2 hi4 = (s.vox[pos + sg * axis_stride(la)] & kVoxIndirect) ? light4_of<kRaw>(s, lf, pos) : lo4;
 	int ua = (la + 1) % 3, va = (la + 2) % 3;
 	if (lf & 1) {
 		const int tmp = ua;
@@ -729,7 +739,7 @@ constexpr bool show_matches() {
 static_assert(show_matches(), "Show on face classes");
 } // namespace check
 
-// Bytes of (hi, lo) by selector: selector byte 0-3 takes that byte of lo, 4-7 of hi.
+// Bytes of (hi, lo) by selector: selector byte 0-3 takes that byte of lo, 4-7 of hi, 12 is zero.
 __device__ __forceinline__ uint32_t byte_perm(uint32_t hi, uint32_t lo, uint32_t sel) {
 	return __builtin_amdgcn_perm(hi, lo, sel);
 }
@@ -757,7 +767,7 @@ __device__ __forceinline__ void row_planes(const uint32_t tm[16], uint32_t p0[3]
 	p0[2] = byte_perm(r[6], r[4], 0x07050301u), p1[2] = byte_perm(r[7], r[5], 0x07050301u);
 }
 
-// A halo row's planes (templates tm[0 .. 17] of x = -1 .. 16) to where the rows beside it read them; for a
+// A halo row's planes (first template words tm[0 .. 17] of x = -1 .. 16) to where the rows beside it read them; for a
 // row of the chunk also its visible x faces, which need no other row.
 template <int NT> __device__ __forceinline__ void put_planes(Smem<NT> &s, int hy, int hz, const uint32_t tm[18]) {
 	uint32_t p0[3], p1[3];
@@ -841,14 +851,6 @@ template <int NT> __device__ __forceinline__ void visibility_row(Smem<NT> &s, in
 // goes to the transparent pass.
 constexpr uint32_t kDescTrans = 0x8000u;
 static_assert(kTasks * 256 <= (int)kDescTrans, "descriptors of 15 bits");
-
-// Halo index of the block owning a face, and which of its faces it is.
-__device__ __forceinline__ int face_owner(uint32_t desc, int &face) {
-	const int t = (desc >> 8) & 127, u = (desc >> 4) & 15, v = desc & 15;
-	const int A = task_axis(t), layer = task_layer(t);
-	face = 2 * A + (task_plus(t) ^ 1);
-	return (layer + 1) * axis_stride(A) + (u + 1) * axis_stride(u_axis(A)) + (v + 1) * axis_stride(v_axis(A));
-}
 
 // Running maximum over the wavefront, as wave_incl_sum.
 __device__ __forceinline__ uint32_t wave_incl_max(uint32_t v) {
@@ -951,11 +953,17 @@ template <int NT> __device__ __forceinline__ uint32_t face_desc(const Smem<NT> &
 // four of x and bits 28-30 of y and the transparent-pass flag in bit 31. Faces merge only if their words are equal
 // (Light4::operator==, :44, and the texture compare, :367-368). The code's upper three bits and the flag come from
 // the table of codes as they lie in the word.
-template <int NT> __device__ __forceinline__ uint2 face_word(const Smem<NT> &s, uint32_t desc) {
-	int face;
-	const int self = face_owner(desc, face);
-	const uint2 l = light4(s.vox, face, self);
-	const uint32_t tc = row_code(s, vox_pid(s.vox[self]), face);
+template <bool kRaw, int NT> __device__ __forceinline__ uint2 face_word(const Smem<NT> &s, uint32_t desc) {
+	const int t = desc >> 8, u = (desc >> 4) & 15, v = desc & 15;
+	const int A = task_axis(t), inv = task_plus(t) ^ 1;
+	// byte strides along the mask's axes and the task's: 1, 18 and 324 voxels
+	constexpr int all = 4 * (kSX + kSY + kSZ);
+	const int su = A == 1 ? 4 * kSZ : 4 * kSY, sv = A == 0 ? 4 * kSZ : 4 * kSX, sa = all - su - sv;
+	const int self = all + task_layer(t) * sa + u * su + v * sv;
+	const bool u_first = inv == int(A == 2); // the winding's first axis (kLookup3v) is U
+	const uint2 l = light4<kRaw>(s, self + (inv ? -sa : sa), u_first ? su : sv, u_first ? sv : su);
+	const uint32_t pid = vox_pid(*reinterpret_cast<const uint32_t *>(reinterpret_cast<const char *>(s.vox) + self));
+	const uint32_t tc = row_code(s, pid, 2 * A + inv);
 	return make_uint2(l.x | tc << 28, l.y | (s.codes[tc] & ~kCodeLow));
 }
 
@@ -1286,7 +1294,7 @@ template <int NT> __device__ __forceinline__ HaloRow halo_row(const Smem<NT> &s,
 }
 
 // One job; s.slots and the state of chunk_init are in place (a barrier after them).
-template <int NT> __device__ __forceinline__ void mesh_chunk(const MeshParams &p, Smem<NT> &s, uint32_t job) {
+template <bool kRaw, int NT> __device__ __forceinline__ void mesh_chunk(const MeshParams &p, Smem<NT> &s, uint32_t job) {
 	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
 	constexpr int CPT = HCM_CHUNK_VOXELS / NT; // custom cells per thread
 
@@ -1353,12 +1361,13 @@ template <int NT> __device__ __forceinline__ void mesh_chunk(const MeshParams &p
 		for (int k = 0; k < 8; ++k)
 			diff |= bw[k] ^ ref2;
 		const bool nonuniform = diff != 0;
-		uint32_t tm[18];
-		tm[0] = s.tmpl_id[bl & 0xffu];
-		tm[17] = s.tmpl_id[br & 0xffu];
+		uint32_t tm[18], words[18];
 #pragma unroll
-		for (int x = 0; x < 16; ++x)
-			tm[x + 1] = s.tmpl_id[(bw[x >> 1] >> (16 * (x & 1))) & 0xffu];
+		for (int x = 0; x < 18; ++x) {
+			const uint32_t b = x == 0 ? bl : (x == 17 ? br : bw[(x - 1) >> 1] >> (16 * ((x - 1) & 1)));
+			const uint2 q = s.tmpl_id[b & 0xffu];
+			tm[x] = q.x, words[x] = q.y;
+		}
 		uint32_t any_meta = 0;
 #pragma unroll
 		for (int x = 0; x < 18; ++x)
@@ -1374,16 +1383,20 @@ template <int NT> __device__ __forceinline__ void mesh_chunk(const MeshParams &p
 			}
 #pragma unroll
 			for (int x = 0; x < 18; ++x) {
-				const uint32_t v = s.pid_vox[full[x]];
-				tm[x] = tm[x] & kTmplMeta ? v : tm[x];
+				const uint2 v = s.pid_vox[full[x]];
+				words[x] = tm[x] & kTmplMeta ? v.y : words[x];
+				tm[x] = tm[x] & kTmplMeta ? v.x : tm[x];
 			}
 		}
 		put_planes(s, hy, hz, tm);
 		uint32_t and_all = ~0u, or_inner = 0;
 		uint32_t *dst = s.vox + row * kHalo;
+		static_assert(kVoxSunBit == 8 && kVoxTorchBit == 16, "light in the low nibbles of two bytes");
 #pragma unroll
 		for (int x = 0; x < 18; ++x) {
-			dst[x] = vox_light((lw[x >> 2] >> (8 * (x & 3))) & 0xffu) | tm[x];
+			const uint32_t w = lw[x >> 2], k = x & 3; // light bytes are sun | torch << 4
+			const uint32_t light = byte_perm((w >> 4) & 0x0f0f0f0fu, w & 0x0f0f0f0fu, 0x0c04000cu + 0x010100u * k);
+			dst[x] = (light & tm[x]) | words[x];
 			and_all &= tm[x];
 			if (x >= 1 && x <= 16)
 				or_inner |= tm[x];
@@ -1399,13 +1412,13 @@ template <int NT> __device__ __forceinline__ void mesh_chunk(const MeshParams &p
 			my_flags |= kFlagMixed;
 		if (inside_yz && (or_inner & kVoxShape))
 			my_flags |= kFlagInnerFaces;
-		if (or_all & kVoxFlow)
+		if (or_all & kTmplFlow)
 			my_flags |= kFlagFlow;
-		if (inside_yz && (or_inner & kVoxMesh)) {
+		if (inside_yz && (or_inner & kTmplMesh)) {
 			uint32_t mesh_bits = 0;
 #pragma unroll
 			for (int x = 0; x < 16; ++x)
-				mesh_bits |= ((tm[x + 1] / kVoxMesh) & 1u) << x;
+				mesh_bits |= ((tm[x + 1] / kTmplMesh) & 1u) << x;
 			const uint32_t cell0 = 16u * (uint32_t(z) + 16u * uint32_t(y));
 			atomicOr(&s.custom_bits[cell0 >> 5], mesh_bits << (cell0 & 31));
 			my_flags |= kFlagCustom;
@@ -1443,7 +1456,7 @@ template <int NT> __device__ __forceinline__ void mesh_chunk(const MeshParams &p
 
 	// 2. liquid-flow cells take the flow mesh's face textures (:221-236)
 	if (flags & kFlagFlow) {
-		constexpr uint32_t kKeep = kVoxSunTorch | kVoxDirect | kVoxIndirect;
+		constexpr uint32_t kKeep = kVoxLight | kVoxDirect;
 		for (int i = tid; i < kHaloVox; i += NT) {
 			if (!(s.vox[i] & kVoxFlow)) // each thread rewrites only its own cells
 				continue;
@@ -1451,17 +1464,16 @@ template <int NT> __device__ __forceinline__ void mesh_chunk(const MeshParams &p
 			const uint32_t pid = vox_pid(s.vox[i]);
 			const uint32_t mesh = s.rows[pid].y >> 24;
 			const Flow f = flow_heights(p, blocks, hx - 1, hy - 1, hz - 1, p.reg.meshes[mesh].flow_height);
-			const uint32_t tmpl = s.pid_vox[p.reg.flow_pid_base + flow_pattern(f)];
+			const uint32_t tmpl = s.pid_vox[p.reg.flow_pid_base + flow_pattern(f)].y;
 			s.vox[i] = (s.vox[i] & kKeep) | (tmpl & ~kKeep);
 		}
 		__syncthreads();
-		// their rows' planes again (the light fields of a voxel word lie below its class bits, which are all
-		// that row_planes takes but for torchlight, in the bits it drops)
+		// their rows' planes again
 		for (int row = tid; row < kHaloRows; row += NT) {
 			uint32_t w[18];
 #pragma unroll
 			for (int x = 0; x < 18; ++x)
-				w[x] = s.vox[row * kHalo + x];
+				w[x] = s.pid_vox[vox_pid(s.vox[row * kHalo + x])].x;
 			put_planes(s, row / kHalo, row % kHalo, w);
 		}
 		__syncthreads();
@@ -1541,7 +1553,7 @@ template <int NT> __device__ __forceinline__ void mesh_chunk(const MeshParams &p
 		for (uint32_t b = wave_u; b * 64 < n; b += NT / 64) {
 			const uint32_t i = 64 * b + lane, desc = face_desc(s, i, g0);
 			if (i < n) {
-				const uint2 word = face_word(s, desc);
+				const uint2 word = face_word<kRaw>(s, desc);
 				s.key[i] = word;
 				s.own[i] = uint16_t(desc | (word.y >> 31 ? kDescTrans : 0u));
 			}
@@ -1662,7 +1674,7 @@ template <int NT> __device__ __forceinline__ void mesh_chunk(const MeshParams &p
 				uint32_t vbase, mk, mj;
 				quad_place(ent.y, vbase, mk, mj);
 				const uint32_t slot = pool_base + (tr ? n0 : 0u) + ent.y;
-				const uint32_t at = emit_custom(p, s, blocks, ent.x & 0xffffu, v & 3, slot, vbase);
+				const uint32_t at = emit_custom<kRaw>(p, s, blocks, ent.x & 0xffffu, v & 3, slot, vbase);
 				quad_done(s, tr, mk, (v & 3) ? ~0u : mj, w0 + e, word_box(at, at), box); // (a split is one lane's to note)
 			}
 		}
@@ -1713,20 +1725,21 @@ template <int NT> __device__ __forceinline__ void mesh_chunk(const MeshParams &p
 	}
 }
 
-template <int NT> __global__ __launch_bounds__(NT, NT >= 512 ? 2 : 3) void mesh_kernel(MeshParams p) {
+template <int NT, bool kRaw> __global__ __launch_bounds__(NT, NT >= 512 ? 2 : 3) void mesh_kernel(MeshParams p) {
 	__shared__ Smem<NT> s;
 	for (int i = threadIdx.x; i < kMaxPid; i += NT) {
 		const bool ok = i < (int)p.reg.n_pid;
 		s.rows[i] = ok ? p.reg.rows[i] : make_uint2(0, 0);
-		s.pid_vox[i] = ok ? p.reg.pid_vox[i] : (uint32_t(i) << kVoxPidShift);
+		s.pid_vox[i] = ok ? p.reg.pid_vox[i] : make_uint2(0, uint32_t(i) << kVoxPidShift);
 	}
 	for (int i = threadIdx.x; i < kMaxCodes; i += NT)
 		s.codes[i] = i < (int)p.reg.n_codes ? p.reg.codes[i] : 0u;
 	for (int i = threadIdx.x; i < 256; i += NT)
 	{
 		const uint32_t q = p.reg.pid_of[65536 + i];
-		s.tmpl_id[i] = q == 0xffu ? kTmplMeta : p.reg.pid_vox[q];
+		s.tmpl_id[i] = q == 0xffu ? make_uint2(kTmplMeta, 0) : p.reg.pid_vox[q];
 	}
+	fill_averages(s);
 	JobClaims claims(p.n_jobs); // lane 0 of wavefront 0 only
 	const int lane = threadIdx.x & 63;
 	const uint32_t given = p.job_base + blockIdx.x; // per-chunk launches: the workgroup's one job
@@ -1747,7 +1760,7 @@ template <int NT> __global__ __launch_bounds__(NT, NT >= 512 ? 2 : 3) void mesh_
 		const uint32_t job = s.job;
 		if (job >= p.n_jobs)
 			break;
-		mesh_chunk(p, s, job);
+		mesh_chunk<kRaw>(p, s, job);
 		if (!p.persistent)
 			break;
 		__syncthreads();
@@ -1877,15 +1890,18 @@ hipError_t launch_reset(Counters *ctr, hipStream_t stream) {
 hipError_t launch_mesh(const MeshParams &p, int threads, int grid, hipStream_t stream) {
 	if (p.halo_in && threads < kHaloRows) // packed halos are staged one row per thread
 		return hipErrorInvalidValue;
+	const auto launch = [&](auto plain, auto raw) {
+		hipLaunchKernelGGL(p.reg.raw_front ? raw : plain, dim3(grid), dim3(threads), 0, stream, p);
+	};
 	switch (threads) {
 	case 128:
-		hipLaunchKernelGGL(mesh_kernel<128>, dim3(grid), dim3(128), 0, stream, p);
+		launch(mesh_kernel<128, false>, mesh_kernel<128, true>);
 		break;
 	case 256:
-		hipLaunchKernelGGL(mesh_kernel<256>, dim3(grid), dim3(256), 0, stream, p);
+		launch(mesh_kernel<256, false>, mesh_kernel<256, true>);
 		break;
 	case 512:
-		hipLaunchKernelGGL(mesh_kernel<512>, dim3(grid), dim3(512), 0, stream, p);
+		launch(mesh_kernel<512, false>, mesh_kernel<512, true>);
 		break;
 	default:
 		return hipErrorInvalidValue;

@@ -114,12 +114,17 @@ __attribute__((noinline)) uint32_t site_dpp(uint32_t old, uint32_t src, uint32_t
 #define __builtin_amdgcn_update_dpp(old, src, ctrl, rm, bm, bc) \
 	((int)::hipcpu::site_dpp((uint32_t)(old), (uint32_t)(src), (ctrl), (rm), (bm), nullptr))
 
-// v_perm_b32: selector bytes 0-3 take a byte of lo, 4-7 of hi (the kernels use no other selector)
+// v_alignbit_b32: (hi, lo) shifted right by the shift's low five bits
+inline uint32_t __builtin_amdgcn_alignbit(uint32_t hi, uint32_t lo, uint32_t shift) {
+	return uint32_t(((uint64_t(hi) << 32) | lo) >> (shift & 31u));
+}
+// v_perm_b32: selector bytes 0-3 take a byte of lo, 4-7 of hi, 12 zero (the kernels use no other selector)
 inline uint32_t __builtin_amdgcn_perm(uint32_t hi, uint32_t lo, uint32_t sel) {
 	const uint64_t v = (uint64_t(hi) << 32) | lo;
 	uint32_t r = 0;
 	for (int i = 0; i < 4; ++i)
-		r |= uint32_t((v >> (8 * ((sel >> (8 * i)) & 7u))) & 0xffu) << (8 * i);
+		if (((sel >> (8 * i)) & 0xffu) != 12u)
+			r |= uint32_t((v >> (8 * ((sel >> (8 * i)) & 7u))) & 0xffu) << (8 * i);
 	return r;
 }
 // v_mbcnt: the set bits of a mask below this lane, added up over its two halves

@@ -85,10 +85,10 @@ def chunk_with_faces(n):
 
 
 @pytest.mark.parametrize("merge", [False, True])
-@pytest.mark.parametrize("faces", [1, 2, 63, 64, 65, 128, 1471, 1472, 1473, 1536, 2944, 2945, 4416, 4417, 8232])
+@pytest.mark.parametrize("faces", [1, 2, 63, 64, 65, 128, 1343, 1344, 1345, 1471, 1472, 1473, 1536, 2688, 2689, 2944, 2945, 4416, 4417, 8232])
 def test_face_counts_at_block_and_group_edges(ctx, oracle, faces, merge):
     """Visible faces are numbered by units of 64 mask bits, handled in blocks of 64 lanes and held in groups of up to
-    1,472: counts at and beside those edges, with light that lets faces merge and light that does not."""
+    1,344: counts at and beside those edges, with light that lets faces merge and light that does not."""
     if faces < 3:  # nothing apart has so few: a slab's top, and two
         b27 = [np.zeros(4096, np.uint16) if d[1] == 1 else np.ones(4096, np.uint16) for d in workloads.SLOT_OFFSETS]
         l27 = [np.zeros(4096, np.uint8)] * 27
@@ -185,5 +185,46 @@ def test_batches_around_a_job_per_cu(n, oracle):
         for j in range(n):
             assert meshdigest.digest(hcm.job_meshes(j, *out)) == want[j & 1], (asked, j)
         batch.close()
+    store.close()
+    ctx.close()
+
+
+@pytest.mark.parametrize("kind,seed,threads", [("mesh", 1, 256), ("face", 2, 256), ("both", 3, 512), ("cubes", 4, 256), ("both", 5, 128)])
+def test_blocks_in_front_that_pass_no_light(tmp_path, kind, seed, threads):
+    """Voxel words hold no light where a block passes none, unless the registry has such a block that a visible face may
+    look at: one with a face that is not opaque, or with a mesh. Blocks that pass none and are opaque cubes need no more."""
+    import cpu_oracle
+
+    reg = cases.RegistryFile(REGISTRY)
+    rng = np.random.default_rng(seed)
+    flags = reg.tex_flags[np.minimum(reg.rows["tex"] & 0x1FFF, len(reg.tex_flags) - 1)]
+    cube = (((reg.rows["tex"] & 0x1FFF) != 0) & ((flags & 5) == 0)).all(axis=1)
+    mesh = reg.rows["mesh"] != 0xFFFF
+    pick = {"mesh": mesh, "face": ~cube & ~mesh, "both": np.ones(len(mesh), bool), "cubes": cube & ~mesh}[kind]
+    assert pick.any()
+    reg.rows["transparency"][pick & (rng.random(len(mesh)) < 0.7)] = 0
+    path = str(tmp_path / f"registry_{kind}.bin")
+    reg.write(path)
+    orc = cpu_oracle.Oracle(path)
+    ids = np.arange(1, 256)
+    values = np.unique(np.concatenate([cases.CUSTOM, ids[reg.row_of[ids] != reg.row_of[255]], ids[:40], ids[:40] | 0x100]))
+    n = 3
+    blocks = np.where(rng.random((27 * n, 4096)) < 0.4, values[rng.integers(0, values.size, (27 * n, 4096))], 0).astype(np.uint16)
+    light = rng.integers(0, 256, blocks.shape).astype(np.uint8)
+    nbr = np.arange(27 * n, dtype=np.uint32).reshape(n, 27)
+    ctx = hcm.Context(pool_quads=1 << 20, registry=reg.c_registry(hcm))
+    ctx.set_tuning(wg_per_cu=0, threads=threads)
+    store = hcm.Store(ctx, blocks.shape[0])
+    store.upload(blocks, light)
+    batch = hcm.Batch(ctx, store, nbr)
+    print(f"no light through {kind}: {threads} threads", flush=True)
+    batch.run()
+    out = batch.download()
+    for j in range(n):
+        b27, l27 = workloads.slice_jobs(blocks, light, nbr, j)
+        want = meshdigest.digest(orc.mesh(b27, l27))
+        assert meshdigest.digest(hcm.job_meshes(j, *out)) == want, f"job {j}"
+        assert meshdigest.digest(ctx.mesh_chunk(b27, l27)) == want, f"job {j}, plain"
+    batch.close()
     store.close()
     ctx.close()
