@@ -1891,7 +1891,7 @@ hipError_t launch_mesh(const MeshParams &p, int threads, int grid, hipStream_t s
 	if (p.halo_in && threads < kHaloRows) // packed halos are staged one row per thread
 		return hipErrorInvalidValue;
 	const auto launch = [&](auto plain, auto raw) {
-		hipLaunchKernelGGL(p.reg.raw_front ? raw : plain, dim3(grid), dim3(threads), 0, stream, p);
+		hipLaunchKernelGGL((p.reg.raw_front ? raw : plain), dim3(grid), dim3(threads), 0, stream, p);
 	};
 	switch (threads) {
 	case 128:
