@@ -43,15 +43,8 @@ constexpr int kTasks = 96;
 __host__ __device__ constexpr int task_axis(int t) { return t >> 5; }
 __host__ __device__ constexpr int task_layer(int t) { return (t >> 1) & 15; }
 __host__ __device__ constexpr int task_plus(int t) { return t & 1; }
-// Entries of the face-word stage. 1,344 keeps the 256-thread workgroup's LDS within three per CU
-// (static_assert below); the tasks of a chunk with more visible faces are taken in several groups.
-constexpr int kListCap = 1344;
-constexpr int kFaceBlocks = kListCap / 64;
 constexpr int kMaskRows = kTasks * 16;
 constexpr int kUnits = kMaskRows / 4; // a unit is four mask rows, 64 faces
-// A group but the last holds more than kListCap - 256 faces (a task has at most 256), of 24,576 at most.
-constexpr int kMaxGroups = kTasks * 256 / (kListCap - 255) + 2;
-static_assert(kListCap % 64 == 0 && kFaceBlocks <= 64, "whole blocks of faces, one lane each");
 constexpr uint32_t kSplitQuads = 16383u; // a BlockMesh holds at most 65,532 vertices (:273-279, :397-403)
 constexpr int kMaxMeshPerPass = 8;
 
@@ -134,6 +127,14 @@ __device__ __forceinline__ uint32_t local16(int x, int y, int z) {
 __device__ __forceinline__ int hidx(int x, int y, int z) { return (x + 1) * kSX + (y + 1) * kSY + (z + 1) * kSZ; }
 
 template <int NT> struct Smem {
+	// Entries of the face-word stage; the tasks of a chunk with more visible faces are taken in several groups. 1,344
+	// keeps the 256-thread workgroup's LDS within three per CU (static_assert below). A 512-thread one has the CU
+	// to itself by its registers, and 64 KB to itself in an LDS instruction's offset: 2,496. One random
+	// chunk of 7,700 quads took 65.2 us in groups of 1,344, 60.5 so.
+	static constexpr int kListCap = NT >= 512 ? 2496 : 1344;
+	static_assert(kListCap % 64 == 0 && kListCap / 64 <= 64, "whole blocks of faces, one lane each");
+	// A group but the last holds more than kListCap - 256 faces (a task has at most 256), of 24,576 at most.
+	static constexpr int kMaxGroups = kTasks * 256 / (kListCap - 255) + 2;
 	uint32_t vox[kHaloVox];
 	union {
 		struct {
@@ -977,8 +978,8 @@ template <int NT> __device__ __forceinline__ void face_links(Smem<NT> &s, uint32
 	const uint32_t ne_u = s.ne[r], ne_d = uint32_t(s.ne[min(r + 1, uint32_t(kMaskRows - 1))]) & (0u - uint32_t(u < 15));
 	const uint2 w = s.key[i];
 	const uint32_t bit = 1u << (v + 16 * (u & 1));
-	const uint32_t ir = min(i + 1, uint32_t(kListCap - 1));
-	const uint32_t id = min(i + 1 + __popc(ne_u >> (v + 1)) + __popc(ne_d & ((1u << v) - 1u)), uint32_t(kListCap - 1));
+	const uint32_t ir = min(i + 1, uint32_t(s.kListCap - 1));
+	const uint32_t id = min(i + 1 + __popc(ne_u >> (v + 1)) + __popc(ne_d & ((1u << v) - 1u)), uint32_t(s.kListCap - 1));
 	const uint2 right = s.key[ir], d = s.key[id];
 	const bool eq_r = v < 15 && ((ne_u >> (v + 1)) & 1u) && ((right.x ^ w.x) | (right.y ^ w.y)) == 0;
 	const bool eq_d = ((ne_d >> v) & 1u) && ((d.x ^ w.x) | (d.y ^ w.y)) == 0;
@@ -1120,7 +1121,7 @@ template <int NT> __device__ __forceinline__ void quad_starts(Smem<NT> &s, int t
 // most 256 faces, always fits). Every wavefront counts the tasks that end within it, two per lane (a search by one
 // thread and a barrier took 0.8 us for each of a dense chunk's groups).
 template <int NT> __device__ __forceinline__ int group_end(const Smem<NT> &s, int t0, uint32_t n_faces) {
-	const uint32_t limit = uint32_t(s.upre[4 * t0]) + (uint32_t)kListCap;
+	const uint32_t limit = uint32_t(s.upre[4 * t0]) + (uint32_t)s.kListCap;
 	if (n_faces <= limit) // the rest fits (the usual case)
 		return kTasks;
 	static_assert(kTasks <= 128, "two tasks per lane");
@@ -1479,9 +1480,9 @@ template <bool kRaw, int NT> __device__ __forceinline__ void mesh_chunk(const Me
 	for (int i = tid; i < kMaskRows / 8; i += NT) {
 		reinterpret_cast<uint4 *>(s.eh)[i] = make_uint4(0, 0, 0, 0);
 		reinterpret_cast<uint4 *>(s.ev)[i] = make_uint4(0, 0, 0, 0);
-		if (i < kListCap / 8)
-			reinterpret_cast<uint4 *>(s.own)[i] = make_uint4(0, 0, 0, 0);
 	}
+	for (int i = tid; i < s.kListCap / 8; i += NT)
+		reinterpret_cast<uint4 *>(s.own)[i] = make_uint4(0, 0, 0, 0);
 	__syncthreads();
 	uint32_t first, cnt[3];
 	const uint32_t n_faces = number_faces(s, first, cnt);
@@ -1527,13 +1528,11 @@ template <bool kRaw, int NT> __device__ __forceinline__ void mesh_chunk(const Me
 #pragma unroll 1
 	for (bool again = false;; again = true) {
 		int t1 = kTasks;
-		if (again || n_faces > (uint32_t)kListCap) {
+		if (again || n_faces > (uint32_t)s.kListCap) {
 			if (again) {
 				__syncthreads(); // the last group's descriptors are read
-				if (tid < kListCap / 8)
-					reinterpret_cast<uint4 *>(s.own)[tid] = make_uint4(0, 0, 0, 0);
-				if (NT < kListCap / 8 && tid + NT < kListCap / 8)
-					reinterpret_cast<uint4 *>(s.own)[tid + NT] = make_uint4(0, 0, 0, 0);
+				for (int i = tid; i < s.kListCap / 8; i += NT)
+					reinterpret_cast<uint4 *>(s.own)[i] = make_uint4(0, 0, 0, 0);
 			}
 			__syncthreads();
 			t1 = group_end(s, t0, n_faces);
@@ -1640,9 +1639,9 @@ template <bool kRaw, int NT> __device__ __forceinline__ void mesh_chunk(const Me
 	if (flags & kFlagCustom) {
 		const uint32_t n_cust = cust0 + cust1;
 #pragma unroll 1
-		for (uint32_t w0 = 0; w0 < n_cust; w0 += kListCap) {
+		for (uint32_t w0 = 0; w0 < n_cust; w0 += s.kListCap) {
 			__syncthreads(); // key is free: the regular quads and the previous window are written
-			const uint32_t w1 = w0 + kListCap;
+			const uint32_t w1 = w0 + s.kListCap;
 			uint32_t io = (uint32_t)cust_pre, it = (uint32_t)(cust_pre >> 32);
 			if (io + it < w1 && io + it + c_o + c_t > w0) {
 				for (uint32_t bits = custom_cells(s); bits && io + it < w1; bits &= bits - 1) {
@@ -1656,7 +1655,7 @@ template <bool kRaw, int NT> __device__ __forceinline__ void mesh_chunk(const Me
 				}
 			}
 			__syncthreads();
-			const uint32_t n = min(n_cust - w0, (uint32_t)kListCap);
+			const uint32_t n = min(n_cust - w0, (uint32_t)s.kListCap);
 			for (uint32_t v = tid; v < 4 * n; v += NT) { // a lane per vertex
 				const uint32_t e = v >> 2;
 				const uint2 ent = s.key[e];

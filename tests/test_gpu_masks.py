@@ -85,7 +85,7 @@ def chunk_with_faces(n):
 
 
 @pytest.mark.parametrize("merge", [False, True])
-@pytest.mark.parametrize("faces", [1, 2, 63, 64, 65, 128, 1343, 1344, 1345, 1471, 1472, 1473, 1536, 2688, 2689, 2944, 2945, 4416, 4417, 8232])
+@pytest.mark.parametrize("faces", [1, 2, 63, 64, 65, 128, 1343, 1344, 1345, 1471, 1472, 1473, 1536, 2496, 2497, 2688, 2689, 2944, 2945, 4416, 4417, 8232])
 def test_face_counts_at_block_and_group_edges(ctx, oracle, faces, merge):
     """Visible faces are numbered by units of 64 mask bits, handled in blocks of 64 lanes and held in groups of up to
     1,344: counts at and beside those edges, with light that lets faces merge and light that does not."""
