@@ -234,6 +234,10 @@ struct hcm_ctx {
 	// device registry buffers
 	uint8_t *d_pid_of = nullptr;
 	uint2 *d_rows = nullptr;
+	uint8_t *d_kept = nullptr; // MeshParams::kept of the batches, all on `stream`; from the first batch on
+	size_t kept_bytes = 0;
+	DevReg *d_reg = nullptr;
+	uint32_t raw_front = 0;
 	uint2 *d_pid_vox = nullptr;
 	uint32_t *d_codes = nullptr;
 	hcm_custom_mesh *d_meshes = nullptr;
@@ -335,6 +339,8 @@ static void free_ctx(hcm_ctx *c) {
 		return;
 	dfree(c->d_pid_of);
 	dfree(c->d_rows);
+	dfree(c->d_kept);
+	dfree(c->d_reg);
 	dfree(c->d_pid_vox);
 	dfree(c->d_codes);
 	dfree(c->d_meshes);
@@ -398,7 +404,6 @@ static int create_impl(hcm_ctx *c, const hcm_registry *registry, uint64_t pool_q
 	c->reg.pid_of = c->d_pid_of;
 	c->reg.rows = c->d_rows;
 	c->reg.pid_vox = c->d_pid_vox;
-	c->reg.raw_front = t.raw_front;
 	c->reg.codes = c->d_codes;
 	c->reg.meshes = c->d_meshes;
 	c->reg.mesh_sums = c->d_mesh_sums;
@@ -409,6 +414,9 @@ static int create_impl(hcm_ctx *c, const hcm_registry *registry, uint64_t pool_q
 	c->reg.flow_trans = t.flow_trans;
 	c->reg.src_id = t.src_id;
 	c->reg.flow_id = t.flow_id;
+	c->raw_front = t.raw_front;
+	HCM_HIP(dmalloc(&c->d_reg, 1));
+	HCM_HIP(hipMemcpy(c->d_reg, &c->reg, sizeof(DevReg), hipMemcpyHostToDevice));
 
 	c->pool_quads = std::min<uint64_t>(pool_quads, 0xffffffffull - (1u << 20));
 	if (c->pool_quads) {
@@ -483,7 +491,8 @@ extern "C" int hcm_get_tuning(hcm_ctx *ctx, hcm_tuning *t) {
 static MeshParams base_params(hcm_ctx *c) {
 	MeshParams p;
 	std::memset(&p, 0, sizeof(p));
-	p.reg = c->reg;
+	p.reg = (const HCM_CONSTANT DevReg *)c->d_reg;
+	p.raw_front = c->raw_front;
 	return p;
 }
 
@@ -510,7 +519,8 @@ int hcm::ctx_info(hcm_ctx *ctx, uint32_t threads, CtxInfo *out) {
 	if (!ctx || !out)
 		return HCM_ERR_INVALID;
 	std::lock_guard<std::mutex> lk(ctx->mu);
-	out->reg = ctx->reg;
+	out->reg = ctx->d_reg;
+	out->raw_front = ctx->raw_front;
 	out->n_cu = ctx->n_cu;
 	out->threads = threads ? threads : ctx->tuning.threads;
 	out->grid = (uint32_t)persistent_grid(ctx, out->threads);
@@ -843,6 +853,14 @@ extern "C" int hcm_batch_create(hcm_ctx *ctx, hcm_store *store, const uint32_t *
 	if (dmalloc(&b->d_read_slots, slots.size()) != hipSuccess ||
 	    hipMemcpy(b->d_read_slots, slots.data(), slots.size() * 4, hipMemcpyHostToDevice) != hipSuccess)
 		return fail();
+	{
+		std::lock_guard<std::mutex> lk(ctx->mu);
+		const size_t bytes = persistent_grid(ctx, 256) * kKeptBytes;
+		if (!ctx->d_kept && dmalloc(&ctx->d_kept, bytes) == hipSuccess)
+			ctx->kept_bytes = bytes;
+		else if (!ctx->d_kept)
+			(void)hipGetLastError(); // (dense chunks do without)
+	}
 	*out = b;
 	return HCM_OK;
 }
@@ -973,6 +991,7 @@ static int batch_run(hcm_batch *b, uint32_t mode, uint32_t times) {
 		p.persistent = 1;
 		p.self_reset = 1; // the counters start at zero and the run's last workgroup zeroes them again
 		const int grid = (int)std::min((uint32_t)persistent_grid(c, threads), b->n_jobs);
+		p.kept = grid * kKeptBytes <= c->kept_bytes ? c->d_kept : nullptr; // (c->stream's launches follow each other)
 		HCM_HIP(hipEventRecord(b->ev0, st));
 		for (uint32_t k = 0; k < times; ++k) {
 			if (b->light_mode == HCM_LIGHT_REBUILD)

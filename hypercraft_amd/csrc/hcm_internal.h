@@ -52,7 +52,6 @@ struct DevReg {
 	const uint32_t *mesh_sums;     // [n_meshes]: faces | (bit j: face j goes to the transparent pass) << 16
 	uint32_t n_pid, n_codes, flow_pid_base;
 	uint32_t flow_tex, flow_trans, src_id, flow_id;
-	uint32_t raw_front; // a block that passes no indirect light may stand in front of a visible face (or have a mesh)
 };
 
 // The persistent kernels' job list is cut into kQueues contiguous parts, one per XCD (gfx950 has 8,
@@ -78,8 +77,24 @@ struct Counters {
 	uint32_t total_quads, total_meshes;
 };
 
+// Memory of a workgroup for the words (8 bytes) and descriptors (2) of a dense chunk's faces, from when it computes them
+// until it emits their quads: the first 8,192, past which it computes them twice, as it does all without the memory.
+// 1,000 chunks of random blocks (7,757 quads each) took 202.4 us computing all groups but the last twice, 181.6 so.
+constexpr uint32_t kKeptFaces = 8192;
+constexpr size_t kKeptBytes = kKeptFaces * 10;
+
+// Device memory that no kernel writes: read by scalar loads where it is used.
+#ifdef __HIP_DEVICE_COMPILE__
+#define HCM_CONSTANT __attribute__((address_space(4)))
+#else
+#define HCM_CONSTANT
+#endif
+
 struct MeshParams {
-	DevReg reg;
+	// By pointer: its members among the kernel's arguments were held in scalar registers from the start, which spilled
+	// (4,096 cave chunks 78.5 us, 77.1 so).
+	const HCM_CONSTANT DevReg *reg;
+	uint32_t raw_front; // a block that passes no indirect light may stand in front of a visible face (or have a mesh)
 	const uint16_t *blocks; // store: slot * 4096 + local
 	const uint8_t *light;
 	const uint32_t *nbr;    // 27 slots per job
@@ -100,6 +115,7 @@ struct MeshParams {
 	// the store). Launches of 512 threads. Any alignment, device or pinned host memory.
 	const uint16_t *halo_in;
 	const uint8_t *halo_in_light;
+	uint8_t *kept;  // per workgroup kKeptBytes, or null
 	uint32_t alone; // the launch's one job: its output starts at quad and record 0, the counters are not touched
 };
 
@@ -203,7 +219,8 @@ int light_lds_bytes();
 
 // Context internals the serving loop needs (hcm_api.cpp)
 struct CtxInfo {
-	DevReg reg;
+	const DevReg *reg;          // in device memory
+	uint32_t raw_front;
 	int n_cu;
 	uint32_t threads;
 	uint32_t grid;              // persistent grid for `threads`

@@ -173,6 +173,7 @@ template <int NT> struct Smem {
 	uint32_t job, flags, n_events;
 	uint32_t wave_ref[NT / 64];
 	uint32_t pool_base, mesh_base;
+	JobClaims claims;
 };
 
 constexpr uint32_t kFlagNonUniform = 1u, kFlagCustom = 2u, kFlagFlow = 4u;
@@ -198,7 +199,7 @@ template <int NT> __device__ __forceinline__ uint32_t row_code(const Smem<NT> &s
 // Texture row of a block value: from LDS for most ids, from the full table for meta-dependent ones.
 template <int NT> __device__ __forceinline__ uint32_t block_pid(const MeshParams &p, const Smem<NT> &s, uint32_t b) {
 	const uint2 q = s.tmpl_id[b & 0xffu];
-	return q.x & kTmplMeta ? p.reg.pid_of[b] : vox_pid(q.y);
+	return q.x & kTmplMeta ? p.reg->pid_of[b] : vox_pid(q.y);
 }
 
 // AO of a light4_init vertex (:126-130) by side, corner and side cell direct-pass bits and the front cell's:
@@ -410,7 +411,7 @@ __device__ __forceinline__ uint32_t flow_vh(int nb, int a, int b, int c) {
 
 __device__ __forceinline__ Flow flow_heights(const MeshParams &p, const JobBlocks &blocks, int x, int y, int z,
                                           uint32_t nb_height) {
-	const uint32_t src = p.reg.src_id, fid = p.reg.flow_id;
+	const uint32_t src = p.reg->src_id, fid = p.reg->flow_id;
 	// neighbours (:291-300): 0 (-1,-1) 1 (0,-1) 2 (1,-1) 3 (-1,0) 4 (1,0) 5 (-1,1) 6 (0,1) 7 (1,1) in (x, z)
 	const uint32_t b0 = blocks.at(x - 1, y, z - 1), b1 = blocks.at(x, y, z - 1);
 	const uint32_t b2 = blocks.at(x + 1, y, z - 1), b3 = blocks.at(x - 1, y, z);
@@ -516,7 +517,7 @@ __device__ __forceinline__ CustomCell custom_cell(const MeshParams &p, const Sme
 	const int x = cell & 15, z = (cell >> 4) & 15, y = cell >> 8;
 	// the voxel word has the block's row but for flow cells, whose words took a row of face textures
 	uint32_t pid = vox_pid(s.vox[hidx(x, y, z)]);
-	if (pid >= p.reg.flow_pid_base)
+	if (pid >= p.reg->flow_pid_base)
 		pid = block_pid(p, s, blocks.at(x, y, z));
 	CustomCell c;
 	c.mesh = s.rows[pid].y >> 24;
@@ -524,12 +525,12 @@ __device__ __forceinline__ CustomCell custom_cell(const MeshParams &p, const Sme
 	c.trans = 0;
 	c.flow_set = 0;
 	c.fl.h = 0, c.fl.liq_side = 0;
-	const uint32_t sum = p.reg.mesh_sums[c.mesh]; // (one load: the faces' textures and flags would be two per face)
+	const uint32_t sum = p.reg->mesh_sums[c.mesh]; // (one load: the faces' textures and flags would be two per face)
 	if (c.flow) {
-		c.fl = flow_heights(p, blocks, x, y, z, p.reg.meshes[c.mesh].flow_height);
+		c.fl = flow_heights(p, blocks, x, y, z, p.reg->meshes[c.mesh].flow_height);
 		c.flow_set = flow_face_set(c.fl);
 		c.count = __popc(c.flow_set);
-		if (p.reg.flow_trans)
+		if (p.reg->flow_trans)
 			c.trans = (1u << c.count) - 1u;
 	} else {
 		c.count = sum & 0x1fu;
@@ -548,11 +549,11 @@ template <int NT> __device__ __forceinline__ uint32_t custom_cells(const Smem<NT
 
 __device__ __forceinline__ hcm_mesh_face custom_face(const MeshParams &p, const CustomCell &c, int j) {
 	if (!c.flow)
-		return p.reg.meshes[c.mesh].faces[j];
+		return p.reg->meshes[c.mesh].faces[j];
 	uint32_t set = c.flow_set;
 	for (int i = 0; i < j; ++i)
 		set &= set - 1u;
-	return flow_face(c.fl, __ffs(set) - 1, uint16_t(p.reg.flow_tex));
+	return flow_face(c.fl, __ffs(set) - 1, uint16_t(p.reg->flow_tex));
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1287,6 +1288,32 @@ template <int NT> __device__ __forceinline__ HaloRow halo_row(const Smem<NT> &s,
 	return r;
 }
 
+// The words and descriptors of a group of n faces to the workgroup's part of p.kept, from its face g0 on, and back; a
+// thread reads what it wrote, all of it on its way at once.
+template <int NT> __device__ __forceinline__ void store_kept(const MeshParams &p, const Smem<NT> &s, uint32_t g0, uint32_t n) {
+	uint2 *words = reinterpret_cast<uint2 *>(p.kept + blockIdx.x * kKeptBytes);
+	uint16_t *desc = reinterpret_cast<uint16_t *>(words + kKeptFaces);
+#pragma unroll 1
+	for (uint32_t i = threadIdx.x; i < n; i += NT)
+		words[g0 + i] = s.key[i], desc[g0 + i] = s.own[i];
+}
+template <int NT> __device__ __forceinline__ void load_kept(const MeshParams &p, Smem<NT> &s, uint32_t g0, uint32_t n) {
+	const uint2 *words = reinterpret_cast<const uint2 *>(p.kept + blockIdx.x * kKeptBytes);
+	const uint16_t *desc = reinterpret_cast<const uint16_t *>(words + kKeptFaces);
+	constexpr int kSteps = (Smem<NT>::kListCap + NT - 1) / NT;
+	uint2 w[kSteps];
+	uint16_t d[kSteps];
+#pragma unroll
+	for (int k = 0; k < kSteps; ++k) {
+		const uint32_t i = g0 + min(uint32_t(threadIdx.x + k * NT), n - 1);
+		w[k] = words[i], d[k] = desc[i];
+	}
+#pragma unroll
+	for (int k = 0; k < kSteps; ++k)
+		if (uint32_t(threadIdx.x + k * NT) < n)
+			s.key[threadIdx.x + k * NT] = w[k], s.own[threadIdx.x + k * NT] = d[k];
+}
+
 // One job; s.slots and the state of chunk_init are in place (a barrier after them).
 template <bool kRaw, int NT> __device__ __forceinline__ void mesh_chunk(const MeshParams &p, Smem<NT> &s, uint32_t job) {
 	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -1373,7 +1400,7 @@ template <bool kRaw, int NT> __device__ __forceinline__ void mesh_chunk(const Me
 #pragma unroll
 			for (int x = 0; x < 18; ++x) {
 				const uint32_t b = x == 0 ? bl : (x == 17 ? br : (bw[(x - 1) >> 1] >> (16 * ((x - 1) & 1))) & 0xffffu);
-				full[x] = p.reg.pid_of[b];
+				full[x] = p.reg->pid_of[b];
 			}
 #pragma unroll
 			for (int x = 0; x < 18; ++x) {
@@ -1457,8 +1484,8 @@ template <bool kRaw, int NT> __device__ __forceinline__ void mesh_chunk(const Me
 			const int hx = i % kHalo, rest = i / kHalo, hz = rest % kHalo, hy = rest / kHalo;
 			const uint32_t pid = vox_pid(s.vox[i]);
 			const uint32_t mesh = s.rows[pid].y >> 24;
-			const Flow f = flow_heights(p, blocks, hx - 1, hy - 1, hz - 1, p.reg.meshes[mesh].flow_height);
-			const uint32_t tmpl = s.pid_vox[p.reg.flow_pid_base + flow_pattern(f)].y;
+			const Flow f = flow_heights(p, blocks, hx - 1, hy - 1, hz - 1, p.reg->meshes[mesh].flow_height);
+			const uint32_t tmpl = s.pid_vox[p.reg->flow_pid_base + flow_pattern(f)].y;
 			s.vox[i] = (s.vox[i] & kKeep) | (tmpl & ~kKeep);
 		}
 		__syncthreads();
@@ -1511,7 +1538,8 @@ template <bool kRaw, int NT> __device__ __forceinline__ void mesh_chunk(const Me
 
 	// 4. groups of tasks whose visible faces fit the stage, twice: first every group's faces, links and quads
 	// (one group but in dense chunks), which gives the chunk's quad counts; then, from the last group, whose
-	// words are still in the stage, the emission, for which an earlier group's words are computed again. A
+	// words are still in the stage, the emission, for which an earlier group's words are read back from the
+	// workgroup's part of p.kept, or computed again where that is not given or too small. A
 	// quad's place in its pass is its start's among the faces, counted by ballots over blocks of 64 faces.
 	const uint32_t wave_u = __builtin_amdgcn_readfirstlane(wave);
 	uint32_t base_o = cust0, base_t = cust1;       // quads of each pass before the group
@@ -1528,26 +1556,34 @@ template <bool kRaw, int NT> __device__ __forceinline__ void mesh_chunk(const Me
 #pragma unroll 1
 	for (bool again = false;; again = true) {
 		int t1 = kTasks;
+		uint32_t n = n_faces;
+		bool loaded = false;
 		if (again || n_faces > (uint32_t)s.kListCap) {
-			if (again) {
-				__syncthreads(); // the last group's descriptors are read
+			__syncthreads(); // s.upre is complete; the last group's descriptors are read
+			t1 = group_end(s, t0, n_faces);
+			const uint32_t end = __builtin_amdgcn_readfirstlane(s.upre[4 * t1]);
+			n = end - g0;
+			if (!collect && p.kept && end <= kKeptFaces) {
+				load_kept(p, s, g0, n);
+				loaded = true;
+			} else if (again) {
 				for (int i = tid; i < s.kListCap / 8; i += NT)
 					reinterpret_cast<uint4 *>(s.own)[i] = make_uint4(0, 0, 0, 0);
+				__syncthreads();
 			}
-			__syncthreads();
-			t1 = group_end(s, t0, n_faces);
 		}
-		mark_units(s, t0, t1, g0, first, cnt);
-		__syncthreads();
-		const uint32_t n = __builtin_amdgcn_readfirstlane(s.upre[4 * t1]) - g0;
-		// face words
+		if (!loaded) {
+			mark_units(s, t0, t1, g0, first, cnt);
+			__syncthreads();
+			// face words
 #pragma unroll 1
-		for (uint32_t b = wave_u; b * 64 < n; b += NT / 64) {
-			const uint32_t i = 64 * b + lane, desc = face_desc(s, i, g0);
-			if (i < n) {
-				const uint2 word = face_word<kRaw>(s, desc);
-				s.key[i] = word;
-				s.own[i] = uint16_t(desc | (word.y >> 31 ? kDescTrans : 0u));
+			for (uint32_t b = wave_u; b * 64 < n; b += NT / 64) {
+				const uint32_t i = 64 * b + lane, desc = face_desc(s, i, g0);
+				if (i < n) {
+					const uint2 word = face_word<kRaw>(s, desc);
+					s.key[i] = word;
+					s.own[i] = uint16_t(desc | (word.y >> 31 ? kDescTrans : 0u));
+				}
 			}
 		}
 		__syncthreads();
@@ -1575,6 +1611,8 @@ template <bool kRaw, int NT> __device__ __forceinline__ void mesh_chunk(const Me
 			const uint32_t tot = (uint32_t)__builtin_amdgcn_readlane((int)inc, 63);
 			n0 = base_o + (tot & 0xffffu), n1 = base_t + (tot >> 16);
 			if (t1 < kTasks) { // the group waits for the others' counts
+				if (p.kept && g0 + n <= kKeptFaces)
+					store_kept(p, s, g0, n);
 				if (tid == 0)
 					s.grp[n_saved] = make_uint2(uint32_t(t0) | base_o << 8, base_t);
 				++n_saved;
@@ -1717,19 +1755,20 @@ template <bool kRaw, int NT> __device__ __forceinline__ void mesh_chunk(const Me
 template <int NT, bool kRaw> __global__ __launch_bounds__(NT, NT >= 512 ? 2 : 3) void mesh_kernel(MeshParams p) {
 	__shared__ Smem<NT> s;
 	for (int i = threadIdx.x; i < kMaxPid; i += NT) {
-		const bool ok = i < (int)p.reg.n_pid;
-		s.rows[i] = ok ? p.reg.rows[i] : make_uint2(0, 0);
-		s.pid_vox[i] = ok ? p.reg.pid_vox[i] : make_uint2(0, uint32_t(i) << kVoxPidShift);
+		const bool ok = i < (int)p.reg->n_pid;
+		s.rows[i] = ok ? p.reg->rows[i] : make_uint2(0, 0);
+		s.pid_vox[i] = ok ? p.reg->pid_vox[i] : make_uint2(0, uint32_t(i) << kVoxPidShift);
 	}
 	for (int i = threadIdx.x; i < kMaxCodes; i += NT)
-		s.codes[i] = i < (int)p.reg.n_codes ? p.reg.codes[i] : 0u;
+		s.codes[i] = i < (int)p.reg->n_codes ? p.reg->codes[i] : 0u;
 	for (int i = threadIdx.x; i < 256; i += NT)
 	{
-		const uint32_t q = p.reg.pid_of[65536 + i];
-		s.tmpl_id[i] = q == 0xffu ? make_uint2(kTmplMeta, 0) : p.reg.pid_vox[q];
+		const uint32_t q = p.reg->pid_of[65536 + i];
+		s.tmpl_id[i] = q == 0xffu ? make_uint2(kTmplMeta, 0) : p.reg->pid_vox[q];
 	}
 	fill_averages(s);
-	JobClaims claims(p.n_jobs); // lane 0 of wavefront 0 only
+	if (threadIdx.x == 0) // (only this lane uses it)
+		s.claims.init(p.n_jobs);
 	const int lane = threadIdx.x & 63;
 	const uint32_t given = p.job_base + blockIdx.x; // per-chunk launches: the workgroup's one job
 	for (;;) {
@@ -1737,7 +1776,7 @@ template <int NT, bool kRaw> __global__ __launch_bounds__(NT, NT >= 512 ? 2 : 3)
 		if (threadIdx.x < 64) {
 			uint32_t job = ~0u;
 			if (lane == 0) {
-				job = p.persistent ? claims.next(p.ctr) : given;
+				job = p.persistent ? s.claims.next(p.ctr) : given;
 				s.job = job;
 			}
 			job = (uint32_t)__builtin_amdgcn_readfirstlane((int)job);
@@ -1880,7 +1919,7 @@ hipError_t launch_mesh(const MeshParams &p, int threads, int grid, hipStream_t s
 	if (p.halo_in && threads < kHaloRows) // packed halos are staged one row per thread
 		return hipErrorInvalidValue;
 	const auto launch = [&](auto plain, auto raw) {
-		hipLaunchKernelGGL((p.reg.raw_front ? raw : plain), dim3(grid), dim3(threads), 0, stream, p);
+		hipLaunchKernelGGL((p.raw_front ? raw : plain), dim3(grid), dim3(threads), 0, stream, p);
 	};
 	switch (threads) {
 	case 128:

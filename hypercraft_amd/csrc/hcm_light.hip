@@ -306,7 +306,9 @@ __global__ __launch_bounds__(256) void light_prep_kernel(LightParams p) {
 
 __global__ __launch_bounds__(kLightThreads, 8) void light_kernel(LightParams p) {
 	__shared__ LightSmem s;
-	JobClaims claims(p.n_jobs); // lane 0 of wavefront 0 only
+	__shared__ JobClaims claims;
+	if (threadIdx.x == 0) // (only this lane uses it)
+		claims.init(p.n_jobs);
 	for (;;) {
 		if (threadIdx.x < 64) { // wavefront 0 claims the next job and loads its slot list and levels
 			uint32_t job = ~0u;

@@ -517,7 +517,8 @@ struct hcm_server {
 			}
 			MeshParams p;
 			std::memset(&p, 0, sizeof(p));
-			p.reg = info.reg;
+			p.reg = (const HCM_CONSTANT DevReg *)info.reg;
+			p.raw_front = info.raw_front;
 			p.blocks = d_blocks;
 			p.light = d_light;
 			p.nbr = nbr;

@@ -228,3 +228,34 @@ def test_blocks_in_front_that_pass_no_light(tmp_path, kind, seed, threads):
     batch.close()
     store.close()
     ctx.close()
+
+
+@pytest.mark.parametrize("n,wg_per_cu,threads", [(3, 0, 0), (300, 0, 0), (2, 0, 128), (3, 0, 512), (1030, 4, 128)])
+def test_dense_chunks_past_the_kept_faces(n, wg_per_cu, threads, oracle):
+    """A batch's workgroups keep the words of a dense chunk's first 8,192 faces until its quads are written, as many of them
+    as the memory was made for; past either they are computed again. Checkerboards of 12,288 faces and fewer."""
+    rng = np.random.default_rng(n)
+    y, z, x = np.indices((16, 16, 16))
+    odd = ((x + y + z) & 1).reshape(-1) == 1
+    solid = np.array([1, 2, 3, 9, 10, 4], np.uint16)
+    blocks = np.where(odd & (rng.random((54, 4096)) < 0.9), solid[rng.integers(0, solid.size, (54, 4096))], 0).astype(np.uint16)
+    blocks[26] = np.where(odd, 1, 0)  # the first job's own chunk (the neighbour slot of all coordinates 0)
+    light = rng.integers(0, 256, blocks.shape).astype(np.uint8)
+    nbr = np.tile(np.arange(54, dtype=np.uint32).reshape(2, 27), (n, 1))[:n]
+    want = [meshdigest.digest(oracle.mesh(*workloads.slice_jobs(blocks, light, nbr, j))) for j in range(2)]
+    ctx = hcm.Context(pool_quads=n * 13000)
+    if threads:
+        ctx.set_tuning(wg_per_cu=wg_per_cu, threads=threads)
+    store = hcm.Store(ctx, 54)
+    store.upload(blocks, light)
+    batch = hcm.Batch(ctx, store, nbr)
+    print(f"{n} dense jobs, {wg_per_cu} x {threads} threads", flush=True)
+    for _ in range(2):
+        batch.run()
+    out = batch.download()
+    assert out[0]["quad_count"][0] > 11000
+    for j in range(0, n, 1 if n < 10 else 23):
+        assert meshdigest.digest(hcm.job_meshes(j, *out)) == want[j & 1], j
+    batch.close()
+    store.close()
+    ctx.close()
