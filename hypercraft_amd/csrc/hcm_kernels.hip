@@ -1409,7 +1409,6 @@ template <bool kRaw, int NT> __device__ __forceinline__ void mesh_chunk(const Me
 				tm[x] = tm[x] & kTmplMeta ? v.x : tm[x];
 			}
 		}
-		put_planes(s, hy, hz, tm);
 		uint32_t and_all = ~0u, or_inner = 0;
 		uint32_t *dst = s.vox + row * kHalo;
 		static_assert(kVoxSunBit == 8 && kVoxTorchBit == 16, "light in the low nibbles of two bytes");
@@ -1422,6 +1421,7 @@ template <bool kRaw, int NT> __device__ __forceinline__ void mesh_chunk(const Me
 			if (x >= 1 && x <= 16)
 				or_inner |= tm[x];
 		}
+		put_planes(s, hy, hz, tm);
 		const uint32_t or_all = or_inner | tm[0] | tm[17];
 		const bool inside_yz = (unsigned)y < 16u && (unsigned)z < 16u;
 		// every voxel an opaque cube: the shape bits that the cube has set are set in all, the others in none
