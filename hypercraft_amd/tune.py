@@ -1,7 +1,7 @@
 """Autotuner for the batched meshing kernel: workgroup size x workgroups per CU x job order.
 
 The persistent kernel's cost per chunk depends on the workgroup size (how many lanes share the
-102 visibility tasks, the face-word pass and the emission), on how many workgroups each CU holds
+96 visibility tasks, the face-word pass and the emission), on how many workgroups each CU holds
 (LDS occupancy vs latency hiding), and on the order of the job list: the kernel cuts the list into
 eight contiguous parts, one per XCD, so the order decides which chunks share an XCD's L2 (a chunk's
 halo is read by its 26 neighbours' jobs too) and, within a part, which jobs run last: a persistent launch
