@@ -36,6 +36,7 @@ template <typename T> hipError_t dmalloc(T **p, size_t count) {
 
 // Registry flattened for the kernels (see hcm_internal.h for the word layouts).
 struct DeviceTables {
+	MeshTables tables;
 	std::vector<uint8_t> pid_of;
 	std::vector<uint2> rows;
 	std::vector<uint2> pid_vox;
@@ -151,21 +152,29 @@ int build_tables(const hcm_registry *r, DeviceTables *t) {
 		const uint32_t pass = tex_flags(uint16_t(tex)) & HCM_TEX_TRANS_PASS ? kCodeTransPass : 0u;
 		t->codes.push_back((vertex & kCodeVertex) | uint32_t(i >> 4) << 28 | pass);
 	}
-	t->pid_of.resize(65536 + 256);
+	t->pid_of.resize(65536);
 	for (uint32_t d = 0; d < 65536; ++d) {
 		if (r->row_of[d] >= r->n_rows)
 			return HCM_ERR_INVALID;
 		t->pid_of[d] = (uint8_t)r->row_of[d];
 	}
-	// per block id: its row when no meta value changes it (kept in LDS by the kernel), else 0xff
-	for (uint32_t id = 0; id < 256; ++id) {
-		uint8_t v = t->pid_of[id];
-		for (uint32_t meta = 1; meta < 256; ++meta)
-			if (t->pid_of[id | meta << 8] != v) {
-				v = 0xff;
-				break;
-			}
-		t->pid_of[65536 + id] = v;
+	// what the kernel holds in LDS
+	MeshTables &m = t->tables;
+	std::memset(&m, 0, sizeof(m));
+	std::copy(t->rows.begin(), t->rows.end(), m.rows);
+	std::copy(t->codes.begin(), t->codes.end(), m.codes);
+	for (uint32_t pid = 0; pid < (uint32_t)kMaxPid; ++pid)
+		m.pid_vox[pid] = pid < t->pid_vox.size() ? t->pid_vox[pid] : make_uint2(0, pid << kVoxPidShift);
+	for (uint32_t id = 0; id < 256; ++id) { // a block id's template when no meta value changes its row
+		const uint8_t pid = t->pid_of[id];
+		bool same = true;
+		for (uint32_t meta = 1; meta < 256 && same; ++meta)
+			same = t->pid_of[id | meta << 8] == pid;
+		m.tmpl_id[id] = same ? t->pid_vox[pid] : make_uint2(kTmplMeta, 0);
+	}
+	for (uint32_t k = 0; k < 256; ++k) {
+		m.sun_of[k] = uint8_t((k & 63u) * 4u / ((k >> 6) + 1u) << 2);
+		m.torch_of[k] = uint8_t((k >> 2) * 4u / ((k & 3u) + 1u));
 	}
 	// the light rebuild's view of a block: Block::GetLightLevel, GetIndirectLightPass and
 	// GetVerticalLightPass (Block.hpp:69-71)
@@ -233,13 +242,11 @@ struct hcm_ctx {
 	DevReg reg{};
 	// device registry buffers
 	uint8_t *d_pid_of = nullptr;
-	uint2 *d_rows = nullptr;
+	MeshTables *d_tables = nullptr;
 	uint8_t *d_kept = nullptr; // MeshParams::kept of the batches, all on `stream`; from the first batch on
 	size_t kept_bytes = 0;
 	DevReg *d_reg = nullptr;
 	uint32_t raw_front = 0;
-	uint2 *d_pid_vox = nullptr;
-	uint32_t *d_codes = nullptr;
 	hcm_custom_mesh *d_meshes = nullptr;
 	uint32_t *d_mesh_sums = nullptr;
 	uint8_t *d_light_info = nullptr;
@@ -338,11 +345,9 @@ static void free_ctx(hcm_ctx *c) {
 	if (!c)
 		return;
 	dfree(c->d_pid_of);
-	dfree(c->d_rows);
+	dfree(c->d_tables);
 	dfree(c->d_kept);
 	dfree(c->d_reg);
-	dfree(c->d_pid_vox);
-	dfree(c->d_codes);
 	dfree(c->d_meshes);
 	dfree(c->d_mesh_sums);
 	dfree(c->d_light_info);
@@ -393,31 +398,22 @@ static int create_impl(hcm_ctx *c, const hcm_registry *registry, uint64_t pool_q
 	HCM_HIP(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
 
 	HCM_HIP(dmalloc(&c->d_pid_of, t.pid_of.size()));
-	HCM_HIP(dmalloc(&c->d_rows, t.rows.size()));
-	HCM_HIP(dmalloc(&c->d_pid_vox, t.pid_vox.size()));
-	HCM_HIP(dmalloc(&c->d_codes, t.codes.size()));
+	HCM_HIP(dmalloc(&c->d_tables, 1));
 	HCM_HIP(dmalloc(&c->d_meshes, t.meshes.size()));
 	HCM_HIP(dmalloc(&c->d_mesh_sums, t.mesh_sums.size()));
 	HCM_HIP(dmalloc(&c->d_light_info, t.light_info.size()));
 	HCM_HIP(hipMemcpy(c->d_light_info, t.light_info.data(), t.light_info.size(), hipMemcpyHostToDevice));
 	c->light_info = t.light_info;
 	HCM_HIP(hipMemcpy(c->d_pid_of, t.pid_of.data(), t.pid_of.size(), hipMemcpyHostToDevice));
-	HCM_HIP(hipMemcpy(c->d_rows, t.rows.data(), t.rows.size() * sizeof(uint2), hipMemcpyHostToDevice));
-	HCM_HIP(hipMemcpy(c->d_pid_vox, t.pid_vox.data(), t.pid_vox.size() * sizeof(uint2), hipMemcpyHostToDevice));
-	HCM_HIP(hipMemcpy(c->d_codes, t.codes.data(), t.codes.size() * 4, hipMemcpyHostToDevice));
+	HCM_HIP(hipMemcpy(c->d_tables, &t.tables, sizeof(MeshTables), hipMemcpyHostToDevice));
 	if (!t.meshes.empty())
 		HCM_HIP(hipMemcpy(c->d_meshes, t.meshes.data(), t.meshes.size() * sizeof(hcm_custom_mesh),
 		                  hipMemcpyHostToDevice));
 	if (!t.mesh_sums.empty())
 		HCM_HIP(hipMemcpy(c->d_mesh_sums, t.mesh_sums.data(), t.mesh_sums.size() * 4, hipMemcpyHostToDevice));
 	c->reg.pid_of = c->d_pid_of;
-	c->reg.rows = c->d_rows;
-	c->reg.pid_vox = c->d_pid_vox;
-	c->reg.codes = c->d_codes;
 	c->reg.meshes = c->d_meshes;
 	c->reg.mesh_sums = c->d_mesh_sums;
-	c->reg.n_pid = (uint32_t)t.rows.size();
-	c->reg.n_codes = (uint32_t)t.codes.size();
 	c->reg.flow_pid_base = t.flow_pid_base;
 	c->reg.flow_tex = t.flow_tex;
 	c->reg.flow_trans = t.flow_trans;
@@ -502,6 +498,7 @@ static MeshParams base_params(hcm_ctx *c) {
 	std::memset(&p, 0, sizeof(p));
 	p.reg = (const HCM_CONSTANT DevReg *)c->d_reg;
 	p.raw_front = c->raw_front;
+	p.tables = c->d_tables;
 	return p;
 }
 
@@ -530,6 +527,7 @@ int hcm::ctx_info(hcm_ctx *ctx, uint32_t threads, CtxInfo *out) {
 	std::lock_guard<std::mutex> lk(ctx->mu);
 	out->reg = ctx->d_reg;
 	out->raw_front = ctx->raw_front;
+	out->tables = ctx->d_tables;
 	out->n_cu = ctx->n_cu;
 	out->threads = threads ? threads : ctx->tuning.threads;
 	out->grid = (uint32_t)persistent_grid(ctx, out->threads);

@@ -41,16 +41,25 @@ constexpr uint32_t kCodeTransPass = 1u << 31;
 // Texture-row flag (in rows[pid].y): a halo made of this row's block alone has visible faces.
 constexpr uint32_t kRowSelfShow = 1u << 16;
 
+// What a mesh workgroup holds in LDS for all its jobs, laid out in device memory as it is there: copied by one load per
+// thread or two, where filling it from separate tables took dependent loads (37 plant chunks 22.9 us per pass, 22.15 so).
+struct MeshTables {
+	uint2 rows[kMaxPid];       // x = tc0..tc3 (8 bits each), y = tc4 | tc5 << 8 | kRowSelfShow | mesh << 24
+	uint2 pid_vox[kMaxPid];    // templates by texture row
+	uint2 tmpl_id[256];        // template by block id when the meta byte does not change it, else kTmplMeta
+	uint32_t codes[kMaxCodes];
+	// (sum << 2) / count of light4_init for every sum of lights of 0 to 15, by the fields of a sum of voxel words:
+	// sunlight by sum | (count - 1) << 6 and moved up by the two bits a face word has it at, torchlight by
+	// (count - 1) | sum << 2
+	uint8_t sun_of[256], torch_of[256];
+};
+static_assert(sizeof(MeshTables) % 16 == 0, "copied in 16-byte words");
+
 struct DevReg {
-	const uint8_t *pid_of;         // [65536] Block::m_data -> texture row (pid); then [256] by block id:
-	                               // the row when the meta byte does not change it, else 0xff
-	const uint2 *rows;             // [n_pid]: x = tc0..tc3 (8 bits each),
-	                               // y = tc4 | tc5 << 8 | kRowSelfShow | mesh << 24
-	const uint2 *pid_vox;          // [n_pid]: templates
-	const uint32_t *codes;         // [n_codes]
+	const uint8_t *pid_of;         // [65536] Block::m_data -> texture row (pid)
 	const hcm_custom_mesh *meshes; // [n_meshes]
 	const uint32_t *mesh_sums;     // [n_meshes]: faces | (bit j: face j goes to the transparent pass) << 16
-	uint32_t n_pid, n_codes, flow_pid_base;
+	uint32_t flow_pid_base;
 	uint32_t flow_tex, flow_trans, src_id, flow_id;
 };
 
@@ -94,6 +103,7 @@ struct MeshParams {
 	// By pointer: its members among the kernel's arguments were held in scalar registers from the start, which spilled
 	// (4,096 cave chunks 78.5 us, 77.1 so).
 	const HCM_CONSTANT DevReg *reg;
+	const MeshTables *tables;
 	uint32_t raw_front; // a block that passes no indirect light may stand in front of a visible face (or have a mesh)
 	const uint16_t *blocks; // store: slot * 4096 + local
 	const uint8_t *light;
@@ -220,6 +230,7 @@ int light_lds_bytes();
 // Context internals the serving loop needs (hcm_api.cpp)
 struct CtxInfo {
 	const DevReg *reg;          // in device memory
+	const MeshTables *tables;   // likewise
 	uint32_t raw_front;
 	int n_cu;
 	uint32_t threads;

@@ -160,12 +160,8 @@ template <int NT> struct Smem {
 	uint16_t upre[kUnits + 2]; // visible faces before each unit (the dense face order; at most 24,576), and in all
 	uint32_t bcnt[64];         // per 64 faces of the group: quads that start there, opaque | transparent << 16
 	uint2 grp[kMaxGroups];     // per group of tasks: its first task, and the quads of the groups before it
-	uint2 rows[kMaxPid];
-	uint2 pid_vox[kMaxPid];    // templates by texture row
-	uint32_t codes[kMaxCodes];
+	alignas(16) MeshTables tables;
 	uint32_t custom_bits[128]; // in-chunk cells with a custom mesh
-	uint2 tmpl_id[256];        // template by block id when the meta byte does not change it, else kTmplMeta
-	uint8_t sun_of[256], torch_of[256]; // averages of light4_init (fill_averages)
 	uint32_t aabb[2][kMaxMeshPerPass][6];
 	uint32_t events[16][2];
 	uint32_t scan_w[NT / 64][4]; // per wavefront: its totals of block_excl_sums
@@ -191,14 +187,14 @@ constexpr uint32_t kVoxOpaqueCube = 0x555u << kVoxClassShift; // opaque on all s
 __device__ __forceinline__ uint32_t vox_pid(uint32_t vox) { return (vox >> kVoxPidShift) & kVoxPidMask; }
 
 template <int NT> __device__ __forceinline__ uint32_t row_code(const Smem<NT> &s, uint32_t pid, int face) {
-	const uint2 r = s.rows[pid];
+	const uint2 r = s.tables.rows[pid];
 	const uint32_t w = face < 4 ? r.x : r.y;
 	return (w >> (8 * (face & 3))) & 0xffu;
 }
 
 // Texture row of a block value: from LDS for most ids, from the full table for meta-dependent ones.
 template <int NT> __device__ __forceinline__ uint32_t block_pid(const MeshParams &p, const Smem<NT> &s, uint32_t b) {
-	const uint2 q = s.tmpl_id[b & 0xffu];
+	const uint2 q = s.tables.tmpl_id[b & 0xffu];
 	return q.x & kTmplMeta ? p.reg->pid_of[b] : vox_pid(q.y);
 }
 
@@ -217,15 +213,6 @@ constexpr uint32_t ao_table() {
 constexpr uint32_t kAoTable = ao_table();
 static_assert(kAoTable == 0xe9849040u, "AO table");
 constexpr uint32_t rotate_left(uint32_t v, int n) { return n ? v << n | v >> (32 - n) : v; }
-
-// (sum << 2) / count for every sum of lights of 0 to 15, as bytes by the fields of a sum of voxel words: sunlight by
-// sum | (count - 1) << 6 and moved up by the two bits a face word has it at, torchlight by (count - 1) | sum << 2.
-template <int NT> __device__ __forceinline__ void fill_averages(Smem<NT> &s) {
-	for (uint32_t i = threadIdx.x; i < 256; i += NT) {
-		s.sun_of[i] = uint8_t((i & 63u) * 4u / ((i >> 6) + 1u) << 2);
-		s.torch_of[i] = uint8_t((i >> 2) * 4u / ((i & 3u) + 1u));
-	}
-}
 
 // A cell's word in a light4_init sum when it passes indirect light (:132-161). Voxel words have no light where their
 // block does not pass it, so that words are added as they are, unless the registry has such a block in front of
@@ -263,7 +250,7 @@ template <bool kRaw, int NT> __device__ __forceinline__ uint2 light4(const Smem<
 	const uint32_t s0 = light_sum(qm, c0, pm, fqm), s1 = light_sum(qm, c1, pp, fqm);
 	const uint32_t s2 = light_sum(qp, c2, pp, fqp), s3 = light_sum(qp, c3, pm, fqp);
 	const auto vertex = [&s](uint32_t sum) {
-		return uint32_t(s.sun_of[(sum >> kVoxSunBit) & 0xffu]) | uint32_t(s.torch_of[(sum >> (kVoxTorchBit - 2)) & 0xffu]) << 8;
+		return uint32_t(s.tables.sun_of[(sum >> kVoxSunBit) & 0xffu]) | uint32_t(s.tables.torch_of[(sum >> (kVoxTorchBit - 2)) & 0xffu]) << 8;
 	};
 	uint32_t x = vertex(s0) | vertex(s1) << 14, y = vertex(s2) | vertex(s3) << 14;
 	// AO: bits 1 to 4 of a word, of which bit 0 is zero, rotate the table by the two bits of each cell's flag
@@ -520,8 +507,8 @@ __device__ __forceinline__ CustomCell custom_cell(const MeshParams &p, const Sme
 	if (pid >= p.reg->flow_pid_base)
 		pid = block_pid(p, s, blocks.at(x, y, z));
 	CustomCell c;
-	c.mesh = s.rows[pid].y >> 24;
-	c.flow = (s.pid_vox[pid].x & kTmplFlow) ? 1u : 0u;
+	c.mesh = s.tables.rows[pid].y >> 24;
+	c.flow = (s.tables.pid_vox[pid].x & kTmplFlow) ? 1u : 0u;
 	c.trans = 0;
 	c.flow_set = 0;
 	c.fl.h = 0, c.fl.liq_side = 0;
@@ -620,7 +607,7 @@ __device__ __forceinline__ Box emit_quad(const Smem<NT> &s, uint32_t desc, uint3
 	const uint32_t second = base + (height_first ? pu : pv), opposite = base + pu + pv, fourth = base + (height_first ? pv : pu);
 	// BlockVertex word 1 (client/include/client/BlockVertex.hpp:13-14): texture, face, and the vertex's light
 	const uint32_t code = (word.x >> 28) | ((word.y >> 24) & 0x70u);
-	const uint32_t common = (s.codes[code] & kCodeVertex) | uint32_t(2 * A + (plus ^ 1)) << 13;
+	const uint32_t common = (s.tables.codes[code] & kCodeVertex) | uint32_t(2 * A + (plus ^ 1)) << 13;
 	constexpr uint32_t kLight = 0x3fff0000u;
 	uint4 *vp = verts + 2 * (size_t)i;
 	vp[0] = make_uint4(base, common | (word.x << 16 & kLight), second, common | (word.x << 2 & kLight));
@@ -966,7 +953,7 @@ template <bool kRaw, int NT> __device__ __forceinline__ uint2 face_word(const Sm
 	const uint2 l = light4<kRaw>(s, self + (inv ? -sa : sa), u_first ? su : sv, u_first ? sv : su);
 	const uint32_t pid = vox_pid(*reinterpret_cast<const uint32_t *>(reinterpret_cast<const char *>(s.vox) + self));
 	const uint32_t tc = row_code(s, pid, 2 * A + inv);
-	return make_uint2(l.x | tc << 28, l.y | (s.codes[tc] & ~kCodeLow));
+	return make_uint2(l.x | tc << 28, l.y | (s.tables.codes[tc] & ~kCodeLow));
 }
 
 // Equal-to-right and equal-to-below bits of the visible face with dense index i (local to the group): its
@@ -1386,7 +1373,7 @@ template <bool kRaw, int NT> __device__ __forceinline__ void mesh_chunk(const Me
 #pragma unroll
 		for (int x = 0; x < 18; ++x) {
 			const uint32_t b = x == 0 ? bl : (x == 17 ? br : bw[(x - 1) >> 1] >> (16 * ((x - 1) & 1)));
-			const uint2 q = s.tmpl_id[b & 0xffu];
+			const uint2 q = s.tables.tmpl_id[b & 0xffu];
 			tm[x] = q.x, words[x] = q.y;
 		}
 		uint32_t any_meta = 0;
@@ -1404,7 +1391,7 @@ template <bool kRaw, int NT> __device__ __forceinline__ void mesh_chunk(const Me
 			}
 #pragma unroll
 			for (int x = 0; x < 18; ++x) {
-				const uint2 v = s.pid_vox[full[x]];
+				const uint2 v = s.tables.pid_vox[full[x]];
 				words[x] = tm[x] & kTmplMeta ? v.y : words[x];
 				tm[x] = tm[x] & kTmplMeta ? v.x : tm[x];
 			}
@@ -1466,7 +1453,7 @@ template <bool kRaw, int NT> __device__ __forceinline__ void mesh_chunk(const Me
 	// one block value everywhere hides every face when the block's opposite textures do not show to each
 	// other (true of every registered block; a registry may define one whose do)
 	const bool uniform_hidden =
-	    !(flags & kFlagNonUniform) && !(s.rows[block_pid(p, s, s.wave_ref[0])].y & kRowSelfShow);
+	    !(flags & kFlagNonUniform) && !(s.tables.rows[block_pid(p, s, s.wave_ref[0])].y & kRowSelfShow);
 	if (!(flags & kFlagCustom) && (uniform_hidden || !(flags & kFlagMixed) || !(flags & kFlagInnerFaces))) {
 		// one block value everywhere whose faces hide each other, opaque cubes only, or no chunk voxel
 		// with a face: no quads
@@ -1483,9 +1470,9 @@ template <bool kRaw, int NT> __device__ __forceinline__ void mesh_chunk(const Me
 				continue;
 			const int hx = i % kHalo, rest = i / kHalo, hz = rest % kHalo, hy = rest / kHalo;
 			const uint32_t pid = vox_pid(s.vox[i]);
-			const uint32_t mesh = s.rows[pid].y >> 24;
+			const uint32_t mesh = s.tables.rows[pid].y >> 24;
 			const Flow f = flow_heights(p, blocks, hx - 1, hy - 1, hz - 1, p.reg->meshes[mesh].flow_height);
-			const uint32_t tmpl = s.pid_vox[p.reg->flow_pid_base + flow_pattern(f)].y;
+			const uint32_t tmpl = s.tables.pid_vox[p.reg->flow_pid_base + flow_pattern(f)].y;
 			s.vox[i] = (s.vox[i] & kKeep) | (tmpl & ~kKeep);
 		}
 		__syncthreads();
@@ -1494,7 +1481,7 @@ template <bool kRaw, int NT> __device__ __forceinline__ void mesh_chunk(const Me
 			uint32_t w[18];
 #pragma unroll
 			for (int x = 0; x < 18; ++x)
-				w[x] = s.pid_vox[vox_pid(s.vox[row * kHalo + x])].x;
+				w[x] = s.tables.pid_vox[vox_pid(s.vox[row * kHalo + x])].x;
 			put_planes(s, row / kHalo, row % kHalo, w);
 		}
 		__syncthreads();
@@ -1754,23 +1741,12 @@ template <bool kRaw, int NT> __device__ __forceinline__ void mesh_chunk(const Me
 
 template <int NT, bool kRaw> __global__ __launch_bounds__(NT, NT >= 512 ? 2 : 3) void mesh_kernel(MeshParams p) {
 	__shared__ Smem<NT> s;
-	for (int i = threadIdx.x; i < kMaxPid; i += NT) {
-		const bool ok = i < (int)p.reg->n_pid;
-		s.rows[i] = ok ? p.reg->rows[i] : make_uint2(0, 0);
-		s.pid_vox[i] = ok ? p.reg->pid_vox[i] : make_uint2(0, uint32_t(i) << kVoxPidShift);
-	}
-	for (int i = threadIdx.x; i < kMaxCodes; i += NT)
-		s.codes[i] = i < (int)p.reg->n_codes ? p.reg->codes[i] : 0u;
-	for (int i = threadIdx.x; i < 256; i += NT)
-	{
-		const uint32_t q = p.reg->pid_of[65536 + i];
-		s.tmpl_id[i] = q == 0xffu ? make_uint2(kTmplMeta, 0) : p.reg->pid_vox[q];
-	}
-	fill_averages(s);
 	if (threadIdx.x == 0) // (only this lane uses it)
 		s.claims.init(p.n_jobs);
 	const int lane = threadIdx.x & 63;
 	const uint32_t given = p.job_base + blockIdx.x; // per-chunk launches: the workgroup's one job
+	for (uint32_t i = threadIdx.x; i < sizeof(MeshTables) / 16; i += NT)
+		reinterpret_cast<uint4 *>(&s.tables)[i] = reinterpret_cast<const uint4 *>(p.tables)[i];
 	for (;;) {
 		// wavefront 0 claims the next job and loads its slot list while the others set up its LDS state
 		if (threadIdx.x < 64) {

@@ -519,6 +519,7 @@ struct hcm_server {
 			std::memset(&p, 0, sizeof(p));
 			p.reg = (const HCM_CONSTANT DevReg *)info.reg;
 			p.raw_front = info.raw_front;
+			p.tables = info.tables;
 			p.blocks = d_blocks;
 			p.light = d_light;
 			p.nbr = nbr;
