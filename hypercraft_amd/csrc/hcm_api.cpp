@@ -1074,8 +1074,9 @@ static int export_run(hcm_batch *b, bool results, bool recs, bool quads, Exporte
 	p.rec_cap = b->rec_cap;
 	if (recs && (p.out_recs = reinterpret_cast<hcm_mesh_rec *>(place((size_t)b->rec_cap * sizeof(hcm_mesh_rec)))))
 		p.recs = b->d_recs;
-	if (quads) {
-		p.quad_cap = (uint32_t)((kPoutBytes - at - 32) / 44);
+	if (quads && at + 32 < kPoutBytes) {
+		// (the run's total counts allocations that did not fit the pool: no more than the pool holds may be copied)
+		p.quad_cap = (uint32_t)std::min<uint64_t>((kPoutBytes - at - 32) / 44, c->pool_quads);
 		p.out_verts = reinterpret_cast<uint2 *>(place((size_t)p.quad_cap * 4 * sizeof(uint2)));
 		p.out_idx = reinterpret_cast<uint16_t *>(place((size_t)p.quad_cap * 12));
 		if (p.out_verts && p.out_idx)
@@ -1088,7 +1089,7 @@ static int export_run(hcm_batch *b, bool results, bool recs, bool quads, Exporte
 		what->results = p.out_results;
 	if (p.recs)
 		what->recs = p.out_recs;
-	if (p.verts && what->quads <= p.quad_cap && what->quads <= c->pool_quads)
+	if (p.verts && what->quads <= p.quad_cap)
 		what->verts = p.out_verts, what->idx = p.out_idx;
 	return HCM_OK;
 }

@@ -1,6 +1,9 @@
 // The CPU build's lane scheduler and runtime calls (see hip/hip_runtime.h).
 #include <hip/hip_runtime.h>
 
+#include <sys/mman.h>
+#include <unistd.h>
+
 #include <map>
 #include <mutex>
 
@@ -218,9 +221,30 @@ void submit(hipStream_t s, const std::function<void()> &work) {
 
 using namespace hipcpu;
 
+// With HIPCPU_GUARD set, every allocation ends (to 16 bytes) where an inaccessible page begins, so that an access past
+// it ends the process.
+struct Guarded {
+	void *base;
+	size_t bytes;
+};
+static std::map<void *, Guarded> g_guarded; // g_mu
+static hipError_t guarded_malloc(void **p, size_t n) {
+	const size_t page = (size_t)sysconf(_SC_PAGESIZE), m = (std::max<size_t>(n, 1) + 15) / 16 * 16;
+	const size_t data = (m + page - 1) / page * page;
+	char *base = (char *)mmap(nullptr, data + page, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS, -1, 0);
+	if (base == MAP_FAILED || mprotect(base + data, page, PROT_NONE) != 0)
+		return hipErrorOutOfMemory;
+	*p = base + data - m;
+	std::lock_guard<std::mutex> lk(g_mu);
+	g_guarded[*p] = Guarded{base, data + page};
+	return hipSuccess;
+}
+
 extern "C" {
 
 hipError_t hipMalloc(void **p, size_t n) {
+	if (std::getenv("HIPCPU_GUARD"))
+		return guarded_malloc(p, n);
 	const size_t m = (n + 255) / 256 * 256;
 	*p = std::aligned_alloc(256, m ? m : 256);
 	if (*p)
@@ -228,6 +252,15 @@ hipError_t hipMalloc(void **p, size_t n) {
 	return *p ? hipSuccess : hipErrorOutOfMemory;
 }
 hipError_t hipFree(void *p) {
+	{
+		std::lock_guard<std::mutex> lk(g_mu);
+		auto it = g_guarded.find(p);
+		if (it != g_guarded.end()) {
+			munmap(it->second.base, it->second.bytes);
+			g_guarded.erase(it);
+			return hipSuccess;
+		}
+	}
 	std::free(p);
 	return hipSuccess;
 }

@@ -1,0 +1,69 @@
+"""Memory faults and allocations of the library, on the CPU build of its sources (tests/cpp/hipcpu; no GPU). With
+HIPCPU_GUARD every device and pinned allocation ends at an inaccessible page, so that an access past one ends the
+process: each check runs in one of its own."""
+import os
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+LIB = os.path.join(ROOT, "hypercraft_amd", "_build", "cpu", "libhcm_cpu.so")
+
+
+def dense(n):
+    """n jobs whose own chunks are checkerboards of 12,288 faces, one quad each: two blocks in turn."""
+    y, z, x = np.indices((16, 16, 16))
+    odd = ((x + y + z) & 1).reshape(-1) == 1
+    blocks = np.zeros((27, 4096), np.uint16)
+    blocks[26] = np.where(odd, np.where(np.arange(4096) & 32, 1, 2), 0)
+    light = np.random.default_rng(7).integers(0, 256, blocks.shape).astype(np.uint8)
+    return blocks, light, np.tile(np.arange(27, dtype=np.uint32), (n, 1))
+
+
+def batch_of(hcm, ctx, n):
+    blocks, light, nbr = dense(n)
+    store = hcm.Store(ctx, 27)
+    store.upload(blocks, light)
+    return hcm.Batch(ctx, store, nbr)
+
+
+def check_download_of_a_full_pool(pool_quads):
+    """A run that wants more quads than the pool has: what fits is handed out, and nothing past the pool is read."""
+    from hypercraft_amd import hcm
+
+    ctx = hcm.Context(pool_quads=pool_quads)
+    batch = batch_of(hcm, ctx, 3)
+    batch.run()
+    wanted = batch.totals()[0]
+    res, _, verts, idx = batch.download()
+    full = res["status"] == hcm.HCM_ERR_POOL_FULL
+    assert full.any() and wanted == res["quad_count"].sum() > pool_quads and wanted < 45000
+    kept = int(res["quad_count"][~full].sum())  # the first chunks that fit: 12,288 quads each
+    assert verts[: 4 * kept].any(axis=1).all() and not verts[4 * pool_quads :].any()
+    assert idx.reshape(-1, 6)[:kept].any(axis=1).all() and not idx[6 * pool_quads :].any()
+
+
+@pytest.fixture(scope="module", autouse=True)
+def library():
+    subprocess.run(["make", "-s", "-j4", "-C", os.path.join(ROOT, "tests", "cpp", "hipcpu")], check=True, timeout=900,
+                   stderr=subprocess.DEVNULL)
+
+
+def run(check, *args):
+    env = dict(os.environ, HCM_LIB=LIB, HIPCPU_GUARD="1")
+    p = subprocess.run([sys.executable, __file__, check.__name__, *map(str, args)], capture_output=True, text=True,
+                       timeout=600, env=env)
+    assert p.returncode == 0, f"exit status {p.returncode}\n" + (p.stdout + p.stderr)[-4000:]
+
+
+# smaller than a chunk's 12,288 quads, one chunk's, two and a half chunks'
+@pytest.mark.parametrize("pool_quads", [1000, 12288, 30000])
+def test_download_of_a_full_pool(pool_quads):
+    run(check_download_of_a_full_pool, pool_quads)
+
+
+if __name__ == "__main__":
+    sys.path.insert(0, ROOT)
+    globals()[sys.argv[1]](*map(int, sys.argv[2:]))
