@@ -163,6 +163,7 @@ struct hcm_server {
 	hcm_server_config cfg{};
 	CtxInfo info{};
 	hipStream_t s_copy = nullptr, s_comp = nullptr;
+	hipStream_t s_read = nullptr; // hcm_server_chunk_mesh's (world_mu): it waits for no upload or batch
 	uint16_t *d_blocks = nullptr;
 	uint8_t *d_light = nullptr;
 	int8_t *d_heights = nullptr;  // HCM_LIGHT_REBUILD: [slot][256] sunlight heights
@@ -775,6 +776,8 @@ static void free_server(hcm_server *s) {
 		(void)hipStreamDestroy(s->s_copy);
 	if (s->s_comp)
 		(void)hipStreamDestroy(s->s_comp);
+	if (s->s_read)
+		(void)hipStreamDestroy(s->s_read);
 	delete s->pool;
 	delete s;
 }
@@ -793,6 +796,7 @@ static int server_init(hcm_server *s) {
 		return r;
 	HCM_CHECK(hipStreamCreateWithFlags(&s->s_copy, hipStreamNonBlocking));
 	HCM_CHECK(hipStreamCreateWithFlags(&s->s_comp, hipStreamNonBlocking));
+	HCM_CHECK(hipStreamCreateWithFlags(&s->s_read, hipStreamNonBlocking));
 	HCM_CHECK(dalloc(&s->d_blocks, (size_t)c.max_chunks * HCM_CHUNK_VOXELS));
 	HCM_CHECK(dalloc(&s->d_light, (size_t)c.max_chunks * HCM_CHUNK_VOXELS));
 	if (s->relight()) {
@@ -969,8 +973,8 @@ extern "C" int hcm_server_drain(hcm_server *s) {
 	return s->error;
 }
 
-static int copy_meshes(const std::vector<hcm_mesh_rec> &recs, const uint2 *verts, const uint16_t *idx, bool device,
-                       hcm_host_result *out) {
+// The counts of a chunk's meshes into *out, and whether its buffers hold them.
+static int check_capacity(const std::vector<hcm_mesh_rec> &recs, hcm_host_result *out) {
 	uint64_t nv = 0, ni = 0;
 	for (auto &m : recs)
 		nv += 4ull * m.quad_count, ni += 6ull * m.quad_count;
@@ -978,6 +982,14 @@ static int copy_meshes(const std::vector<hcm_mesh_rec> &recs, const uint2 *verts
 	if (nv > out->vertex_capacity || ni > out->index_capacity || recs.size() > out->mesh_capacity ||
 	    (nv && (!out->vertices || !out->indices)) || (!recs.empty() && !out->meshes))
 		return HCM_ERR_CAPACITY;
+	return HCM_OK;
+}
+
+static int copy_meshes(const std::vector<hcm_mesh_rec> &recs, const uint2 *verts, const uint16_t *idx, bool device,
+                       hcm_host_result *out) {
+	const int r = check_capacity(recs, out);
+	if (r != HCM_OK)
+		return r;
 	uint32_t vb = 0, ib = 0;
 	for (size_t m = 0; m < recs.size(); ++m) {
 		const hcm_mesh_rec &rc = recs[m];
@@ -1012,16 +1024,19 @@ extern "C" int hcm_server_chunk_mesh(hcm_server *s, int32_t cx, int32_t cy, int3
 	const Chunk &c = it->second;
 	if (c.mesh.count == 0 || c.mesh.count > kPinnedQuads)
 		return copy_meshes(c.recs, s->d_verts, s->d_idx, true, out);
-	// the chunk's quads lie together: one kernel brings them to pinned memory (on the copy stream: they were made
-	// by a finished batch, and later ones may be running)
+	const int fits = check_capacity(c.recs, out);
+	if (fits != HCM_OK)
+		return fits;
+	// the chunk's quads lie together: one kernel brings them to pinned memory (they were made by a finished batch, and
+	// later ones may be running)
 	ExportParams e;
 	e.given_quads = e.quad_cap = (uint32_t)c.mesh.count;
 	e.verts = s->d_verts + 4 * c.mesh.first;
 	e.idx = s->d_idx + 6 * c.mesh.first;
 	e.out_verts = reinterpret_cast<uint2 *>(s->h_mesh);
 	e.out_idx = reinterpret_cast<uint16_t *>(s->h_mesh + (size_t)kPinnedQuads * 32);
-	HCM_CHECK(launch_export(e, s->s_copy));
-	HCM_CHECK(hipStreamSynchronize(s->s_copy));
+	HCM_CHECK(launch_export(e, s->s_read));
+	HCM_CHECK(hipStreamSynchronize(s->s_read));
 	std::vector<hcm_mesh_rec> recs = c.recs;
 	for (auto &rec : recs)
 		rec.first_quad -= (uint32_t)c.mesh.first;
