@@ -34,6 +34,7 @@
 #include <mutex>
 #include <thread>
 #include <unordered_map>
+#include <unordered_set>
 #include <vector>
 
 #include "hcm_internal.h"
@@ -461,16 +462,19 @@ struct hcm_server {
 		for (uint32_t i = 0; i < n_up; ++i)
 			if (!uploads[i].reload)
 				b.h_moves[n_fresh++] = make_uint2(i, uploads[i].slot);
-		for (uint32_t i = 0, k = n_fresh; i < n_up; ++i)
-			if (uploads[i].reload)
-				b.h_moves[k++] = make_uint2(i, uploads[i].slot);
+		// (of several reloads of a chunk the last: the launch's workgroups run in any order)
+		uint32_t n_moves = n_fresh;
+		std::unordered_set<uint32_t> reloaded;
+		for (uint32_t i = n_up; i-- > 0;)
+			if (uploads[i].reload && reloaded.insert(uploads[i].slot).second)
+				b.h_moves[n_moves++] = make_uint2(i, uploads[i].slot);
 		if (n_fresh) {
 			HCM_CHECK(launch_upload_scatter(b.h_blocks, b.h_light, b.h_heights, b.h_moves, n_fresh, d_blocks, d_light,
 			                                d_heights, s_copy));
 			HCM_CHECK(hipEventRecord(b.ev_up, s_copy));
 			HCM_CHECK(hipStreamWaitEvent(s_comp, b.ev_up, 0));
 		}
-		HCM_CHECK(launch_upload_scatter(b.h_blocks, b.h_light, b.h_heights, b.h_moves + n_fresh, n_up - n_fresh, d_blocks,
+		HCM_CHECK(launch_upload_scatter(b.h_blocks, b.h_light, b.h_heights, b.h_moves + n_fresh, n_moves - n_fresh, d_blocks,
 		                                d_light, d_heights, s_comp));
 		uploads.erase(uploads.begin(), uploads.begin() + n_up);
 

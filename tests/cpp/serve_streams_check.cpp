@@ -3,6 +3,7 @@
 // the gate is open, so that requests can be held back until one batch takes them all. Exit status 0 when all holds.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <condition_variable>
 #include <cstdio>
 #include <map>
@@ -168,9 +169,35 @@ static void check_read_back(uint32_t mode) {
 	CHECK(rec::exports[0] != w.s->s_copy && rec::exports[0] != w.s->s_comp);
 }
 
+// A chunk that is loaded again and again before a batch takes the loads: the last one counts, and no launch writes a slot
+// twice (its workgroups run in any order).
+static void check_repeated_loads(uint32_t mode) {
+	World w(mode);
+	rec::gate = false;
+	w.load(0, 0, 0, 2); // goes ahead alone; the others gather behind it
+	w.wait_uploads(0);
+	for (uint16_t block : {3, 4, 5}) {
+		w.load(0, 0, 0, block);
+		w.load(0, 1, 0, block);
+		w.load(5, 5, 5, block); // the first of these is a first load
+	}
+	w.wait_uploads(9);
+	rec::clear();
+	rec::gate = true;
+	CHECK(hcm_server_drain(w.s) == HCM_OK);
+	size_t n = 0;
+	for (rec::Scatter &s : rec::scatters) {
+		n += s.slots.size();
+		std::sort(s.slots.begin(), s.slots.end());
+		CHECK(std::adjacent_find(s.slots.begin(), s.slots.end()) == s.slots.end());
+	}
+	CHECK(n == 4); // three chunks, one of them also for the first time
+	CHECK(w.center_block() == 5);
+}
+
 int main() {
 	for (uint32_t mode : {HCM_LIGHT_STORE, HCM_LIGHT_REBUILD})
-		check_read_back(mode);
+		check_read_back(mode), check_repeated_loads(mode);
 	if (g_fail)
 		return 1;
 	std::printf("serve_streams_check: all checks passed\n");
