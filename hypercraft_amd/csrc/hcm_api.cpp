@@ -243,8 +243,9 @@ struct hcm_ctx {
 	// device registry buffers
 	uint8_t *d_pid_of = nullptr;
 	MeshTables *d_tables = nullptr;
-	uint8_t *d_kept = nullptr; // MeshParams::kept of the batches, all on `stream`; from the first batch on
+	uint8_t *d_kept = nullptr; // MeshParams::kept of the batches, all on `stream` (want_kept)
 	size_t kept_bytes = 0;
+	size_t kept_refused = SIZE_MAX; // the least that could not be allocated
 	DevReg *d_reg = nullptr;
 	uint32_t raw_front = 0;
 	hcm_custom_mesh *d_meshes = nullptr;
@@ -519,6 +520,34 @@ static int persistent_grid(hcm_ctx *c, uint32_t threads) {
 // and 41.0).
 static uint32_t batch_threads(const hcm_ctx *c, uint32_t n_jobs) {
 	return !c->threads_given && n_jobs <= (uint32_t)c->n_cu ? 512u : c->tuning.threads;
+}
+
+// Memory for the dense chunks of a persistent launch of `grid` workgroups (context lock held): made by the batch that
+// first needs as much, so that a context of small batches holds little. A tuning with many workgroups per CU does
+// without it past kKeptMax (12 workgroups of each of 256 CUs, four times what their LDS holds), as does a launch for
+// which there is no memory: words are then computed twice.
+constexpr size_t kKeptMax = size_t(256) << 20;
+static void want_kept(hcm_ctx *c, size_t grid) {
+	const size_t bytes = grid * kKeptBytes;
+	if (bytes <= c->kept_bytes || bytes > kKeptMax || bytes >= c->kept_refused)
+		return;
+	uint8_t *grown = nullptr;
+	if (dmalloc(&grown, bytes) != hipSuccess) {
+		(void)hipGetLastError();
+		c->kept_refused = bytes;
+		return;
+	}
+	if (c->d_kept) { // earlier launches may still be using it
+		(void)hipStreamSynchronize(c->stream);
+		dfree(c->d_kept);
+	}
+	c->d_kept = grown;
+	c->kept_bytes = bytes;
+}
+
+// Workgroups of a persistent launch of n_jobs.
+static int batch_grid(hcm_ctx *c, uint32_t n_jobs) {
+	return (int)std::min((uint32_t)persistent_grid(c, batch_threads(c, n_jobs)), n_jobs);
 }
 
 int hcm::ctx_info(hcm_ctx *ctx, uint32_t threads, CtxInfo *out) {
@@ -862,11 +891,8 @@ extern "C" int hcm_batch_create(hcm_ctx *ctx, hcm_store *store, const uint32_t *
 		return fail();
 	{
 		std::lock_guard<std::mutex> lk(ctx->mu);
-		const size_t bytes = persistent_grid(ctx, 256) * kKeptBytes;
-		if (!ctx->d_kept && dmalloc(&ctx->d_kept, bytes) == hipSuccess)
-			ctx->kept_bytes = bytes;
-		else if (!ctx->d_kept)
-			(void)hipGetLastError(); // (dense chunks do without)
+		ctx->kept_refused = SIZE_MAX;
+		want_kept(ctx, batch_grid(ctx, n_jobs));
 	}
 	*out = b;
 	return HCM_OK;
@@ -997,7 +1023,8 @@ static int batch_run(hcm_batch *b, uint32_t mode, uint32_t times) {
 		b->ctr_clean = false;
 		p.persistent = 1;
 		p.self_reset = 1; // the counters start at zero and the run's last workgroup zeroes them again
-		const int grid = (int)std::min((uint32_t)persistent_grid(c, threads), b->n_jobs);
+		const int grid = batch_grid(c, b->n_jobs);
+		want_kept(c, grid); // (the tuning may have changed since the batch was made)
 		p.kept = grid * kKeptBytes <= c->kept_bytes ? c->d_kept : nullptr; // (c->stream's launches follow each other)
 		HCM_HIP(hipEventRecord(b->ev0, st));
 		for (uint32_t k = 0; k < times; ++k) {

@@ -215,8 +215,9 @@ typedef struct hcm_batch hcm_batch;
 #define HCM_RUN_PER_CHUNK 1u  /* one kernel launch per chunk (the plain per-chunk path) */
 
 /* A batch of n_jobs chunk jobs over a store: nbr holds 27 slot indices per job (host array, copied
- * to the device). Output meshes go to the context's quad pool. A context's first batch also allocates the
- * kernels' working memory for dense chunks (80 KB per workgroup of the persistent grid), which the context holds. */
+ * to the device). Output meshes go to the context's quad pool. The context also holds the
+ * kernels' working memory for dense chunks, 80 KB per workgroup of its batches' largest launch (at most 256 MiB): it
+ * grows where a batch is made or, after a change of tuning, run. */
 int hcm_batch_create(hcm_ctx *ctx, hcm_store *store, const uint32_t *nbr, uint32_t n_jobs, hcm_batch **out);
 void hcm_batch_destroy(hcm_batch *batch);
 /* Enqueues one meshing pass over every job (resets the pool first). Asynchronous. */

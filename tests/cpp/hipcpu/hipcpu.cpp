@@ -225,7 +225,7 @@ using namespace hipcpu;
 // it ends the process.
 struct Guarded {
 	void *base;
-	size_t bytes;
+	size_t bytes, asked;
 };
 static std::map<void *, Guarded> g_guarded; // g_mu
 static hipError_t guarded_malloc(void **p, size_t n) {
@@ -236,11 +236,20 @@ static hipError_t guarded_malloc(void **p, size_t n) {
 		return hipErrorOutOfMemory;
 	*p = base + data - m;
 	std::lock_guard<std::mutex> lk(g_mu);
-	g_guarded[*p] = Guarded{base, data + page};
+	g_guarded[*p] = Guarded{base, data + page, n};
 	return hipSuccess;
 }
 
 extern "C" {
+
+// The bytes of all allocations made with HIPCPU_GUARD and not freed.
+size_t hipcpu_allocated() {
+	std::lock_guard<std::mutex> lk(g_mu);
+	size_t sum = 0;
+	for (auto &g : g_guarded)
+		sum += g.second.asked;
+	return sum;
+}
 
 hipError_t hipMalloc(void **p, size_t n) {
 	if (std::getenv("HIPCPU_GUARD"))

@@ -1,6 +1,7 @@
 """Memory faults and allocations of the library, on the CPU build of its sources (tests/cpp/hipcpu; no GPU). With
 HIPCPU_GUARD every device and pinned allocation ends at an inaccessible page, so that an access past one ends the
 process: each check runs in one of its own."""
+import ctypes
 import os
 import subprocess
 import sys
@@ -45,6 +46,48 @@ def check_download_of_a_full_pool(pool_quads):
     assert idx.reshape(-1, 6)[:kept].any(axis=1).all() and not idx[6 * pool_quads :].any()
 
 
+KEPT = 8192 * 10  # bytes of a workgroup's memory for dense chunks; the CPU build has two CUs
+
+
+def allocated(hcm):
+    f = hcm.lib().hipcpu_allocated
+    f.restype = ctypes.c_size_t
+    return f()
+
+
+def check_dense_memory_of_one_job():
+    """The memory for dense chunks is that of the workgroups a batch can launch, whatever the tuning allows."""
+    from hypercraft_amd import hcm
+
+    ctx = hcm.Context(pool_quads=1 << 14)
+    ctx.set_tuning(wg_per_cu=64, threads=256)
+    before = allocated(hcm)
+    batch = batch_of(hcm, ctx, 1)
+    assert allocated(hcm) - before < 1 << 20  # (its store is 0.34 MB)
+    batch.run()
+    assert allocated(hcm) - before < 1 << 20 and batch.totals() == (12288, 1)
+
+
+def check_dense_memory_grows():
+    """A batch whose launches grow beyond the workgroups the memory was made for gets more of it, once."""
+    from hypercraft_amd import hcm
+    import meshdigest
+
+    ctx = hcm.Context(pool_quads=12 * 12288)
+    ctx.set_tuning(wg_per_cu=1, threads=256)
+    batch = batch_of(hcm, ctx, 12)
+    digests = []
+    sizes = [allocated(hcm)]
+    for wg_per_cu in (1, 3, 1, 3):
+        ctx.set_tuning(wg_per_cu=wg_per_cu, threads=256)
+        batch.run()
+        sizes.append(allocated(hcm))
+        out = batch.download()
+        digests.append({meshdigest.digest(hcm.job_meshes(j, *out)) for j in range(12)})
+    assert np.diff(sizes).tolist() == [0, 4 * KEPT, 0, 0], np.diff(sizes)
+    assert len(digests[0]) == 1 and digests == digests[:1] * 4
+
+
 @pytest.fixture(scope="module", autouse=True)
 def library():
     subprocess.run(["make", "-s", "-j4", "-C", os.path.join(ROOT, "tests", "cpp", "hipcpu")], check=True, timeout=900,
@@ -64,6 +107,14 @@ def test_download_of_a_full_pool(pool_quads):
     run(check_download_of_a_full_pool, pool_quads)
 
 
+def test_dense_memory_of_one_job():
+    run(check_dense_memory_of_one_job)
+
+
+def test_dense_memory_grows():
+    run(check_dense_memory_grows)
+
+
 if __name__ == "__main__":
-    sys.path.insert(0, ROOT)
+    sys.path[:0] = [ROOT, os.path.join(ROOT, "tests")]
     globals()[sys.argv[1]](*map(int, sys.argv[2:]))
