@@ -279,8 +279,7 @@ struct hcm_ctx {
 	float *d_depth = nullptr;
 	size_t depth_cap = 0; // floats
 	DepthPyramid hiz;
-	hcm_tuning tuning{0, 256, {0, 0}};
-	bool threads_given = false; // hcm_set_tuning named the workgroup size: no launch takes another
+	hcm_tuning tuning{0, 256, {1, 0}}; // reserved[0]: no workgroup size was asked for
 };
 
 struct hcm_store {
@@ -482,7 +481,8 @@ extern "C" int hcm_set_tuning(hcm_ctx *ctx, const hcm_tuning *t) {
 	std::lock_guard<std::mutex> lk(ctx->mu);
 	ctx->tuning = *t;
 	ctx->tuning.threads = th;
-	ctx->threads_given = t->threads != 0;
+	// (a size that was asked for is every launch's)
+	ctx->tuning.reserved[0] = t->threads == 0 || (t->reserved[0] == 1 && th == 256);
 	return HCM_OK;
 }
 
@@ -519,7 +519,7 @@ static int persistent_grid(hcm_ctx *c, uint32_t threads) {
 // such workgroup fills a CU's registers, so that past that many jobs it is the slower (400 jobs: 35.8 and 38.5, 28.9
 // and 41.0).
 static uint32_t batch_threads(const hcm_ctx *c, uint32_t n_jobs) {
-	return !c->threads_given && n_jobs <= (uint32_t)c->n_cu ? 512u : c->tuning.threads;
+	return c->tuning.reserved[0] && n_jobs <= (uint32_t)c->n_cu ? 512u : c->tuning.threads;
 }
 
 // Memory for the dense chunks of a persistent launch of `grid` workgroups (context lock held): made by the batch that

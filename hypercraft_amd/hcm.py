@@ -293,14 +293,14 @@ class Context:
         except Exception:
             pass
 
-    def set_tuning(self, wg_per_cu=0, threads=256):
-        t = TuningC(wg_per_cu, threads, (ctypes.c_uint32 * 2)(0, 0))
+    def set_tuning(self, wg_per_cu=0, threads=256, default_threads=False):
+        t = TuningC(wg_per_cu, threads, (ctypes.c_uint32 * 2)(int(default_threads), 0))
         check("hcm_set_tuning", lib().hcm_set_tuning(self._ptr, ctypes.byref(t)))
 
     def get_tuning(self):
         t = TuningC()
         check("hcm_get_tuning", lib().hcm_get_tuning(self._ptr, ctypes.byref(t)))
-        return {"wg_per_cu": t.wg_per_cu, "threads": t.threads}
+        return {"wg_per_cu": t.wg_per_cu, "threads": t.threads, "default_threads": t.reserved[0] == 1}
 
     def mesh_chunk(self, blocks27, light27):
         """Plain path: meshes slot 26 of 27 host chunks; returns the reference's list of BlockMesh."""

@@ -301,6 +301,8 @@ int hcm_batch_cull_occlusion(hcm_batch *batch, const float view_position[3], con
 typedef struct hcm_tuning {
 	uint32_t wg_per_cu; /* persistent workgroups per compute unit */
 	uint32_t threads;   /* workgroup size: 128, 256 or 512; 0: 256, and 512 for batches of few jobs */
+	/* reserved[0]: hcm_get_tuning sets it to 1 when threads is the default's (it then reads 256), so that
+	 * hcm_set_tuning of what it gave, or of that with another wg_per_cu, leaves the default as it was; else 0 */
 	uint32_t reserved[2];
 } hcm_tuning;
 int hcm_set_tuning(hcm_ctx *ctx, const hcm_tuning *t);

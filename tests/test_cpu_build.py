@@ -88,6 +88,28 @@ def check_dense_memory_grows():
     assert len(digests[0]) == 1 and digests == digests[:1] * 4
 
 
+def check_tuning_round_trip():
+    """What hcm_get_tuning returns, given back, changes nothing: with no workgroup size set, batches of few jobs still
+    take another than the one it names."""
+    from hypercraft_amd import hcm
+
+    ctx = hcm.Context(pool_quads=1 << 14)
+    fresh = ctx.get_tuning()
+    assert fresh == {"wg_per_cu": 0, "threads": 256, "default_threads": True}
+    ctx.set_tuning(**fresh)
+    assert ctx.get_tuning() == fresh
+    ctx.set_tuning(**dict(fresh, wg_per_cu=2))
+    assert ctx.get_tuning() == dict(fresh, wg_per_cu=2)
+    for threads in (128, 256, 512):
+        ctx.set_tuning(wg_per_cu=2, threads=threads)
+        asked = ctx.get_tuning()
+        assert asked == {"wg_per_cu": 2, "threads": threads, "default_threads": False}
+        ctx.set_tuning(**asked)
+        assert ctx.get_tuning() == asked
+    ctx.set_tuning(threads=0)
+    assert ctx.get_tuning() == fresh
+
+
 @pytest.fixture(scope="module", autouse=True)
 def library():
     subprocess.run(["make", "-s", "-j4", "-C", os.path.join(ROOT, "tests", "cpp", "hipcpu")], check=True, timeout=900,
@@ -113,6 +135,10 @@ def test_dense_memory_of_one_job():
 
 def test_dense_memory_grows():
     run(check_dense_memory_grows)
+
+
+def test_tuning_round_trip():
+    run(check_tuning_round_trip)
 
 
 if __name__ == "__main__":
