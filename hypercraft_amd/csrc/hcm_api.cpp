@@ -34,6 +34,20 @@ template <typename T> hipError_t dmalloc(T **p, size_t count) {
 	return hipMalloc(reinterpret_cast<void **>(p), std::max<size_t>(count, 1) * sizeof(T));
 }
 
+// Memory made by the first call that needs it; after a failure the next call tries again.
+template <typename T> hipError_t ensure(T **p, size_t count) { return *p ? hipSuccess : dmalloc(p, count); }
+template <typename T> hipError_t ensure_zero(T **p, hipStream_t st) { // one, zero for what st launches from now on
+	if (*p)
+		return hipSuccess;
+	T *made = nullptr;
+	hipError_t e = dmalloc(&made, 1);
+	if (e == hipSuccess && (e = hipMemsetAsync(made, 0, sizeof(T), st)) != hipSuccess)
+		(void)hipFree(made);
+	if (e == hipSuccess)
+		*p = made;
+	return e;
+}
+
 // Registry flattened for the kernels (see hcm_internal.h for the word layouts).
 struct DeviceTables {
 	MeshTables tables;
@@ -905,16 +919,10 @@ extern "C" int hcm_batch_set_light(hcm_batch *b, uint32_t light_mode) {
 	std::lock_guard<std::mutex> lk(c->mu);
 	if (light_mode == HCM_LIGHT_REBUILD) {
 		hcm_store *st = b->store;
-		if (!st->d_packed) {
-			HCM_HIP(dmalloc(&st->d_packed, (size_t)st->n_slots * kLightSlotBytes / 2));
-			HCM_HIP(dmalloc(&st->d_levels, st->n_slots));
-		}
-		if (!b->d_lctr) { // zero once: each light run's last workgroup clears the queues again
-			HCM_HIP(dmalloc(&b->d_lctr, 1));
-			HCM_HIP(hipMemset(b->d_lctr, 0, sizeof(Counters)));
-		}
-		if (!b->d_halo_light)
-			HCM_HIP(dmalloc(&b->d_halo_light, (size_t)b->n_jobs * kLightJobBytes));
+		HCM_HIP(ensure(&st->d_packed, (size_t)st->n_slots * kLightSlotBytes / 2));
+		HCM_HIP(ensure(&st->d_levels, st->n_slots));
+		HCM_HIP(ensure_zero(&b->d_lctr, c->stream)); // each light run's last workgroup clears the queues again
+		HCM_HIP(ensure(&b->d_halo_light, (size_t)b->n_jobs * kLightJobBytes));
 	}
 	b->light_mode = light_mode;
 	return HCM_OK;
@@ -1159,13 +1167,10 @@ extern "C" int hcm_batch_mesh_infos(hcm_batch *b, const int32_t *chunk_pos, hcm_
 	hcm_ctx *c = b->ctx;
 	std::lock_guard<std::mutex> lk(c->mu);
 	hipStream_t st = c->stream;
-	if (!b->d_infos) {
-		HCM_HIP(dmalloc(&b->d_chunk_pos, 3ull * b->n_jobs));
-		HCM_HIP(dmalloc(&b->d_infos, b->rec_cap));
-		HCM_HIP(dmalloc(&b->d_draws, 2ull * b->rec_cap));
-		HCM_HIP(dmalloc(&b->d_draw_counts, 1));
-		HCM_HIP(hipMemsetAsync(b->d_draw_counts, 0, sizeof(CullCounts), st)); // zero once: each cull clears them again
-	}
+	HCM_HIP(ensure(&b->d_chunk_pos, 3ull * b->n_jobs));
+	HCM_HIP(ensure(&b->d_infos, b->rec_cap));
+	HCM_HIP(ensure(&b->d_draws, 2ull * b->rec_cap));
+	HCM_HIP(ensure_zero(&b->d_draw_counts, st)); // each cull clears them again
 	// one launch from and to pinned memory where the positions and the infos fit, else by way of the device
 	const size_t pos_bytes = 12ull * b->n_jobs, at_infos = 64 + (pos_bytes + 15) / 16 * 16;
 	const bool pinned = at_infos + (size_t)b->rec_cap * sizeof(hcm_mesh_info) <= kPoutBytes;

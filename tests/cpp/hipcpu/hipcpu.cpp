@@ -240,7 +240,11 @@ static hipError_t guarded_malloc(void **p, size_t n) {
 	return hipSuccess;
 }
 
+static int g_fail_in = 0; // the g_fail_in-th allocation from now fails
+
 extern "C" {
+
+void hipcpu_fail_allocation(int in) { g_fail_in = in; }
 
 // The bytes of all allocations made with HIPCPU_GUARD and not freed.
 size_t hipcpu_allocated() {
@@ -252,6 +256,8 @@ size_t hipcpu_allocated() {
 }
 
 hipError_t hipMalloc(void **p, size_t n) {
+	if (g_fail_in && --g_fail_in == 0)
+		return hipErrorOutOfMemory;
 	if (std::getenv("HIPCPU_GUARD"))
 		return guarded_malloc(p, n);
 	const size_t m = (n + 255) / 256 * 256;

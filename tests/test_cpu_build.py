@@ -110,6 +110,30 @@ def check_tuning_round_trip():
     assert ctx.get_tuning() == fresh
 
 
+def check_retry_after_failed_allocation(n):
+    """A call whose n-th allocation failed can be made again."""
+    from hypercraft_amd import hcm, workloads
+
+    ctx = hcm.Context(pool_quads=1 << 14)
+    batch = batch_of(hcm, ctx, 1)
+
+    def twice(call):
+        hcm.lib().hipcpu_fail_allocation(n)
+        try:
+            call()
+        except hcm.HcmError:
+            pass
+        hcm.lib().hipcpu_fail_allocation(0)
+        return call()
+
+    twice(lambda: batch.set_light(hcm.LIGHT_REBUILD))
+    batch.run()
+    assert batch.results()["status"][0] == 0
+    infos = twice(lambda: batch.mesh_infos(np.zeros((1, 3), np.int32)))
+    opaque, clear = batch.cull(np.array([8, 8, -20], np.float32), workloads.look_at_projection(np.array([8, 8, -20], np.float32), (8, 8, 8)))
+    assert len(infos) == len(opaque) + len(clear) == 1
+
+
 @pytest.fixture(scope="module", autouse=True)
 def library():
     subprocess.run(["make", "-s", "-j4", "-C", os.path.join(ROOT, "tests", "cpp", "hipcpu")], check=True, timeout=900,
@@ -139,6 +163,11 @@ def test_dense_memory_grows():
 
 def test_tuning_round_trip():
     run(check_tuning_round_trip)
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 4])
+def test_retry_after_failed_allocation(n):
+    run(check_retry_after_failed_allocation, n)
 
 
 if __name__ == "__main__":
