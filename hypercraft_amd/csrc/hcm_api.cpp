@@ -281,6 +281,7 @@ struct hcm_ctx {
 	// records, up to kPlainFastQuads quads and the rebuilt light
 	uint8_t *h_halo_in = nullptr;
 	uint8_t *h_pout = nullptr;
+	size_t pout_touched = 0; // its first bytes that the host has written
 	// this device's copy of `scratch` (hcm_mesh_halos_noalloc); host code uses this address, never the
 	// array's name, which on the host is only a stand-in
 	uint8_t *d_scratch = nullptr;
@@ -389,13 +390,22 @@ static void free_ctx(hcm_ctx *c) {
 	delete c;
 }
 
-// Pinned memory, written once: the first touch of each of its pages by the host faults, about 600 us for the 2 MiB that
-// a first download would otherwise meet (the download of 333 chunks' meshes 770 us, 150 so).
 template <typename T> static hipError_t pinned(T **p, size_t bytes) {
-	const hipError_t e = hipHostMalloc(reinterpret_cast<void **>(p), bytes);
-	if (e == hipSuccess)
-		std::memset(*p, 0, bytes);
-	return e;
+	return hipHostMalloc(reinterpret_cast<void **>(p), bytes);
+}
+
+// Writes the first `bytes` of the context's pinned output once (context lock held: no kernel is writing there). The
+// host's first touch of each of its pages faults, 0.4 ms per MiB: that is paid by what may use it, 64 KB with the
+// context and 6 KB (128 quads and their records) for each job of a batch when it is made. With none of it touched
+// before, the first download of 333 chunks' meshes took 770 us instead of 150; with all of it touched in every context
+// a context took 1.8 ms to make beside others, 0.9 so.
+constexpr size_t kTouchContext = 64 << 10, kTouchJob = 6 << 10;
+static void touch_output(hcm_ctx *c, size_t bytes) {
+	bytes = std::min(bytes, kPoutBytes);
+	if (bytes > c->pout_touched) {
+		std::memset(c->h_pout + c->pout_touched, 0, bytes - c->pout_touched);
+		c->pout_touched = bytes;
+	}
 }
 
 static int create_impl(hcm_ctx *c, const hcm_registry *registry, uint64_t pool_quads) {
@@ -450,6 +460,8 @@ static int create_impl(hcm_ctx *c, const hcm_registry *registry, uint64_t pool_q
 	HCM_HIP(pinned(&c->h_pblocks, 27 * HCM_CHUNK_VOXELS * 2));
 	HCM_HIP(pinned(&c->h_halo_in, kHaloBytes));
 	HCM_HIP(pinned(&c->h_pout, kPoutBytes));
+	std::memset(c->h_halo_in, 0, kHaloBytes);
+	touch_output(c, kTouchContext);
 	HCM_HIP(pinned(&c->h_pheights, 27 * 256));
 	HCM_HIP(dmalloc(&c->d_ppacked, 27 * kLightSlotBytes / 2));
 	HCM_HIP(dmalloc(&c->d_plevels, 27));
@@ -907,6 +919,7 @@ extern "C" int hcm_batch_create(hcm_ctx *ctx, hcm_store *store, const uint32_t *
 		std::lock_guard<std::mutex> lk(ctx->mu);
 		ctx->kept_refused = SIZE_MAX;
 		want_kept(ctx, batch_grid(ctx, n_jobs));
+		touch_output(ctx, kTouchContext + (size_t)n_jobs * kTouchJob);
 	}
 	*out = b;
 	return HCM_OK;

@@ -226,9 +226,10 @@ using namespace hipcpu;
 struct Guarded {
 	void *base;
 	size_t bytes, asked;
+	bool pinned;
 };
 static std::map<void *, Guarded> g_guarded; // g_mu
-static hipError_t guarded_malloc(void **p, size_t n) {
+static hipError_t guarded_malloc(void **p, size_t n, bool pinned) {
 	const size_t page = (size_t)sysconf(_SC_PAGESIZE), m = (std::max<size_t>(n, 1) + 15) / 16 * 16;
 	const size_t data = (m + page - 1) / page * page;
 	char *base = (char *)mmap(nullptr, data + page, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS, -1, 0);
@@ -236,7 +237,7 @@ static hipError_t guarded_malloc(void **p, size_t n) {
 		return hipErrorOutOfMemory;
 	*p = base + data - m;
 	std::lock_guard<std::mutex> lk(g_mu);
-	g_guarded[*p] = Guarded{base, data + page, n};
+	g_guarded[*p] = Guarded{base, data + page, n, pinned};
 	return hipSuccess;
 }
 
@@ -255,11 +256,26 @@ size_t hipcpu_allocated() {
 	return sum;
 }
 
+// The bytes of pinned ones that have been touched, in whole pages.
+size_t hipcpu_pinned_touched() {
+	const size_t page = (size_t)sysconf(_SC_PAGESIZE);
+	std::lock_guard<std::mutex> lk(g_mu);
+	size_t sum = 0;
+	for (auto &g : g_guarded)
+		if (g.second.pinned) {
+			std::vector<unsigned char> in(g.second.bytes / page);
+			if (mincore(g.second.base, g.second.bytes, in.data()) == 0)
+				for (unsigned char c : in)
+					sum += (c & 1) * page;
+		}
+	return sum;
+}
+
 hipError_t hipMalloc(void **p, size_t n) {
 	if (g_fail_in && --g_fail_in == 0)
 		return hipErrorOutOfMemory;
 	if (std::getenv("HIPCPU_GUARD"))
-		return guarded_malloc(p, n);
+		return guarded_malloc(p, n, false);
 	const size_t m = (n + 255) / 256 * 256;
 	*p = std::aligned_alloc(256, m ? m : 256);
 	if (*p)
@@ -279,7 +295,9 @@ hipError_t hipFree(void *p) {
 	std::free(p);
 	return hipSuccess;
 }
-hipError_t hipHostMalloc(void **p, size_t n, unsigned) { return hipMalloc(p, n); }
+hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
+	return std::getenv("HIPCPU_GUARD") ? guarded_malloc(p, n, true) : hipMalloc(p, n);
+}
 hipError_t hipHostFree(void *p) { return hipFree(p); }
 hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) {
 	if (n)

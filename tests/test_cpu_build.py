@@ -49,10 +49,14 @@ def check_download_of_a_full_pool(pool_quads):
 KEPT = 8192 * 10  # bytes of a workgroup's memory for dense chunks; the CPU build has two CUs
 
 
-def allocated(hcm):
-    f = hcm.lib().hipcpu_allocated
+def count(hcm, name):
+    f = getattr(hcm.lib(), "hipcpu_" + name)
     f.restype = ctypes.c_size_t
     return f()
+
+
+def allocated(hcm):
+    return count(hcm, "allocated")
 
 
 def check_dense_memory_of_one_job():
@@ -86,6 +90,22 @@ def check_dense_memory_grows():
         digests.append({meshdigest.digest(hcm.job_meshes(j, *out)) for j in range(12)})
     assert np.diff(sizes).tolist() == [0, 4 * KEPT, 0, 0], np.diff(sizes)
     assert len(digests[0]) == 1 and digests == digests[:1] * 4
+
+
+def check_pinned_memory_touched():
+    """A context touches little of its pinned memory before it has batches, and then as much as they are large."""
+    from hypercraft_amd import hcm
+
+    ctx = hcm.Context(pool_quads=1 << 14)
+    touched = [count(hcm, "pinned_touched")]
+    for n in (1, 37, 400, 37, 1000):
+        batch_of(hcm, ctx, n)
+        touched.append(count(hcm, "pinned_touched"))
+    made, one, few, many, after, most = touched
+    assert made <= 128 << 10
+    assert made <= one <= made + (16 << 10)
+    assert 37 * 5000 < few - made < 37 * 10000
+    assert 2 << 20 <= many <= (2 << 20) + (128 << 10) and many == after == most
 
 
 def check_tuning_round_trip():
@@ -159,6 +179,10 @@ def test_dense_memory_of_one_job():
 
 def test_dense_memory_grows():
     run(check_dense_memory_grows)
+
+
+def test_pinned_memory_touched():
+    run(check_pinned_memory_touched)
 
 
 def test_tuning_round_trip():
