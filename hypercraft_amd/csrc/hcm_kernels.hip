@@ -1771,11 +1771,11 @@ template <int NT, bool kRaw> __global__ __launch_bounds__(NT, NT >= 512 ? 2 : 3)
 	}
 	// every claim and allocation of this workgroup precedes its increment of `done`, so the last
 	// workgroup to increment it sees final totals and may clear the counters for the next run. They are
-	// atomics whose results this workgroup has (JobClaims::done for the last), and nothing else of it is read before
-	// the launch ends: no fence, which would write back the XCD's L2 once per workgroup (the cave batch 95.0 -> 86.2 us
+	// atomics that have returned, and nothing else of this workgroup is read before the launch ends: no fence, which would write back the XCD's L2 once per workgroup (the cave batch 95.0 -> 86.2 us
 	// without, 1,000 random chunks 258 -> 230 us).
 	if (p.self_reset && threadIdx.x == 0) {
-		if (atomicAdd(&p.ctr->done, s.claims.done()) == gridDim.x - 1) {
+		claims_returned();
+		if (atomicAdd(&p.ctr->done, 1u) == gridDim.x - 1) {
 			p.ctr->total_quads = atomicAdd(&p.ctr->pool_cursor, 0u);
 			p.ctr->total_meshes = atomicAdd(&p.ctr->mesh_cursor, 0u);
 			for (uint32_t q = 0; q < kQueues; ++q)

@@ -330,7 +330,8 @@ __global__ __launch_bounds__(kLightThreads, 8) void light_kernel(LightParams p) 
 	}
 	// as in the mesh kernel: the last workgroup to finish clears the queues for the next run
 	if (p.self_reset && threadIdx.x == 0) {
-		if (atomicAdd(&p.ctr->done, claims.done()) == gridDim.x - 1) {
+		claims_returned();
+		if (atomicAdd(&p.ctr->done, 1u) == gridDim.x - 1) {
 			for (uint32_t q = 0; q < kQueues; ++q)
 				p.ctr->queue[q].v = 0;
 			p.ctr->dry.v = 0;

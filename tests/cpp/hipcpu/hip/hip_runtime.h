@@ -91,6 +91,7 @@ inline dim3 grid_dim() { return current()->gdim; }
 
 #define __syncthreads() ::hipcpu::wait_barrier()
 #define __threadfence() ((void)0)
+#define __builtin_amdgcn_s_waitcnt(counts) ((void)0)
 namespace hipcpu {
 // wavefront operations: a call site is told apart by the return address into its caller (each
 // inlined copy of a caller has its own); the last argument is unused
