@@ -21,10 +21,10 @@
 //   4. greedy merge: one lane per task replays the reference's merge row by row on the bit masks:
 //      the quads starting in a row are the row's uncovered visible runs split where the face word
 //      changes; each extends downward while every column of it continues (equal and uncovered).
-//   5. block-wide prefix sums give every quad its index in its pass and its position in the
-//      reference's emission order; one atomic per chunk allocates its output range; quads are then
-//      described into an LDS list and written one lane per quad as packed BlockVertex words and u16
-//      indices, with the reference's 65,532-vertex mesh split, per-mesh AABBs and mesh order.
+//   5. ballots over blocks of 64 faces and a scan of the blocks' counts give every quad its index in its
+//      pass; one atomic per chunk and list allocates its output range; one lane per face that starts a quad
+//      writes it as packed BlockVertex words and u16 indices (custom meshes: one lane per vertex), with the
+//      reference's 65,532-vertex mesh split, per-mesh AABBs and mesh order.
 // All arithmetic is integer. References are to client/include/client/BlockMeshAlgo.hpp unless noted.
 #include <hip/hip_runtime.h>
 
@@ -53,8 +53,6 @@ constexpr int kSX = 1, kSZ = kHalo, kSY = kHalo * kHalo;
 __host__ __device__ constexpr int axis_stride(int a) { return a == 0 ? kSX : (a == 1 ? kSY : kSZ); }
 // Mask axes per slice axis (BlockAlgo.hpp:70-81 with the YZX swizzle): x -> (U=y, V=z), y -> (U=z, V=x),
 // z -> (U=y, V=x).
-__host__ __device__ constexpr int u_axis(int a) { return a == 1 ? 2 : 1; }
-__host__ __device__ constexpr int v_axis(int a) { return a == 0 ? 2 : 0; }
 
 // The light4_init cell pattern (kLookup3v, :75-108). Vertex k of face F reads, in the plane of the front
 // cell, a side cell c0 offset along plane axis Q, the corner cell c1 offset along P and Q, and a side cell
@@ -1771,8 +1769,9 @@ template <int NT, bool kRaw> __global__ __launch_bounds__(NT, NT >= 512 ? 2 : 3)
 	}
 	// every claim and allocation of this workgroup precedes its increment of `done`, so the last
 	// workgroup to increment it sees final totals and may clear the counters for the next run. They are
-	// atomics that have returned, and nothing else of this workgroup is read before the launch ends: no fence, which would write back the XCD's L2 once per workgroup (the cave batch 95.0 -> 86.2 us
-	// without, 1,000 random chunks 258 -> 230 us).
+	// atomics that have returned, and nothing else of this workgroup is read before the launch ends: no fence, which
+	// would write back the XCD's L2 once per workgroup (the cave batch 95.0 -> 86.2 us without, 1,000 random chunks
+	// 258 -> 230 us).
 	if (p.self_reset && threadIdx.x == 0) {
 		claims_returned();
 		if (atomicAdd(&p.ctr->done, 1u) == gridDim.x - 1) {

@@ -40,10 +40,11 @@ constexpr int kLightWaves = kLightThreads / 64;
 // row's neighbours along z are the neighbouring lanes', those along y are in the lane's own registers but for
 // the wavefront's first and last layer, which go through LDS. A level step of a layer is 16 VALU instructions
 // and no LDS; eight wavefronts of six layers at 64 registers fill a CU's wavefronts four workgroups deep. The
-// step is bound by VALU issue (88.6 M instructions for 4,096 jobs of the lit cave region, 144 us at full issue,
-// 174 us measured). The earlier kernel kept the whole window in LDS, one row per thread and step, with six LDS
-// reads and a write per row: 223 us. Six wavefronts of eight layers took 207 us, a wavefront skipping steps that
-// can change none of its rows 181 us (the skipped work is less than the bookkeeping).
+// step is bound by VALU issue (91.1 M instructions for 4,096 jobs of the lit cave region, 148 us at full issue,
+// 183 us measured; on another region of the kind, that of the figures below, 88.6 M, 144 and 174). The earlier kernel
+// kept the whole window in LDS, one row per thread and step, with six LDS reads and a write per row: 223 us. Six
+// wavefronts of eight layers took 207 us, a wavefront skipping steps that can change none of its rows 181 us (the
+// skipped work is less than the bookkeeping).
 constexpr int kPlanes = 6;
 static_assert(kLightWaves * kPlanes >= kW && kW <= 64, "the wavefronts' layers cover the window");
 constexpr int kEdgeLanes = 48; // rows of an exchanged layer: 46 and two that are always empty

@@ -7,10 +7,12 @@
 //   copy stream:    first-time chunk loads -> their fresh slots (no running batch reads a fresh slot), by a
 //                   kernel that reads them where the host staged them, in pinned memory;
 //   compute stream: wait for those copies; reloads of resident chunks (in stream order, after every
-//                   earlier batch that may read them); the batch's voxel edits; then up to max_batch stale
-//                   chunks meshed by the persistent kernel into an arena taken from the vertex pool, and
-//                   the per-chunk results written back to pinned memory.
-// Uploads of batch i+1 overlap the meshing of batch i. A batch meshes chunks only when every pending data
+//                   earlier batch that may read them), read from pinned memory too; the batch's voxel edits;
+//                   then up to max_batch stale chunks meshed by the persistent kernel into an arena taken from
+//                   the vertex pool, and the per-chunk results written back to pinned memory.
+// First-time loads of batch i+1 overlap the meshing of batch i; its reloads follow it. (Reloads copied to the
+// device on the copy stream first, and scattered there, were slower: one reload 100 against 68 us, bursts of
+// 64, 256 and 1,728 of them 250, 650 and 3,500 against 210, 560 and 3,270.) A batch meshes chunks only when every pending data
 // change has been flushed into it, so its meshes reflect all requests up to the epoch at its launch; a
 // batch that cannot flush everything (upload or edit limits) carries data only, and its "applied epoch"
 // is the last epoch before the first change it left pending. A request completes when a finished batch
