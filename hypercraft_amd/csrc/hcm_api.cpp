@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <bitset>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
@@ -235,7 +236,8 @@ constexpr size_t kPoutLight = kPoutIdx + kPlainFastQuads * 6 * 2;
 // quads, mesh infos, draws. Its size is what a context may hold of it and touch (touch_output), not where copies
 // become the better way: a download of 43,700 quads takes 108 us through it and 135 by copies, and through 4 MiB one of
 // 77,600 quads 188 against 212, through 8 MiB one of 117,000 283 against 316, past which they are level.
-constexpr size_t kPoutBytes = size_t(2) << 20;
+constexpr size_t kPoutBytes = size_t(2) << 20, kPage = 4096;
+static_assert(kPoutBytes % kPage == 0, "whole pages");
 static_assert(kPoutLight + kLightJobBytes <= kPoutBytes, "a one-chunk call's output fits");
 static_assert(kPoutVerts % 16 == 0 && kPoutIdx % 16 == 0 && kPoutLight % 4 == 0 && HCM_HALO_BLOCKS * 2 % 16 == 0,
               "aligned for the kernels' widest stores and loads");
@@ -283,7 +285,7 @@ struct hcm_ctx {
 	// records, up to kPlainFastQuads quads and the rebuilt light
 	uint8_t *h_halo_in = nullptr;
 	uint8_t *h_pout = nullptr;
-	size_t pout_touched = 0; // its first bytes that the host has written
+	std::bitset<kPoutBytes / kPage> pout_touched; // its pages that the host has written (touch_output)
 	// this device's copy of `scratch` (hcm_mesh_halos_noalloc); host code uses this address, never the
 	// array's name, which on the host is only a stand-in
 	uint8_t *d_scratch = nullptr;
@@ -396,18 +398,30 @@ template <typename T> static hipError_t pinned(T **p, size_t bytes) {
 	return hipHostMalloc(reinterpret_cast<void **>(p), bytes);
 }
 
-// Writes the first `bytes` of the context's pinned output once (context lock held: no kernel is writing there). The
-// host's first touch of each of its pages faults, 0.4 ms per MiB: that is paid by what may use it, 64 KB with the
-// context and 6 KB (128 quads and their records) for each job of a batch when it is made. With none of it touched
-// before, the first download of 333 chunks' meshes took 770 us instead of 150; with all of it touched in every context
-// a context took 1.8 ms to make beside others, 0.9 so.
-constexpr size_t kTouchContext = 64 << 10, kTouchJob = 6 << 10;
-static void touch_output(hcm_ctx *c, size_t bytes) {
-	bytes = std::min(bytes, kPoutBytes);
-	if (bytes > c->pout_touched) {
-		std::memset(c->h_pout + c->pout_touched, 0, bytes - c->pout_touched);
-		c->pout_touched = bytes;
-	}
+// The host's first touch of a page of pinned memory faults, 0.4 ms per MiB. It is paid by what may use the page before
+// it does so: a context when it is made touches what one-chunk calls read and what a chunk of some 500 quads returns,
+// a batch what its download of 128 quads a job returns. With none touched before, the first download of 333
+// chunks' meshes took 770 us instead of 150 and a first hcm_mesh_chunk_relight 200 instead of 95; with all of it touched in
+// every context a context took 1.8 ms to make beside others, now 0.95.
+constexpr uint32_t kTouchChunkQuads = 1024, kTouchJobQuads = 128;
+static void touch_pages(uint8_t *at, size_t bytes) {
+	for (size_t k = 0; k < bytes; k += kPage)
+		*const_cast<volatile uint8_t *>(at + k) = 0;
+}
+// The pages of the context's pinned output from `at` on (context lock held: no kernel is writing there).
+static void touch_output(hcm_ctx *c, size_t at, size_t bytes) {
+	const size_t end = std::min(at + bytes, kPoutBytes);
+	for (size_t k = at / kPage; k * kPage < end; ++k)
+		if (!c->pout_touched[k]) {
+			touch_pages(c->h_pout + k * kPage, 1);
+			c->pout_touched[k] = true;
+		}
+}
+
+// Where a run's quads go in the pinned output behind `at` bytes of results and records: as many as fit and as the pool
+// holds, first their vertices, then their indices.
+static uint32_t export_quads(const hcm_ctx *c, size_t at) {
+	return at + 32 < kPoutBytes ? (uint32_t)std::min<uint64_t>((kPoutBytes - at - 32) / 44, c->pool_quads) : 0u;
 }
 
 static int create_impl(hcm_ctx *c, const hcm_registry *registry, uint64_t pool_quads) {
@@ -462,8 +476,11 @@ static int create_impl(hcm_ctx *c, const hcm_registry *registry, uint64_t pool_q
 	HCM_HIP(pinned(&c->h_pblocks, 27 * HCM_CHUNK_VOXELS * 2));
 	HCM_HIP(pinned(&c->h_halo_in, kHaloBytes));
 	HCM_HIP(pinned(&c->h_pout, kPoutBytes));
-	std::memset(c->h_halo_in, 0, kHaloBytes);
-	touch_output(c, kTouchContext);
+	touch_pages(reinterpret_cast<uint8_t *>(c->h_pblocks), 27 * HCM_CHUNK_VOXELS * 2);
+	touch_pages(c->h_halo_in, kHaloBytes);
+	touch_output(c, 0, kPoutVerts + kTouchChunkQuads * 32);
+	touch_output(c, kPoutIdx, kTouchChunkQuads * 12);
+	touch_output(c, kPoutLight, kLightJobBytes);
 	HCM_HIP(pinned(&c->h_pheights, 27 * 256));
 	HCM_HIP(dmalloc(&c->d_ppacked, 27 * kLightSlotBytes / 2));
 	HCM_HIP(dmalloc(&c->d_plevels, 27));
@@ -921,7 +938,10 @@ extern "C" int hcm_batch_create(hcm_ctx *ctx, hcm_store *store, const uint32_t *
 		std::lock_guard<std::mutex> lk(ctx->mu);
 		ctx->kept_refused = SIZE_MAX;
 		want_kept(ctx, batch_grid(ctx, n_jobs));
-		touch_output(ctx, kTouchContext + (size_t)n_jobs * kTouchJob);
+		const size_t at = 64 + (size_t)n_jobs * sizeof(hcm_job_result) + (size_t)b->rec_cap * sizeof(hcm_mesh_rec);
+		const size_t room = export_quads(ctx, at), quads = std::min<size_t>((size_t)n_jobs * kTouchJobQuads, room);
+		touch_output(ctx, 0, at + quads * 32);
+		touch_output(ctx, at + room * 32, quads * 12);
 	}
 	*out = b;
 	return HCM_OK;
@@ -1124,9 +1144,9 @@ static int export_run(hcm_batch *b, bool results, bool recs, bool quads, Exporte
 	p.rec_cap = b->rec_cap;
 	if (recs && (p.out_recs = reinterpret_cast<hcm_mesh_rec *>(place((size_t)b->rec_cap * sizeof(hcm_mesh_rec)))))
 		p.recs = b->d_recs;
-	if (quads && at + 32 < kPoutBytes) {
+	if (quads && export_quads(c, at)) {
 		// (the run's total counts allocations that did not fit the pool: no more than the pool holds may be copied)
-		p.quad_cap = (uint32_t)std::min<uint64_t>((kPoutBytes - at - 32) / 44, c->pool_quads);
+		p.quad_cap = export_quads(c, at);
 		p.out_verts = reinterpret_cast<uint2 *>(place((size_t)p.quad_cap * 4 * sizeof(uint2)));
 		p.out_idx = reinterpret_cast<uint16_t *>(place((size_t)p.quad_cap * 12));
 		if (p.out_verts && p.out_idx)

@@ -93,19 +93,22 @@ def check_dense_memory_grows():
 
 
 def check_pinned_memory_touched():
-    """A context touches little of its pinned memory before it has batches, and then as much as they are large."""
+    """A context touches its pinned input and little of its 2 MiB of pinned output before it has batches, and then as much
+    as they are large."""
     from hypercraft_amd import hcm
 
-    ctx = hcm.Context(pool_quads=1 << 14)
+    ctx = hcm.Context(pool_quads=1 << 16)
     touched = [count(hcm, "pinned_touched")]
     for n in (1, 37, 400, 37, 1000):
         batch_of(hcm, ctx, n)
         touched.append(count(hcm, "pinned_touched"))
     made, one, few, many, after, most = touched
-    assert made <= 128 << 10
-    assert made <= one <= made + (16 << 10)
-    assert 37 * 5000 < few - made < 37 * 10000
-    assert 2 << 20 <= many <= (2 << 20) + (128 << 10) and many == after == most
+    inputs = 27 * 4096 * 2 + 14400 + 5832
+    assert inputs <= made <= inputs + (96 << 10)
+    assert made <= one <= made + (96 << 10)  # (room for 1,027 records)
+    assert 37 * 128 * 44 < few - made < 37 * 128 * 44 + (112 << 10)
+    assert inputs + (2 << 20) - (64 << 10) <= many <= inputs + (2 << 20) + (64 << 10)
+    assert many <= after <= most <= inputs + (2 << 20) + (64 << 10)
 
 
 def check_tuning_round_trip():
